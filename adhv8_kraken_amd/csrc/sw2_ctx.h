@@ -186,7 +186,8 @@ struct Ctx {
     std::vector<int> tb_h_nt, tb_h_inst;   // host copies: each band's panels and model
     size_t tb_size;
     TBand *tb_bands;
-    double *tb_AB, *tb_LI, *tb_UI, *tb_xb, *tb_yb, *tb_panel;
+    double *tb_AB, *tb_LI, *tb_UI, *tb_xb, *tb_yb, *tb_zb;
+    int *tb_int, *tb_guard;   // sweep tickets [2 bands], then a guard flag per tile (tb_guard)
     // block ILU(0) in multicolour order (preconditioner 3), built on demand
     int ilu_ready, ilu_ncolor, ilu_Rp, ilu_f32;
     size_t ilu_nl, ilu_nu;                 // lower / upper slots (64 per slice slot)

@@ -19,25 +19,31 @@
 // dimension 2 wp the band is a column-major dense matrix, so tiles are
 // strided blocks.
 //
-// Factorisation, per panel of TB columns (two launches over all bands at once:
-// a model's node blocks, or every block of every model of an ensemble):
-//   k_tb_trsm  a workgroup per 64-row tile of L (rows below the panel:
-//              L = A U~^-1 by substitution, U~ = U with the guarded pivots)
-//              and per 64-column tile of U (right of the panel: U = L^-1 A);
-//   k_tb_gemm  the trailing w x w window -= L U, 64 x 64 tiles, 2 x 4
-//              register blocks per thread from LDS; the workgroup of the
-//              first tile, the next panel's diagonal block, then factors it
-//              (eight waves, row t in lane t, 8 columns per wave, blocked by
-//              waves) while the other tiles are updated.
-// k_tb_diag factors panel 0's diagonal block the same way.
-// Then k_tb_inv forms the inverses of every diagonal block's unit-lower and
-// upper factors (all blocks in parallel) and k_tb_scale multiplies every
-// off-diagonal tile by its column's inverse, so that each step of the
-// substitutions is independent matrix-vector work: the forward sweep is one
-// launch per tile (block 0 y_k = L_kk^-1 x_k, the blocks below
-// x_i -= (L_ik L_kk^-1) x_k), the backward sweep likewise upwards.
+// Factorisation, one launch per panel of TB columns over all bands at once (a
+// model's node blocks, or every block of every model of an ensemble):
+//   k_tb_step  a workgroup per 64 x 64 tile of the trailing w x w window, which
+//              takes (A U~^-1) (L^-1 A) of its row and column of the panel (U~: U
+//              with the guarded pivots) on the matrix cores; the workgroup of the
+//              first tile, the next panel's diagonal block, goes on to factor
+//              it and to invert both factors (lu64).
+// k_tb_diag factors panel 0's diagonal block.  Then k_tb_inv forms G_k = U~^-1
+// L^-1 of every diagonal block and k_tb_scale multiplies every off-diagonal tile
+// by its column's, so that the substitutions are matrix-vector work in which
+// only a tile's input is serial: k_tb_sweep runs both as one dataflow kernel
+// (y_i = x_i - sum (A_ik G_k) y_k, then upwards), k_tb_apply the diagonal inverses.
+//
+// A chain of m / 64 dependent panels bounds both.  200 x 100 cells (m 60,903,
+// w 308, 952 panels): a panel 22.2 us, of which the diagonal block's LU 11.7
+// (189 cycles per pivot in the panel wave, which issues on 150 of them),
+// the tile's three products 3.8 at the matrix cores' FP64 rate, the rest load
+// latency and the launch (substitution and update in two launches, vector FMAs,
+// LU by readlane broadcasts: 9.6 + 21.7 us); a sweep step 1.9 us (a launch
+// per tile: 3.5).
+#include <limits.h>
+
 #include <algorithm>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "sw2_ctx.h"
@@ -45,9 +51,9 @@
 namespace sw2 {
 
 constexpr int TB = 64;          // tile and panel width (DOFs)
-constexpr int LW = 8;           // columns (rows) per wave in the blocked factor and solves
-constexpr int NWV = TB / LW;    // waves per workgroup of those kernels
-constexpr int NT = 64 * NWV;    // their threads
+constexpr int NT = 512;         // threads of the factorisation and sweep workgroups (eight waves)
+
+using d4 = double __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ size_t tb_idx(const TBand &B, int i, int j) {
     return B.off + (size_t)(B.wp + i - j) + (size_t)j * (2 * B.wp + 1);
@@ -60,6 +66,12 @@ __device__ __forceinline__ double lane_bcast(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
     const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
     return __hiloint2double(hi, lo);
+}
+
+// D (16 x 16) += X (16 x 4) Y (4 x 16) on the matrix cores: lane l holds
+// X[l % 16][l / 16], Y[l / 16][l % 16] and D[l / 16 + 4 r][l % 16], r = 0..3
+__device__ __forceinline__ d4 mfma4(double x, double y, d4 d) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, d, 0, 0, 0);
 }
 
 // Band record b in SGPRs at once: the empty asm statement uses every field, so
@@ -103,369 +115,475 @@ __global__ void k_tb_load(int N, const int *node_blk, const TBand *bands, double
     }
 }
 
-// LU of a 64 x 64 diagonal block, blocked by LW = 8 columns: lane t of each of
-// the eight waves holds row t (r[LW]), wave w columns 8 w .. 8 w + 7.  Wave
-// P factors its 8 columns (right-looking: the pivot read from lane p with
-// readlane, the multipliers as entry times the reciprocal guarded pivot),
-// publishes them in LDS, and after one barrier the waves to its right update
-// their columns with them (the same right-looking steps, multipliers read
-// from LDS); then wave P + 1 factors its (updated) columns.  Eight barriers
-// per block instead of one per pivot; the serial part of each phase, one
-// wave's pivots and the next wave's update, is half what 16-column groups
-// give, and every entry takes the same updates in the same order as with any
-// grouping.  Then the factors go back into the band and
-// [strict U by rows | strict L by columns | 1 / guarded pivots] into the
-// band's panel copy P for k_tb_trsm (zeros on and across the diagonal let it
-// update every column at every step).  pan: [2][TB][LW + 1] and rd: [TB] in LDS.
-constexpr int TB_PANEL = 2 * TB * TB + TB;   // doubles of one band's panel copy
-__device__ __forceinline__ void diag_lu_store(double (&r)[LW], double (*pan)[TB][LW + 1], double *rd, double *AB,
-                                              const TBand &B, double *P, int c0, int kb, int lane, int wv) {
+// ---- LU of a 64 x 64 diagonal block with the inverses of its factors ---------
+// 16-column panels on single waves, 16 x 16 block products on the matrix cores.
+//
+// A panel wave's lane holds a row; the wave's four 16-lane rows are the four
+// block rows.  The pivot row's broadcast is the DPP operand of the multiply-add
+// itself (row_newbcast), so every 16-lane row carries its own copy of the
+// panel's diagonal block.  A step's order is fixed by scheduling barriers: the
+// next pivot's column first, then its reciprocal's chain in the shadow of the
+// other columns, each source of a DPP read at least two instructions old (the
+// compiler does not look into the asm; only the first after them needs a s_nop).
+#define SW2_FM(D, S) "v_fmac_f64_dpp %" #D ", %" #S ", %[f] row_newbcast:%[p] row_mask:0xf bank_mask:0xf\n\t"
+// d[J .. J + NJ) += f * (row P's s[J .. J + NJ)), s another array than d
+template <int P, int J, int NJ>
+__device__ __forceinline__ void rank1(double *d, const double *s, double f) {
+    if constexpr (NJ >= 3) {
+        asm(SW2_FM(0, 3) SW2_FM(1, 4) SW2_FM(2, 5)
+            : "+v"(d[J]), "+v"(d[J + 1]), "+v"(d[J + 2])
+            : "v"(s[J]), "v"(s[J + 1]), "v"(s[J + 2]), [f] "v"(f), [p] "n"(P));
+        rank1<P, J + 3, NJ - 3>(d, s, f);
+    } else if constexpr (NJ >= 1) {
+        asm(SW2_FM(0, 1) : "+v"(d[J]) : "v"(s[J]), [f] "v"(f), [p] "n"(P));
+        rank1<P, J + 1, NJ - 1>(d, s, f);
+    }
+}
+// the same within one array: d[j] += f * (row P's d[j])
+template <int P, int J, int NJ>
+__device__ __forceinline__ void rank1(double *d, double f) {
+    if constexpr (NJ >= 3) {
+        asm(SW2_FM(0, 0) SW2_FM(1, 1) SW2_FM(2, 2)
+            : "+v"(d[J]), "+v"(d[J + 1]), "+v"(d[J + 2]) : [f] "v"(f), [p] "n"(P));
+        rank1<P, J + 3, NJ - 3>(d, f);
+    } else if constexpr (NJ >= 1) {
+        asm(SW2_FM(0, 0) : "+v"(d[J]) : [f] "v"(f), [p] "n"(P));
+        rank1<P, J + 1, NJ - 1>(d, f);
+    }
+}
+#undef SW2_FM
+#define SW2_ORDER() __builtin_amdgcn_sched_barrier(0)
+// row P's d[P] in every lane
+template <int P>
+__device__ __forceinline__ double pivot_of(const double *d) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(d[P]), 0x150 + P, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(d[P]), 0x150 + P, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// its reciprocal from the hardware's estimate r (e = 1 - piv r about 2^-23) by
+// one cubic step r (1 + e + e^2), guarded (solv_blk_profile.c:66-71)
+__device__ __forceinline__ double pivot_end(double piv, double r, double e2, bool &small) {
+    small = !(fabs(piv) > SMALL);
+    r = fma(r, e2, r);
+    return small ? 1.0 / SMALL : r;
+}
+__device__ __forceinline__ double pivot_whole(double piv, bool &small) {
+    const double r = __builtin_amdgcn_rcp(piv), e = fma(-piv, r, 1.0);
+    return pivot_end(piv, r, fma(e, e, e), small);
+}
+// a <- a U^-1 for the lane's row a (forward substitution with the reciprocal
+// guarded pivots), U from the LU of the block whose row the lane holds in d; r:
+// pivot P's reciprocal.  Rows of d above the pivot are finished and not read
+// again, so no lane is masked.  A finished column of a goes to C.
+template <int P>
+__device__ __forceinline__ void panel_rows(double (&d)[16], double (&a)[16], double *C, double r, bool &hit) {
+    const double nl = -a[P] * r, f = -d[P] * r;
+    C[P] = -nl;
+    if constexpr (P < 15) {
+        constexpr int M = 14 - P;   // columns after the next pivot's
+        SW2_ORDER();
+        asm volatile("s_nop 1");
+        rank1<P, P + 1, 1>(a, d, nl);
+        rank1<P, P + 1, 1>(d, f);
+        SW2_ORDER();
+        const double piv = pivot_of<P + 1>(d);
+        const double r0 = __builtin_amdgcn_rcp(piv);
+        SW2_ORDER();
+        rank1<P, P + 2, M>(a, d, nl);
+        SW2_ORDER();
+        const double e = fma(-piv, r0, 1.0);
+        SW2_ORDER();
+        rank1<P, P + 2, M / 2>(d, f);
+        SW2_ORDER();
+        const double e2 = fma(e, e, e);
+        SW2_ORDER();
+        rank1<P, P + 2 + M / 2, M - M / 2>(d, f);
+        SW2_ORDER();
+        bool small;
+        const double rn = pivot_end(piv, r0, e2, small);
+        hit = hit || small;
+        panel_rows<P + 1>(d, a, C, rn, hit);
+    }
+}
+// the LU of the block whose row the lane holds, in place, with the inverse of
+// the unit lower factor below the diagonal in the multipliers' place
+template <int P>
+__device__ __forceinline__ void lower_inverse(double (&d)[16], double r, int row) {
+    const double f = row > P ? -d[P] * r : 0.0;
+    if (row > P) d[P] = f;
+    if constexpr (P < 15) {
+        constexpr int M = 14 - P;
+        SW2_ORDER();
+        asm volatile("s_nop 1");
+        rank1<P, P + 1, 1>(d, f);
+        SW2_ORDER();
+        const double piv = pivot_of<P + 1>(d);
+        const double r0 = __builtin_amdgcn_rcp(piv);
+        SW2_ORDER();
+        rank1<P, 0, P>(d, f);
+        rank1<P, P + 2, M / 3>(d, f);
+        SW2_ORDER();
+        const double e = fma(-piv, r0, 1.0);
+        SW2_ORDER();
+        rank1<P, P + 2 + M / 3, M / 3>(d, f);
+        SW2_ORDER();
+        const double e2 = fma(e, e, e);
+        SW2_ORDER();
+        rank1<P, P + 2 + 2 * (M / 3), M - 2 * (M / 3)>(d, f);
+        SW2_ORDER();
+        bool small;
+        lower_inverse<P + 1>(d, pivot_end(piv, r0, e2, small), row);
+    }
+}
+
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// 16 x 16 blocks in LDS, rows of 18: whole rows (16 bytes a lane) and both operand
+// layouts of the matrix cores read distinct banks
+constexpr int BLD = 18, BS = 16 * BLD;
+struct Lu64 {
+    double col[2][4][BS];   // block column s, by step parity: its blocks, then those times U_ss^-1
+    double row[2][4][BS];   // block row s: its blocks, then L_ss^-1 times those
+    double li[BS], ui[BS];  // L_ss^-1, U_ss^-1
+    double one[BS];         // the identity
+    int hit;
+};
+__device__ __forceinline__ void blk_put(double *dst, const d4 &v, int lo, int hi) {
 #pragma unroll
-    for (int Q = 0; Q < NWV; Q++) {
-        if (wv == Q) {
+    for (int r = 0; r < 4; r++) dst[BLD * lo + hi + 4 * r] = v[r];
+}
+__device__ __forceinline__ d4 blk_get(const double *src, int lo, int hi) {
+    d4 v;
 #pragma unroll
-            for (int pj = 0; pj < LW; pj++) {
-                const int p = LW * Q + pj;
-                const double rden = 1.0 / guarded(lane_bcast(r[pj], p));
-                if (lane == p) rd[p] = rden;
-                const double l = lane > p ? r[pj] * rden : 0.0;
-                if (lane > p) r[pj] = l;
+    for (int r = 0; r < 4; r++) v[r] = src[BLD * lo + hi + 4 * r];
+    return v;
+}
+// Eight waves: wave (wi, wj) holds blocks (wi, 2 wj) and (wi, 2 wj + 1) in
+// registers, element (row, col) of a block in lane row + 16 (col % 4), register
+// col / 4 -- the matrix cores' operand and result layout of the transposed
+// product.  Step s, in place:
+//   wave 0   C_i = D_is U_ss^-1 for the four block rows (block row s: U_ss^-1
+//            itself, from rows of the identity); beside it wave 1 L_ss^-1
+//   then     R_j = L_ss^-1 D_sj, a wave each
+//   then     D_ij -= C_i R_j, D_is <- -C_i L_ss^-1 (i > s), D_sj <- -U_ss^-1 R_j (j > s)
+// after which the blocks below the diagonal are L^-1's and those above U^-1's
+// (with the guarded pivots).  LI: L^-1 column-major, UI: U^-1 row-major, 64 x 64
+// each, the blocks on the other side of the diagonal not written.  *guard: a
+// pivot took the guard.
+__device__ __forceinline__ void lu64(d4 (&D)[2], Lu64 &S, double *LI, double *UI, int *guard, int lane, int wi, int wj) {
+    const int lo = lane & 15, hi = lane >> 4;
+    if (threadIdx.x == 0) S.hit = 0;
+    if (threadIdx.x < 256) S.one[BLD * (threadIdx.x >> 4) + (threadIdx.x & 15)] = threadIdx.x % 17 == 0 ? 1.0 : 0.0;
+    // not unrolled: a workgroup runs this once, so its instructions come from
+    // beyond the instruction cache, and four copies cost more to fetch than to run
+#pragma unroll 1
+    for (int s = 0; s < 4; s++) {
+        double (*col)[BS] = S.col[s & 1], (*row)[BS] = S.row[s & 1];
+        // block row and column s into LDS (the diagonal block with the column)
 #pragma unroll
-                for (int qj = pj + 1; qj < LW; qj++) r[qj] = fma(-l, lane_bcast(r[qj], p), r[qj]);
-            }
-#pragma unroll
-            for (int j = 0; j < LW; j++) pan[Q & 1][lane][j] = r[j];
+        for (int t = 0; t < 2; t++) {
+            const int bj = 2 * wj + t;
+            if (bj == s) blk_put(col[wi], D[t], lo, hi);
+            else if (wi == s) blk_put(row[bj], D[t], lo, hi);
         }
         __syncthreads();
-        if (wv > Q) {
+        if (wj == 0 && wi < 2) {
+            double d[16];
 #pragma unroll
-            for (int sj = 0; sj < LW; sj++) {
-                const int sp = LW * Q + sj;
-                const double l = lane > sp ? pan[Q & 1][lane][sj] : 0.0;
+            for (int j = 0; j < 16; j++) d[j] = col[s][BLD * lo + j];
+            if (wi == 0) {
+                double a[16];
+                const double *A = hi == s ? S.one : col[hi];
 #pragma unroll
-                for (int j = 0; j < LW; j++) r[j] = fma(-l, lane_bcast(r[j], sp), r[j]);
+                for (int j = 0; j < 16; j++) a[j] = A[BLD * lo + j];
+                bool hit = false;
+                const double r = pivot_whole(pivot_of<0>(d), hit);
+                panel_rows<0>(d, a, (hi == s ? S.ui : col[hi]) + BLD * lo, r, hit);
+                if (hit) S.hit = 1;
+            } else {
+                bool small;
+                lower_inverse<0>(d, pivot_whole(pivot_of<0>(d), small), lo);
+                if (hi == 0) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) S.li[BLD * lo + j] = j < lo ? d[j] : (j == lo ? 1.0 : 0.0);
+                }
             }
         }
-    }
-    __syncthreads();
+        __syncthreads();
+        const d4 zero = {0.0, 0.0, 0.0, 0.0};
+        const int wv = threadIdx.x >> 6;
+        if (wv < 4 && wv != s) {   // a wave on each SIMD
+            double *R = row[wv];
+            double x[4], y[4];
+            d4 acc = zero;
 #pragma unroll
-    for (int j = 0; j < LW; j++) {
-        const int col = LW * wv + j;
-        if (lane < kb && col < kb) tb_at(AB, B, c0 + lane, c0 + col) = r[j];
-        P[TB * lane + col] = col > lane ? r[j] : 0.0;              // U strictly above the diagonal, row `lane`
-        P[TB * TB + TB * col + lane] = col < lane ? r[j] : 0.0;    // L, column `col` (unit diagonal not stored)
+            for (int q = 0; q < 4; q++) { x[q] = R[BLD * (hi + 4 * q) + lo]; y[q] = S.li[BLD * lo + hi + 4 * q]; }
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc = mfma4(x[q], y[q], acc);
+            wave_sync();
+            blk_put(R, acc, lo, hi);
+        } else if (wv == s + 4) {   // the diagonal block's own factors are final
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                LI[64 * (16 * s + hi + 4 * r) + 16 * s + lo] = S.li[BLD * lo + hi + 4 * r];
+                UI[64 * (16 * s + hi + 4 * r) + 16 * s + lo] = S.ui[BLD * (hi + 4 * r) + lo];
+            }
+        }
+        __syncthreads();
+        // every unfinished block as base - left right
+        d4 acc[2];
+        if (wi > s || 2 * wj + 1 > s) {
+            const double *left = wi == s ? S.ui : col[wi];
+            double x[2][4], y[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) y[q] = -left[BLD * lo + hi + 4 * q];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int bj = 2 * wj + t;
+                const double *right = bj == s ? S.li : row[bj];
+#pragma unroll
+                for (int q = 0; q < 4; q++) x[t][q] = right[BLD * (hi + 4 * q) + lo];
+                acc[t] = (wi == s || bj == s) ? zero : D[t];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) acc[t] = mfma4(x[t][q], y[q], acc[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int bj = 2 * wj + t;
+            if (wi > s || bj > s) D[t] = acc[t];
+            else if (wi == s && bj < s) D[t] = blk_get(row[bj], lo, hi);
+            else if (bj == s && wi < s) D[t] = blk_get(col[wi], lo, hi);
+        }
     }
-    if (wv == 0) P[2 * TB * TB + lane] = lane < kb ? rd[lane] : 0.0;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int bj = 2 * wj + t;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int i = 16 * wi + lo, j = 16 * bj + hi + 4 * r;
+            if (wi > bj) LI[64 * j + i] = D[t][r];
+            else if (wi < bj) UI[64 * i + j] = D[t][r];
+        }
+    }
+    if (threadIdx.x == 0) *guard = S.hit;   // every pivot was before the last barriers
 }
 
 // Panel 0's diagonal block, one workgroup per band (every later panel's is
-// factored by k_tb_gemm of the panel before, which updates it last).
-__global__ void __launch_bounds__(NT) k_tb_diag(const TBand *bands, double *AB, double *panel, int k,
-                                                const int *mask) {
-    __shared__ double pan[2][TB][LW + 1];   // a factored column group (double-buffered by group parity)
-    __shared__ double rd[TB];           // 1 / guarded pivots
+// factored by k_tb_step of the panel before, which updates it last).
+__global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const double *AB, double *LI, double *UI,
+                                                   int *guard, const int *mask) {
+    __shared__ Lu64 S;
     const TBand B = band_rec(bands, blockIdx.x);
-    if (k >= B.nt || (mask && !mask[B.inst])) return;
-    const int c0 = k * TB, kb = min(TB, B.m - c0);
+    if (mask && !mask[B.inst]) return;
+    const int kb = min(TB, B.m);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tc = min(lane, kb - 1);
-    double r[LW];
-    // loads at clamped (in-band) positions, then zeroed outside the block: the
-    // rows and columns past a short last block are zero, their pivots guarded
-    // and their multipliers zero
+    const int wi = wv & 3, wj = wv >> 2, lo = lane & 15, hi = lane >> 4;
+    d4 D[2];
+    const int i = 16 * wi + lo;
 #pragma unroll
-    for (int j = 0; j < LW; j++) {
-        const int col = LW * wv + j;
-        const double v = tb_get(AB, B, c0 + tc, c0 + min(col, kb - 1));
-        r[j] = (lane < kb && col < kb) ? v : 0.0;
-    }
-    diag_lu_store(r, pan, rd, AB, B, panel + (size_t)TB_PANEL * blockIdx.x, c0, kb, lane, wv);
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {   // past a short block: the identity
+            const int j = 32 * wj + 16 * t + hi + 4 * r;
+            const double v = tb_get(AB, B, min(i, kb - 1), min(j, kb - 1));
+            D[t][r] = (i < kb && j < kb) ? v : (i == j ? 1.0 : 0.0);
+        }
+    lu64(D, S, LI + 4096 * B.toff, UI + 4096 * B.toff, guard + B.toff, lane, wi, wj);
 }
 
-// Panel k's L tiles (blockIdx.x < gl: 64 rows each below the panel) and U
-// tiles (blockIdx.x >= gl: 64 columns each right of it), one workgroup of
-// eight waves per tile, blocked by 8 as k_tb_diag.  L side: lane t holds row
-// t of the tile, wave w its columns 8 w .. 8 w + 7; wave P forms the
-// multipliers of its 8 columns, publishes them in LDS, and after one barrier
-// the waves to its right take the rank-8 update.  U side: lane t holds
-// column t, wave w its rows 8 w .. 8 w + 7; wave P finishes its rows and
-// the waves below take their update.  The diagonal block's entries come from
-// an LDS copy of the half of the panel block the side uses (broadcast reads;
-// strict triangles, so every update runs over whole column groups): the
-// L side the strict U rows and the reciprocal guarded pivots, the U side the
-// strict L columns.  LDS: that copy, and one region that is the U side's
-// transpose buffer before and after the blocked steps and the published
-// column (row) groups during them -- 66.5 KB, two workgroups per CU.
-__global__ void __launch_bounds__(NT) k_tb_trsm(const TBand *bands, double *AB, const double *panel, int k,
-                                                int gl, const int *mask) {
-    __shared__ double sm[2 * TB * (TB + 1)];
-    double (*T)[TB + 1] = reinterpret_cast<double (*)[TB + 1]>(sm);          // U side: the tile, transposed
-    double (*pan)[TB][LW + 1] = reinterpret_cast<double (*)[TB][LW + 1]>(sm);   // a finished group, by parity
-    double *Pl = sm + TB * (TB + 1);                                         // the panel half
+// Panel k: the trailing window A[r0:r1, r0:r1] -= (A[r0:r1, panel] U_k^-1) (L_k^-1 A[panel, r0:r1])
+// with L_k, U_k the factors of the panel's (updated) diagonal block, one 64 x 64
+// tile per workgroup of eight waves, on the matrix cores: first the tile's L and
+// U panels (triangular inverses: 10 of 16 block products each, two block columns
+// per wave that make up five), then their product.  Block columns and rows of
+// a panel are left in the band as they stand at its elimination, which is what
+// the sweeps read (scaled, k_tb_scale).  Every tile forms its own L and U panel:
+// 2.25 times the flops of separate launches, but one dependent launch per panel,
+// and at the usual band widths (a few tiles) the launch and the next diagonal
+// block, not the matrix cores, are what a panel waits for.  The workgroup of the
+// window's first tile, the next panel's diagonal block, goes on to factor it.
+__global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, double *AB, double *LI, double *UI, int *guard,
+                                                int k, int gt, const int *mask) {
+    constexpr int LD = TB + 2;   // operand reads of 16 rows x 2 columns hit distinct banks
+    __shared__ union {
+        struct { double Xs[TB * LD], Us[TB * LD], Ls[4][16][64]; } p;
+        Lu64 S;
+    } sm;
     const TBand B = band_rec(bands, blockIdx.y);
-    if (k >= B.nt || (mask && !mask[B.inst])) return;
-    const int c0 = k * TB, kb = min(TB, B.m - c0);
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = c0 + kb, r1 = min(B.m, r0 + B.w);
-    const bool lside = (int)blockIdx.x < gl;
-    const int g = lside ? blockIdx.x : blockIdx.x - gl;
-    const int base = r0 + TB * g;
-    if (base >= r1) return;
-    // the panel half: [strict U rows | 1 / guarded pivots] (L side) or strict
-    // L columns (U side); a thread's loads all issued before its LDS stores
-    const double *Pg = panel + (size_t)TB_PANEL * blockIdx.y + (lside ? 0 : TB * TB);
-    {
-        constexpr int NP = TB * TB / NT;
-        double v[NP];
-#pragma unroll
-        for (int u = 0; u < NP; u++) v[u] = Pg[threadIdx.x + NT * u];
-        const double rv = lside && threadIdx.x < TB ? Pg[2 * TB * TB + threadIdx.x] : 0.0;
-#pragma unroll
-        for (int u = 0; u < NP; u++) Pl[threadIdx.x + NT * u] = v[u];
-        if (lside && threadIdx.x < TB) Pl[TB * TB + threadIdx.x] = rv;
-    }
-    double r[LW];
-    if (lside) {
-        const double *U = Pl, *R = Pl + TB * TB;
-        const int i = base + lane;
-        const bool act = i < r1;
-        const int ic = min(i, r1 - 1);
-#pragma unroll
-        for (int j = 0; j < LW; j++) {
-            const int col = LW * wv + j;
-            const double v = tb_get(AB, B, ic, c0 + min(col, kb - 1));   // clamped: in flight together
-            r[j] = (act && col < kb) ? v : 0.0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int P = 0; P < NWV; P++) {
-            if (wv == P) {
-#pragma unroll
-                for (int pj = 0; pj < LW; pj++) {
-                    const int p = LW * P + pj;
-                    const double l = r[pj] * R[p];
-                    r[pj] = l;
-#pragma unroll
-                    for (int qj = pj + 1; qj < LW; qj++) r[qj] = fma(-l, U[TB * p + LW * P + qj], r[qj]);
-                }
-#pragma unroll
-                for (int j = 0; j < LW; j++) pan[P & 1][lane][j] = r[j];
-            }
-            __syncthreads();
-            if (wv > P) {
-#pragma unroll
-                for (int sj = 0; sj < LW; sj++) {
-                    const double l = pan[P & 1][lane][sj];
-#pragma unroll
-                    for (int j = 0; j < LW; j++) r[j] = fma(-l, U[TB * (LW * P + sj) + LW * wv + j], r[j]);
-                }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < LW; j++) {
-            const int col = LW * wv + j;
-            if (act && col < kb) tb_at(AB, B, i, c0 + col) = r[j];
-        }
-    } else {
-        const double *L = Pl;
-        const int ncol = min(TB, r1 - base);
-        constexpr int NU = TB * TB / NT;
-        double tv[NU];
-#pragma unroll
-        for (int u = 0; u < NU; u++) {
-            const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;   // down a column
-            tv[u] = tb_get(AB, B, c0 + min(row, kb - 1), base + min(col, ncol - 1));
-        }
-#pragma unroll
-        for (int u = 0; u < NU; u++) {
-            const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
-            T[row][col] = (row < kb && col < ncol) ? tv[u] : 0.0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < LW; j++) r[j] = T[LW * wv + j][lane];
-        __syncthreads();   // the groups below overwrite the transpose buffer
-#pragma unroll
-        for (int P = 0; P < NWV; P++) {
-            if (wv == P) {
-#pragma unroll
-                for (int pj = 0; pj < LW; pj++) {
-                    const int p = LW * P + pj;
-#pragma unroll
-                    for (int qj = pj + 1; qj < LW; qj++) r[qj] = fma(-L[TB * p + LW * P + qj], r[pj], r[qj]);
-                }
-#pragma unroll
-                for (int j = 0; j < LW; j++) pan[P & 1][lane][j] = r[j];
-            }
-            __syncthreads();
-            if (wv > P) {
-#pragma unroll
-                for (int sj = 0; sj < LW; sj++) {
-                    const double u = pan[P & 1][lane][sj];
-#pragma unroll
-                    for (int j = 0; j < LW; j++) r[j] = fma(-L[TB * (LW * P + sj) + LW * wv + j], u, r[j]);
-                }
-            }
-        }
-        // the last group reads ended before the last barrier above
-#pragma unroll
-        for (int j = 0; j < LW; j++) T[LW * wv + j][lane] = r[j];
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NU; u++) {
-            const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
-            if (row < kb && col < ncol) tb_at(AB, B, c0 + row, base + col) = T[row][col];
-        }
-    }
-}
-
-// Trailing window of panel k: A[r0:r1, r0:r1] -= L[r0:r1, panel] U[panel, r0:r1],
-// one 64 x 64 tile per workgroup (512 threads, a 2 x 4 block each).  The
-// workgroup of the window's first tile -- panel k + 1's diagonal block, which
-// no later update of panel k touches -- goes on to factor that block
-// (diag_lu_store), while the other tiles are updated: panel k + 1's diagonal
-// LU leaves the critical path of the rank-64 update.
-__global__ void __launch_bounds__(NT) k_tb_gemm(const TBand *bands, double *AB, double *panel, int k, int gt,
-                                                const int *mask) {
-    __shared__ double sm[TB * TB + TB * (TB + 1)];
-    double (*Ls)[TB] = reinterpret_cast<double (*)[TB]>(sm);                 // Ls[p][row]
-    double (*Us)[TB + 1] = reinterpret_cast<double (*)[TB + 1]>(sm + TB * TB);   // Us[p][col]
-    const TBand B = band_rec(bands, blockIdx.y);
-    if (k >= B.nt || (mask && !mask[B.inst])) return;
-    const int c0 = k * TB, kb = min(TB, B.m - c0);
-    const int r0 = c0 + kb, r1 = min(B.m, r0 + B.w);
+    if (k + 1 >= B.nt || (mask && !mask[B.inst])) return;   // the last panel has no window
+    const int c0 = k * TB;
+    const int r0 = c0 + TB, r1 = min(B.m, r0 + B.w);
     const int I = blockIdx.x % gt, J = blockIdx.x / gt;
     const int i0 = r0 + TB * I, j0 = r0 + TB * J;
-    const bool next = I == 0 && J == 0 && k + 1 < B.nt;   // the tile is panel k + 1's diagonal block
+    const bool next = I == 0 && J == 0;   // the tile is panel k + 1's diagonal block
     if (!next && (i0 >= r1 || j0 >= r1)) return;
     // the next diagonal block is read whole (rows and columns past the window
     // keep their values: their products are zero), other tiles in the window
     const int cl = next ? min(B.m, r0 + TB) : r1;
-    const int t = threadIdx.x;
-    const int tr = t & 31, tc = t >> 5;   // rows 2 tr, 2 tr + 1, columns 4 tc .. 4 tc + 3
-    // this thread's 8 entries of the tile, fetched first (clamped positions)
-    // so that their loads overlap the product
-    double cv[2][4];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wi = wv & 3, wj = wv >> 2, lo = lane & 15, hi = lane >> 4;
+    const int i = i0 + 16 * wi + lo, ja = j0 + 32 * wj + hi;   // the lane's row; its columns ja + 16 t + 4 r
+    // all loads in flight together: A[panel, columns] (staged), the factors' inverses, A[rows, panel], the tile
+    double xv[8], lv[20], uv[20], av[16];
+    d4 C[2];
 #pragma unroll
-    for (int v = 0; v < 4; v++)
+    for (int u = 0; u < 8; u++) {
+        const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
+        xv[u] = tb_get(AB, B, c0 + row, min(j0 + col, r1 - 1));
+    }
+    // the wave's block columns of both products: wj and 3 - wj, with wj + 1 and 4 - wj blocks
+    const double *Lk = LI + 4096 * (B.toff + k), *Uk = UI + 4096 * (B.toff + k);
 #pragma unroll
-        for (int u = 0; u < 2; u++)
-            cv[u][v] = tb_get(AB, B, min(i0 + 2 * tr + u, cl - 1), min(j0 + 4 * tc + v, cl - 1));
-    // both tiles read down their columns (consecutive addresses across threads)
-    constexpr int NU = TB * TB / NT;
-    double lv[NU], uv[NU];   // all loads in flight before the LDS stores
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-        const int e = t + NT * u, lo = e & (TB - 1), hi = e >> 6;
-        lv[u] = tb_get(AB, B, min(i0 + lo, r1 - 1), c0 + min(hi, kb - 1));
-        uv[u] = tb_get(AB, B, c0 + min(lo, kb - 1), min(j0 + hi, r1 - 1));
+    for (int z = 0; z < 20; z++) {
+        const int blk = z < 4 * (wj + 1) ? wj : 3 - wj, q = z < 4 * (wj + 1) ? z : z - 4 * (wj + 1);
+        lv[z] = Lk[64 * (4 * q + hi) + 16 * blk + lo];
+        uv[z] = Uk[64 * (4 * q + hi) + 16 * blk + lo];
     }
 #pragma unroll
-    for (int u = 0; u < NU; u++) {
-        const int e = t + NT * u, lo = e & (TB - 1), hi = e >> 6;
-        Ls[hi][lo] = (hi < kb && i0 + lo < r1) ? lv[u] : 0.0;   // row lo, panel column hi
-        Us[lo][hi] = (lo < kb && j0 + hi < r1) ? uv[u] : 0.0;   // panel row lo, column hi
+    for (int q = 0; q < 16; q++) av[q] = tb_get(AB, B, min(i, r1 - 1), c0 + 4 * q + hi);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) C[t][r] = tb_get(AB, B, min(i, cl - 1), min(ja + 16 * t + 4 * r, cl - 1));
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
+        sm.p.Xs[LD * col + row] = j0 + col < r1 ? xv[u] : 0.0;
     }
+#pragma unroll
+    for (int q = 0; q < 16; q++) av[q] = i < r1 ? av[q] : 0.0;
     __syncthreads();
-    double acc[2][4] = {};
-#pragma unroll 8
-    for (int p = 0; p < kb; p++) {
-        double a[2], b[4];
+    const d4 zero = {0.0, 0.0, 0.0, 0.0};
+    // L panel: rows of block wi, block columns wj and 3 - wj; U panel: columns of
+    // block wi, block rows wj and 3 - wj (wave-uniform trip counts)
+    auto panels = [&](auto WJ) {
+        constexpr int J0 = decltype(WJ)::value;
+        d4 l0 = zero, l1 = zero, u0 = zero, u1 = zero;
 #pragma unroll
-        for (int u = 0; u < 2; u++) a[u] = Ls[p][2 * tr + u];
-#pragma unroll
-        for (int v = 0; v < 4; v++) b[v] = Us[p][4 * tc + v];
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[u][v] = fma(a[u], b[v], acc[u][v]);
-    }
-    if (next) {
-        // the updated block through LDS into the diagonal LU's layout
-        double (*D)[TB + 1] = reinterpret_cast<double (*)[TB + 1]>(sm);
-        __syncthreads();   // the product's LDS reads are done
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) D[2 * tr + u][4 * tc + v] = cv[u][v] - acc[u][v];
-        __syncthreads();
-        const int kb1 = min(TB, B.m - r0);
-        const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
-        double r[LW];
-#pragma unroll
-        for (int j = 0; j < LW; j++) {
-            const int col = LW * wv + j;
-            r[j] = (lane < kb1 && col < kb1) ? D[lane][col] : 0.0;
+        for (int q = 0; q < 16 - 4 * J0; q++) {
+            const double x = sm.p.Xs[LD * (16 * wi + lo) + 4 * q + hi];
+            if (q < 4 * (J0 + 1)) {
+                l0 = mfma4(uv[q], av[q], l0);
+                u0 = mfma4(x, lv[q], u0);
+            }
+            l1 = mfma4(uv[4 * (J0 + 1) + q], av[q], l1);
+            u1 = mfma4(x, lv[4 * (J0 + 1) + q], u1);
         }
-        double (*pan)[TB][LW + 1] = reinterpret_cast<double (*)[TB][LW + 1]>(sm + TB * (TB + 1));
-        double *rd = sm + TB * (TB + 1) + 2 * TB * (LW + 1);
-        diag_lu_store(r, pan, rd, AB, B, panel + (size_t)TB_PANEL * blockIdx.y, r0, kb1, lane, wv);
-        return;
-    }
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int j = j0 + 4 * tc + v;
-        if (j >= r1) continue;
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int i = i0 + 2 * tr + u;
-            if (i < r1) tb_at(AB, B, i, j) = cv[u][v] - acc[u][v];
+        for (int r = 0; r < 4; r++) {
+            sm.p.Ls[wi][4 * J0 + r][lane] = l0[r];
+            sm.p.Ls[wi][4 * (3 - J0) + r][lane] = l1[r];
+            sm.p.Us[LD * (16 * wi + hi + 4 * r) + 16 * J0 + lo] = u0[r];
+            sm.p.Us[LD * (16 * wi + hi + 4 * r) + 16 * (3 - J0) + lo] = u1[r];
         }
+    };
+    if (wj == 0) panels(std::integral_constant<int, 0>());
+    else panels(std::integral_constant<int, 1>());
+    __syncthreads();
+    d4 acc[2] = {zero, zero};
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const double l = sm.p.Ls[wi][q][lane];
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[t] = mfma4(sm.p.Us[LD * (32 * wj + 16 * t + lo) + 4 * q + hi], l, acc[t]);
     }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int j = ja + 16 * t + 4 * r;
+            C[t][r] = C[t][r] - acc[t][r];
+            if (i < cl && j < cl) tb_at(AB, B, i, j) = C[t][r];
+        }
+    if (!next) return;
+    const int kb1 = min(TB, B.m - r0);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {   // past a short last block: the identity
+            const int ii = i - r0, jj = ja + 16 * t + 4 * r - r0;
+            if (ii >= kb1 || jj >= kb1) C[t][r] = ii == jj ? 1.0 : 0.0;
+        }
+    __syncthreads();   // the products' LDS reads are done
+    lu64(C, sm.S, LI + 4096 * (B.toff + k + 1), UI + 4096 * (B.toff + k + 1), guard + B.toff + k + 1, lane, wi, wj);
 }
 
-// Inverses of every diagonal block's factors for the substitutions: LI the
-// unit-lower one, UI the upper one with the pivots themselves; 64 x 64
-// column-major per tile (padding rows and columns of a short last tile are
-// identity).  One wave per tile: lane j forms column j.
+// Every panel's diagonal block inverse for the sweeps, in the place of its
+// factors' inverses: G_k = U_k^-1 L_k^-1 (column-major) for the forward sweep
+// and the backward sweep's UI_k.  Where no pivot of the block took the guard
+// the two are the same.  Where one did, the reference's backward substitution
+// divides by the pivot itself (solv_blk_solve.c:50-52) after an elimination
+// with the guarded one: U^-1 L^-1 with L's multipliers guarded and U's own
+// diagonal, formed column by column from the block's LU (rare).  One workgroup
+// of a wave per tile, column t in lane t.
 __global__ void __launch_bounds__(64) k_tb_inv(const TBand *bands, const double *AB, double *LI, double *UI,
-                                                const int *mask) {
+                                               const int *guard, const int *mask) {
     __shared__ double D[TB][TB + 1];
-    __shared__ double T[TB][TB + 1];
+    __shared__ double X[TB][TB + 1];
     const TBand B = band_rec(bands, blockIdx.y);
     const int k = blockIdx.x;
     if (k >= B.nt || (mask && !mask[B.inst])) return;
     const int c0 = k * TB, kb = min(TB, B.m - c0), t = threadIdx.x;
+    double *Lk = LI + 4096 * (B.toff + k), *Uk = UI + 4096 * (B.toff + k);
+    const int lo = t & 15, hi = t >> 4;
+    // G by 16 x 16 blocks: G^T[j][i] = sum_m L^-1[m][j] U^-1[i][m] over blocks m >= max(i, j)
+    for (int j = 0; j < 64; j++) {   // the blocks of the other triangle were not written
+        D[t][j] = j >= (t & ~15) ? Uk[64 * t + j] : 0.0;
+        X[j][t] = j >= (t & ~15) ? Lk[64 * t + j] : 0.0;
+    }
+    __syncthreads();
+    for (int bi = 0; bi < 4; bi++)
+        for (int bj = 0; bj < 4; bj++) {
+            d4 acc = {0.0, 0.0, 0.0, 0.0};
+            for (int q = 4 * max(bi, bj); q < 16; q++)
+                acc = mfma4(X[4 * q + hi][16 * bj + lo], D[16 * bi + lo][4 * q + hi], acc);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                Lk[64 * (16 * bj + hi + 4 * r) + 16 * bi + lo] = acc[r];
+                Uk[64 * (16 * bj + hi + 4 * r) + 16 * bi + lo] = acc[r];
+            }
+        }
+    if (!guard[B.toff + k]) return;
+    __syncthreads();
     for (int j = 0; j < TB; j++)
         D[t][j] = (t < kb && j < kb) ? tb_get(AB, B, c0 + t, c0 + j) : (t == j ? 1.0 : 0.0);
     __syncthreads();
-    double x[TB];
-    // unit lower: x_i = delta_ij - sum_{q<i} L_iq x_q
-#pragma unroll
-    for (int i = 0; i < TB; i++) {
-        double s = i == t ? 1.0 : 0.0;
-#pragma unroll
-        for (int q = 0; q < i; q++) s = fma(-D[i][q], x[q], s);
-        x[i] = s;
+    for (int p = 0; p < TB; p++) {   // LU in place, lane t row t
+        const double rden = 1.0 / guarded(D[p][p]);
+        if (t > p) {
+            const double l = D[t][p] * rden;
+            D[t][p] = l;
+            for (int j = p + 1; j < TB; j++) D[t][j] = fma(-l, D[p][j], D[t][j]);
+        }
+        __syncthreads();
     }
-    const size_t o = 4096 * (B.toff + k);
-#pragma unroll
-    for (int i = 0; i < TB; i++) T[i][t] = x[i];
-    __syncthreads();
-    for (int j = 0; j < TB; j++) LI[o + 64 * j + t] = T[t][j];
-    __syncthreads();
-    // upper: x_i = (delta_ij - sum_{q>i} U_iq x_q) / U_ii
-#pragma unroll
-    for (int i = TB - 1; i >= 0; i--) {
+    for (int i = 0; i < TB; i++) {   // lane t column t: L y = e_t
         double s = i == t ? 1.0 : 0.0;
-#pragma unroll
-        for (int q = i + 1; q < TB; q++) s = fma(-D[i][q], x[q], s);
-        x[i] = s / D[i][i];
+        for (int q = 0; q < i; q++) s = fma(-D[i][q], X[q][t], s);
+        X[i][t] = s;
     }
-#pragma unroll
-    for (int i = 0; i < TB; i++) T[i][t] = x[i];
+    for (int i = TB - 1; i >= 0; i--) {   // U x = y
+        double s = X[i][t];
+        for (int q = i + 1; q < TB; q++) s = fma(-D[i][q], X[q][t], s);
+        X[i][t] = s / D[i][i];
+    }
     __syncthreads();
-    for (int j = 0; j < TB; j++) UI[o + 64 * j + t] = T[t][j];
+    for (int j = 0; j < TB; j++) Uk[64 * j + t] = X[t][j];
 }
 
-// After k_tb_inv: every off-diagonal tile of L (below a diagonal block) times
-// that block's LI, and of U (above it) times its UI, in place, so that a sweep
-// step's off-diagonal update reads one tile and no inverse: x_i -= (L_ik LI_k)
-// x_k = L_ik y_k, y_i -= (U_ik UI_k) y_k = U_ik z_k.  The products fill at most
+// After the factorisation: every off-diagonal tile below a diagonal block times
+// that block's G, and above it times its UI, in place, so that a sweep step's
+// off-diagonal update reads one tile and no inverse: x_i -= (A_ik G_k) x_k,
+// y_i -= (A_ik UI_k) y_k.  The products fill at most
 // the band's TB extra diagonals (entries within w + 63 of the diagonal), which
 // is what they are stored for.  One workgroup of 256 threads per tile, a 4 x 4
 // register block each from LDS.
-__global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB, const double *LI, const double *UI,
+__global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB, const double *G, const double *UI,
                                                   int gf, const int *mask) {
     __shared__ double As[TB][TB];       // As[q][row]: the tile, column q
     __shared__ double Ms[TB][TB + 1];   // Ms[q][col]: the inverse
@@ -481,7 +599,7 @@ __global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB
     const int i1 = low ? min(tr0 + TB, min(B.m, c0 + kb + B.w)) : tr0 + TB;
     if (i0 >= i1) return;
     const int t = threadIdx.x;
-    const double *M = (low ? LI : UI) + 4096 * (B.toff + k);
+    const double *M = (low ? G : UI) + 4096 * (B.toff + k);
     double av[16], mv[16];   // all loads in flight before the LDS stores
 #pragma unroll
     for (int u = 0; u < 16; u++) {
@@ -521,124 +639,276 @@ __global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB
     }
 }
 
-// sliced node vector <-> band-ordered vector (nodes of no block skipped; the
-// scatter leaves a model that has converged, or is outside the mask, as it is)
-__global__ void k_tb_gather(int N, const int *node_blk, const TBand *bands, const double *x, double *xb) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
-    const int bk = node_blk[a];
-    if (bk < 0) return;
-    const TBand B = bands[bk];
-    for (int v = 0; v < 3; v++) xb[B.xoff + 3 * (a - B.n0) + v] = x[vidx3(a, v)];
+// ---- substitutions ----------------------------------------------------------
+// One kernel runs both sweeps as a dataflow over 64-row tiles: a workgroup takes
+// the next tile row in order (a ticket), adds up its tiles' products as the
+// rows they need are finished, and publishes its 64 values.  A value is its own
+// ready flag: the output vectors hold NOT_YET until it is stored, values travel
+// by agent-scope atomic stores and loads (past the XCDs' private L2s), and a
+// reader polls the value itself, so a hand-over is one store and one load and
+// needs no fence.  Tickets make it free of deadlock whatever is resident: rows
+// are claimed in order, so the lowest unfinished row belongs to a running
+// workgroup and waits only for finished ones.
+constexpr unsigned long long NOT_YET = 0xfff8dead0badf00dull;   // a NaN no arithmetic produces
+
+__device__ __forceinline__ void publish(double *p, double v) {
+    unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    if (u == NOT_YET) u = 0x7ff8000000000000ull;
+    __hip_atomic_store((unsigned long long *)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__global__ void k_tb_scatter(int N, const int *node_blk, const TBand *bands, const double *xb, double *x,
-                             const KScal *sc, const int *mask) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
-    const int bk = node_blk[a];
-    if (bk < 0) return;
-    const TBand B = bands[bk];
-    if ((sc && sc[B.inst].done) || (mask && !mask[B.inst])) return;
-    for (int v = 0; v < 3; v++) x[vidx3(a, v)] = xb[B.xoff + 3 * (a - B.n0) + v];
+__device__ __forceinline__ unsigned long long peek(const double *p) {
+    return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the value at p in every lane with `want`, waiting until all of the wave's are there
+__device__ __forceinline__ double await_value(const double *p, bool want) {
+    unsigned long long u = want ? peek(p) : 0ull;
+    while (__any(u == NOT_YET)) {
+        __builtin_amdgcn_s_sleep(1);
+        if (u == NOT_YET) u = peek(p);
+    }
+    return __longlong_as_double((long long)u);
 }
 
-// Sweep kernels: four waves per workgroup split a tile's 64 columns (16
-// each); lane r accumulates row r over its wave's columns (the column value
-// broadcast from lane c) and the four partial sums are added in LDS in wave
-// order.  Block 0 applies the diagonal block's inverse; block g >= 1 the
-// off-diagonal tile scaled by it (k_tb_scale), to the same input slice, so
-// the blocks of a step are independent and each reads one tile: all of a
-// block's loads are issued at once after a single band-record fetch.
-__device__ __forceinline__ double tile_mv_part(const double (&m)[16], double xr, int wv) {
+// The right-hand side into band order (nodes of no block skipped), the two
+// output vectors to NOT_YET, the tickets to zero.
+__global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, const int *node_blk, const TBand *bands,
+                                                   const double *x, double *xb, double *yb, double *zb, int *tick) {
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int b = a; b < 2 * nband; b += gridDim.x * blockDim.x) tick[b] = 0;
+    if (a >= N) return;
+    const int bk = node_blk[a];
+    if (bk < 0) return;
+    const TBand B = bands[bk];
+    const size_t o = B.xoff + 3 * (size_t)(a - B.n0);
+    const double ny = __longlong_as_double((long long)NOT_YET);
+    for (int v = 0; v < 3; v++) {
+        xb[o + v] = x[vidx3(a, v)];
+        yb[o + v] = ny;
+        zb[o + v] = ny;
+    }
+}
+
+// One sweep of a band by this workgroup.  FWD: y_i = x_i - sum_{k < i} (A_ik
+// G_k) y_k into out = yb; else z_i = y_i - sum_{k > i} (A_ik UI_k) z_k into out
+// = zb (the diagonal inverse is applied afterwards, k_tb_apply).  Eight waves
+// take 8 columns each of every tile, lane r row r; the ninth wave polls the
+// values the tiles multiply (so that no poll queues behind a tile's loads),
+// hands them over in LDS, adds the row's partial sums in wave order and
+// publishes it.  A product's tile was fetched SW_PF products earlier, across
+// rows, so a step of the chain is the hand-over and one 64 x 64 product; the
+// order of every sum is fixed, whichever workgroup runs the row.
+constexpr int SW_W = 8;                  // product waves
+constexpr int SW_NT = 64 * (SW_W + 1);   // threads of a sweep workgroup
+constexpr int SW_PF = 4;                 // tiles fetched ahead
+constexpr int SW_RING = 32;              // values handed over between two barriers
+struct SweepLds {
+    double x[SW_RING][TB];
+    double part[2][SW_W][TB];
+    int ready;       // values handed over since the last barrier
+    int rows[2][4];  // the next row and those claimed after it
+};
+template <bool FWD>
+__device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const double *in, double *out, int *tick,
+                                         SweepLds &S) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool server = wv == SW_W;
+    // t-th row in sweep order; its number of tiles; the j-th of them in the order their values finish
+    auto row_of = [&](int t) { return FWD ? t : B.nt - 1 - t; };
+    auto ntiles = [&](int i) {
+        if (FWD) {
+            const int d = TB * i - TB - B.w;   // column tile k reaches row tile i when 64 k > d
+            return i - (d < 0 ? 0 : d / TB + 1);
+        }
+        return min(B.nt - 1, (TB * i + TB + B.w - 1) / TB) - i;
+    };
+    auto kcol = [&](int i, int n, int j) { return FWD ? i - n + j : i + n - j; };
+    if (threadIdx.x == 64 * SW_W) {
+        S.rows[0][0] = atomicAdd(tick, 1);
+        S.ready = 0;
+    }
+    __syncthreads();
+    int cur = __builtin_amdgcn_readfirstlane(S.rows[0][0]);
+    __syncthreads();
+    // an LDS pointer by type: a generic one would make the polls flat loads,
+    // which queue behind the tiles' loads
+    using lds_int = __attribute__((address_space(3))) volatile int;
+    lds_int *ready = (lds_int *)&S.ready;
+    int parity = 0;
+    if (server) {
+        // rows claimed ahead (INT_MAX: not yet), one when a row's first value has
+        // arrived -- by then the other workgroups have theirs, so neighbouring
+        // rows go to different workgroups -- and one more after a row while the
+        // product waves cannot see SW_PF tiles ahead
+        int q0 = INT_MAX, q1 = INT_MAX, q2 = INT_MAX;
+        auto claim = [&]() {
+            if (q2 != INT_MAX) return;
+            int t = 0;
+            if (lane == 0) t = atomicAdd(tick, 1);
+            t = __builtin_amdgcn_readfirstlane(t);
+            if (q0 == INT_MAX) q0 = t;
+            else if (q1 == INT_MAX) q1 = t;
+            else q2 = t;
+        };
+        while (cur < B.nt) {
+            const int i = row_of(cur), n = ntiles(i), r = TB * i + lane;
+            const double xi = FWD ? in[B.xoff + min(r, B.m - 1)] : await_value(in + B.xoff + min(r, B.m - 1), true);
+            if (n == 0) claim();
+            for (int j = 0; j < n; j++) {
+                const int d = TB * kcol(i, n, j) + lane;
+                const double v = await_value(out + B.xoff + min(d, B.m - 1), d < B.m);
+                S.x[j % SW_RING][lane] = v;   // 0 past the band's last row
+                wave_sync();                  // LDS keeps a wave's order: the value, then the count
+                if (lane == 0) *ready = j % SW_RING + 1;
+                if (j == 0) claim();
+                if (j % SW_RING == SW_RING - 1 && j + 1 < n) {   // the ring is full: wait for the products
+                    __syncthreads();
+                    if (lane == 0) *ready = 0;
+                    __syncthreads();
+                }
+            }
+            if (lane < 3) S.rows[parity][lane] = lane == 0 ? q0 : (lane == 1 ? q1 : q2);
+            __syncthreads();   // the row's partial sums are in LDS
+            if (lane == 0) *ready = 0;
+            double s = S.part[parity][0][lane];
+#pragma unroll
+            for (int w = 1; w < SW_W; w++) s += S.part[parity][w][lane];
+            if (r < B.m) publish(out + B.xoff + r, xi - s);
+            cur = q0;
+            q0 = q1;
+            q1 = q2;
+            q2 = INT_MAX;
+            parity ^= 1;
+            __syncthreads();   // the next row's hand-overs count from zero
+            if ((n < SW_PF ? q1 : q0) == INT_MAX) claim();
+        }
+    } else {
+        const int c8 = 8 * wv;
+        double m[SW_PF][8];
+        long long tag[SW_PF];   // row (in sweep order) and tile whose entries m[s] holds
+        auto id = [&](int t, int j) { return ((long long)t << 32) | j; };
+        auto fetch = [&](double (&d)[8], int t, int j) {
+            const int i = row_of(t), n = ntiles(i), k = kcol(i, n, j);
+            const int ck = TB * k, kb = min(TB, B.m - ck), r = TB * i + lane;
+            const int rc = FWD ? min(r, min(B.m, ck + TB + B.w) - 1) : max(r, max(0, ck - B.w));
+            const double *p = AB + tb_idx(B, rc, ck);
+#pragma unroll
+            for (int u = 0; u < 8; u++) d[u] = p[(size_t)min(c8 + u, kb - 1) * (2 * B.wp)];
+        };
+        int q[2] = {INT_MAX, INT_MAX};   // the rows after cur, as far as they are known
+        int j = 0, n = cur < B.nt ? ntiles(row_of(cur)) : 0;
+        // the entries of the `ahead`-th tile from (cur, j) into d, and its tag.  Always
+        // eight loads, so that the number in flight is known where one is waited
+        // for: past the known rows an earlier tile again (row 1 has one
+        // wherever there is a second row), under no tag.
+        auto prefetch = [&](double (&d)[8], int ahead) {
+            int t = cur, jj = j + ahead, nn = n;
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+                if (jj >= nn && t < B.nt) {
+                    jj -= nn;
+                    t = q[a];
+                    nn = t < B.nt ? ntiles(row_of(t)) : 0;
+                }
+            const bool got = t < B.nt && jj < nn;
+            if (!got) { t = 1; jj = 0; }
+            fetch(d, t, jj);
+            return got ? id(t, jj) : -1LL;
+        };
+        if (B.nt > 1) {
+#pragma unroll
+            for (int s = 0; s < SW_PF; s++) tag[s] = prefetch(m[s], s);
+        }
+        double acc = 0.0;
+        while (cur < B.nt) {
+#pragma unroll
+            for (int s = 0; s < SW_PF; s++) {
+                while (j == n) {   // the row is done
+                    S.part[parity][wv][lane] = acc;
+                    __syncthreads();
+                    cur = __builtin_amdgcn_readfirstlane(S.rows[parity][0]);
+                    q[0] = __builtin_amdgcn_readfirstlane(S.rows[parity][1]);
+                    q[1] = __builtin_amdgcn_readfirstlane(S.rows[parity][2]);
+                    parity ^= 1;
+                    j = 0;
+                    acc = 0.0;
+                    n = cur < B.nt ? ntiles(row_of(cur)) : -1;
+                    __syncthreads();
+                }
+                if (n < 0) break;   // no rows left
+                const int i = row_of(cur), k = kcol(i, n, j), ck = TB * k, r = TB * i + lane;
+                if (tag[s] != id(cur, j)) {   // its row was not known in time
+                    fetch(m[s], cur, j);
+                    // used here, so that this path waits here and the other keeps its fetches in flight
+                    asm volatile("" : "+v"(m[s][0]), "+v"(m[s][1]), "+v"(m[s][2]), "+v"(m[s][3]), "+v"(m[s][4]),
+                                 "+v"(m[s][5]), "+v"(m[s][6]), "+v"(m[s][7]));
+                }
+                while (*ready <= j % SW_RING) __builtin_amdgcn_s_sleep(1);
+                wave_sync();
+                const double xv = S.x[j % SW_RING][c8 + (lane & 7)];
+                double p = 0.0;
+#pragma unroll
+                for (int u = 0; u < 8; u++) p = fma(m[s][u], lane_bcast(xv, u), p);
+                // rows the column tile does not reach were read clamped
+                const bool in_reach = FWD ? r < min(B.m, ck + TB + B.w) : r >= ck - B.w;
+                acc += in_reach ? p : 0.0;
+                if (j % SW_RING == SW_RING - 1 && j + 1 < n) {
+                    __syncthreads();
+                    __syncthreads();
+                }
+                tag[s] = prefetch(m[s], SW_PF);
+                j++;
+            }
+        }
+    }
+    __syncthreads();   // the LDS is free for the next sweep
+}
+
+__global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, const double *AB, const double *xb, double *yb,
+                                                    double *zb, int *tick, const int *done, const int *mask,
+                                                    const KScal *sc) {
+    __shared__ SweepLds S;
+    const int stop = *done;   // the band record and the flag fetched together
+    const TBand B = band_rec(bands, blockIdx.y, stop);
+    // ensembles: the band's model, converged or outside the mask, is skipped
+    if (stop || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
+    tb_sweep<true>(B, AB, xb, yb, tick + 2 * blockIdx.y, S);
+    tb_sweep<false>(B, AB, yb, zb, tick + 2 * blockIdx.y + 1, S);
+}
+
+// The backward sweep's diagonal inverses, and back into node order: x_k = UI_k z_k,
+// one workgroup of four waves per tile (16 columns each, partial sums added in
+// wave order).  A model that has converged, or is outside the mask, keeps x.
+__global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, const double *UI, const double *zb, double *x,
+                                                  const int *done, const int *mask, const KScal *sc) {
+    __shared__ double part[4][TB];
+    const int stop = *done;
+    const TBand B = band_rec(bands, blockIdx.y, stop);
+    const int k = blockIdx.x;
+    if (stop || k >= B.nt || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c0 = TB * k, kb = min(TB, B.m - c0);
+    const double *M = UI + 4096 * (B.toff + k);
+    double m[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) m[u] = M[64 * (16 * wv + u) + lane];
+    const double zv = zb[B.xoff + c0 + min(lane, kb - 1)];
+    const double zr = lane < kb ? zv : 0.0;
     double s = 0.0;
 #pragma unroll
-    for (int u = 0; u < 16; u++) s = fma(m[u], lane_bcast(xr, 16 * wv + u), s);
-    return s;
-}
-__device__ __forceinline__ double sum4(double (*part)[TB], int lane) {
-    return ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
-}
-
-// Forward step k: block 0 stores y_k = LI_k x_k in yb; block g >= 1 takes
-// x[tile k + g] -= (L LI_k)[tile k + g, tile k] x_k.
-__global__ void __launch_bounds__(256) k_tb_fwd(const TBand *bands, const double *AB, const double *LI, double *xb,
-                                                double *yb, int k, const int *done, const int *mask,
-                                                const KScal *sc) {
-    __shared__ double part[4][TB];
-    const int stop = *done;   // the band record and the flag fetched together
-    const TBand B = band_rec(bands, blockIdx.y, stop);
-    // ensembles: the band's model, converged or outside the mask, is skipped
-    if (stop || k >= B.nt || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
-    const int c0 = k * TB, kb = min(TB, B.m - c0), g = blockIdx.x;
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rmax = min(B.m, c0 + kb + B.w);
-    if (g > 0 && c0 + TB * g >= rmax) return;
-    const int i = c0 + TB * g + lane, ic = min(i, rmax - 1);
-    const double xv = xb[B.xoff + c0 + min(lane, kb - 1)];
-    double m[16], xi = 0.0;
-    if (g == 0) {
-        const double *M = LI + 4096 * (B.toff + k);
-#pragma unroll
-        for (int u = 0; u < 16; u++) m[u] = M[64 * (16 * wv + u) + lane];
-    } else {
-#pragma unroll
-        for (int u = 0; u < 16; u++) m[u] = tb_get(AB, B, ic, c0 + min(16 * wv + u, kb - 1));
-        xi = xb[B.xoff + ic];
-    }
-    const double xr = lane < kb ? xv : 0.0;
-    part[wv][lane] = tile_mv_part(m, xr, wv);
+    for (int u = 0; u < 16; u++) s = fma(m[u], lane_bcast(zr, 16 * wv + u), s);
+    part[wv][lane] = s;
     __syncthreads();
-    if (wv != 0) return;
-    if (g == 0) {
-        if (lane < kb) yb[B.xoff + c0 + lane] = sum4(part, lane);
-    } else if (i < rmax) {
-        xb[B.xoff + i] = xi - sum4(part, lane);
-    }
-}
-
-// Backward step k: block 0 stores z_k = UI_k y_k in xb; block g >= 1 takes
-// y[tile k - g] -= (U UI_k)[tile k - g, tile k] y_k.
-__global__ void __launch_bounds__(256) k_tb_bwd(const TBand *bands, const double *AB, const double *UI, double *xb,
-                                                double *yb, int k, const int *done, const int *mask,
-                                                const KScal *sc) {
-    __shared__ double part[4][TB];
-    const int stop = *done;   // the band record and the flag fetched together
-    const TBand B = band_rec(bands, blockIdx.y, stop);
-    // ensembles: the band's model, converged or outside the mask, is skipped
-    if (stop || k >= B.nt || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
-    const int c0 = k * TB, kb = min(TB, B.m - c0), g = blockIdx.x;
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rmin = max(0, c0 - B.w);
-    if (g > 0 && c0 - TB * g + TB <= rmin) return;
-    const int i = c0 - TB * g + lane, ic = max(i, rmin);
-    const double yv = yb[B.xoff + c0 + min(lane, kb - 1)];
-    double m[16], yi = 0.0;
-    if (g == 0) {
-        const double *M = UI + 4096 * (B.toff + k);
-#pragma unroll
-        for (int u = 0; u < 16; u++) m[u] = M[64 * (16 * wv + u) + lane];
-    } else {
-#pragma unroll
-        for (int u = 0; u < 16; u++) m[u] = tb_get(AB, B, ic, c0 + min(16 * wv + u, kb - 1));
-        yi = yb[B.xoff + ic];
-    }
-    const double yr = lane < kb ? yv : 0.0;
-    part[wv][lane] = tile_mv_part(m, yr, wv);
-    __syncthreads();
-    if (wv != 0) return;
-    if (g == 0) {
-        if (lane < kb) xb[B.xoff + c0 + lane] = sum4(part, lane);
-    } else if (i >= rmin) {
-        yb[B.xoff + i] = yi - sum4(part, lane);
-    }
+    if (wv != 0 || lane >= kb) return;
+    const int d = c0 + lane;
+    x[vidx3(B.n0 + d / 3, d % 3)] = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
 }
 
 void tband_free(Ctx *c) {
     for (void *p : {(void *)c->tb_bands, (void *)c->tb_AB, (void *)c->tb_LI, (void *)c->tb_UI, (void *)c->tb_xb,
-                    (void *)c->tb_yb, (void *)c->tb_panel})
+                    (void *)c->tb_yb, (void *)c->tb_zb, (void *)c->tb_int})
         if (p) (void)hipFree(p);
-    c->tb_bands = nullptr; c->tb_AB = nullptr; c->tb_LI = nullptr; c->tb_UI = nullptr; c->tb_panel = nullptr;
-    c->tb_xb = nullptr; c->tb_yb = nullptr;
+    c->tb_bands = nullptr; c->tb_AB = nullptr; c->tb_LI = nullptr; c->tb_UI = nullptr; c->tb_int = nullptr;
+    c->tb_xb = nullptr; c->tb_yb = nullptr; c->tb_zb = nullptr;
     c->tb_nband = 0; c->tb_maxnt = 0; c->tb_gt = 0; c->tb_gf = 0; c->tb_size = 0;
     c->tb_h_nt.clear(); c->tb_h_inst.clear();
 }
@@ -673,7 +943,8 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     }
     size_t freeb = 0, totalb = 0;
     (void)hipMemGetInfo(&freeb, &totalb);
-    const size_t need = sizeof(double) * (off + 2 * 4096 * toff + 2 * xoff);
+    const size_t nint = toff + 2 * (size_t)nblk;   // a guard flag per tile, two tickets per band
+    const size_t need = sizeof(double) * (off + 2 * 4096 * toff + 3 * xoff) + sizeof(int) * nint;
     if (need + ((size_t)2 << 30) > freeb)
         return "tiled band LU: " + std::to_string(need >> 20) + " MiB of band storage do not fit in the free " +
                std::to_string(freeb >> 20) + " MiB; raise nblock" +
@@ -685,7 +956,8 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
         hipMalloc((void **)&c->tb_UI, sizeof(double) * 4096 * toff) != hipSuccess ||
         hipMalloc((void **)&c->tb_xb, sizeof(double) * xoff) != hipSuccess ||
         hipMalloc((void **)&c->tb_yb, sizeof(double) * xoff) != hipSuccess ||
-        hipMalloc((void **)&c->tb_panel, sizeof(double) * TB_PANEL * nblk) != hipSuccess) {
+        hipMalloc((void **)&c->tb_zb, sizeof(double) * xoff) != hipSuccess ||
+        hipMalloc((void **)&c->tb_int, sizeof(int) * nint) != hipSuccess) {
         tband_free(c);
         return "hipMalloc failed for the tiled band LU";
     }
@@ -697,6 +969,7 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     c->tb_gt = (maxw + TB - 1) / TB;
     c->tb_gf = (maxw + 2 * TB - 2) / TB;   // tiles below (above) a panel that its L (U) reaches
     c->tb_size = off;
+    c->tb_guard = c->tb_int + 2 * nblk;
     return "";
 }
 
@@ -722,16 +995,13 @@ void launch_tband_setup(Ctx *c) {
     hipLaunchKernelGGL(k_tb_load, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->node_blk,
                        c->tb_bands, c->tb_AB, c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, mask);
     const int gt = std::max(1, c->tb_gt);
-    hipLaunchKernelGGL(k_tb_diag, dim3(c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_panel,
-                       0, mask);
-    for (int k = 0; k < nt; k++) {
-        hipLaunchKernelGGL(k_tb_trsm, dim3(2 * gt, c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_panel, k, gt, mask);
-        hipLaunchKernelGGL(k_tb_gemm, dim3(gt * gt, c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_panel, k, gt, mask);
-    }
-    hipLaunchKernelGGL(k_tb_inv, dim3(nt, c->tb_nband), dim3(64), 0, c->stream, c->tb_bands, c->tb_AB,
-                       c->tb_LI, c->tb_UI, mask);
+    hipLaunchKernelGGL(k_tb_diag, dim3(c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
+                       c->tb_UI, c->tb_guard, mask);
+    for (int k = 0; k + 1 < nt; k++)
+        hipLaunchKernelGGL(k_tb_step, dim3(gt * gt, c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB,
+                           c->tb_LI, c->tb_UI, c->tb_guard, k, gt, mask);
+    hipLaunchKernelGGL(k_tb_inv, dim3(nt, c->tb_nband), dim3(64), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
+                       c->tb_UI, c->tb_guard, mask);
     const int gf = std::max(1, c->tb_gf);
     hipLaunchKernelGGL(k_tb_scale, dim3(nt, 2 * gf, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands,
                        c->tb_AB, c->tb_LI, c->tb_UI, gf, mask);
@@ -741,22 +1011,22 @@ void launch_tband_setup(Ctx *c) {
 // null outside the iteration loop
 void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     const int *mask = tb_mask(c);
-    const dim3 gn(nblocks_for(c->N, 256));
-    hipLaunchKernelGGL(k_tb_gather, gn, dim3(256), 0, c->stream, c->N, c->node_blk, c->tb_bands, x, c->tb_xb);
-    const dim3 g(1 + c->tb_gf, c->tb_nband);
+    const int nt = tb_active_nt(c);
+    if (nt == 0) return;
+    hipLaunchKernelGGL(k_tb_gather, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->tb_nband,
+                       c->node_blk, c->tb_bands, x, c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int);
     // one model: its done flag, or the first band record's pad (always 0),
     // read beside the band record; ensembles: each band's model's flag
     const int *done = (sc && !mask) ? &sc->done : &c->tb_bands[0].pad;
     const KScal *msc = mask ? sc : nullptr;
-    const int nt = tb_active_nt(c);
-    for (int k = 0; k < nt; k++)
-        hipLaunchKernelGGL(k_tb_fwd, g, dim3(256), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI, c->tb_xb, c->tb_yb,
-                           k, done, mask, msc);
-    for (int k = nt - 1; k >= 0; k--)
-        hipLaunchKernelGGL(k_tb_bwd, g, dim3(256), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_UI, c->tb_xb, c->tb_yb,
-                           k, done, mask, msc);
-    hipLaunchKernelGGL(k_tb_scatter, gn, dim3(256), 0, c->stream, c->N, c->node_blk, c->tb_bands, c->tb_xb, x, sc,
-                       mask);
+    // a workgroup per tile of a row's reach and one more keep the chain's next
+    // row always waiting; any number is correct, and with many bands one
+    // workgroup each already fills the chip
+    const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 512 / c->tb_nband));
+    hipLaunchKernelGGL(k_tb_sweep, dim3(g, c->tb_nband), dim3(SW_NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_xb,
+                       c->tb_yb, c->tb_zb, c->tb_int, done, mask, msc);
+    hipLaunchKernelGGL(k_tb_apply, dim3(nt, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_UI, c->tb_zb, x,
+                       done, mask, msc);
 }
 
 }  // namespace sw2

@@ -674,12 +674,20 @@ __global__ void __launch_bounds__(256) k_pl_omega(int N, KVecs<P> V, double *par
 // solv_return_old (src/solver/solv_return_old.c:23-30): sol = (u + u0) * scale,
 // u0 the initial guess held in sol.  ZERO: the caller zeroed the guess (the
 // Newton step does), so u0 = +0 enters as a constant and the kernel gives the
-// same sol however often it runs.
+// same sol however often it runs.  r (one LU of the whole matrix, or null): a
+// model whose solve ended at the prologue takes its preconditioned residual
+// r = M^-1 (b - A u), which the prologue has formed to test it, as one step of
+// refinement: the LU's rounding error enters squared.
 template <typename T, bool ZERO>
-__global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol) {
+__global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, const double *r, const KScal *sc,
+                          const int *node_inst) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N3) return;
     double x = (double)u[i];
+    if (r) {
+        const int m = node_inst ? node_inst[64 * (i / 192) + (i & 63)] : 0;
+        if (m >= 0 && sc[m].done && sc[m].it == 0) x += r[i];
+    }
     x += ZERO ? 0.0 : sol[i];
     x *= scale[i];
     sol[i] = x;
@@ -839,13 +847,19 @@ void launch_krylov_iters(Ctx *c, int k) {
 void launch_krylov_epilogue(Ctx *c, bool zero_guess) {
     int n3 = 3 * c->Np;
     dim3 g(nblocks_for(n3, 256));
+    const bool lu = c->opts.preconditioner == 1 && c->opts.krylov == 0 && c->band_tiled && c->opts.nblock == 1;
+    const double *r = lu ? c->kr : nullptr;
+    const int *ni = c->ninst ? c->node_inst : nullptr;
+#define SW2_EPI(T, Z, U) \
+    hipLaunchKernelGGL((k_bcg_epi<T, Z>), g, dim3(256), 0, c->stream, n3, U, c->scale, c->sol, r, c->ksc, ni)
     if (c->opts.precision == 2) {
-        if (zero_guess) hipLaunchKernelGGL((k_bcg_epi<float, true>), g, dim3(256), 0, c->stream, n3, c->fu, c->scale, c->sol);
-        else hipLaunchKernelGGL((k_bcg_epi<float, false>), g, dim3(256), 0, c->stream, n3, c->fu, c->scale, c->sol);
+        if (zero_guess) SW2_EPI(float, true, c->fu);
+        else SW2_EPI(float, false, c->fu);
     } else {
-        if (zero_guess) hipLaunchKernelGGL((k_bcg_epi<double, true>), g, dim3(256), 0, c->stream, n3, c->ku, c->scale, c->sol);
-        else hipLaunchKernelGGL((k_bcg_epi<double, false>), g, dim3(256), 0, c->stream, n3, c->ku, c->scale, c->sol);
+        if (zero_guess) SW2_EPI(double, true, c->ku);
+        else SW2_EPI(double, false, c->ku);
     }
+#undef SW2_EPI
 }
 
 }  // namespace sw2
