@@ -8,11 +8,12 @@
 // factors are those of the skyline LU; only the rounding order of the
 // updates differs).
 //
-// One workgroup factors one block (right-looking band update, a barrier per
-// pivot); one wavefront solves one block (forward unit-lower, backward
-// upper), keeping the block's right-hand side in LDS.  This is the robust
-// preconditioner for steps with large Courant numbers, where 3x3 block
-// Jacobi stalls; its cost grows with block size times bandwidth squared.
+// Here: the partition, and the LU of blocks of at most a tile (64 DOFs), one
+// workgroup per block (right-looking band update, a barrier per pivot) and one
+// wavefront per solve (forward unit-lower, backward upper, the block's
+// right-hand side in LDS).  Larger blocks go to the tiled band LU (sw2_lu.hip).
+// This is the robust preconditioner for steps with large Courant numbers, where
+// 3x3 block Jacobi stalls.
 #include <algorithm>
 #include <string>
 
@@ -178,24 +179,34 @@ std::string band_structure(Ctx *c, int nblock) {
         max_n = std::max(max_n, nb);
         off[b + 1] = off[b] + (size_t)nb * (2 * w[b] + 1);
     }
-    // blocks beyond the one-workgroup band LU (its solve keeps a block's
-    // right-hand side in LDS), ensembles, or when asked for: the tiled band LU
-    if (c->ninst || max_n > BAND_MAX_DOF || off[nbk] * sizeof(double) > BAND_MAX_BYTES || c->opts.lu_tiled) {
+    // The tiled band LU takes every partition whose largest block exceeds a
+    // tile: the one-workgroup LU pays a global-memory round trip and a barrier
+    // per pivot (set-up + one application, 40 x 20 cells: one block of 2,583
+    // DOFs 12.9 + 2.7 ms against 1.0 + 0.21, ten of 258 1.2 + 0.32 against
+    // 0.19 + 0.07, 41 of 63 0.09 + 0.09 against 0.08 + 0.05).  Below, the one-
+    // workgroup LU is the faster one and needs no 64 x 64 inverses per block
+    // (300 x 100 cells, 7,600 blocks of 12 DOFs: 0.16 + 0.19 ms against 0.83 +
+    // 0.35, and 20 MB against 1.1 GB).  Ensembles always take the tiled LU, and so
+    // does opts.lu_tiled; a partition whose tiles do not fit in device memory
+    // falls back to the one-workgroup LU where that can hold its blocks.
+    const bool small_ok = !c->ninst && !c->opts.lu_tiled && max_n <= BAND_MAX_DOF &&
+                          off[nbk] * sizeof(double) <= BAND_MAX_BYTES;
+    if (!small_ok || max_n > 64) {
         if (hipMalloc((void **)&c->node_blk, sizeof(int) * N) != hipSuccess ||
             hipMemcpy(c->node_blk, node_blk.data(), sizeof(int) * N, hipMemcpyHostToDevice) != hipSuccess) {
             band_free(c);
             return "hipMalloc failed for the profile-LU blocks";
         }
         std::string err = tband_structure(c, s0, s1, binst, w);
-        if (!err.empty()) {
-            band_free(c);
-            return err;
+        if (err.empty()) {
+            c->band_tiled = 1;
+            c->band_nblock = nblock;
+            c->band_nb = nbk;
+            c->band_max_n = max_n;
+            return "";
         }
-        c->band_tiled = 1;
-        c->band_nblock = nblock;
-        c->band_nb = nbk;
-        c->band_max_n = max_n;
-        return "";
+        band_free(c);
+        if (!small_ok) return err;
     }
     // one model: consecutive blocks, n0[b + 1] = the end of block b
     std::vector<int> n0(s0);
