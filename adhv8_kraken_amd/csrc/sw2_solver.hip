@@ -677,7 +677,15 @@ __global__ void __launch_bounds__(256) k_pl_omega(int N, KVecs<P> V, double *par
 // same sol however often it runs.  r (one LU of the whole matrix, or null): a
 // model whose solve ended at the prologue takes its preconditioned residual
 // r = M^-1 (b - A u), which the prologue has formed to test it, as one step of
-// refinement: the LU's rounding error enters squared.
+// refinement when the factorisation has lost digits (|r| above REFINE_ABOVE
+// times the right-hand side's norm): the LU's rounding error then enters
+// squared.  A well-conditioned model stands at 1e-13 and below (angle_source
+// deck 3e-14) and returns u as the reference does; a nearly singular one (the
+// partly dry floodplain, 224 x 112 nodes) was seen at 8e-7, and without the
+// step its Newton history left the oracle's by 2.4e-7 of its first entry,
+// with it by 1.2e-8.
+constexpr double REFINE_ABOVE = 1e-12;
+
 template <typename T, bool ZERO>
 __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, const double *r, const KScal *sc,
                           const int *node_inst) {
@@ -686,7 +694,7 @@ __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, 
     double x = (double)u[i];
     if (r) {
         const int m = node_inst ? node_inst[64 * (i / 192) + (i & 63)] : 0;
-        if (m >= 0 && sc[m].done && sc[m].it == 0) x += r[i];
+        if (m >= 0 && sc[m].done && sc[m].it == 0 && sc[m].rnorm > REFINE_ABOVE * sc[m].bnorm) x += r[i];
     }
     x += ZERO ? 0.0 : sol[i];
     x *= scale[i];
@@ -847,7 +855,8 @@ void launch_krylov_iters(Ctx *c, int k) {
 void launch_krylov_epilogue(Ctx *c, bool zero_guess) {
     int n3 = 3 * c->Np;
     dim3 g(nblocks_for(n3, 256));
-    const bool lu = c->opts.preconditioner == 1 && c->opts.krylov == 0 && c->band_tiled && c->opts.nblock == 1;
+    const bool lu = c->opts.preconditioner == 1 && c->opts.krylov == 0 && c->band_tiled && c->opts.nblock == 1 &&
+                    c->opts.precision != 2;
     const double *r = lu ? c->kr : nullptr;
     const int *ni = c->ninst ? c->node_inst : nullptr;
 #define SW2_EPI(T, Z, U) \
