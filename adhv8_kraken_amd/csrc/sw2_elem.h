@@ -99,6 +99,10 @@ struct ElemData {
 HDF double elem_dt(const ElemData &D, int ie) { return D.dt_inst ? D.dt_inst[D.elem_inst[ie]] : D.dt; }
 HDF double edge_dt(const ElemData &D, int ie) { return D.dt_inst ? D.dt_inst[D.edge_inst[ie]] : D.dt; }
 
+// Dirichlet kinds of a node string in two bits (0: none of them), and back
+HDF int bc_code(int bc) { return bc == BCT_PRS_DIR ? 1 : bc == BCT_VEL_DIR ? 2 : bc == BCT_VEL_PRS_DIR ? 3 : 0; }
+HDF int code_bc(int code) { return code == 1 ? BCT_PRS_DIR : code == 2 ? BCT_VEL_DIR : code == 3 ? BCT_VEL_PRS_DIR : 0; }
+
 // Correctly rounded x / b from y = RN(1/b): one multiply and two FMAs
 // instead of a full division.  Markstein's correction step (P. Markstein,
 // "Computation of elementary functions on the IBM RISC System/6000
@@ -202,13 +206,26 @@ HDF double drag_coef(double depth, double rh, const crlog::tables *T) {
 }
 
 // ---------------------------------------------------------------- wet/dry
+// integrate_triangle_dphi_f_f_h (:864-884): the factors of h_0, h_1, h_2 ...
+HDF void flux_ff(const double *f, double *p) {
+    double f1_2 = f[0] * f[0], f2_2 = f[1] * f[1], f3_2 = f[2] * f[2];
+    p[0] = (3 * f1_2 + 2 * f[0] * f[1] + f2_2 + (2 * f[0] + f[1]) * f[2] + f3_2);
+    p[1] = (f1_2 + 2 * f[0] * f[1] + 3 * f2_2 + (f[0] + 2 * f[1]) * f[2] + f3_2);
+    p[2] = (f1_2 + f[0] * f[1] + f2_2 + 2 * (f[0] + f[1]) * f[2] + 3 * f3_2);
+}
+// ... and the integral, c the flux's factor (-1 dt)
+HDF double flux_ffh(const double *p, const double *h, double djac, double c) {
+    return djac * one_30 * c * (p[0] * h[0] + p[1] * h[1] + p[2] * h[2]);
+}
+
 // integrand selectors for the wet/dry wrapper (fe_sw2_wet_dry_integrations.c)
 enum { WD_INTEGRATE_F = 0, WD_CONT_TEMPORAL, WD_CONVECTION, WD_GLS_CONVECTION, WD_PRESSURE, WD_BODYFORCE,
        WD_BOUNDARY_PRESSURE };
 
 template <int FN>
 HDF void wd_apply(const v3 *x, const double *h, const v2 *gp, v2 vconst, const v2 *vwd, const double *fwd, double djac,
-                  double dt, double c, d3 *rhs) {
+                  double dt, double c, d3 *rhs, const double *flux = nullptr) {
+    // flux (convection): the u u h and v v h integrals where the caller has them
     if (FN == WD_INTEGRATE_F) {  // :95-116
         double t1 = div_rn(h[0] + h[1] + h[2], 3.0, RN_ONE_THIRD), t2 = 0.0, t3 = 0.0;
         if (vwd) {
@@ -251,16 +268,19 @@ HDF void wd_apply(const v3 *x, const double *h, const v2 *gp, v2 vconst, const v
             for (int i = 0; i < 3; i++) rx[i] += con * gp[i].y;
         }
         // integrate_triangle_dphi_f_f_h :864-884, once with uu (x) and once with vv (y)
-        for (int pass = 0; pass < 2; pass++) {
-            const double *f = pass == 0 ? uu : vv;
-            double f1_2 = f[0] * f[0], f2_2 = f[1] * f[1], f3_2 = f[2] * f[2];
-            double p1 = (3 * f1_2 + 2 * f[0] * f[1] + f2_2 + (2 * f[0] + f[1]) * f[2] + f3_2);
-            double p2 = (f1_2 + 2 * f[0] * f[1] + 3 * f2_2 + (f[0] + 2 * f[1]) * f[2] + f3_2);
-            double p3 = (f1_2 + f[0] * f[1] + f2_2 + 2 * (f[0] + f[1]) * f[2] + 3 * f3_2);
-            double con = djac * one_30 * c * (p1 * h[0] + p2 * h[1] + p3 * h[2]);
-            if (pass == 0) for (int i = 0; i < 3; i++) rx[i] += con * gp[i].x;
-            else for (int i = 0; i < 3; i++) ry[i] += con * gp[i].y;
+        double cuu, cvv;
+        if (flux) {
+            cuu = flux[0];
+            cvv = flux[1];
+        } else {
+            double p[3];
+            flux_ff(uu, p);
+            cuu = flux_ffh(p, h, djac, c);
+            flux_ff(vv, p);
+            cvv = flux_ffh(p, h, djac, c);
         }
+        for (int i = 0; i < 3; i++) rx[i] += cuu * gp[i].x;
+        for (int i = 0; i < 3; i++) ry[i] += cvv * gp[i].y;
         for (int i = 0; i < 3; i++) {
             rhs[i].c_eq += rc[i];
             rhs[i].x_eq += rx[i];
@@ -454,14 +474,23 @@ HD double wd_factor(const v3 *x, const double *h, double djac) {
 }
 
 // fe_sw2_wd_average (src/fe/sw2/fe_sw2_wet_dry_integrations.c:42-61)
-template <bool WET = false>
-HDF void wd_average(const v3 *x, const double *depth, const v2 *v_wd, double djac, double *f_avg, v2 *v_avg) {
+// inv: RN(1 / djac) where the caller has it and the triangle is fully wet (wet_area
+// is djac then), so that the quotients take two FMAs each; 0 otherwise.
+template <bool WET = false, bool INV = false>
+HDF void wd_average(const v3 *x, const double *depth, const v2 *v_wd, double djac, double *f_avg, v2 *v_avg,
+                    double inv = 0.0) {
     d3 av[3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
     double factor = wd_wrapper<WD_INTEGRATE_F, false, true, true, false, WET>(av, x, depth, nullptr, v2{0., 0.}, v_wd, depth,
                                                                         djac, 1., 1.);
     *f_avg = 0.;
     v_avg->x = 0.;
     v_avg->y = 0.;
+    if constexpr (WET && INV) {
+        *f_avg = div_rn(av[0].c_eq, djac, inv);
+        v_avg->x = div_rn(av[0].x_eq, djac, inv);
+        v_avg->y = div_rn(av[0].y_eq, djac, inv);
+        return;
+    }
     if (factor > 0.0) {
         double wet_area = djac * factor;
         *f_avg = av[0].c_eq / wet_area;
@@ -563,13 +592,34 @@ HD void elem_old_terms(const ElemData &D, int ie, double *pre) {
 // Where body_resid reads one triangle's inputs: the model arrays themselves
 // (GlobalSrc), or a copy a kernel has staged in LDS (sw2_kernels.hip).  Node
 // fields are addressed by the triangle's local node 0..2.
+//
+// A source that evaluates one triangle many times may also carry terms of its
+// unperturbed state (has_base: Base, formed once by base_terms with the
+// operations body_resid_src performs to reach them); body_resid_src takes those
+// that a perturbation leaves as they are.
+struct Base {
+    double rough;      // drag coefficient
+    double speed[3];   // |velocity| at the nodes
+    double tau_le;     // SUPG: tau_pg sqrt(area * old wet/dry factor)
+    double inv_djac;   // RN(1 / djac)
+    double puu[3], pvv[3];   // momentum flux u u h, v v h: the factors of h_0, h_1, h_2 ...
+    double cuu, cvv;         // ... and the integrals (fully wet triangles)
+};
+constexpr int NBASE = sizeof(Base) / sizeof(double);
+// constant eddy viscosity of a material: 0 streamwise, 1 transverse
+HDF double evs_viscosity(const ElemData &D, int imat, int k) {
+    double exx = D.mat_ev[3 * imat], eyy = D.mat_ev[3 * imat + 1];
+    exx += D.visc;
+    eyy += D.visc;
+    return k == 0 ? fabs(exx - eyy) : dmin(exx, eyy);
+}
 struct GlobalSrc {
-    static constexpr bool has_rough0 = false;   // see body_resid_src's friction coefficient
+    static constexpr bool has_base = false;
     const ElemData &D;
     const int *nd;
     int ie;
     const double *pre_;
-    HDM double rough0() const { return 0.0; }
+    HDM double base(int) const { return 0.0; }
     HDM double x(int i) const { return D.x[nd[i]]; }
     HDM double y(int i) const { return D.y[nd[i]]; }
     HDM double z(int i) const { return D.z[nd[i]]; }
@@ -577,6 +627,7 @@ struct GlobalSrc {
     HDM double u(int i) const { return D.u[nd[i]]; }
     HDM double v(int i) const { return D.v[nd[i]]; }
     HDM int node_bc(int i) const { return D.node_bc[nd[i]]; }
+    HDM bool any_bc() const { return true; }
     HDM double grad(int k) const { return D.grad[6 * ie + k]; }
     HDM double djac() const { return D.djac[ie]; }
     HDM int mat() const { return D.mat[ie]; }
@@ -585,10 +636,15 @@ struct GlobalSrc {
     HDM int src_flag() const { return D.src_flag[ie]; }
     HDM double src() const { return D.src[ie]; }
     HDM double pre(int k) const { return pre_[k]; }
+    HDM double dt() const { return elem_dt(D, ie); }
+    HDM int turb() const { return D.mat_turb[D.mat[ie]]; }
+    HDM double cor() const { return D.mat_cor[D.mat[ie]]; }
+    HDM double ev(int k) const { return evs_viscosity(D, D.mat[ie], k); }
 };
 
-template <bool WET = false, typename SRC>
-HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int pnode, int pvar, int psign,
+constexpr int PV_ARG = -2;
+template <bool WET = false, int PV = PV_ARG, typename SRC>
+HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int pnode, int pvar_arg, int psign,
                        bool dry_rule, d3 *elem_rhs, const int *nd);
 
 template <bool WET = false>
@@ -600,11 +656,9 @@ HD void body_resid(const ElemData &D, const double *pre, int ie, double pert, in
     body_resid_src<WET>(D, GlobalSrc{D, nd, ie, pre}, ie, pert, pnode, pvar, psign, dry_rule, elem_rhs, nd);
 }
 
-// The drag coefficient of the triangle at its unperturbed state, by the
-// operations body_resid_src performs to reach it (node coordinates and
-// depths, wd_average's depth average, the SMALL floor, drag_coef).
+// The triangle's terms at its unperturbed state.
 template <bool WET, typename SRC>
-HD double unperturbed_roughness(const ElemData &D, const SRC &S) {
+HD Base base_terms(const ElemData &D, const SRC &S) {
     v3 nds[3];
     double h[3];
     v2 vel[3];
@@ -614,26 +668,41 @@ HD double unperturbed_roughness(const ElemData &D, const SRC &S) {
         h[i] = S.head(i);
         vel[i].x = S.u(i); vel[i].y = S.v(i);
     }
+    Base b;
+    const double djac = S.djac(), ks = S.ks();
+    b.inv_djac = 1.0 / djac;
     double h_wd = int_tri_f(1., 1., h);
     v2 vwd;
-    wd_average<WET>(nds, h, vel, S.djac(), &h_wd, &vwd);
-    const double ks = S.ks();
-    return ks > SMALL ? drag_coef(dmax(h_wd, SMALL), ks, D.logt) : 0.0;
+    wd_average<WET>(nds, h, vel, djac, &h_wd, &vwd);
+    b.rough = ks > SMALL ? drag_coef(dmax(h_wd, SMALL), ks, D.logt) : 0.0;
+    for (int i = 0; i < 3; i++) b.speed[i] = sqrt(vel[i].x * vel[i].x + vel[i].y * vel[i].y);
+    b.tau_le = D.tau_pg * sqrt(djac * S.pre(18));
+    const double uu[3] = {vel[0].x, vel[1].x, vel[2].x}, vv[3] = {vel[0].y, vel[1].y, vel[2].y};
+    const double c = -1 * S.dt();
+    flux_ff(uu, b.puu);
+    flux_ff(vv, b.pvv);
+    b.cuu = flux_ffh(b.puu, h, djac, c);
+    b.cvv = flux_ffh(b.pvv, h, djac, c);
+    return b;
 }
+// index of a Base member among its doubles
+enum : int { B_ROUGH = 0, B_SPEED = 1, B_TAULE = 4, B_INVDJ = 5, B_PUU = 6, B_PVV = 9, B_CUU = 12, B_CVV = 13 };
 
 // The body residual with its inputs read through S (GlobalSrc or a staged
-// copy); nd is only used by the dry-node rule and the winds.
-template <bool WET, typename SRC>
-HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int pnode, int pvar, int psign,
+// copy); nd is only used by the dry-node rule and the winds.  PV: the perturbed
+// variable where the caller knows it at compile time (else the argument): the
+// code for the others, and the jumps around it, then go.
+template <bool WET, int PV, typename SRC>
+HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int pnode, int pvar_arg, int psign,
                        bool dry_rule, d3 *elem_rhs, const int *nd) {
+    const int pvar = PV == PV_ARG ? pvar_arg : PV;
     int PRESSURE_FLAG = 1;
     v2 gs[3];
     for (int i = 0; i < 3; i++) {
         gs[i].x = S.grad(2 * i);
         gs[i].y = S.grad(2 * i + 1);
     }
-    const double alpha = D.alpha, dt = elem_dt(D, ie), djac = S.djac(), g = D.g, dll = D.dll, dul = D.dul;
-    const int imat = S.mat();
+    const double alpha = D.alpha, dt = S.dt(), djac = S.djac(), g = D.g, dll = D.dll, dul = D.dul;
     const int wd_flag = S.wd_flag();
     double t1;
 
@@ -653,10 +722,17 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
     if (pvar == PERTURB_U || pvar == PERTURB_V) PRESSURE_FLAG = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        if (i != pnode) continue;
-        if (pvar == PERTURB_H) h[i] += psign * pert;
-        else if (pvar == PERTURB_U) vel[i].x += psign * pert;
-        else if (pvar == PERTURB_V) vel[i].y += psign * pert;
+        if constexpr (PV == PV_ARG) {
+            if (i != pnode) continue;
+            if (pvar == PERTURB_H) h[i] += psign * pert;
+            else if (pvar == PERTURB_U) vel[i].x += psign * pert;
+            else if (pvar == PERTURB_V) vel[i].y += psign * pert;
+        } else {   // selects, not jumps
+            const bool p = i == pnode;
+            if (PV == PERTURB_H) { const double t = h[i] + psign * pert; h[i] = p ? t : h[i]; }
+            else if (PV == PERTURB_U) { const double t = vel[i].x + psign * pert; vel[i].x = p ? t : vel[i].x; }
+            else if (PV == PERTURB_V) { const double t = vel[i].y + psign * pert; vel[i].y = p ? t : vel[i].y; }
+        }
     }
     // baroclinic density and lid pressures are zero for the supported decks
     const double elem_density[3] = {0., 0., 0.};
@@ -678,43 +754,38 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
     }
     ggw.x = ggz.x + ggh.x;
     ggw.y = ggz.y + ggh.y;
-    const double vmag = sqrt(elem_u_avg * elem_u_avg + elem_v_avg * elem_v_avg);
-    const double vst_i = elem_u_avg / dmax(vmag, 1.E-8);
-    const double vst_j = elem_v_avg / dmax(vmag, 1.E-8);
-
     double factor;
     const double factor_old = S.pre(18);
     double h_wd = elem_h_avg;
     v2 vwd;
-    wd_average<WET>(nds, h, vel, djac, &h_wd, &vwd);
+    if constexpr (WET && SRC::has_base) wd_average<WET, true>(nds, h, vel, djac, &h_wd, &vwd, S.base(B_INVDJ));
+    else wd_average<WET>(nds, h, vel, djac, &h_wd, &vwd);
     factor = wd_factor<WET>(nds, h, djac);
     const double vwd_mag = sqrt(vwd.x * vwd.x + vwd.y * vwd.y);
 
     const double h_fric = dmax(h_wd, SMALL);
     const double ks = S.ks();
+    const bool pert_vel = pvar == PERTURB_U || pvar == PERTURB_V;
     // h_wd depends on the depths alone (wd_average's f_avg), so under a u or v
-    // perturbation the drag coefficient is the unperturbed triangle's; a source
-    // that carries it (computed once per triangle by unperturbed_roughness, the
-    // same operations on the same inputs) saves its log for those columns
+    // perturbation the drag coefficient, whose log is the most expensive single
+    // piece here, is the unperturbed triangle's
     double roughness;
-    if constexpr (SRC::has_rough0) {
-        if (pvar == PERTURB_U || pvar == PERTURB_V) roughness = S.rough0();
+    if constexpr (SRC::has_base) {
+        if (pert_vel) roughness = S.base(B_ROUGH);
         else roughness = ks > SMALL ? drag_coef(h_fric, ks, D.logt) : 0.0;
     } else {
         roughness = ks > SMALL ? drag_coef(h_fric, ks, D.logt) : 0.0;
     }
 
     double ev_st = 0., ev_tr = 0.;
-    const int turb = D.mat_turb[imat];
+    const int turb = S.turb();
     if (turb == TURB_EVS) {
-        double exx = D.mat_ev[3 * imat], eyy = D.mat_ev[3 * imat + 1];
-        exx += D.visc;
-        eyy += D.visc;
-        ev_st = fabs(exx - eyy);
-        ev_tr = dmin(exx, eyy);
+        ev_st = S.ev(0);
+        ev_tr = S.ev(1);
     } else if (turb == TURB_EEV) {  // fe_sw2_get_EEVF (src/fe/sw2/fe_sw2_get_EEVF.c:33-60)
-        int mode = D.mat_eev_mode[imat];
-        double coef = D.mat_eev_coef[imat];
+        const double vmag = sqrt(elem_u_avg * elem_u_avg + elem_v_avg * elem_v_avg);
+        int mode = D.mat_eev_mode[S.mat()];
+        double coef = D.mat_eev_coef[S.mat()];
         double ev_min = 0., vmin = 0.1 * sqrt(g * dll);
         if (mode == 1) {
             ev_st = 0.0;
@@ -765,7 +836,27 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
 
     // advection :434-461
     for (int i = 0; i < 3; i++) { rhs[i].x_eq = 0.; rhs[i].y_eq = 0.; rhs[i].c_eq = 0.; }
-    wd_wrapper<WD_CONVECTION, true, true, false, true, WET>(rhs, nds, h, gs, v2{0., 0.}, vel, nullptr, djac, dt, -1);
+    if constexpr (WET && SRC::has_base) {
+        // a u perturbation leaves the v v h integral, a v one the u u h integral, and
+        // a depth perturbation both integrals' factors
+        double flux[2], p[3];
+        const double c = -1 * dt;
+        if (pvar == PERTURB_V) flux[0] = S.base(B_CUU);
+        else {
+            if (pvar == PERTURB_H) for (int i = 0; i < 3; i++) p[i] = S.base(B_PUU + i);
+            else flux_ff(eu, p);
+            flux[0] = flux_ffh(p, h, djac, c);
+        }
+        if (pvar == PERTURB_U) flux[1] = S.base(B_CVV);
+        else {
+            if (pvar == PERTURB_H) for (int i = 0; i < 3; i++) p[i] = S.base(B_PVV + i);
+            else flux_ff(ev, p);
+            flux[1] = flux_ffh(p, h, djac, c);
+        }
+        wd_apply<WD_CONVECTION>(nds, h, gs, v2{0., 0.}, vel, nullptr, djac, dt, -1, rhs, flux);
+    } else {
+        wd_wrapper<WD_CONVECTION, true, true, false, true, WET>(rhs, nds, h, gs, v2{0., 0.}, vel, nullptr, djac, dt, -1);
+    }
     for (int i = 0; i < 3; i++) {
         elem_rhs[i].c_eq += rhs[i].c_eq;
         elem_rhs[i].x_eq += rhs[i].x_eq;
@@ -790,10 +881,21 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
         if (h_wd < dul) temp = dul;
         for (int i = 0; i < 3; i++) { rxq[i] = 0.; ryq[i] = 0.; }
         v2 dfx, dfy;
-        dfx.x = 2. * ev_st * vst_i * (vst_i * ggu.x + vst_j * ggu.y) + 2. * ev_tr * ggu.x;
-        dfx.y = ev_st * vst_j * (vst_j * ggu.y + vst_i * ggu.x + vst_i * ggv.x + vst_j * ggv.y) + ev_tr * (ggu.y + ggv.x);
-        dfy.x = ev_st * vst_i * (vst_j * ggu.y + vst_i * ggu.x + vst_i * ggv.x + vst_j * ggv.y) + ev_tr * (ggu.y + ggv.x);
-        dfy.y = 2. * ev_st * vst_j * (vst_j * ggv.y + vst_i * ggv.x) + 2. * ev_tr * ggv.y;
+        if (ev_st != 0.) {
+            const double vmag = sqrt(elem_u_avg * elem_u_avg + elem_v_avg * elem_v_avg);
+            const double vst_i = elem_u_avg / dmax(vmag, 1.E-8);
+            const double vst_j = elem_v_avg / dmax(vmag, 1.E-8);
+            dfx.x = 2. * ev_st * vst_i * (vst_i * ggu.x + vst_j * ggu.y) + 2. * ev_tr * ggu.x;
+            dfx.y = ev_st * vst_j * (vst_j * ggu.y + vst_i * ggu.x + vst_i * ggv.x + vst_j * ggv.y) + ev_tr * (ggu.y + ggv.x);
+            dfy.x = ev_st * vst_i * (vst_j * ggu.y + vst_i * ggu.x + vst_i * ggv.x + vst_j * ggv.y) + ev_tr * (ggu.y + ggv.x);
+            dfy.y = 2. * ev_st * vst_j * (vst_j * ggv.y + vst_i * ggv.x) + 2. * ev_tr * ggv.y;
+        } else {
+            // the streamwise terms are zeros, and the sign of a zero is lost in the
+            // integrals' sums, which start from +0: bit for bit the sums above
+            dfx.x = 2. * ev_tr * ggu.x;
+            dfx.y = dfy.x = ev_tr * (ggu.y + ggv.x);
+            dfy.y = 2. * ev_tr * ggv.y;
+        }
         int_tri_gradPhi_dot_vbar(gs, djac, temp, dfx, rxq);
         int_tri_gradPhi_dot_vbar(gs, djac, temp, dfy, ryq);
         t1 = dt * factor;
@@ -806,11 +908,22 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
     // friction :557-594
     const double resistance = roughness / (2.0 * g);
     {
-        double fx[3], fy[3];
+        double fx[3], fy[3], sp[3];
+        if constexpr (SRC::has_base) {   // the perturbed node's speed alone is new
+            for (int i = 0; i < 3; i++) sp[i] = S.base(B_SPEED + i);
+            if (pert_vel) {   // from the source by index: indexing vel would put it in scratch memory
+                v2 q = {S.u(pnode), S.v(pnode)};
+                if (pvar == PERTURB_U) q.x += psign * pert;
+                else q.y += psign * pert;
+                const double sq = sqrt(q.x * q.x + q.y * q.y);
+                for (int i = 0; i < 3; i++) sp[i] = i == pnode ? sq : sp[i];
+            }
+        } else {
+            for (int i = 0; i < 3; i++) sp[i] = sqrt(vel[i].x * vel[i].x + vel[i].y * vel[i].y);
+        }
         for (int i = 0; i < 3; i++) {
-            t1 = sqrt(vel[i].x * vel[i].x + vel[i].y * vel[i].y);
-            fx[i] = vel[i].x * t1;
-            fy[i] = vel[i].y * t1;
+            fx[i] = vel[i].x * sp[i];
+            fy[i] = vel[i].y * sp[i];
         }
         for (int i = 0; i < 3; i++) { rxq[i] = 0.; ryq[i] = 0.; }
         t1 = dt * g * resistance * factor;
@@ -825,9 +938,10 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
     bed_stress.x = resistance * vwd.x * vwd_mag;
     bed_stress.y = resistance * vwd.y * vwd_mag;
 
-    // coriolis :639-652
-    const double cor = D.mat_cor[imat];
-    {
+    // coriolis :639-652; without it the terms are zeros, and a sum that began at
+    // +0 is never -0, so leaving them out changes no bit
+    const double cor = S.cor();
+    if (cor != 0.) {
         for (int i = 0; i < 3; i++) { rxq[i] = 0.; ryq[i] = 0.; }
         t1 = dt * factor * cor;
         int_tri_phi_f_g(djac, -t1, h, ev, rxq);
@@ -855,7 +969,7 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
             wind_stress.x += shear_x;
             wind_stress.y += shear_y;
         }
-        const double watt = D.mat_windatt[imat];
+        const double watt = D.mat_windatt[S.mat()];
         wind_stress.x *= (watt * watt) / (3 * D.density);
         wind_stress.y *= (watt * watt) / (3 * D.density);
         total_stress.x = wind_stress.x + 0.0;   // + wave stress
@@ -911,18 +1025,29 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
         const double denom = dmax(h_wd, NOT_QUITE_SMALL);
         double tau;
         {   // fe_get_supg_tau_sw (src/fe/fe_get_supg_tau.c:43-80), le = sqrt(area*factor_old) (:289)
-            double le = sqrt(area * factor_old);
             double cs2 = g_factor * denom;
             if (denom <= 0.0) cs2 = 0.;
             double sr = sqrt(vwd.x * vwd.x + vwd.y * vwd.y + cs2 + SMALL);
-            tau = D.tau_pg * le / sr;
+            if constexpr (SRC::has_base) tau = S.base(B_TAULE) / sr;
+            else tau = D.tau_pg * sqrt(area * factor_old) / sr;
         }
         d3 dfdt[3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
         d3 adv[3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
         double dudt = S.pre(19), dvdt = S.pre(20), dhdt = S.pre(21);   // -(old-state integrals), :1012-1013
         factor = wd_wrapper<WD_INTEGRATE_F, false, true, true, false, WET>(dfdt, nds, h, nullptr, v2{0., 0.}, vel, h, djac, 1, 1);
         dudt += dfdt[0].x_eq; dvdt += dfdt[0].y_eq; dhdt += dfdt[0].c_eq;
-        factor = wd_wrapper<WD_GLS_CONVECTION, true, true, true, false, WET>(adv, nds, h, gs, v2{0., 0.}, vel, h, djac, dt, 1);
+        if constexpr (WET) {
+            // WD_GLS_CONVECTION (:361-381) with the gradients formed above (they differ
+            // from its own at most in the sign of a zero, which the sums lose)
+            const double h_avg = one_3 * (h[0] + h[1] + h[2]);
+            const double u_avg = one_3 * (vel[0].x + vel[1].x + vel[2].x);
+            const double v_avg = one_3 * (vel[0].y + vel[1].y + vel[2].y);
+            adv[0].c_eq += djac * dt * (u_avg * ggh.x + h_avg * ggu.x + v_avg * ggh.y + h_avg * ggv.y);
+            adv[0].x_eq += djac * dt * (u_avg * ggu.x + v_avg * ggu.y);
+            adv[0].y_eq += djac * dt * (u_avg * ggv.x + v_avg * ggv.y);
+        } else {
+            factor = wd_wrapper<WD_GLS_CONVECTION, true, true, true, false, WET>(adv, nds, h, gs, v2{0., 0.}, vel, h, djac, dt, 1);
+        }
         double x_pressure = g_factor * (ggh.x + ggz.x) * dt * factor + ggp.x * dt * factor;
         double y_pressure = g_factor * (ggh.y + ggz.y) * dt * factor + ggp.y * dt * factor;
         double x_friction = g * bed_stress.x * dt * factor;
@@ -930,8 +1055,10 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
         double x_coriolis = -vwd.y * cor;
         double y_coriolis = vwd.x * cor;
         double c_eq = dhdt + adv[0].c_eq + factor * src * djac * dt;
-        double x_eq = dudt + adv[0].x_eq + (x_pressure + x_friction / denom) * djac + (x_coriolis - total_stress.x / denom) * djac * factor * dt;
-        double y_eq = dvdt + adv[0].y_eq + (y_pressure + y_friction / denom) * djac + (y_coriolis - total_stress.y / denom) * djac * factor * dt;
+        // no winds: 0 / denom
+        const double sx = D.wind ? total_stress.x / denom : 0., sy = D.wind ? total_stress.y / denom : 0.;
+        double x_eq = dudt + adv[0].x_eq + (x_pressure + x_friction / denom) * djac + (x_coriolis - sx) * djac * factor * dt;
+        double y_eq = dvdt + adv[0].y_eq + (y_pressure + y_friction / denom) * djac + (y_coriolis - sy) * djac * factor * dt;
         for (int i = 0; i < 3; i++) {
             rcq[i] = (gs[i].x * (tau * vwd.x * c_eq + tau * h_wd * x_eq) + gs[i].y * (tau * vwd.y * c_eq + tau * h_wd * y_eq));
             rxq[i] = (gs[i].x * (tau * g_factor * h_wd * c_eq + tau * vwd.x * h_wd * x_eq) + gs[i].y * (tau * vwd.y * h_wd * x_eq));
@@ -945,6 +1072,7 @@ HD void body_resid_src(const ElemData &D, const SRC &S, int ie, double pert, int
     }
 
     // Dirichlet :1239-1256
+    if (!S.any_bc()) return;
     for (int i = 0; i < 3; i++) {
         int bc = S.node_bc(i);
         if (bc == BCT_PRS_DIR) {
@@ -1107,8 +1235,9 @@ HD void jac_column(const ElemData &D, int ie, int j, int var, double *col) {
 // applied to one column (node j, var) of the element matrix.  The reference
 // reads the node string with the LOCAL index i (fe_sw2_load.c:103, :165), so
 // the node-string flags come from nodes 0..NN-1 of the mesh; `loc_bc` holds them.
+// dry: old depth <= 0 at the element's nodes.
 template <int NN>
-HDF void jac_column_db(const ElemData &D, const int *nodes, const int *loc_bc, int j, int var, double *col) {
+HDF void jac_column_db(const bool *dry, const int *loc_bc, int j, int var, double *col) {
 #pragma unroll
     for (int k = 0; k < NN; k++) {
         // mom: zero rows k (x,y) in all columns, zero columns (k,u),(k,v), unit diagonal
@@ -1132,12 +1261,19 @@ HDF void jac_column_db(const ElemData &D, const int *nodes, const int *loc_bc, i
             }
         };
         // the reference's order of edits for local node k
-        if (D.old_head[nodes[k]] <= 0.) mom();
+        if (dry[k]) mom();
         const int nb = loc_bc[k];
         if (nb == BCT_PRS_DIR) dacont();
         else if (nb == BCT_VEL_DIR) mom();
         else if (nb == BCT_VEL_PRS_DIR) { dacont(); mom(); }
     }
+}
+
+template <int NN>
+HDF void jac_column_db(const ElemData &D, const int *nodes, const int *loc_bc, int j, int var, double *col) {
+    bool dry[NN];
+    for (int k = 0; k < NN; k++) dry[k] = D.old_head[nodes[k]] <= 0.;
+    jac_column_db<NN>(dry, loc_bc, j, var, col);
 }
 
 }  // namespace sw2

@@ -12,6 +12,7 @@
 // fe_assemble_matrix.c:166-224) -- so sums are bit-identical to it without
 // atomics.
 #include <algorithm>
+#include <type_traits>
 
 #include "sw2_ctx.h"
 
@@ -266,51 +267,72 @@ __global__ void __launch_bounds__(BS) k_jac2d_cols(ElemData D, const int *list, 
     }
 }
 
-// The column-uniform layout with every triangle's inputs staged in LDS
-// first.  Each wave copies the inputs of its 32 triangles -- node
-// coordinates, depths and velocities, P1 gradients, the 24 old-state terms,
-// djac, roughness, rain, material, wet/dry flag and the nodes' boundary flags
-// -- with 29 loads per lane issued back to back (lanes l and l + 32 share a
-// triangle and take alternate fields), waits once, and then evaluates the
-// residuals reading those inputs from LDS.  In the global-memory layouts
-// many of these loads sit deep in the element code, each waited for on its
-// own; here they cost one round trip per triangle group.  Same arithmetic,
-// same results.
-constexpr int LREC = 58;   // doubles per staged triangle (integers held as exact doubles)
-enum : int { LR_NODE = 0, LR_GRAD = 18, LR_PRE = 24, LR_DJAC = 48, LR_KS = 49, LR_SRC = 50, LR_MAT = 51,
-             LR_WD = 52, LR_SRCF = 53, LR_NBC = 54, LR_ROUGH0 = 57 };
+// The column-uniform layout with every triangle's inputs staged in LDS first.
+// Each wave copies the inputs of its 32 triangles (lanes l and l + 32 share a
+// triangle and take alternate fields) with loads issued back to back, waits
+// once, and then evaluates the residuals reading those inputs from LDS.  Same
+// arithmetic, same results as the global-memory layouts.
+//
+// Everything a column reads is in the record, down to the positions its
+// entries go to, the Dirichlet edits' flags and the material's constants: a
+// load in the column loop would queue behind the previous columns' stores (the
+// memory counter retires in order) and cost a round trip of the store to
+// memory per column.  Jumps cost next (a taken one refetches): the perturbed
+// variable is a template argument, the perturbed node a select, and the
+// Dirichlet edits are behind one test of the record's flags.  Terms that a
+// perturbation leaves as they are come from the record (Base).  At 1M triangles,
+// refined / FP64 form: 747 / 806 us (1,086 / 1,174 before), 305M of 374M VALU
+// instructions; what is left is latency at two waves per SIMD (254 registers;
+// at 168, three waves, the code spills and is slower).
+//
+// LREC doubles per triangle, odd so that 32 records' fields lie in distinct banks.
+enum : int { LR_NODE = 0, LR_GRAD = 18, LR_PRE = 24, LR_DJAC = 46, LR_KS = 47, LR_SRC = 48, LR_DT = 49, LR_COR = 50,
+             LR_EV = 51, LR_META = 53, LR_BLK = 54, LR_BASE = 59, LREC = LR_BASE + NBASE };
+static_assert(LREC % 2 == 1, "an even record length would put a field of two triangles in one bank");
+// LR_META: the material, then these bits (two-bit fields by bc_code; the Dirichlet edits' topmost)
+enum : int { MB_WD = 0, MB_SRCF = 2, MB_TURB = 3, MB_NBC = 5, MB_LBC = 11, MB_DRY = 17 };
 
-// R0: the record also carries the unperturbed drag coefficient (LR_ROUGH0),
-// which the residual then uses for u and v perturbations
-template <bool R0>
+// BASE: the record also carries the unperturbed triangle's terms (Base)
+template <bool BASE>
 struct LdsSrcT {
-    static constexpr bool has_rough0 = R0;
+    static constexpr bool has_base = BASE;
     const double *r;   // the triangle's staged record (LDS)
-    __device__ __forceinline__ double rough0() const { return r[LR_ROUGH0]; }
+    int meta;
+    __device__ __forceinline__ double base(int k) const { return r[LR_BASE + k]; }
     __device__ __forceinline__ double x(int i) const { return r[6 * i]; }
     __device__ __forceinline__ double y(int i) const { return r[6 * i + 1]; }
     __device__ __forceinline__ double z(int i) const { return r[6 * i + 2]; }
     __device__ __forceinline__ double head(int i) const { return r[6 * i + 3]; }
     __device__ __forceinline__ double u(int i) const { return r[6 * i + 4]; }
     __device__ __forceinline__ double v(int i) const { return r[6 * i + 5]; }
-    __device__ __forceinline__ int node_bc(int i) const { return (int)r[LR_NBC + i]; }
+    __device__ __forceinline__ int node_bc(int i) const { return code_bc((meta >> (MB_NBC + 2 * i)) & 3); }
+    __device__ __forceinline__ bool any_bc() const { return (meta >> MB_NBC) & 63; }
+    __device__ __forceinline__ bool any_db() const { return meta >> MB_LBC; }   // a Dirichlet edit of the column
+    __device__ __forceinline__ int loc_bc(int i) const { return code_bc((meta >> (MB_LBC + 2 * i)) & 3); }
+    __device__ __forceinline__ bool dry(int i) const { return (meta >> (MB_DRY + i)) & 1; }
     __device__ __forceinline__ double grad(int k) const { return r[LR_GRAD + k]; }
     __device__ __forceinline__ double djac() const { return r[LR_DJAC]; }
-    __device__ __forceinline__ int mat() const { return (int)r[LR_MAT]; }
-    __device__ __forceinline__ int wd_flag() const { return (int)r[LR_WD]; }
+    __device__ __forceinline__ int mat() const { return ((const int *)(r + LR_META))[0]; }
+    __device__ __forceinline__ int wd_flag() const { return (meta >> MB_WD) & 3; }
     __device__ __forceinline__ double ks() const { return r[LR_KS]; }
-    __device__ __forceinline__ int src_flag() const { return (int)r[LR_SRCF]; }
+    __device__ __forceinline__ int src_flag() const { return (meta >> MB_SRCF) & 1; }
     __device__ __forceinline__ double src() const { return r[LR_SRC]; }
     __device__ __forceinline__ double pre(int k) const { return r[LR_PRE + k]; }
+    __device__ __forceinline__ double dt() const { return r[LR_DT]; }
+    __device__ __forceinline__ int turb() const { return (meta >> MB_TURB) & 3; }
+    __device__ __forceinline__ double cor() const { return r[LR_COR]; }
+    __device__ __forceinline__ double ev(int k) const { return r[LR_EV + k]; }
+    __device__ __forceinline__ int blkpos(int k) const { return ((const int *)(r + LR_BLK))[k]; }
 };
-using LdsSrc = LdsSrcT<false>;
 
-// The triangle's 57 inputs into rec: lane half 0 takes one field of each
-// pair, half 1 the other (both fields of a step come from one array where
-// possible, so a step is one load instruction for the whole wave).
-__device__ __forceinline__ void stage_triangle(const ElemData &D, int ie, const int *nd, int half, double *rec) {
-    double val[29];
-    int fld[29];
+// The triangle's inputs into rec: lane half 0 takes one field of each pair,
+// half 1 the other (both fields of a step come from one array where possible,
+// so a step is one load instruction for the whole wave).
+__device__ __forceinline__ void stage_triangle(const ElemData &D, int ie, const int *nd, int half, int b0, int b1,
+                                               int b2, const int *blkpos, double *rec) {
+    constexpr int NF = 25;
+    double val[NF];
+    int fld[NF];
     const int na = half ? nd[1] : nd[0];
     // node fields of nodes 0 and 1
     const double *narr[6] = {D.x, D.y, D.z, D.head, D.u, D.v};
@@ -334,36 +356,54 @@ __device__ __forceinline__ void stage_triangle(const ElemData &D, int ie, const 
     }
     const double *pre = D.pre + PRE_STRIDE * (size_t)ie;
 #pragma unroll
-    for (int m = 0; m < 12; m++) {
+    for (int m = 0; m < 11; m++) {   // pre[22..23] are padding
         val[12 + m] = pre[2 * m + half];
         fld[12 + m] = LR_PRE + 2 * m + half;
     }
-    val[24] = half ? D.ks[ie] : D.djac[ie];
-    fld[24] = half ? LR_KS : LR_DJAC;
-    val[25] = D.src[ie];
-    fld[25] = LR_SRC;   // both halves write the same value
-    val[26] = (double)(half ? D.wd_flag[ie] : D.mat[ie]);
-    fld[26] = half ? LR_WD : LR_MAT;
-    val[27] = (double)(half ? D.node_bc[nd[0]] : D.src_flag[ie]);
-    fld[27] = half ? LR_NBC : LR_SRCF;
-    val[28] = (double)D.node_bc[half ? nd[2] : nd[1]];
-    fld[28] = LR_NBC + 1 + half;
+    val[23] = half ? D.ks[ie] : D.djac[ie];
+    fld[23] = half ? LR_KS : LR_DJAC;
+    val[24] = half ? elem_dt(D, ie) : D.src[ie];
+    fld[24] = half ? LR_DT : LR_SRC;
+    // where the nine blocks go: half 0 five of them, half 1 four
+    int bp[5];
 #pragma unroll
-    for (int k = 0; k < 29; k++) rec[fld[k]] = val[k];
+    for (int k = 0; k < 5; k++) bp[k] = blkpos[9 * (size_t)ie + min(5 * half + k, 8)];
+    // integers
+    const int mat = D.mat[ie];
+    int meta = (D.wd_flag[ie] & 3) << MB_WD | (D.src_flag[ie] ? 1 << MB_SRCF : 0);
+    const int *lbi = D.loc_bc_inst ? D.loc_bc_inst + 3 * D.elem_inst[ie] : nullptr;
+    const int lb[3] = {lbi ? lbi[0] : b0, lbi ? lbi[1] : b1, lbi ? lbi[2] : b2};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        meta |= bc_code(D.node_bc[nd[k]]) << (MB_NBC + 2 * k) | bc_code(lb[k]) << (MB_LBC + 2 * k);
+        meta |= D.old_head[nd[k]] <= 0. ? 1 << (MB_DRY + k) : 0;
+    }
+    meta |= (D.mat_turb[mat] & 3) << MB_TURB;
+#pragma unroll
+    for (int k = 0; k < NF; k++) rec[fld[k]] = val[k];
+#pragma unroll
+    for (int k = 0; k < 5; k++) ((int *)(rec + LR_BLK))[5 * half + k] = bp[k];   // the tenth is padding
+    if (half) {
+        rec[LR_EV] = evs_viscosity(D, mat, 0);
+        rec[LR_EV + 1] = evs_viscosity(D, mat, 1);
+    } else {
+        rec[LR_COR] = D.mat_cor[mat];
+        ((int *)(rec + LR_META))[0] = mat;
+        ((int *)(rec + LR_META))[1] = meta;
+    }
 }
 
 // One Jacobian column (node j, variable var) of the staged triangle: the
 // +eps residual on lanes 0-31, the -eps one on lanes 32-63, the difference
 // quotient, the Dirichlet edits, and the stores of the +eps lanes.
-template <bool WET, typename SRC>
+template <bool WET, int VAR, typename SRC>
 __device__ __forceinline__ void lds_column(const ElemData &DL, const SRC &S, int ie, const int *nodes, int j,
-                                           int var, bool minus, bool act, int b0, int b1, int b2,
-                                           const int *blkpos, double *EM, float *EM32) {
+                                           bool minus, bool act, double *EM, float *EM32) {
+    constexpr int var = VAR, PV = VAR == 0 ? PERTURB_U : (VAR == 1 ? PERTURB_V : PERTURB_H);
     const double val = var == 0 ? S.u(j) : (var == 1 ? S.v(j) : S.head(j));
     const double eps = num_diff_eps(val), eps2 = 2.0 * eps;
-    const int pv = var == 0 ? PERTURB_U : (var == 1 ? PERTURB_V : PERTURB_H);
     d3 r[3];
-    body_resid_src<WET>(DL, S, ie, eps, j, pv, minus ? -1 : +1, false, r, nodes);
+    body_resid_src<WET, PV>(DL, S, ie, minus ? -eps : eps, j, PV, 1, false, r, nodes);
     double col[9];
     const double inv = 1.0 / eps2;
 #pragma unroll
@@ -375,12 +415,14 @@ __device__ __forceinline__ void lds_column(const ElemData &DL, const SRC &S, int
         col[3 * i + 2] = div_rn(r[i].c_eq - mc, eps2, inv);
     }
     if (minus || !act) return;
-    const int *lbi = DL.loc_bc_inst ? DL.loc_bc_inst + 3 * DL.elem_inst[ie] : nullptr;
-    const int lb[3] = {lbi ? lbi[0] : b0, lbi ? lbi[1] : b1, lbi ? lbi[2] : b2};
-    jac_column_db<3>(DL, nodes, lb, j, var, col);
+    if (S.any_db()) {
+        const bool dry[3] = {S.dry(0), S.dry(1), S.dry(2)};
+        const int lb[3] = {S.loc_bc(0), S.loc_bc(1), S.loc_bc(2)};
+        jac_column_db<3>(dry, lb, j, var, col);
+    }
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const size_t o = 9 * (size_t)blkpos[9 * ie + 3 * i + j];
+        const size_t o = 9 * (size_t)S.blkpos(3 * i + j);
 #pragma unroll
         for (int rr = 0; rr < 3; rr++) {
             if (EM32) EM32[o + 3 * rr + var] = (float)col[3 * i + rr];
@@ -389,24 +431,21 @@ __device__ __forceinline__ void lds_column(const ElemData &DL, const SRC &S, int
     }
 }
 
-// GROUP = false: wave w takes column w % 9 of group w / 9 (as the
-// column-uniform layout) and stages its group's inputs for that one column.
-// GROUP = true: wave w takes all nine columns of group w, one after the
-// other, from one staging of the group's inputs; the nine column stores of a
-// triangle then come from one wave, so its element blocks are completed in
-// one L2 rather than in partial lines from several XCDs.
-template <bool WET, int BS, bool GROUP>
+// A wave takes COLS of a 32-triangle group's nine columns from one staging:
+// all nine, one node's three, or one (unit w: group w / (9 / COLS), part w
+// mod that).  With more than one column the terms of the unperturbed triangles
+// (Base) are formed once after the staging.
+template <bool WET, int BS, int COLS>
 __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list, const int *count, int b0, int b1,
                                                   int b2, const int *blkpos, double *EM, float *EM32) {
-    constexpr int WPB = BS / 64;
+    constexpr int WPB = BS / 64, PARTS = 9 / COLS;
     __shared__ double srec[WPB][32][LREC];
     __shared__ crlog::tables slog;
     const int n = *count;
-    const int ngroups = (n + 31) >> 5;
-    const int nunits = GROUP ? ngroups : 9 * ngroups;
+    const int nunits = PARTS * ((n + 31) >> 5);
     if ((int)blockIdx.x * WPB >= nunits) return;   // the whole block has no unit (uniform exit)
-    // the friction law's log table (4 KB) copied to LDS: its lookup is the
-    // one data-dependent load of the element code
+    // the friction law's log table copied to LDS: its lookup is the one
+    // data-dependent load of the element code
     {
         const double *src = (const double *)D.logt;
         double *dst = (double *)&slog;
@@ -423,7 +462,7 @@ __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list
     // software pipeline: the triangle id two units ahead and its node ids one
     // unit ahead are loaded while the current unit is computed
     auto tri_of = [&](int w) {
-        const int g = GROUP ? w : w / 9, l = g * 32 + (lane & 31);
+        const int g = w / PARTS, l = g * 32 + (lane & 31);
         return list[l < n ? l : g * 32];
     };
     int w = blockIdx.x * WPB + wib;
@@ -433,8 +472,7 @@ __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list
     if (w < nunits)
         for (int k = 0; k < 3; k++) nd_a[k] = D.e2d[3 * ie_a + k];
     for (; w < nunits; w += wstride) {
-        const int grp = GROUP ? w : w / 9;
-        const int li = grp * 32 + (lane & 31);
+        const int li = (w / PARTS) * 32 + (lane & 31);
         const bool act = li < n;   // idle lanes of a last group recompute its first triangle, store nothing
         const int ie = ie_a;
         const int nodes[3] = {nd_a[0], nd_a[1], nd_a[2]};
@@ -445,29 +483,39 @@ __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list
         // the previous group's reads are done before the records are rewritten
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        stage_triangle(D, ie, nodes, minus ? 1 : 0, rec);
+        stage_triangle(D, ie, nodes, minus ? 1 : 0, b0, b1, b2, blkpos, rec);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if constexpr (GROUP) {
-            // the unperturbed drag coefficient, once for the six u and v columns
-            const double rough0 = unperturbed_roughness<WET>(DL, LdsSrc{rec});
-            if (!minus) rec[LR_ROUGH0] = rough0;
+        if constexpr (COLS > 1) {
+            const LdsSrcT<false> S0{rec, ((const int *)(rec + LR_META))[1]};
+            const Base base = base_terms<WET>(DL, S0);
+            if (!minus) {
+#pragma unroll
+                for (int k = 0; k < NBASE; k++) rec[LR_BASE + k] = reinterpret_cast<const double *>(&base)[k];
+            }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
         }
-        const LdsSrcT<GROUP> S{rec};
-        if constexpr (GROUP) {
-#pragma unroll 1
-            for (int q = 0; q < 9; q++) {
-                // keeps the record's reads inside the column loop (hoisted
-                // out of it they would hold the whole record in registers)
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                lds_column<WET>(DL, S, ie, nodes, q / 3, q % 3, minus, act, b0, b1, b2, blkpos, EM, EM32);
-            }
+        // keeps the record's reads inside a column (hoisted out of the loop they
+        // would hold the whole record in registers)
+        auto fresh = [&]() {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            return LdsSrcT<(COLS > 1)>{rec, ((const int *)(rec + LR_META))[1]};
+        };
+        const int q0 = (w % PARTS) * COLS;
+        if constexpr (COLS == 1) {
+            const int j = q0 / 3, var = q0 % 3;
+            if (var == 0) lds_column<WET, 0>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
+            else if (var == 1) lds_column<WET, 1>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
+            else lds_column<WET, 2>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
         } else {
-            const int q = w % 9;
-            lds_column<WET>(DL, S, ie, nodes, q / 3, q % 3, minus, act, b0, b1, b2, blkpos, EM, EM32);
+#pragma unroll 1
+            for (int j = q0 / 3; j < (q0 + COLS) / 3; j++) {
+                lds_column<WET, 0>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
+                lds_column<WET, 1>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
+                lds_column<WET, 2>(DL, fresh(), ie, nodes, j, minus, act, EM, EM32);
+            }
         }
     }
 }
@@ -646,23 +694,38 @@ static void launch_split(Ctx *c) {
     c->split_valid = 1;
 }
 
+// Columns a wave of the LDS layout takes of its 32 triangles.  The GPU holds two
+// of its waves on each of 1,024 SIMDs, and a wave's nine columns are one serial
+// chain (63 us at any size that fits): one column a wave while nine waves per
+// group fit at once, one node's three while the groups are fewer than two
+// rounds of waves, else all nine (staging and Base terms formed once).
+// Measured, us for 9 / 3 / 1 columns: 50 groups 61 / 31 / 21, 394 groups 63 /
+// 31 / 35, 1,000 69 / 55 / 69, 2,000 88 / 84 / 112, 4,050 139 / 141 / 198,
+// 31,250 747 / 893 / 1,282.
+constexpr int JAC_WAVES = 2048;
+static int jac_columns(int groups) {
+    if (9 * groups <= JAC_WAVES) return 1;
+    return groups < 2 * JAC_WAVES ? 3 : 9;
+}
+
 // Grid-stride list launches.  Block size and grid size change only the
 // schedule (every triangle's arithmetic and output slot are fixed), so they
 // are free parameters: defaults below, or what adh_sw2_hip_autotune measured.
 template <bool WET, int BS>
 static void jac_list_bs(Ctx *c, const ElemData &D, const int *list, const int *count, int grid, int layout) {
-    if (layout == 2) {   // column-uniform waves, inputs staged in LDS
-        const int units = 9 * ((c->E + 31) / 32);
-        hipLaunchKernelGGL((k_jac2d_lds<WET, BS, false>), dim3(std::min(grid, nblocks_for(units, BS / 64))), dim3(BS),
-                           0, c->stream, D, list, count, c->loc_bc[0], c->loc_bc[1], c->loc_bc[2], c->blkpos, c->EM,
-                           em32_of(c));
-        return;
-    }
-    if (layout == 3) {   // a wave per triangle group, its nine columns from one staging
-        const int units = (c->E + 31) / 32;
-        hipLaunchKernelGGL((k_jac2d_lds<WET, BS, true>), dim3(std::min(grid, nblocks_for(units, BS / 64))), dim3(BS),
-                           0, c->stream, D, list, count, c->loc_bc[0], c->loc_bc[1], c->loc_bc[2], c->blkpos, c->EM,
-                           em32_of(c));
+    if (layout >= 2) {   // column-uniform waves, inputs staged in LDS
+        const int groups = (c->E + 31) / 32;
+        auto launch = [&](auto cols) {
+            constexpr int COLS = decltype(cols)::value;
+            const int units = 9 / COLS * groups;
+            hipLaunchKernelGGL((k_jac2d_lds<WET, BS, COLS>), dim3(std::min(grid, nblocks_for(units, BS / 64))),
+                               dim3(BS), 0, c->stream, D, list, count, c->loc_bc[0], c->loc_bc[1], c->loc_bc[2],
+                               c->blkpos, c->EM, em32_of(c));
+        };
+        const int cols = layout == 2 ? 1 : jac_columns(groups);
+        if (cols == 1) launch(std::integral_constant<int, 1>());
+        else if (cols == 3) launch(std::integral_constant<int, 3>());
+        else launch(std::integral_constant<int, 9>());
         return;
     }
     if (layout == 1) {   // column-uniform waves: 9 waves per 32 triangles
