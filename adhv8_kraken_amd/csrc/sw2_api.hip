@@ -289,6 +289,9 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     c.N = m->nnodes; c.E = m->nelems2d; c.B = m->nelems1d; c.M = m->nmat;
     c.Np = (c.N + 63) & ~63;
     c.kgraph_prec = -1;
+    c.run_cap[0] = c.run_cap[1] = c.run_prec = -1;
+    c.run_max_blocks = nblocks_for(c.N, 256);
+    c.run_limit = 200000;   // 2 ms: a hand-over takes 2 to 5 us when every block is resident
     if (opts) {
         int rc0 = check_opts(opts);
         if (rc0) { delete h; return rc0; }
@@ -514,6 +517,16 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     const size_t nmod = ninst > 0 ? (size_t)ninst : 1;
     UP(ksc, (const KScal *)nullptr, nmod);
     UP(norms, (const Norms *)nullptr, nmod);
+    {
+        const unsigned long long empty = 0xfff8dead0badf00dull;   // Slot<double>::EMPTY of sw2_run.hip
+        // the one-kernel solve's hand-over storage; a single model beyond RUN_BLOCKS never takes it
+        const bool may = ninst > 0 || c.run_max_blocks <= RUN_BLOCKS;
+        std::vector<double> w(may ? run_slot_words(c.run_max_blocks) : 1);
+        for (double &x : w) memcpy(&x, &empty, sizeof x);
+        UP(run_slots, w.data(), w.size());
+        UP(run_xch, (const double *)nullptr, may ? run_vector_words(c.Np) : 1);
+    }
+    UP(run_quit, (const int *)nullptr, 2 * nmod);
     c.red.maxblocks = nblocks_for(N, 256) + 8;
     UP(red.part, (const double *)nullptr, 4 * (size_t)c.red.maxblocks);
     UP(red.count, (const unsigned *)nullptr, 8);
@@ -948,6 +961,25 @@ static void chunk_plan(const Ctx &c, int &first, int &more) {
     more = graphs ? 4 : 2;
 }
 
+// The solve as one kernel where the models fit on the GPU (sw2_run.hip).
+// *done: every model finished; otherwise a hand-over timed out or the system
+// does not take this form, and the caller solves from the prologue.  After a
+// time-out the next solves are left to the other form: what held the CUs
+// (another stream's or program's long kernels) may still do.
+constexpr int RUN_PAUSE = 64;
+static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
+    *done = false;
+    if (c.run_pause > 0) { c.run_pause--; return 0; }
+    if (!launch_krylov_run(&c, zero_guess)) return 0;
+    const int n = c.ninst ? c.ninst : 1;
+    HIPCHK(hipMemcpyAsync(c.h_ksc, c.ksc, sizeof(KScal) * n, hipMemcpyDeviceToHost, c.stream));
+    HIPCHK(hipStreamSynchronize(c.stream));
+    *done = true;
+    for (int i = 0; i < n; i++) *done = *done && c.h_ksc[i].done;
+    if (!*done) { c.run_pause = RUN_PAUSE; c.run_dirty = 1; }
+    return 0;
+}
+
 // zero_guess: sol holds a zero initial guess (the Newton step zeroes it), so
 // the epilogue is idempotent and is queued behind every chunk before the
 // convergence flag is read; otherwise it runs once, after the last chunk.
@@ -969,7 +1001,10 @@ static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
     init.rtol = c.opts.lin_rtol;
     init.max_it = lin_it_cap(c);
     HIPCHK(hipMemcpyAsync(c.ksc, &init, sizeof(KScal), hipMemcpyHostToDevice, c.stream));
-    launch_krylov_prologue(&c);
+    bool done_early = false;
+    int rc0 = krylov_one_kernel(c, zero_guess, &done_early);
+    if (rc0) return rc0;
+    if (!done_early) launch_krylov_prologue(&c);
     // first chunk: the previous solve's iteration count (consecutive Newton
     // systems converge alike), then chunks of 2 (chunk_plan).  The device flag
     // makes iterations launched past convergence return at entry, so the
@@ -979,7 +1014,6 @@ static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
     int left = lin_it_cap(c);
     // with the tiled band LU an iteration is two sweeps of a launch per tile:
     // the flag is read after the prologue and after every iteration instead
-    bool done_early = false;
     if (c.opts.preconditioner == 1 && c.band_tiled) {
         first = more = 1;
         HIPCHK(hipMemcpyAsync(c.h_ksc, c.ksc, sizeof(KScal), hipMemcpyDeviceToHost, c.stream));
@@ -1309,7 +1343,10 @@ static int krylov_batch(Ctx &c, const std::vector<int> &active, std::vector<int>
         init[i].max_it = active[i] ? cap : 0;
     }
     HIPCHK(hipMemcpyAsync(c.ksc, init.data(), sizeof(KScal) * n, hipMemcpyHostToDevice, c.stream));
-    launch_krylov_prologue(&c);
+    bool all_done0 = false;
+    int rc0 = krylov_one_kernel(c, true, &all_done0);
+    if (rc0) return rc0;
+    if (!all_done0) launch_krylov_prologue(&c);
     // chunks as in krylov() with a zero guess (newton_batch zeroes sol): no
     // host check between the prologue and the first chunk, the idempotent
     // epilogue queued behind every chunk before the flags are read
@@ -1319,7 +1356,6 @@ static int krylov_batch(Ctx &c, const std::vector<int> &active, std::vector<int>
     int left = cap;
     // the tiled band LU: flags read after the prologue and every iteration,
     // as krylov() does (a direct solve usually ends at the prologue)
-    bool all_done0 = false;
     if (c.opts.preconditioner == 1 && c.band_tiled) {
         first = more = 1;
         HIPCHK(hipMemcpyAsync(c.h_ksc, c.ksc, sizeof(KScal) * n, hipMemcpyDeviceToHost, c.stream));
@@ -1567,6 +1603,8 @@ extern "C" int adh_sw2_hip_batch_create(const adh_sw2_mesh *meshes, int n, const
         dts[i] = meshes[i].dt;
     }
     inst_blk0[n] = (c.N + 255) / 256;
+    c.run_max_blocks = 0;
+    for (int i = 0; i < n; i++) c.run_max_blocks = std::max(c.run_max_blocks, inst_blk0[i + 1] - inst_blk0[i]);
     auto up = [&](auto **dst, const auto *src, size_t cnt) -> int { return dupload(h, dst, src, cnt); };
     if ((rc = up(&c.blk_inst, blk_inst.data(), blk_inst.size())) || (rc = up(&c.inst_blk0, inst_blk0.data(), n + 1)) ||
         (rc = up(&c.inst_nodes, inst_nodes.data(), n)) || (rc = up(&c.node_inst, node_inst.data(), node_inst.size())) ||
@@ -1756,6 +1794,13 @@ extern "C" int adh_sw2_hip_get_tuning(adh_sw2_hip *h, adh_sw2_tuning *out) {
         out->layout[k] = h->c.tune.layout[k];
         out->ms[k] = 0.0;
     }
+    return 0;
+}
+
+extern "C" int adh_sw2_hip_set_solve_wait(adh_sw2_hip *h, long long ticks) {
+    if (!h) return fail(ADH_SW2_EINVAL, "null argument");
+    h->c.run_limit = ticks;
+    h->c.run_pause = 0;
     return 0;
 }
 

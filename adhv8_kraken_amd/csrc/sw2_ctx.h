@@ -171,6 +171,16 @@ struct Ctx {
     int kgraph_prec, kgraph_pc;
     const double *kgraph_band;
     int last_lin_it;       // iterations of the previous solve (sizes the first chunk)
+    // the one-kernel block-Jacobi BiCGSTAB (sw2_run.hip)
+    double *run_slots;     // two sets of hand-over slots, used by turns (run_parity)
+    double *run_xch;       // the hand-over vectors
+    int run_dirty;         // run_xch is to be emptied first
+    int *run_quit;         // [2 max(1, ninst)] give-up flags
+    int run_parity, run_prec;
+    int run_cap[2];        // blocks the GPU holds at once in form run_prec, at one and two a CU (-1: not asked yet)
+    int run_max_blocks;    // 256-node blocks of the largest model
+    int run_pause;         // solves left to the kernel-per-step form after a hand-over timed out
+    long long run_limit;   // bound of a hand-over's wait, 100 MHz ticks
     // profile-LU (OP BLK) preconditioner, built on demand for opts.nblock
     int band_nblock;       // block count of the current band structure (0 = none)
     int band_nb;           // blocks
@@ -285,6 +295,10 @@ void launch_norms(Ctx *c);
 void launch_setup(Ctx *c);
 void launch_krylov_prologue(Ctx *c);
 void launch_krylov_iters(Ctx *c, int k);
+bool launch_krylov_run(Ctx *c, bool zero_guess);   // false: this system takes the kernel-per-step form
+constexpr int RUN_BLOCKS = 1024;   // 256-node blocks of the largest model that form is ever asked for
+size_t run_slot_words(int nblk);
+size_t run_vector_words(int Np);
 void launch_krylov_epilogue(Ctx *c, bool zero_guess);
 void launch_geometry(Ctx *c);
 void launch_zero(Ctx *c, double *p, size_t n);

@@ -12,7 +12,9 @@
 // finisher kernel reduces them in block order and updates the device
 // scalars, so a BiCGSTAB iteration is 6 launches with no host round trip; the
 // host reads the convergence flag every opts.check_every iterations and
-// kernels launched past convergence return at entry.  The same kernels run in FP64 or FP32
+// kernels launched past convergence return at entry.  Models that fit on the
+// GPU at once solve in one kernel instead, with the same operations
+// (sw2_run.hip).  The same kernels run in FP64 or FP32
 // (precision 0), with FP32 matrix and preconditioner and FP64 vectors
 // (precision 1), or all in FP32 (precision 2); dot products accumulate in FP64.
 //
@@ -25,19 +27,9 @@
 #include <type_traits>
 
 #include "sw2_ctx.h"
+#include "sw2_krylov.h"
 
 namespace sw2 {
-
-// FP64 matrix and preconditioner entries are read once per product:
-// non-temporal loads keep them from displacing the gathered vector in L2
-// (57 against 63 us for the FP64 K1 at 1M triangles; the FP32 streams are
-// faster with ordinary loads)
-template <typename T>
-__device__ __forceinline__ T ldnt(const T *p) {
-    if constexpr (sizeof(T) == 8) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-
 
 // model tables of an ensemble (null for one model)
 #define BI(c) ((c)->ninst ? (const int *)(c)->blk_inst : (const int *)nullptr)
@@ -332,13 +324,6 @@ __global__ void __launch_bounds__(256) k_fin(int nparts, const double *part, KSc
 // Off-diagonal blocks come from the SELL-64 slice of this row's wavefront:
 // every lane runs the slice's K block slots (zero padding past the row's
 // length), and entry e of slot j is one coalesced 64-value read per wave.
-// Precision tags of the Krylov solve: matrix/preconditioner storage type M
-// and vector/arithmetic type V (a float matrix entry times a double vector
-// entry is formed in double).
-struct PrecF64 { using M = double; using V = double; };   // precision 0
-struct PrecMix { using M = float; using V = double; };    // precision 1: FP32 matrix, FP64 vectors
-struct PrecF32 { using M = float; using V = float; };     // precision 2: all FP32
-
 template <typename P, int K, typename XF, bool BJ = true>
 __device__ __forceinline__ void amult_prec_row(int n, const typename P::M *diag, const typename P::M *offd,
                                                const int *sell_ptr, const int *sell_col, const typename P::M *dinv,
@@ -409,12 +394,6 @@ struct VecS {  // s = r + (-alpha) Ap, the reference's copy + daxpy
     const T *r, *ap;
     T nalpha;
     __device__ T operator()(size_t i) const { return r[i] + nalpha * ap[i]; }
-};
-
-template <typename P>
-struct KVecs {
-    const typename P::M *diag, *offd, *dinv;
-    typename P::V *b, *r, *p, *Ap, *s, *As, *q, *u;
 };
 
 // prologue part 1: b' = M^-1 b, u = b', ||b'||inf  (solv_bcgstab.c:117-137)
@@ -699,21 +678,6 @@ __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, 
     x += ZERO ? 0.0 : sol[i];
     x *= scale[i];
     sol[i] = x;
-}
-
-template <typename P>
-static KVecs<P> vecs(Ctx *c);
-template <>
-KVecs<PrecF64> vecs<PrecF64>(Ctx *c) {
-    return KVecs<PrecF64>{c->diag, c->offd, c->dinv, c->kb, c->kr, c->kp, c->kAp, c->ks_, c->kAs, c->kq, c->ku};
-}
-template <>
-KVecs<PrecMix> vecs<PrecMix>(Ctx *c) {
-    return KVecs<PrecMix>{c->diag32, c->offd32, c->dinv32, c->kb, c->kr, c->kp, c->kAp, c->ks_, c->kAs, c->kq, c->ku};
-}
-template <>
-KVecs<PrecF32> vecs<PrecF32>(Ctx *c) {
-    return KVecs<PrecF32>{c->diag32, c->offd32, c->dinv32, c->fb, c->fr, c->fp, c->fAp, c->fs, c->fAs, c->fq, c->fu};
 }
 
 template <typename P, int K>

@@ -124,6 +124,7 @@ def lib():
         L.adh_sw2_hip_batch_set_tol.argtypes = [C.c_void_p, C.c_int, C.c_double]
         L.adh_sw2_hip_get_tuning.argtypes = [C.c_void_p, C.POINTER(Tuning)]
         L.adh_sw2_hip_set_tuning.argtypes = [C.c_void_p, C.POINTER(Tuning)]
+        L.adh_sw2_hip_set_solve_wait.argtypes = [C.c_void_p, C.c_longlong]
         L.adh_sw2_hip_autotune.argtypes = [C.c_void_p, C.c_int, C.POINTER(Tuning)]
         L.adh_sw2_hip_batch_residual_norm.argtypes = [C.c_void_p, PD]
         L.adh_sw2_hip_time_kernel.argtypes = [C.c_void_p, C.c_int, C.c_int, PD]
@@ -209,6 +210,11 @@ class _Tunable:
 
     def set_tuning(self, t: Tuning):
         _check(self.L.adh_sw2_hip_set_tuning(self.h, C.byref(t)))
+
+    def set_solve_wait(self, ticks: int):
+        """Bound of a wait inside the one-kernel solve, in 10 ns; below 0: a
+        kernel per step always.  Never changes a result."""
+        _check(self.L.adh_sw2_hip_set_solve_wait(self.h, ticks))
 
 
 class SW2Model(_Tunable):
