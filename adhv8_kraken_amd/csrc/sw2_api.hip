@@ -493,6 +493,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     UP(col, c.h_col.data(), c.nnz);
     UP(sell_ptr, sell_ptr.data(), c.nslice + 1);
     UP(sell_col, sell_col.data(), c.nsell);
+    UP(offd_pos, c.h_offd_pos.data(), c.h_offd_pos.size());
     UP(slot_ptr, slot_ptr.data(), c.ndslots + 1);
     UP(slot_src, slot_src.data(), slot_src.size());
     {   // element block -> its position in the slot-ordered contributor list
@@ -534,7 +535,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     if ((rc = alloc_solver(h))) { adh_sw2_hip_destroy(h); return rc; }
     if (hipHostMalloc((void **)&c.h_ksc, sizeof(KScal) * nmod) != hipSuccess ||
         hipHostMalloc((void **)&c.h_norms, sizeof(Norms) * nmod) != hipSuccess ||
-        hipHostMalloc((void **)&c.h_flag, 64) != hipSuccess) {
+        hipHostMalloc((void **)&c.h_flag, 64) != hipSuccess || c.stage.create() != hipSuccess) {
         adh_sw2_hip_destroy(h);
         return fail(ADH_SW2_ENOMEM, "hipHostMalloc failed");
     }
@@ -584,6 +585,7 @@ extern "C" void adh_sw2_hip_destroy(adh_sw2_hip *h) {
     if (c.h_ksc) (void)hipHostFree(c.h_ksc);
     if (c.h_norms) (void)hipHostFree(c.h_norms);
     if (c.h_flag) (void)hipHostFree(c.h_flag);
+    c.stage.destroy();
     for (int i = 0; i < 8; i++) if (c.ev[i]) (void)hipEventDestroy(c.ev[i]);
     if (c.stream) (void)hipStreamDestroy(c.stream);
     delete h;
@@ -665,22 +667,50 @@ extern "C" int adh_sw2_hip_pattern(adh_sw2_hip *h, int *row_ptr, int *col) {
     return 0;
 }
 
-static int set_pair(Ctx &c, double *dh, double *du, double *dv, const double *hh, const double *vel) {
-    std::vector<double> u(c.N), v(c.N);
-    for (int i = 0; i < c.N; i++) { u[i] = vel[2 * i]; v[i] = vel[2 * i + 1]; }
-    HIPCHK(hipMemcpy(dh, hh, sizeof(double) * c.N, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(du, u.data(), sizeof(double) * c.N, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(dv, v.data(), sizeof(double) * c.N, hipMemcpyHostToDevice));
+static StageMap plain(const void *dev, StageMap::Kind kind = StageMap::PLAIN) {
+    StageMap m{};
+    m.kind = kind;
+    m.a[0] = (void *)dev;
+    m.ndst = 1;
+    return m;
+}
+
+// The three time levels of nodes a .. a + n - 1 from the caller.  Levels given
+// by one and the same array (a start from rest) cross the bus once.
+static int state_from_host(Ctx &c, int a, int n, const double *const (&head)[3], const double *const (&vel)[3]) {
+    double *hd[3] = {c.head, c.old_head, c.older_head}, *ud[3] = {c.u, c.old_u, c.older_u},
+           *vd[3] = {c.v, c.old_v, c.older_v};
+    for (int k = 0; k < 3; k++) {
+        StageMap h{}, w{};
+        h.kind = StageMap::PLAIN;
+        w.kind = StageMap::PAIR;
+        for (int j = k; j < 3; j++) {
+            if (head[j] == head[k]) h.a[h.ndst++] = hd[j] + a;
+            if (vel[j] == vel[k]) { w.a[w.ndst] = ud[j] + a; w.b[w.ndst++] = vd[j] + a; }
+        }
+        if (std::find(head, head + k, head[k]) == head + k) HIPCHK(c.stage.in(c.stream, h, head[k], n));
+        if (std::find(vel, vel + k, vel[k]) == vel + k) HIPCHK(c.stage.in(c.stream, w, vel[k], 2 * (size_t)n));
+    }
+    c.pre_valid = 0;
+    c.split_valid = 0;
+    HIPCHK(c.stage.finish_in());
     return 0;
 }
 
-static int get_pair(Ctx &c, const double *dh, const double *du, const double *dv, double *hh, double *vel) {
-    if (hh) HIPCHK(hipMemcpy(hh, dh, sizeof(double) * c.N, hipMemcpyDeviceToHost));
+// the caller's arrays complete, and the stream with them
+static int finish_out(Ctx &c) {
+    HIPCHK(c.stage.finish_out(c.stream));
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+// one time level to the caller; null: not wanted
+static int pair_to_host(Ctx &c, const double *dh, const double *du, const double *dv, int n, double *head, double *vel) {
+    if (head) HIPCHK(c.stage.out(c.stream, plain(dh), head, n));
     if (vel) {
-        std::vector<double> u(c.N), v(c.N);
-        HIPCHK(hipMemcpy(u.data(), du, sizeof(double) * c.N, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(v.data(), dv, sizeof(double) * c.N, hipMemcpyDeviceToHost));
-        for (int i = 0; i < c.N; i++) { vel[2 * i] = u[i]; vel[2 * i + 1] = v[i]; }
+        StageMap w = plain(du, StageMap::PAIR);
+        w.b[0] = (void *)dv;
+        HIPCHK(c.stage.out(c.stream, w, vel, 2 * (size_t)n));
     }
     return 0;
 }
@@ -690,15 +720,7 @@ extern "C" int adh_sw2_hip_set_state(adh_sw2_hip *h, const double *head, const d
     if (h && h->c.ninst) return fail(ADH_SW2_EINVAL, "an ensemble handle takes the adh_sw2_hip_batch_* calls");
     if (!h || !head || !vel || !old_head || !old_vel || !older_head || !older_vel)
         return fail(ADH_SW2_EINVAL, "null argument");
-    Ctx &c = h->c;
-    HIPCHK(hipStreamSynchronize(c.stream));
-    int rc;
-    if ((rc = set_pair(c, c.head, c.u, c.v, head, vel))) return rc;
-    if ((rc = set_pair(c, c.old_head, c.old_u, c.old_v, old_head, old_vel))) return rc;
-    if ((rc = set_pair(c, c.older_head, c.older_u, c.older_v, older_head, older_vel))) return rc;
-    c.pre_valid = 0;
-    c.split_valid = 0;
-    return 0;
+    return state_from_host(h->c, 0, h->c.N, {head, old_head, older_head}, {vel, old_vel, older_vel});
 }
 
 extern "C" int adh_sw2_hip_get_state(adh_sw2_hip *h, double *head, double *vel, double *old_head, double *old_vel,
@@ -706,12 +728,11 @@ extern "C" int adh_sw2_hip_get_state(adh_sw2_hip *h, double *head, double *vel, 
     if (h && h->c.ninst) return fail(ADH_SW2_EINVAL, "an ensemble handle takes the adh_sw2_hip_batch_* calls");
     if (!h) return fail(ADH_SW2_EINVAL, "null handle");
     Ctx &c = h->c;
-    HIPCHK(hipStreamSynchronize(c.stream));
     int rc;
-    if ((rc = get_pair(c, c.head, c.u, c.v, head, vel))) return rc;
-    if ((rc = get_pair(c, c.old_head, c.old_u, c.old_v, old_head, old_vel))) return rc;
-    if ((rc = get_pair(c, c.older_head, c.older_u, c.older_v, older_head, older_vel))) return rc;
-    return 0;
+    if ((rc = pair_to_host(c, c.head, c.u, c.v, c.N, head, vel))) return rc;
+    if ((rc = pair_to_host(c, c.old_head, c.old_u, c.old_v, c.N, old_head, old_vel))) return rc;
+    if ((rc = pair_to_host(c, c.older_head, c.older_u, c.older_v, c.N, older_head, older_vel))) return rc;
+    return finish_out(c);
 }
 
 static int sync_check(Ctx &c) {
@@ -731,14 +752,11 @@ extern "C" int adh_sw2_hip_init(adh_sw2_hip *h, int *bc_mask, int *wd_flag) {
     if (h && h->c.ninst) return fail(ADH_SW2_EINVAL, "an ensemble handle takes the adh_sw2_hip_batch_* calls");
     if (!h) return fail(ADH_SW2_EINVAL, "null handle");
     Ctx &c = h->c;
-    int *dmask = nullptr;
-    if (bc_mask) HIPCHK(hipMalloc(&dmask, sizeof(int) * 3 * c.N));
-    launch_init(&c, dmask);
-    int rc = sync_check(c);
-    if (!rc && bc_mask) rc = hipMemcpy(bc_mask, dmask, sizeof(int) * 3 * c.N, hipMemcpyDeviceToHost) == hipSuccess ? 0 : fail(ADH_SW2_EHIP, "copy bc_mask");
-    if (dmask) (void)hipFree(dmask);
-    if (!rc && wd_flag) HIPCHK(hipMemcpy(wd_flag, c.wd_flag, sizeof(int) * c.E, hipMemcpyDeviceToHost));
-    return rc;
+    int *mask = bc_mask ? (int *)c.kAs : nullptr;   // a Krylov work vector: free between solves
+    launch_init(&c, mask);
+    if (bc_mask) HIPCHK(c.stage.out(c.stream, plain(mask, StageMap::INTS), bc_mask, 3 * (size_t)c.N));
+    if (wd_flag) HIPCHK(c.stage.out(c.stream, plain(c.wd_flag, StageMap::INTS), wd_flag, c.E));
+    return finish_out(c);
 }
 
 // adh_sw2_hip_init with the boundary mask staged in the device's `scratch`
@@ -761,20 +779,16 @@ extern "C" int adh_sw2_hip_init_noalloc(adh_sw2_hip *h, int *bc_mask, int *wd_fl
 }
 
 // node vectors [3N] / diagonal blocks [9N] between node-major (host) and the
-// device's sliced layout
+// device's sliced layout; to the host: complete after finish_out
 static int nodes_to_host(Ctx &c, const double *dev, double *out, int per) {
-    std::vector<double> t((size_t)per * c.Np);
-    HIPCHK(hipMemcpy(t.data(), dev, sizeof(double) * t.size(), hipMemcpyDeviceToHost));
-    for (int n = 0; n < c.N; n++)
-        for (int k = 0; k < per; k++) out[(size_t)per * n + k] = t[per == 3 ? vidx3(n, k) : didx9(n, k)];
+    HIPCHK(c.stage.out(c.stream, plain(dev, per == 3 ? StageMap::NODE3 : StageMap::NODE9), out, (size_t)per * c.N));
     return 0;
 }
 
 static int nodes_from_host(Ctx &c, double *dev, const double *in, int per) {
-    std::vector<double> t((size_t)per * c.Np, 0.0);
-    for (int n = 0; n < c.N; n++)
-        for (int k = 0; k < per; k++) t[per == 3 ? vidx3(n, k) : didx9(n, k)] = in[(size_t)per * n + k];
-    HIPCHK(hipMemcpy(dev, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
+    launch_zero(&c, dev, (size_t)per * c.Np);   // the padding rows
+    HIPCHK(c.stage.in(c.stream, plain(dev, per == 3 ? StageMap::NODE3 : StageMap::NODE9), in, (size_t)per * c.N));
+    HIPCHK(c.stage.finish_in());
     return 0;
 }
 
@@ -783,32 +797,26 @@ extern "C" int adh_sw2_hip_resid(adh_sw2_hip *h, double *residual) {
     if (!h) return fail(ADH_SW2_EINVAL, "null handle");
     Ctx &c = h->c;
     launch_resid(&c);
-    int rc = sync_check(c);
-    if (rc) return rc;
+    int rc;
     if (residual && (rc = nodes_to_host(c, c.R, residual, 3))) return rc;
-    return 0;
+    return finish_out(c);
 }
 
 // off-diagonal blocks between the reference's row order (host) and SELL-64 (device)
 static int offd_to_host(Ctx &c, double *out) {
-    std::vector<double> sv(9 * c.nsell);
-    if (c.mat32) {   // refined forms: the FP32 matrix (unscaled until the set-up scales it in place)
-        std::vector<float> f(sv.size());
-        HIPCHK(hipMemcpy(f.data(), c.offd32, sizeof(float) * f.size(), hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < f.size(); i++) sv[i] = (double)f[i];
-    } else {
-        HIPCHK(hipMemcpy(sv.data(), c.offd, sizeof(double) * sv.size(), hipMemcpyDeviceToHost));
-    }
-    for (int p = 0; p < c.nnz; p++)
-        for (int e = 0; e < 9; e++) out[9 * (size_t)p + e] = sv[sell_vidx((size_t)c.h_offd_pos[p], e)];
+    // refined forms: the FP32 matrix (unscaled until the set-up scales it in place)
+    StageMap m = plain(c.mat32 ? (const void *)c.offd32 : c.offd, c.mat32 ? StageMap::OFFD32 : StageMap::OFFD);
+    m.pos = c.offd_pos;
+    HIPCHK(c.stage.out(c.stream, m, out, 9 * (size_t)c.nnz));
     return 0;
 }
 
 static int offd_from_host(Ctx &c, const double *in) {
-    std::vector<double> sv(9 * c.nsell, 0.0);
-    for (int p = 0; p < c.nnz; p++)
-        for (int e = 0; e < 9; e++) sv[sell_vidx((size_t)c.h_offd_pos[p], e)] = in[9 * (size_t)p + e];
-    HIPCHK(hipMemcpy(c.offd, sv.data(), sizeof(double) * sv.size(), hipMemcpyHostToDevice));
+    launch_zero(&c, c.offd, 9 * c.nsell);   // the padding blocks
+    StageMap m = plain(c.offd, StageMap::OFFD);
+    m.pos = c.offd_pos;
+    HIPCHK(c.stage.in(c.stream, m, in, 9 * (size_t)c.nnz));
+    HIPCHK(c.stage.finish_in());
     return 0;
 }
 
@@ -818,12 +826,11 @@ extern "C" int adh_sw2_hip_load(adh_sw2_hip *h, double *diagonal, double *offdia
     Ctx &c = h->c;
     launch_jacobian(&c);
     launch_assemble(&c);
-    int rc = sync_check(c);
-    if (rc) return rc;
+    int rc;
     if (diagonal && (rc = nodes_to_host(c, c.diag, diagonal, 9))) return rc;
     if (offdiag && c.nnz && (rc = offd_to_host(c, offdiag))) return rc;
     if (residual && (rc = nodes_to_host(c, c.R, residual, 3))) return rc;
-    return 0;
+    return finish_out(c);
 }
 
 extern "C" int adh_sw2_hip_elem_jacobians(adh_sw2_hip *h, double *em2d, double *em1d) {
@@ -897,10 +904,9 @@ extern "C" int adh_sw2_hip_linear_sys_setup(adh_sw2_hip *h, const double *x, dou
         launch_zero(&c, c.sol, 3 * (size_t)c.Np);
     }
     launch_setup(&c);
-    int rc = sync_check(c);
-    if (rc) return rc;
+    int rc;
     if (scale_vect && (rc = nodes_to_host(c, c.scale, scale_vect, 3))) return rc;
-    return 0;
+    return finish_out(c);
 }
 
 // BiCGSTAB on the scaled device system; returns the reference's YES/NO.
@@ -1052,8 +1058,8 @@ extern "C" int adh_sw2_hip_precond_apply(adh_sw2_hip *h, const double *v, double
     if ((rc = nodes_from_host(c, c.kAs, v, 3))) return rc;
     if (c.opts.preconditioner == 3) launch_ilu_solve(&c, c.kAs, nullptr);
     else launch_band_solve(&c, c.kAs, nullptr);
-    if ((rc = sync_check(c))) return rc;
-    return nodes_to_host(c, c.kAs, y, 3);
+    if ((rc = nodes_to_host(c, c.kAs, y, 3))) return rc;
+    return finish_out(c);
 }
 
 // The ILU(0) node colouring: color[N], *ncolor.
@@ -1073,9 +1079,9 @@ extern "C" int adh_sw2_hip_linear_sys_solve(adh_sw2_hip *h, double *sol, int *li
     int vd = ADH_SW2_NO;
     int rc = krylov(c, lin_it, &vd, false);
     if (rc) return rc;
-    if ((rc = sync_check(c))) return rc;
-    if (verdict) *verdict = vd;
     if (sol && (rc = nodes_to_host(c, c.sol, sol, 3))) return rc;
+    if ((rc = finish_out(c))) return rc;
+    if (verdict) *verdict = vd;
     return 0;
 }
 
@@ -1090,20 +1096,19 @@ extern "C" int adh_sw2_hip_set_system(adh_sw2_hip *h, const double *diagonal, co
     c.sys_scaled = 0;
     c.mat32 = 0;   // the system is now the FP64 one given here
     if ((rc = nodes_from_host(c, c.R, rhs, 3))) return rc;
-    HIPCHK(hipMemset(c.sol, 0, sizeof(double) * 3 * c.Np));
-    return 0;
+    launch_zero(&c, c.sol, 3 * (size_t)c.Np);
+    return sync_check(c);
 }
 
 extern "C" int adh_sw2_hip_get_system(adh_sw2_hip *h, double *diagonal, double *offdiag, double *rhs) {
     if (h && h->c.ninst) return fail(ADH_SW2_EINVAL, "an ensemble handle takes the adh_sw2_hip_batch_* calls");
     if (!h) return fail(ADH_SW2_EINVAL, "null handle");
     Ctx &c = h->c;
-    HIPCHK(hipStreamSynchronize(c.stream));
     int rc;
     if (diagonal && (rc = nodes_to_host(c, c.diag, diagonal, 9))) return rc;
     if (offdiag && c.nnz && (rc = offd_to_host(c, offdiag))) return rc;
     if (rhs && (rc = nodes_to_host(c, c.R, rhs, 3))) return rc;
-    return 0;
+    return finish_out(c);
 }
 
 extern "C" int adh_sw2_hip_probe_math(const double *x, int n, double *log_out, double *sqrt_out, double *div_out) {
@@ -1653,36 +1658,15 @@ extern "C" int adh_sw2_hip_batch_set_state(adh_sw2_hip *h, int i, const double *
     int a, nn, rc;
     if ((rc = model_range(h, i, &a, &nn))) return rc;
     if (!head || !vel || !old_head || !old_vel || !older_head || !older_vel) return fail(ADH_SW2_EINVAL, "null argument");
-    Ctx &c = h->c;
-    HIPCHK(hipStreamSynchronize(c.stream));
-    const double *src[6] = {head, vel, old_head, old_vel, older_head, older_vel};
-    double *hd[3] = {c.head, c.old_head, c.older_head}, *ud[3] = {c.u, c.old_u, c.older_u},
-           *vd[3] = {c.v, c.old_v, c.older_v};
-    std::vector<double> u(nn), v(nn);
-    for (int k = 0; k < 3; k++) {
-        HIPCHK(hipMemcpy(hd[k] + a, src[2 * k], sizeof(double) * nn, hipMemcpyHostToDevice));
-        for (int j = 0; j < nn; j++) { u[j] = src[2 * k + 1][2 * j]; v[j] = src[2 * k + 1][2 * j + 1]; }
-        HIPCHK(hipMemcpy(ud[k] + a, u.data(), sizeof(double) * nn, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(vd[k] + a, v.data(), sizeof(double) * nn, hipMemcpyHostToDevice));
-    }
-    c.pre_valid = 0;
-    c.split_valid = 0;
-    return 0;
+    return state_from_host(h->c, a, nn, {head, old_head, older_head}, {vel, old_vel, older_vel});
 }
 
 extern "C" int adh_sw2_hip_batch_get_state(adh_sw2_hip *h, int i, double *head, double *vel) {
     int a, nn, rc;
     if ((rc = model_range(h, i, &a, &nn))) return rc;
     Ctx &c = h->c;
-    HIPCHK(hipStreamSynchronize(c.stream));
-    if (head) HIPCHK(hipMemcpy(head, c.head + a, sizeof(double) * nn, hipMemcpyDeviceToHost));
-    if (vel) {
-        std::vector<double> u(nn), v(nn);
-        HIPCHK(hipMemcpy(u.data(), c.u + a, sizeof(double) * nn, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(v.data(), c.v + a, sizeof(double) * nn, hipMemcpyDeviceToHost));
-        for (int j = 0; j < nn; j++) { vel[2 * j] = u[j]; vel[2 * j + 1] = v[j]; }
-    }
-    return 0;
+    if ((rc = pair_to_host(c, c.head + a, c.u + a, c.v + a, nn, head, vel))) return rc;
+    return finish_out(c);
 }
 
 extern "C" int adh_sw2_hip_batch_set_dt(adh_sw2_hip *h, int i, double dt) {

@@ -35,6 +35,41 @@ struct Red {
     int maxblocks;
 };
 
+// How an array of the caller's lies on the device (sw2_stage.hip): a[0], on the
+// way in also a[1..ndst-1], which receive the same values
+struct StageMap {
+    enum Kind { PLAIN, INTS, PAIR, NODE3, NODE9, OFFD, OFFD32 } kind;   // PAIR: interleaved a, b
+    void *a[3], *b[3];
+    const int *pos;            // OFFD: SELL slot of each off-diagonal block
+    int ndst;
+};
+
+// The pinned buffer between the caller's memory and the device: two halves,
+// used by turns, each closed with an event.
+struct Stage {
+    static constexpr size_t HALF = (size_t)2 << 20;
+    static constexpr int MAXSEG = 16;
+    struct Seg { void *user; size_t off, bytes; };
+    char *buf;
+    hipEvent_t ev[2];
+    bool pending[2];           // the half's event is recorded and not yet waited for
+    int cur;
+    size_t used;               // bytes of the current half in use
+    Seg seg[2][MAXSEG];        // what the half will be copied to
+    int nseg[2];
+    char *half(int h) const { return buf + h * HALF; }
+    hipError_t create();
+    void destroy();
+    // queue count elements on their way; out: the caller has them after finish_out
+    hipError_t out(hipStream_t st, const StageMap &m, void *user, size_t count);
+    hipError_t in(hipStream_t st, const StageMap &m, const void *user, size_t count);
+    hipError_t finish_out(hipStream_t st);
+    hipError_t finish_in();
+    hipError_t wait(int h);
+    hipError_t drain(int h);
+    hipError_t turn_over(hipStream_t st);
+};
+
 // Newton norms (get_residual_norms, fe_newton.c:40-151)
 struct Norms {
     double maxn, l2, incn, pad;
@@ -145,6 +180,8 @@ struct Ctx {
     Red red;
     Norms *norms, *h_norms;  // [max(1, ninst)]
     int *h_flag;           // pinned scratch
+    Stage stage;
+    int *offd_pos;         // device copy of h_offd_pos
     ElemData ed;
     // Ensemble of independent models sharing one mesh ("batch"): model i owns
     // the node range [inst_node0[i], inst_node0[i] + inst_N[i]) starting on a
