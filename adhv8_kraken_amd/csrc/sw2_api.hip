@@ -978,7 +978,6 @@ static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     if (c.run_pause > 0) { c.run_pause--; return 0; }
     if (!launch_krylov_run(&c, zero_guess)) return 0;
     const int n = c.ninst ? c.ninst : 1;
-    HIPCHK(hipMemcpyAsync(c.h_ksc, c.ksc, sizeof(KScal) * n, hipMemcpyDeviceToHost, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
     *done = true;
     for (int i = 0; i < n; i++) *done = *done && c.h_ksc[i].done;
@@ -1002,11 +1001,7 @@ static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
         *verdict = conv ? ADH_SW2_YES : ADH_SW2_NO;
         return 0;
     }
-    KScal init{};
-    init.atol = c.opts.lin_atol;
-    init.rtol = c.opts.lin_rtol;
-    init.max_it = lin_it_cap(c);
-    HIPCHK(hipMemcpyAsync(c.ksc, &init, sizeof(KScal), hipMemcpyHostToDevice, c.stream));
+    launch_scal_init(&c, lin_it_cap(c));
     bool done_early = false;
     int rc0 = krylov_one_kernel(c, zero_guess, &done_early);
     if (rc0) return rc0;
@@ -1186,7 +1181,6 @@ static float elapsed(Ctx &c, int a, int b) {
 }
 
 static int read_norms(Ctx &c, Norms *out) {
-    HIPCHK(hipMemcpyAsync(c.h_norms, c.norms, sizeof(Norms), hipMemcpyDeviceToHost, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
     *out = *c.h_norms;
     return 0;
@@ -1322,6 +1316,7 @@ extern "C" int adh_sw2_hip_timestep(adh_sw2_hip *h, adh_sw2_report *rep, int *ve
 // same reduction order, same element code.
 
 static int set_mask(Ctx &c, const std::vector<int> &m) {
+    if (m == c.h_inst_mask) return 0;   // the device and the element lists have it already
     c.split_valid = 0;  // the element lists hold the masked models only
     HIPCHK(hipMemcpyAsync(c.inst_mask, m.data(), sizeof(int) * c.ninst, hipMemcpyHostToDevice, c.stream));
     c.h_inst_mask = m;
@@ -1331,7 +1326,6 @@ static int set_mask(Ctx &c, const std::vector<int> &m) {
 }
 
 static int read_norms_all(Ctx &c, std::vector<Norms> &out) {
-    HIPCHK(hipMemcpyAsync(c.h_norms, c.norms, sizeof(Norms) * c.ninst, hipMemcpyDeviceToHost, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
     out.assign(c.h_norms, c.h_norms + c.ninst);
     return 0;
@@ -1340,14 +1334,7 @@ static int read_norms_all(Ctx &c, std::vector<Norms> &out) {
 // BiCGSTAB for the active models (inactive ones start converged)
 static int krylov_batch(Ctx &c, const std::vector<int> &active, std::vector<int> &lin_it, std::vector<int> &vd) {
     const int n = c.ninst, cap = lin_it_cap(c);
-    std::vector<KScal> init(n);
-    for (int i = 0; i < n; i++) {
-        init[i] = KScal{};
-        init[i].atol = c.opts.lin_atol;
-        init[i].rtol = c.opts.lin_rtol;
-        init[i].max_it = active[i] ? cap : 0;
-    }
-    HIPCHK(hipMemcpyAsync(c.ksc, init.data(), sizeof(KScal) * n, hipMemcpyHostToDevice, c.stream));
+    launch_scal_init(&c, cap);   // by the device's mask, which holds `active`
     bool all_done0 = false;
     int rc0 = krylov_one_kernel(c, true, &all_done0);
     if (rc0) return rc0;

@@ -330,6 +330,7 @@ void launch_scale_sol(Ctx *c, double f);          // sol *= f
 void launch_inc_flip(Ctx *c);                     // state += sol, then sol = -sol
 void launch_norms(Ctx *c);
 void launch_setup(Ctx *c);
+void launch_scal_init(Ctx *c, int max_it);
 void launch_krylov_prologue(Ctx *c);
 void launch_krylov_iters(Ctx *c, int k);
 bool launch_krylov_run(Ctx *c, bool zero_guess);   // false: this system takes the kernel-per-step form

@@ -1159,9 +1159,10 @@ __global__ void __launch_bounds__(256) k_norms(int N, const double *R, const dou
     }
 }
 
-// one block: the block partials of k_norms, reduced in block order
+// one block: the block partials of k_norms, reduced in block order; the result
+// also goes straight to the host's pinned copy, so reading it is one wait
 // one block per model (blockIdx.x), over that model's 256-node blocks
-__global__ void __launch_bounds__(256) k_norms_fin(int nparts, int N, const double *part, Norms *out,
+__global__ void __launch_bounds__(256) k_norms_fin(int nparts, int N, const double *part, Norms *out, Norms *host,
                                                    const int *inst_blk0, const int *inst_nodes) {
     __shared__ double smax[256], ssum[256], sinc[256];
     const int m = blockIdx.x;
@@ -1196,9 +1197,12 @@ __global__ void __launch_bounds__(256) k_norms_fin(int nparts, int N, const doub
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        out->maxn = smax[0];
-        out->l2 = sqrt(ssum[0] / (double)(N * 3));
-        out->incn = sinc[0];
+        Norms r{};
+        r.maxn = smax[0];
+        r.l2 = sqrt(ssum[0] / (double)(N * 3));
+        r.incn = sinc[0];
+        *out = r;
+        host[m] = r;
     }
 }
 
@@ -1207,7 +1211,7 @@ void launch_norms(Ctx *c) {
     hipLaunchKernelGGL(k_norms, dim3(nb), dim3(256), 0, c->stream, c->N, c->R, c->sol, c->head, c->old_head,
                        c->red.part);
     hipLaunchKernelGGL(k_norms_fin, dim3(c->ninst ? c->ninst : 1), dim3(256), 0, c->stream, nb, c->N, c->red.part,
-                       c->norms, c->ninst ? c->inst_blk0 : nullptr, c->ninst ? c->inst_nodes : nullptr);
+                       c->norms, c->h_norms, c->ninst ? c->inst_blk0 : nullptr, c->ninst ? c->inst_nodes : nullptr);
 }
 
 }  // namespace sw2

@@ -293,7 +293,7 @@ struct Rows {
 template <typename P, int K, int OCC>
 __global__ void __launch_bounds__(256, OCC)
     k_bcg_run(int N, size_t n3, KVecs<P> V, typename P::V *xch, const int *sell_col, const double *rhs,
-              const double *scale, double *sol, KScal *sc, const int *blk_inst, const int *inst_blk0, double *slots,
+              const double *scale, double *sol, KScal *sc, KScal *host, const int *blk_inst, const int *inst_blk0, double *slots,
               int parity, int *quit, long long limit) {
     using T = typename P::V;
     using MT = typename P::M;
@@ -331,10 +331,11 @@ __global__ void __launch_bounds__(256, OCC)
         if (first) put_raw((float *)(quit + 2 * m + 1 - parity), 0u);
     }
     sc += m;
+    host += m;
     const int max_it = sc->max_it;
     const double atol = sc->atol, rtol = sc->rtol;
     if (blk_inst && max_it <= 0) {   // a model the ensemble's step leaves out
-        if (first && tid == 0) sc->done = 1;
+        if (first && tid == 0) sc->done = host->done = 1;
         return;
     }
     // threads past the model's end repeat its last row and keep the result to themselves
@@ -536,11 +537,14 @@ __global__ void __launch_bounds__(256, OCC)
 #pragma unroll
             for (int j = 0; j < 3; j++) put_raw(xch + t * n3 + own + 64 * j, Slot<T>::EMPTY);
     if (!first || tid != 0) return;
-    sc->bnorm = bnorm;
-    sc->tol = tol;
-    sc->rnorm = rnorm;
-    sc->it = it;
-    sc->done = 1;
+    KScal res = *sc;
+    res.bnorm = bnorm;
+    res.tol = tol;
+    res.rnorm = rnorm;
+    res.it = it;
+    res.done = 1;
+    *sc = res;
+    *host = res;   // pinned: the caller only waits for the kernel
 }
 
 // all hand-over vectors emptied: before the first solve and after one that gave up
@@ -577,9 +581,10 @@ bool run_k(Ctx *c, bool zero_guess) {
         hipLaunchKernelGGL(k_run_empty<T>, dim3((unsigned)((VRING * n3 + 255) / 256)), dim3(256), 0, c->stream,
                            VRING * n3, xch);
     }
+    for (int i = 0; i < (c->ninst ? c->ninst : 1); i++) c->h_ksc[i].done = 0;   // the kernel sets what it finishes
     c->run_parity ^= 1;
     hipLaunchKernelGGL((k_bcg_run<P, K, OCC>), dim3(nb), dim3(256), 0, c->stream, c->N, n3, vecs<P>(c), xch,
-                       c->sell_col, c->R, c->scale, zero_guess ? c->sol : nullptr, c->ksc,
+                       c->sell_col, c->R, c->scale, zero_guess ? c->sol : nullptr, c->ksc, c->h_ksc,
                        c->ninst ? c->blk_inst : nullptr, c->ninst ? c->inst_blk0 : nullptr, c->run_slots,
                        c->run_parity, c->run_quit, c->run_limit);
     return true;

@@ -680,6 +680,24 @@ __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, 
     sol[i] = x;
 }
 
+// every model's scalars at the start of a solve; a model that the mask leaves
+// out may take no iteration
+__global__ void k_scal_init(int n, KScal *sc, double atol, double rtol, int max_it, const int *mask) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= n) return;
+    KScal r{};
+    r.atol = atol;
+    r.rtol = rtol;
+    r.max_it = mask && !mask[m] ? 0 : max_it;
+    sc[m] = r;
+}
+
+void launch_scal_init(Ctx *c, int max_it) {
+    const int n = NFIN(c);
+    hipLaunchKernelGGL(k_scal_init, dim3(nblocks_for(n, 64)), dim3(64), 0, c->stream, n, c->ksc, c->opts.lin_atol,
+                       c->opts.lin_rtol, max_it, c->ninst ? c->inst_mask : nullptr);
+}
+
 template <typename P, int K>
 static void prologue_k(Ctx *c) {
     int nb = nblocks_for(c->N, 256);
