@@ -432,7 +432,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     // ---- device arrays
     hipError_t he = hipStreamCreate(&c.stream);
     if (he != hipSuccess) { delete h; return fail(ADH_SW2_EHIP, "hipStreamCreate failed"); }
-    for (int i = 0; i < 8; i++) (void)hipEventCreate(&c.ev[i]);
+    for (int i = 0; i < 2; i++) (void)hipEventCreate(&c.ev[i]);
     std::vector<int> zeros_i(N, 0);
     std::vector<double> zeros_d;
 #define UP(dst, src, n)                                    \
@@ -535,10 +535,16 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     if ((rc = alloc_solver(h))) { adh_sw2_hip_destroy(h); return rc; }
     if (hipHostMalloc((void **)&c.h_ksc, sizeof(KScal) * nmod) != hipSuccess ||
         hipHostMalloc((void **)&c.h_norms, sizeof(Norms) * nmod) != hipSuccess ||
-        hipHostMalloc((void **)&c.h_flag, 64) != hipSuccess || c.stage.create() != hipSuccess) {
+        hipHostMalloc((void **)&c.h_flag, 64) != hipSuccess ||
+        hipHostMalloc((void **)&c.h_ts, sizeof(long long) * TS_N) != hipSuccess || c.stage.create() != hipSuccess) {
         adh_sw2_hip_destroy(h);
         return fail(ADH_SW2_ENOMEM, "hipHostMalloc failed");
     }
+    int dev = 0, khz = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+        khz = 100000;
+    c.ts_ms = 1.0 / khz;
     {   // scale_vect starts at 1.0 (fe_main.c:263)
         std::vector<double> ones(3 * (size_t)c.Np, 1.0);
         HIPCHK(hipMemcpy(c.scale, ones.data(), sizeof(double) * ones.size(), hipMemcpyHostToDevice));
@@ -585,8 +591,9 @@ extern "C" void adh_sw2_hip_destroy(adh_sw2_hip *h) {
     if (c.h_ksc) (void)hipHostFree(c.h_ksc);
     if (c.h_norms) (void)hipHostFree(c.h_norms);
     if (c.h_flag) (void)hipHostFree(c.h_flag);
+    if (c.h_ts) (void)hipHostFree(c.h_ts);
     c.stage.destroy();
-    for (int i = 0; i < 8; i++) if (c.ev[i]) (void)hipEventDestroy(c.ev[i]);
+    for (int i = 0; i < 2; i++) if (c.ev[i]) (void)hipEventDestroy(c.ev[i]);
     if (c.stream) (void)hipStreamDestroy(c.stream);
     delete h;
 }
@@ -985,10 +992,11 @@ static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     return 0;
 }
 
-// zero_guess: sol holds a zero initial guess (the Newton step zeroes it), so
+// zero_guess: the initial guess is zero (the Newton step's; sol is not read), so
 // the epilogue is idempotent and is queued behind every chunk before the
 // convergence flag is read; otherwise it runs once, after the last chunk.
 static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
+    launch_scal_init(&c, lin_it_cap(c));
     if (c.opts.krylov == 1) {   // restarted GMRES: host-driven cycles
         std::string err = gmres_alloc(&c);
         if (!err.empty()) return fail(ADH_SW2_ENOMEM, err);
@@ -1001,7 +1009,6 @@ static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
         *verdict = conv ? ADH_SW2_YES : ADH_SW2_NO;
         return 0;
     }
-    launch_scal_init(&c, lin_it_cap(c));
     bool done_early = false;
     int rc0 = krylov_one_kernel(c, zero_guess, &done_early);
     if (rc0) return rc0;
@@ -1174,11 +1181,8 @@ extern "C" int adh_sw2_hip_time_kernel(adh_sw2_hip *h, int which, int reps, doub
     return 0;
 }
 
-static float elapsed(Ctx &c, int a, int b) {
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, c.ev[a], c.ev[b]);
-    return ms;
-}
+// ms between two phases' start times; the stream has been waited for
+static double elapsed(const Ctx &c, int a, int b) { return (double)(c.h_ts[b] - c.h_ts[a]) * c.ts_ms; }
 
 static int read_norms(Ctx &c, Norms *out) {
     HIPCHK(hipStreamSynchronize(c.stream));
@@ -1204,42 +1208,31 @@ static int newton(Ctx &c, adh_sw2_report *rep, int *verdict) {
     int rc;
     if ((rc = ensure_band(c))) return rc;
     Norms nm;
-    (void)hipEventRecord(c.ev[0], c.stream);
     launch_init(&c, nullptr);
-    (void)hipEventRecord(c.ev[1], c.stream);
-    launch_resid(&c);
-    launch_norms(&c);
-    (void)hipEventRecord(c.ev[2], c.stream);
+    launch_resid(&c, true);
     if ((rc = read_norms(c, &nm))) return rc;
-    if (rep) rep->ms_resid += elapsed(c, 1, 2);
+    if (rep) rep->ms_resid += elapsed(c, TS_RESID, TS_NORMS);
     hist(rep, nm, 0);
     int it = 0, solv_flag = ADH_SW2_YES, keep = 0;
     do {
         int lin_it = 0, vd = ADH_SW2_YES;
-        (void)hipEventRecord(c.ev[3], c.stream);
         launch_jacobian(&c);
         launch_assemble(&c);
-        launch_zero(&c, c.sol, 3 * (size_t)c.Np);
-        (void)hipEventRecord(c.ev[4], c.stream);
-        launch_setup(&c);
-        (void)hipEventRecord(c.ev[5], c.stream);
-        if ((rc = krylov(c, &lin_it, &vd, true))) return rc;   // sol zeroed above
-        (void)hipEventRecord(c.ev[6], c.stream);
+        launch_setup(&c, false);
+        if ((rc = krylov(c, &lin_it, &vd, true))) return rc;   // a zero guess
         // FP64: the reference's rule, a Krylov failure fails the Newton step.
         // FP32-refined forms: an unconverged inner solve is still a
         // correction; the FP64 residual tests and the line search decide.
         solv_flag = (o.precision >= 1) ? ADH_SW2_YES : vd;
         launch_inc_flip(&c);   // state += sol; sol = -sol for the line search
         double old_l2 = nm.l2;
-        launch_resid(&c);
-        launch_norms(&c);
-        (void)hipEventRecord(c.ev[7], c.stream);
+        launch_resid(&c, true);
         if ((rc = read_norms(c, &nm))) return rc;
         if (rep) {
-            rep->ms_load += elapsed(c, 3, 4);
-            rep->ms_setup += elapsed(c, 4, 5);
-            rep->ms_solve += elapsed(c, 5, 6);
-            rep->ms_resid += elapsed(c, 6, 7);
+            rep->ms_load += elapsed(c, TS_LOAD, TS_SETUP);
+            rep->ms_setup += elapsed(c, TS_SETUP, TS_SOLVE);
+            rep->ms_solve += elapsed(c, TS_SOLVE, TS_INC);
+            rep->ms_resid += elapsed(c, TS_INC, TS_NORMS);
             rep->lin_iterations += lin_it;
         }
         if (isnan(nm.l2) || isinf(nm.l2)) solv_flag = ADH_SW2_NO;
@@ -1247,8 +1240,7 @@ static int newton(Ctx &c, adh_sw2_report *rep, int *verdict) {
         while (nm.maxn > o.tol_nonlin && nm.l2 > old_l2 && cuts < o.max_cuts) {
             launch_scale_sol(&c, 0.5);
             launch_inc(&c, 1.0);
-            launch_resid(&c);
-            launch_norms(&c);
+            launch_resid(&c, true);
             if ((rc = read_norms(c, &nm))) return rc;
             cuts++;
         }
@@ -1263,7 +1255,7 @@ static int newton(Ctx &c, adh_sw2_report *rep, int *verdict) {
         rep->iterations += it;
         rep->converged = !failed;
         rep->solv_fail = solv_flag != ADH_SW2_YES;
-        rep->ms_total += elapsed(c, 0, 7);
+        rep->ms_total += elapsed(c, TS_INIT, TS_NORMS);
     }
     if (failed) {
         launch_init(&c, nullptr);  // fe_newton.c:883
@@ -1339,7 +1331,7 @@ static int krylov_batch(Ctx &c, const std::vector<int> &active, std::vector<int>
     int rc0 = krylov_one_kernel(c, true, &all_done0);
     if (rc0) return rc0;
     if (!all_done0) launch_krylov_prologue(&c);
-    // chunks as in krylov() with a zero guess (newton_batch zeroes sol): no
+    // chunks as in krylov() with a zero guess: no
     // host check between the prologue and the first chunk, the idempotent
     // epilogue queued behind every chunk before the flags are read
     int first, more;
@@ -1396,8 +1388,7 @@ static int newton_batch(Ctx &c, const std::vector<int> &run, adh_sw2_report *rep
     if ((rc = ensure_band(c))) return rc;   // the profile LU's bands, once per partition
     if ((rc = set_mask(c, run))) return rc;
     launch_init(&c, nullptr);   // masked: only the models of this attempt
-    launch_resid(&c);
-    launch_norms(&c);
+    launch_resid(&c, true);
     if ((rc = read_norms_all(c, nm))) return rc;
     std::vector<int> active(run), it(n, 0), solv(n, ADH_SW2_YES), lin_it, vd;
     for (int i = 0; i < n; i++)
@@ -1407,8 +1398,7 @@ static int newton_batch(Ctx &c, const std::vector<int> &run, adh_sw2_report *rep
         if ((rc = set_mask(c, active))) return rc;
         launch_jacobian(&c);
         launch_assemble(&c);
-        launch_zero(&c, c.sol, 3 * (size_t)c.Np);
-        launch_setup(&c);
+        launch_setup(&c, false);
         if ((rc = krylov_batch(c, active, lin_it, vd))) return rc;
         for (int i = 0; i < n; i++)
             if (active[i]) solv[i] = (o.precision >= 1) ? ADH_SW2_YES : vd[i];
@@ -1416,8 +1406,7 @@ static int newton_batch(Ctx &c, const std::vector<int> &run, adh_sw2_report *rep
         launch_inc_flip(&c);   // state += sol; sol = -sol for the line search
         std::vector<double> old_l2(n);
         for (int i = 0; i < n; i++) old_l2[i] = nm[i].l2;
-        launch_resid(&c);
-        launch_norms(&c);
+        launch_resid(&c, true);
         {
             // finished models keep their last norms (their correction
             // vector no longer belongs to them)
@@ -1437,8 +1426,7 @@ static int newton_batch(Ctx &c, const std::vector<int> &run, adh_sw2_report *rep
             if ((rc = set_mask(c, cut))) return rc;
             launch_scale_sol(&c, 0.5);
             launch_inc(&c, 1.0);
-            launch_resid(&c);
-            launch_norms(&c);
+            launch_resid(&c, true);
             std::vector<Norms> nm2;
             if ((rc = read_norms_all(c, nm2))) return rc;
             for (int i = 0; i < n; i++)
@@ -1709,8 +1697,7 @@ extern "C" int adh_sw2_hip_batch_residual_norm(adh_sw2_hip *h, double *maxn) {
     std::vector<Norms> nm;
     if ((rc = set_mask(c, std::vector<int>(c.ninst, 1)))) return rc;
     launch_init(&c, nullptr);
-    launch_resid(&c);
-    launch_norms(&c);
+    launch_resid(&c, true);
     if ((rc = read_norms_all(c, nm))) return rc;
     for (int i = 0; i < c.ninst; i++) maxn[i] = nm[i].maxn;
     return sync_check(c);

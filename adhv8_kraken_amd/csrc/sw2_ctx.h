@@ -90,13 +90,19 @@ struct TBand {
     size_t xoff;   // first DOF in the band-ordered vectors
 };
 
+enum { TS_INIT, TS_RESID, TS_LOAD, TS_SETUP, TS_SOLVE, TS_INC, TS_NORMS, TS_N };
+
 struct Ctx {
     int N, E, B, M, nnz;
     int Np;                // N rounded up to a multiple of 64 (node-slice padding)
     adh_sw2_opts opts;
     double dt;
     hipStream_t stream;
-    hipEvent_t ev[8];
+    hipEvent_t ev[2];      // autotuning
+    // Start times of a Newton step's phases, 100 MHz ticks: kernels store them in
+    // pinned memory (timed events would put a wait between the phases, 3 us each)
+    long long *h_ts;       // [TS_N]
+    double ts_ms;          // a tick in ms
 
     // node fields
     double *x, *y, *z;
@@ -252,6 +258,10 @@ struct Ctx {
     double *gm_host;       // pinned copy of gm_dev
 };
 
+__device__ __forceinline__ void stamp(long long *ts) {
+    if (ts && blockIdx.x == 0 && threadIdx.x == 0) *ts = wall_clock64();
+}
+
 // 3x3 block inverse by Gauss-Jordan with partial pivoting (block-Jacobi set-up)
 __device__ __forceinline__ void inv3(const double (&d)[9], double (&inv)[9]) {
     double a[3][6];
@@ -320,7 +330,7 @@ __device__ __forceinline__ int xcd_block() {
 
 // launchers (sw2_kernels.hip / sw2_solver.hip)
 void launch_old_terms(Ctx *c);
-void launch_resid(Ctx *c);
+void launch_resid(Ctx *c, bool norms = false);   // norms: with the Newton norms, into h_norms
 void launch_jacobian(Ctx *c);
 void launch_assemble(Ctx *c);
 void launch_init(Ctx *c, int *bc_mask_dev);
@@ -328,8 +338,7 @@ void launch_shift(Ctx *c);
 void launch_inc(Ctx *c, double factor_on_sol);   // state += sol
 void launch_scale_sol(Ctx *c, double f);          // sol *= f
 void launch_inc_flip(Ctx *c);                     // state += sol, then sol = -sol
-void launch_norms(Ctx *c);
-void launch_setup(Ctx *c);
+void launch_setup(Ctx *c, bool guess = true);   // guess: sol holds an initial guess, scaled with the system
 void launch_scal_init(Ctx *c, int max_it);
 void launch_krylov_prologue(Ctx *c);
 void launch_krylov_iters(Ctx *c, int k);

@@ -94,6 +94,7 @@ struct ElemData {
     const double *wind;
     const double *mat_windatt;
     double density;
+    long long *ts;             // where a Jacobian kernel stores its start time (null: nowhere)
 };
 
 HDF double elem_dt(const ElemData &D, int ie) { return D.dt_inst ? D.dt_inst[D.elem_inst[ie]] : D.dt; }

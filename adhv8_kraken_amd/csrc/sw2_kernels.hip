@@ -78,62 +78,158 @@ __global__ void __launch_bounds__(128) k_resid1d(ElemData D, int B, double *ER1)
 // residual[3n..] = -(sum of element contributions) in ascending element
 // order, 2D first then 1D; dry-node momentum contributions are dropped and
 // dry-node velocities zeroed (fe_sw2_resid.c:85-93, :154-162).
-__global__ void k_resid_gather(int N, const int *n2e_ptr, const int *n2e, const int *n2b_ptr, const int *n2b,
-                               const double *ER, const double *ER1, const double *old_head, double *u, double *v,
-                               double *R) {
-    int n = xcd_block() * blockDim.x + threadIdx.x;   // a node's elements are shared with its neighbours
-    if (n >= N) return;
-    bool dry = old_head[n] <= 0.;
-    double rx = 0.0, ry = 0.0, rc = 0.0;
-    const int k0 = n2e_ptr[n], k1 = n2e_ptr[n + 1];
-    int k = k0;
-    // batches of up to 8 contributions: the indices, then the values, are
-    // loaded before the (in-order) sums, so their latencies overlap
-    for (; k < k1; k += 8) {
-        const int m = min(8, k1 - k);
-        int sidx[8];
+// NORMS: also get_residual_norms (fe_newton.c:79-150) with
+// include_node_in_residual (:177-187), max norms over nodes with
+// min(h, h_old) > 0, l2 over all DOFs: block partials here, while the values
+// are in registers, reduced in block order by k_norms_fin.
+template <bool NORMS>
+__global__ void __launch_bounds__(256) k_resid_gather(int N, const int *n2e_ptr, const int *n2e,
+                                                      const int *n2b_ptr, const int *n2b, const double *ER,
+                                                      const double *ER1, const double *old_head, double *u, double *v,
+                                                      double *R, const double *sol, const double *h, double *part) {
+    const int lb = xcd_block();   // a node's elements are shared with its neighbours
+    const int n = lb * blockDim.x + threadIdx.x;
+    double rmax = 0.0, rsum = 0.0, imax = 0.0;
+    if (n < N) {
+        bool dry = old_head[n] <= 0.;
+        double rx = 0.0, ry = 0.0, rc = 0.0;
+        const int k0 = n2e_ptr[n], k1 = n2e_ptr[n + 1];
+        int k = k0;
+        // batches of up to 8 contributions: the indices, then the values, are
+        // loaded before the (in-order) sums, so their latencies overlap
+        for (; k < k1; k += 8) {
+            const int m = min(8, k1 - k);
+            int sidx[8];
 #pragma unroll
-        for (int t = 0; t < 8; t++) sidx[t] = t < m ? n2e[k + t] : 0;
-        double vx[8], vy[8], vc[8];
+            for (int t = 0; t < 8; t++) sidx[t] = t < m ? n2e[k + t] : 0;
+            double vx[8], vy[8], vc[8];
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const double *o = ER + 9 * (size_t)(sidx[t] / 3) + 3 * (sidx[t] % 3);
-            vx[t] = t < m ? o[0] : 0.0;
-            vy[t] = t < m ? o[1] : 0.0;
-            vc[t] = t < m ? o[2] : 0.0;
+            for (int t = 0; t < 8; t++) {
+                const double *o = ER + 3 * (size_t)sidx[t];   // 9 a triangle, 3 a node of it
+                vx[t] = t < m ? o[0] : 0.0;
+                vy[t] = t < m ? o[1] : 0.0;
+                vc[t] = t < m ? o[2] : 0.0;
+            }
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                if (t < m) {
+                    if (!dry) { rx -= vx[t]; ry -= vy[t]; }
+                    rc -= vc[t];
+                }
+            }
         }
+        for (int k = n2b_ptr[n]; k < n2b_ptr[n + 1]; k++) {
+            int s = n2b[k];
+            const double *o = ER1 + 3 * (size_t)s;
+            if (!dry) { rx -= o[0]; ry -= o[1]; }
+            rc -= o[2];
+        }
+        R[vidx3(n, 0)] = rx;
+        R[vidx3(n, 1)] = ry;
+        R[vidx3(n, 2)] = rc;
+        if (dry && (n2e_ptr[n + 1] > n2e_ptr[n] || n2b_ptr[n + 1] > n2b_ptr[n])) {
+            u[n] = 0.;
+            v[n] = 0.;
+        }
+        if constexpr (NORMS) {
+            const double r[3] = {rx, ry, rc};
+            const bool inc = dmin(h[n], old_head[n]) > 0;
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            if (t < m) {
-                if (!dry) { rx -= vx[t]; ry -= vy[t]; }
-                rc -= vc[t];
+            for (int j = 0; j < 3; j++) {
+                const double q = sol[vidx3(n, j)];
+                if (inc && fabs(r[j]) > rmax) rmax = fabs(r[j]);
+                if (inc && fabs(q) > imax) imax = fabs(q);
+                rsum += r[j] * r[j];
             }
         }
     }
-    for (int k = n2b_ptr[n]; k < n2b_ptr[n + 1]; k++) {
-        int s = n2b[k];
-        const double *o = ER1 + 6 * (size_t)(s / 2) + 3 * (s % 2);
-        if (!dry) { rx -= o[0]; ry -= o[1]; }
-        rc -= o[2];
-    }
-    R[vidx3(n, 0)] = rx;
-    R[vidx3(n, 1)] = ry;
-    R[vidx3(n, 2)] = rc;
-    if (dry && (n2e_ptr[n + 1] > n2e_ptr[n] || n2b_ptr[n + 1] > n2b_ptr[n])) {
-        u[n] = 0.;
-        v[n] = 0.;
+    if constexpr (NORMS) {
+        __shared__ double smax[256], ssum[256], sinc[256];
+        smax[threadIdx.x] = rmax; ssum[threadIdx.x] = rsum; sinc[threadIdx.x] = imax;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (threadIdx.x < w) {
+                smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + w]);
+                ssum[threadIdx.x] += ssum[threadIdx.x + w];
+                sinc[threadIdx.x] = fmax(sinc[threadIdx.x], sinc[threadIdx.x + w]);
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            part[3 * lb] = smax[0];
+            part[3 * lb + 1] = ssum[0];
+            part[3 * lb + 2] = sinc[0];
+        }
     }
 }
 
-void launch_resid(Ctx *c) {
+// the block partials of k_resid_gather, reduced in block order; the result
+// also goes straight to the host's pinned copy, so reading it is one wait
+// one block per model (blockIdx.x), over that model's 256-node blocks
+__global__ void __launch_bounds__(256) k_norms_fin(int nparts, int N, const double *part, Norms *out, Norms *host,
+                                                   const int *inst_blk0, const int *inst_nodes,
+                                                   long long *ts) {
+    __shared__ double smax[256], ssum[256], sinc[256];
+    const int m = blockIdx.x;
+    const int k0 = inst_blk0 ? inst_blk0[m] : 0, k1 = inst_blk0 ? inst_blk0[m + 1] : nparts;
+    if (inst_nodes) N = inst_nodes[m];
+    out += m;
+    double a = 0.0, b = 0.0, cc = 0.0;
+    // 8 strided partials per thread loaded together, folded in block order
+    const int bd = blockDim.x;
+    for (int k = k0 + threadIdx.x; k < k1; k += 8 * bd) {
+        double x[8][3];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+            for (int e = 0; e < 3; e++) x[u][e] = k + u * bd < k1 ? part[3 * (k + u * bd) + e] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k + u * bd < k1) {
+                a = fmax(a, x[u][0]);
+                b += x[u][1];
+                cc = fmax(cc, x[u][2]);
+            }
+    }
+    smax[threadIdx.x] = a; ssum[threadIdx.x] = b; sinc[threadIdx.x] = cc;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + w]);
+            ssum[threadIdx.x] += ssum[threadIdx.x + w];
+            sinc[threadIdx.x] = fmax(sinc[threadIdx.x], sinc[threadIdx.x + w]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        Norms r{};
+        r.maxn = smax[0];
+        r.l2 = sqrt(ssum[0] / (double)(N * 3));
+        r.incn = sinc[0];
+        *out = r;
+        host[m] = r;
+        if (m == 0) *ts = wall_clock64();
+    }
+}
+
+void launch_resid(Ctx *c, bool norms) {
     if (!c->pre_valid) launch_old_terms(c);
     ElemData D = c->ed;
     D.first_elem = c->first_elem;
     launch_resid2d_split(c, D);
-    if (c->B) hipLaunchKernelGGL(k_resid1d, dim3(nblocks_for(c->B, 128)), dim3(128), 0, c->stream, D, c->B,
-                                 c->ER + 9 * (size_t)c->E);
-    hipLaunchKernelGGL(k_resid_gather, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->n2e_ptr,
-                       c->n2e, c->n2b_ptr, c->n2b, c->ER, c->ER + 9 * (size_t)c->E, c->old_head, c->u, c->v, c->R);
+    double *er1 = c->ER + 9 * (size_t)c->E;
+    if (c->B) hipLaunchKernelGGL(k_resid1d, dim3(nblocks_for(c->B, 128)), dim3(128), 0, c->stream, D, c->B, er1);
+    const int nb = nblocks_for(c->N, 256);
+    if (!norms) {
+        hipLaunchKernelGGL(k_resid_gather<false>, dim3(nb), dim3(256), 0, c->stream, c->N, c->n2e_ptr, c->n2e,
+                           c->n2b_ptr, c->n2b, c->ER, er1, c->old_head, c->u, c->v, c->R, c->sol, c->head, c->red.part);
+        return;
+    }
+    hipLaunchKernelGGL(k_resid_gather<true>, dim3(nb), dim3(256), 0, c->stream, c->N, c->n2e_ptr, c->n2e, c->n2b_ptr,
+                       c->n2b, c->ER, er1, c->old_head, c->u, c->v, c->R, c->sol, c->head, c->red.part);
+    hipLaunchKernelGGL(k_norms_fin, dim3(c->ninst ? c->ninst : 1), dim3(256), 0, c->stream, nb, c->N, c->red.part,
+                       c->norms, c->h_norms, c->ninst ? c->inst_blk0 : nullptr, c->ninst ? c->inst_nodes : nullptr,
+                       c->h_ts + TS_NORMS);
 }
 
 // ------------------------------------------------------------------ Jacobian
@@ -150,6 +246,7 @@ template <bool WET, int BS, int OCC>
 __global__ void __launch_bounds__(BS, OCC > 0 ? OCC : 1) k_jac2d_list(ElemData D, const int *list, const int *count,
                                                                       int b0, int b1, int b2, const int *blkpos,
                                                                       double *EM, float *EM32) {
+    if (WET) stamp(D.ts);
     const int nt = 18 * *count;
     const int stride = gridDim.x * blockDim.x;
     int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -220,6 +317,7 @@ __global__ void __launch_bounds__(BS, OCC > 0 ? OCC : 1) k_jac2d_list(ElemData D
 template <bool WET, int BS>
 __global__ void __launch_bounds__(BS) k_jac2d_cols(ElemData D, const int *list, const int *count, int b0, int b1,
                                                    int b2, const int *blkpos, double *EM, float *EM32) {
+    if (WET) stamp(D.ts);
     constexpr int WPB = BS / 64;
     const int n = *count;
     const int nunits = 9 * ((n + 31) >> 5);
@@ -438,6 +536,7 @@ __device__ __forceinline__ void lds_column(const ElemData &DL, const SRC &S, int
 template <bool WET, int BS, int COLS>
 __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list, const int *count, int b0, int b1,
                                                   int b2, const int *blkpos, double *EM, float *EM32) {
+    if (WET) stamp(D.ts);
     constexpr int WPB = BS / 64, PARTS = 9 / COLS;
     __shared__ double srec[WPB][32][LREC];
     __shared__ crlog::tables slog;
@@ -568,8 +667,9 @@ __device__ __forceinline__ void split_class(int ie, int E, const int *e2d, const
 }
 
 __global__ void __launch_bounds__(256) k_split_count(int E, const int *e2d, const double *head, const int *elem_inst,
-                                                     const int *mask, int *bcount) {
+                                                     const int *mask, int *bcount, long long *ts) {
     __shared__ int wc[2][4];
+    stamp(ts);
     const int ie = blockIdx.x * blockDim.x + threadIdx.x;
     bool w, g;
     split_class(ie, E, e2d, head, elem_inst, mask, w, g);
@@ -585,84 +685,31 @@ __global__ void __launch_bounds__(256) k_split_count(int E, const int *e2d, cons
     }
 }
 
-// exclusive scans of the two block-count arrays (one block of 1024 threads,
-// each owning a contiguous run of up to SCAN_R counts of both arrays, held in
-// registers from one load to the write-back, so the kernel waits on memory
-// once); counts[0] = wet total, counts[1] = general total.  Longer runs
-// (more than 8,192 count blocks, i.e. over 2M triangles) loop over chunks.
-constexpr int SCAN_T = 1024, SCAN_R = 8;
-__device__ __forceinline__ void scan_pair(int s0, int s1, int &run0, int &run1, int &tot0, int &tot1) {
-    __shared__ int wsum[2][SCAN_T / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int x0 = s0, x1 = s1;   // inclusive scans within the wave
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y0 = __shfl_up(x0, o, 64), y1 = __shfl_up(x1, o, 64);
-        if (lane >= o) { x0 += y0; x1 += y1; }
-    }
-    if (lane == 63) { wsum[0][wid] = x0; wsum[1][wid] = x1; }
-    __syncthreads();
-    run0 = x0 - s0; run1 = x1 - s1; tot0 = 0; tot1 = 0;
-    for (int w = 0; w < SCAN_T / 64; w++) {
-        if (w < wid) { run0 += wsum[0][w]; run1 += wsum[1][w]; }
-        tot0 += wsum[0][w];
-        tot1 += wsum[1][w];
-    }
-}
-
-__global__ void __launch_bounds__(SCAN_T) k_split_scan(int nb, int *bcount, int *counts) {
-    int *bc0 = bcount, *bc1 = bcount + nb;
-    const int per = (nb + SCAN_T - 1) / SCAN_T, b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
-    int run0, run1, tot0, tot1;
-    if (per <= SCAN_R) {
-        int v0[SCAN_R], v1[SCAN_R], s0 = 0, s1 = 0;
-#pragma unroll
-        for (int u = 0; u < SCAN_R; u++) {
-            v0[u] = b0 + u < b1 ? bc0[b0 + u] : 0;
-            v1[u] = b0 + u < b1 ? bc1[b0 + u] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < SCAN_R; u++) { s0 += v0[u]; s1 += v1[u]; }
-        scan_pair(s0, s1, run0, run1, tot0, tot1);
-#pragma unroll
-        for (int u = 0; u < SCAN_R; u++)
-            if (b0 + u < b1) {
-                bc0[b0 + u] = run0; run0 += v0[u];
-                bc1[b0 + u] = run1; run1 += v1[u];
-            }
-    } else {
-        int s0 = 0, s1 = 0;
-        for (int b = b0; b < b1; b += SCAN_R) {
-            int v0[SCAN_R], v1[SCAN_R];
-#pragma unroll
-            for (int u = 0; u < SCAN_R; u++) {
-                v0[u] = b + u < b1 ? bc0[b + u] : 0;
-                v1[u] = b + u < b1 ? bc1[b + u] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < SCAN_R; u++) { s0 += v0[u]; s1 += v1[u]; }
-        }
-        scan_pair(s0, s1, run0, run1, tot0, tot1);
-        for (int b = b0; b < b1; b += SCAN_R) {
-            int v0[SCAN_R], v1[SCAN_R];
-#pragma unroll
-            for (int u = 0; u < SCAN_R; u++) {
-                v0[u] = b + u < b1 ? bc0[b + u] : 0;
-                v1[u] = b + u < b1 ? bc1[b + u] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < SCAN_R; u++)
-                if (b + u < b1) {
-                    bc0[b + u] = run0; run0 += v0[u];
-                    bc1[b + u] = run1; run1 += v1[u];
-                }
-        }
-    }
-    if (threadIdx.x == 0) { counts[0] = tot0; counts[1] = tot1; }
-}
-
+// A block's place in the two lists is the sum of the counts before it, which
+// it adds up itself: 1M triangles, 3,906 counts, take less time that way than
+// a scan kernel's launch (3.5 us), and fewer take next to none.  The last block
+// leaves the totals in counts.
 __global__ void __launch_bounds__(256) k_split_write(int E, const int *e2d, const double *head, const int *elem_inst,
-                                                     const int *mask, const int *boff, int *wet, int *gen) {
-    __shared__ int wc[2][4];
+                                                     const int *mask, const int *bcount, int *counts, int *wet,
+                                                     int *gen) {
+    __shared__ int wc[2][4], before[2][4];
+    {
+        int s0 = 0, s1 = 0;
+        constexpr int U = 4;
+        for (int b = threadIdx.x; b < (int)blockIdx.x; b += U * 256) {
+            int x[U][2];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool in = b + u * 256 < (int)blockIdx.x;
+                x[u][0] = in ? bcount[b + u * 256] : 0;
+                x[u][1] = in ? bcount[gridDim.x + b + u * 256] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) { s0 += x[u][0]; s1 += x[u][1]; }
+        }
+        for (int o = 32; o > 0; o >>= 1) { s0 += __shfl_xor(s0, o, 64); s1 += __shfl_xor(s1, o, 64); }
+        if ((threadIdx.x & 63) == 0) { before[0][threadIdx.x >> 6] = s0; before[1][threadIdx.x >> 6] = s1; }
+    }
     const int ie = blockIdx.x * blockDim.x + threadIdx.x;
     bool w, g;
     split_class(ie, E, e2d, head, elem_inst, mask, w, g);
@@ -673,11 +720,16 @@ __global__ void __launch_bounds__(256) k_split_write(int E, const int *e2d, cons
         wc[1][wid] = __popcll(bg);
     }
     __syncthreads();
-    int bef_w = 0, bef_g = 0;  // triangles of each class in earlier waves of this block
+    int bef_w = before[0][0] + before[0][1] + before[0][2] + before[0][3];   // of each class before this wave
+    int bef_g = before[1][0] + before[1][1] + before[1][2] + before[1][3];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        counts[0] = bef_w + wc[0][0] + wc[0][1] + wc[0][2] + wc[0][3];
+        counts[1] = bef_g + wc[1][0] + wc[1][1] + wc[1][2] + wc[1][3];
+    }
     for (int k = 0; k < wid; k++) { bef_w += wc[0][k]; bef_g += wc[1][k]; }
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    if (w) wet[boff[blockIdx.x] + bef_w + __popcll(bw & below)] = ie;
-    if (g) gen[boff[gridDim.x + blockIdx.x] + bef_g + __popcll(bg & below)] = ie;
+    if (w) wet[bef_w + __popcll(bw & below)] = ie;
+    if (g) gen[bef_g + __popcll(bg & below)] = ie;
 }
 
 // ordered wet / general triangle lists for the current depths (and, for
@@ -687,10 +739,9 @@ static void launch_split(Ctx *c) {
     const int nb = nblocks_for(c->E, 256);
     const int *mask = c->ninst ? c->inst_mask : nullptr;
     hipLaunchKernelGGL(k_split_count, dim3(nb), dim3(256), 0, c->stream, c->E, c->e2d, c->head, c->elem_inst, mask,
-                       c->esplit);
-    hipLaunchKernelGGL(k_split_scan, dim3(1), dim3(SCAN_T), 0, c->stream, nb, c->esplit, c->ecount);
+                       c->esplit, c->h_ts + TS_RESID);
     hipLaunchKernelGGL(k_split_write, dim3(nb), dim3(256), 0, c->stream, c->E, c->e2d, c->head, c->elem_inst, mask,
-                       c->esplit, c->elist_wet, c->elist_gen);
+                       c->esplit, c->ecount, c->elist_wet, c->elist_gen);
     c->split_valid = 1;
 }
 
@@ -796,6 +847,7 @@ void launch_jacobian(Ctx *c) {
     if (!c->pre_valid) launch_old_terms(c);
     ElemData D = c->ed;
     D.first_elem = nullptr;
+    D.ts = c->h_ts + TS_LOAD;
     c->em32 = em32_of(c) != nullptr;
     launch_jac2d_split(c, D);
     if (c->B)
@@ -941,7 +993,8 @@ void launch_assemble_only(Ctx *c) { launch_assemble(c); }
 // fe_sw2_init (fe_sw2_init.c:33-79)
 __global__ void k_init_nodes(int N, const double *old_head, const double *old_u, const double *old_v, double *head,
                              double *u, double *v, const int *node_bc, const double *bcval, int *bc_mask,
-                             int *wd_tmp, const int *node_inst, const int *mask) {
+                             int *wd_tmp, const int *node_inst, const int *mask, long long *ts) {
+    stamp(ts);
     int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
     if (mask && (node_inst[n] < 0 || !mask[node_inst[n]])) return;  // gap nodes (-1) never change
@@ -1005,7 +1058,7 @@ void launch_init(Ctx *c, int *bc_mask_dev) {
     const int *mask = c->ninst ? c->inst_mask : nullptr;
     hipLaunchKernelGGL(k_init_nodes, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->old_head,
                        c->old_u, c->old_v, c->head, c->u, c->v, c->node_bc, c->node_bc_val, bc_mask_dev, c->wd_tmp,
-                       c->node_inst, mask);
+                       c->node_inst, mask, c->h_ts + TS_INIT);
     if (c->E) {
         hipLaunchKernelGGL(k_wd_mark, dim3(nblocks_for(c->E, 256)), dim3(256), 0, c->stream, c->E, c->e2d, c->head,
                            c->wd_tmp, c->elem_inst, mask);
@@ -1053,7 +1106,8 @@ void launch_inc(Ctx *c, double) {
 // fe_sw2_inc, then sol = -sol (what the line search steps back along), in one
 // pass over the nodes: the same operations as k_inc followed by k_scale_vec(-1)
 __global__ void k_inc_flip(int N, double *sol, double *h, double *u, double *v, const int *node_inst,
-                           const int *mask) {
+                           const int *mask, long long *ts) {
+    stamp(ts);
     int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
     if (mask && (node_inst[n] < 0 || !mask[node_inst[n]])) return;  // gap nodes (-1) never change
@@ -1069,7 +1123,7 @@ __global__ void k_inc_flip(int N, double *sol, double *h, double *u, double *v, 
 void launch_inc_flip(Ctx *c) {
     c->split_valid = 0;
     hipLaunchKernelGGL(k_inc_flip, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->sol, c->head, c->u,
-                       c->v, c->node_inst, c->ninst ? c->inst_mask : nullptr);
+                       c->v, c->node_inst, c->ninst ? c->inst_mask : nullptr, c->h_ts + TS_INC);
 }
 
 // x *= f over a sliced node vector; entry i belongs to node 64 (i / 192) + i mod 64
@@ -1124,94 +1178,5 @@ void launch_probe(const double *x, int n, const crlog::tables *t, double *lg, do
     hipLaunchKernelGGL(k_probe, dim3(nblocks_for(n, 256)), dim3(256), 0, 0, x, n, t, lg, sq, dv);
 }
 
-// ------------------------------------------------------------------- norms
-// get_residual_norms (fe_newton.c:79-150) with include_node_in_residual
-// (:177-187): max norms over nodes with min(h, h_old) > 0, l2 over all DOFs.
-// Block partials, then a one-block finisher reduces them in block order.
-__global__ void __launch_bounds__(256) k_norms(int N, const double *R, const double *sol, const double *h,
-                                               const double *oh, double *part) {
-    __shared__ double smax[256], ssum[256], sinc[256];
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
-    double m = 0.0, s = 0.0, in = 0.0;
-    if (n < N) {
-        bool inc = dmin(h[n], oh[n]) > 0;
-        for (int j = 0; j < 3; j++) {
-            double r = R[vidx3(n, j)], q = sol[vidx3(n, j)];
-            if (inc && fabs(r) > m) m = fabs(r);
-            if (inc && fabs(q) > in) in = fabs(q);
-            s += r * r;
-        }
-    }
-    smax[threadIdx.x] = m; ssum[threadIdx.x] = s; sinc[threadIdx.x] = in;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + w]);
-            ssum[threadIdx.x] += ssum[threadIdx.x + w];
-            sinc[threadIdx.x] = fmax(sinc[threadIdx.x], sinc[threadIdx.x + w]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[3 * blockIdx.x] = smax[0];
-        part[3 * blockIdx.x + 1] = ssum[0];
-        part[3 * blockIdx.x + 2] = sinc[0];
-    }
-}
-
-// one block: the block partials of k_norms, reduced in block order; the result
-// also goes straight to the host's pinned copy, so reading it is one wait
-// one block per model (blockIdx.x), over that model's 256-node blocks
-__global__ void __launch_bounds__(256) k_norms_fin(int nparts, int N, const double *part, Norms *out, Norms *host,
-                                                   const int *inst_blk0, const int *inst_nodes) {
-    __shared__ double smax[256], ssum[256], sinc[256];
-    const int m = blockIdx.x;
-    const int k0 = inst_blk0 ? inst_blk0[m] : 0, k1 = inst_blk0 ? inst_blk0[m + 1] : nparts;
-    if (inst_nodes) N = inst_nodes[m];
-    out += m;
-    double a = 0.0, b = 0.0, cc = 0.0;
-    // 8 strided partials per thread loaded together, folded in block order
-    const int bd = blockDim.x;
-    for (int k = k0 + threadIdx.x; k < k1; k += 8 * bd) {
-        double x[8][3];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-#pragma unroll
-            for (int e = 0; e < 3; e++) x[u][e] = k + u * bd < k1 ? part[3 * (k + u * bd) + e] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (k + u * bd < k1) {
-                a = fmax(a, x[u][0]);
-                b += x[u][1];
-                cc = fmax(cc, x[u][2]);
-            }
-    }
-    smax[threadIdx.x] = a; ssum[threadIdx.x] = b; sinc[threadIdx.x] = cc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + w]);
-            ssum[threadIdx.x] += ssum[threadIdx.x + w];
-            sinc[threadIdx.x] = fmax(sinc[threadIdx.x], sinc[threadIdx.x + w]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        Norms r{};
-        r.maxn = smax[0];
-        r.l2 = sqrt(ssum[0] / (double)(N * 3));
-        r.incn = sinc[0];
-        *out = r;
-        host[m] = r;
-    }
-}
-
-void launch_norms(Ctx *c) {
-    int nb = nblocks_for(c->N, 256);
-    hipLaunchKernelGGL(k_norms, dim3(nb), dim3(256), 0, c->stream, c->N, c->R, c->sol, c->head, c->old_head,
-                       c->red.part);
-    hipLaunchKernelGGL(k_norms_fin, dim3(c->ninst ? c->ninst : 1), dim3(256), 0, c->stream, nb, c->N, c->red.part,
-                       c->norms, c->h_norms, c->ninst ? c->inst_blk0 : nullptr, c->ninst ? c->inst_nodes : nullptr);
-}
 
 }  // namespace sw2

@@ -80,13 +80,14 @@ template <bool F32, bool BJ, int K, bool SRC32 = false>
 __global__ void __launch_bounds__(256) k_scale_apply(int N, double *diag, double *offd, const int *row_ptr,
                                                      const int *sell_ptr, const int *sell_col, const double *sv,
                                                      double *R, double *sol, double *dinv, float *diag32,
-                                                     float *offd32, float *dinv32) {
+                                                     float *offd32, float *dinv32, long long *ts) {
+    stamp(ts);
     int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
     double rf[3] = {sv[vidx3(n, 0)], sv[vidx3(n, 1)], sv[vidx3(n, 2)]};
     for (int j = 0; j < 3; j++) {
         R[vidx3(n, j)] *= rf[j];
-        sol[vidx3(n, j)] /= rf[j];
+        if (sol) sol[vidx3(n, j)] /= rf[j];
     }
     double d[9];
     for (int j = 0; j < 3; j++)
@@ -148,12 +149,12 @@ __global__ void k_to_f32(size_t n, const double *a, float *b) {
     do {                                                                                                            \
         if (F32 && c->mat32)                                                                                        \
             hipLaunchKernelGGL((k_scale_apply<F32, BJ, K, true>), dim3(nb), dim3(256), 0, c->stream, c->N, c->diag, \
-                               c->offd, c->row_ptr, c->sell_ptr, c->sell_col, c->scale, c->R, c->sol, c->dinv,      \
-                               c->diag32, c->offd32, c->dinv32);                                                    \
+                               c->offd, c->row_ptr, c->sell_ptr, c->sell_col, c->scale, c->R, x0, c->dinv,          \
+                               c->diag32, c->offd32, c->dinv32, c->h_ts + TS_SETUP);                                \
         else                                                                                                        \
             hipLaunchKernelGGL((k_scale_apply<F32, BJ, K, false>), dim3(nb), dim3(256), 0, c->stream, c->N,         \
                                c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, c->scale, c->R, c->sol,      \
-                               c->dinv, c->diag32, c->offd32, c->dinv32);                                           \
+                               c->dinv, c->diag32, c->offd32, c->dinv32, c->h_ts + TS_SETUP);                       \
     } while (0)
 #define SW2_SCALE_SWITCH(F32, BJ)                           \
     switch (c->kuni) {                                      \
@@ -164,7 +165,8 @@ __global__ void k_to_f32(size_t n, const double *a, float *b) {
         default: SW2_SCALE_LAUNCH(F32, BJ, 0); break;       \
     }
 
-void launch_setup(Ctx *c) {
+void launch_setup(Ctx *c, bool guess) {
+    double *x0 = guess ? c->sol : nullptr;
     int nb = nblocks_for(c->N, 256);
     if (!c->scale_valid)   // a matrix the assembly did not produce: its row maxima first
         hipLaunchKernelGGL(k_scale_rows, dim3(nb), dim3(256), 0, c->stream, c->N, c->diag, c->offd, c->row_ptr,
@@ -651,9 +653,9 @@ __global__ void __launch_bounds__(256) k_pl_omega(int N, KVecs<P> V, double *par
 }
 
 // solv_return_old (src/solver/solv_return_old.c:23-30): sol = (u + u0) * scale,
-// u0 the initial guess held in sol.  ZERO: the caller zeroed the guess (the
-// Newton step does), so u0 = +0 enters as a constant and the kernel gives the
-// same sol however often it runs.  r (one LU of the whole matrix, or null): a
+// u0 the initial guess held in sol.  ZERO: the guess is zero (the Newton
+// step's); sol is not read, u0 = +0 enters as a constant and the kernel gives
+// the same sol however often it runs.  r (one LU of the whole matrix, or null): a
 // model whose solve ended at the prologue takes its preconditioned residual
 // r = M^-1 (b - A u), which the prologue has formed to test it, as one step of
 // refinement when the factorisation has lost digits (|r| above REFINE_ABOVE
@@ -682,7 +684,9 @@ __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, 
 
 // every model's scalars at the start of a solve; a model that the mask leaves
 // out may take no iteration
-__global__ void k_scal_init(int n, KScal *sc, double atol, double rtol, int max_it, const int *mask) {
+__global__ void k_scal_init(int n, KScal *sc, double atol, double rtol, int max_it, const int *mask,
+                            long long *ts) {
+    stamp(ts);
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= n) return;
     KScal r{};
@@ -695,7 +699,7 @@ __global__ void k_scal_init(int n, KScal *sc, double atol, double rtol, int max_
 void launch_scal_init(Ctx *c, int max_it) {
     const int n = NFIN(c);
     hipLaunchKernelGGL(k_scal_init, dim3(nblocks_for(n, 64)), dim3(64), 0, c->stream, n, c->ksc, c->opts.lin_atol,
-                       c->opts.lin_rtol, max_it, c->ninst ? c->inst_mask : nullptr);
+                       c->opts.lin_rtol, max_it, c->ninst ? c->inst_mask : nullptr, c->h_ts + TS_SOLVE);
 }
 
 template <typename P, int K>
