@@ -88,6 +88,12 @@ struct TBand {
     size_t off;    // first double of the band
     size_t toff;   // first tile in the per-tile inverse arrays
     size_t xoff;   // first DOF in the band-ordered vectors
+    // A block factored from both ends (sw2_lu.hip) is two bands that share its
+    // middle rows, their rows from 64 na on; else na = nt and part = -1.
+    int na;        // panels before the shared rows
+    int part;      // the other band, -1: none
+    int rev;       // 1: the block's rows from its last one upwards
+    int mtot;      // the block's DOFs
 };
 
 enum { TS_INIT, TS_RESID, TS_LOAD, TS_SETUP, TS_SOLVE, TS_INC, TS_NORMS, TS_N };
@@ -240,7 +246,10 @@ struct Ctx {
     size_t tb_size;
     TBand *tb_bands;
     double *tb_AB, *tb_LI, *tb_UI, *tb_xb, *tb_yb, *tb_zb;
-    int *tb_int, *tb_guard;   // sweep tickets [2 bands], then a guard flag per tile (tb_guard)
+    int *tb_int, *tb_guard;   // sweep tickets [3 bands], then a guard flag per tile (tb_guard)
+    int tb_nbot;           // bands running upwards, before all others; block b's other band is tb_nbot + b
+    int tb_maxs;           // shared rows of the block with most of them
+    std::vector<int> tb_h_na;   // host copy: panels before the shared rows, -1: a block in one band
     // block ILU(0) in multicolour order (preconditioner 3), built on demand
     int ilu_ready, ilu_ncolor, ilu_Rp, ilu_f32;
     size_t ilu_nl, ilu_nu;                 // lower / upper slots (64 per slice slot)

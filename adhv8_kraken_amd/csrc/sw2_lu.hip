@@ -26,19 +26,28 @@
 //              with the guarded pivots) on the matrix cores; the workgroup of the
 //              first tile, the next panel's diagonal block, goes on to factor
 //              it and to invert both factors (lu64).
-// k_tb_diag factors panel 0's diagonal block.  Then k_tb_inv forms G_k = U~^-1
-// L^-1 of every diagonal block and k_tb_scale multiplies every off-diagonal tile
-// by its column's, so that the substitutions are matrix-vector work in which
-// only a tile's input is serial: k_tb_sweep runs both as one dataflow kernel
-// (y_i = x_i - sum (A_ik G_k) y_k, then upwards), k_tb_apply the diagonal inverses.
+// k_tb_diag factors the diagonal blocks that no panel comes before.  Then
+// k_tb_inv forms G_k = U~^-1 L^-1 of every diagonal block and k_tb_scale
+// multiplies every off-diagonal tile by its column's, so that the substitutions
+// are matrix-vector work in which only a tile's input is serial: k_tb_sweep runs
+// both as a dataflow (y_i = x_i - sum (A_ik G_k) y_k, then upwards), k_tb_apply
+// the diagonal inverses.
 //
-// A chain of m / 64 dependent panels bounds both.  200 x 100 cells (m 60,903,
-// w 308, 952 panels): a panel 22.2 us, of which the diagonal block's LU 11.7
-// (189 cycles per pivot in the panel wave, which issues on 150 of them),
-// the tile's three products 3.8 at the matrix cores' FP64 rate, the rest load
-// latency and the launch (substitution and update in two launches, vector FMAs,
-// LU by readlane broadcasts: 9.6 + 21.7 us); a sweep step 1.9 us (a launch
-// per tile: 3.5).
+// A chain of dependent panels bounds both, so a long block is factored from both
+// ends at once: two bands, one of them in reverse order, down to the rows in the
+// middle that both reach (at least w of them).  Those belong to the band from the
+// start, which adds the other's updates (k_tb_merge) and goes on through them.
+// A sweep starts from both ends too, and the shared rows add the two; after them
+// the ends are independent again.  Blocks of all models reach their shared rows
+// at one launch, so each merges where the others do.
+//
+// 200 x 100 cells (m 60,903, w 308, 952 panels; from both ends 473 and 6 shared):
+// factorisation 10.8 ms (21.1 from one end), both sweeps 1.84 ms (3.58).  A panel
+// takes 22.2 us, of which the diagonal block's LU 11.7 (189 cycles per pivot in
+// the panel wave, which issues on 150 of them), the tile's three products 3.8 at
+// the matrix cores' FP64 rate, the rest load latency and the launch
+// (substitution and update in two launches, vector FMAs, LU by readlane
+// broadcasts: 9.6 + 21.7 us); a sweep step 1.9 us (a launch per tile: 3.5).
 #include <limits.h>
 
 #include <algorithm>
@@ -81,7 +90,7 @@ __device__ __forceinline__ d4 mfma4(double x, double y, d4 d) {
 __device__ __forceinline__ TBand band_rec(const TBand *bands, int b, int flag = 0) {
     const TBand B = bands[b];
     asm volatile("" ::"s"(B.m), "s"(B.w), "s"(B.wp), "s"(B.nt), "s"(B.inst), "s"(B.off), "s"(B.toff), "s"(B.xoff),
-                 "s"(flag));
+                 "s"(B.na), "s"(B.part), "s"(B.rev), "s"(B.mtot), "s"(flag));
     return B;
 }
 
@@ -90,19 +99,25 @@ __device__ __forceinline__ double guarded(double piv) { return fabs(piv) > SMALL
 // Scaled matrix (diagonal blocks and SELL off-diagonal blocks) into the bands;
 // the bands are zeroed before.  Ensembles: nodes of no block (the gaps between
 // models) and models outside the mask are skipped.
-__global__ void k_tb_load(int N, const int *node_blk, const TBand *bands, double *AB, const double *diag,
+__global__ void k_tb_load(int N, const int *node_blk, const TBand *bands, int nbot, double *AB, const double *diag,
                           const double *offd, const int *row_ptr, const int *sell_ptr, const int *sell_col,
                           const int *mask) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= N) return;
     const int bk = node_blk[a];
     if (bk < 0) return;
-    const TBand B = bands[bk];
+    const TBand B = bands[nbot + bk];
     if (mask && !mask[B.inst]) return;
-    const int n1 = B.n0 + B.m / 3;
+    const TBand Q = bands[max(B.part, 0)];
+    // what touches a row past the shared ones belongs to the band from the end
+    auto put = [&](int i, int j, double v) {
+        if (i < B.m && j < B.m) tb_at(AB, B, i, j) = v;
+        else tb_at(AB, Q, B.mtot - 1 - i, B.mtot - 1 - j) = v;
+    };
+    const int n1 = B.n0 + B.mtot / 3;
     const int ia = 3 * (a - B.n0);
     for (int r = 0; r < 3; r++)
-        for (int cc = 0; cc < 3; cc++) tb_at(AB, B, ia + r, ia + cc) = diag[didx9(a, 3 * r + cc)];
+        for (int cc = 0; cc < 3; cc++) put(ia + r, ia + cc, diag[didx9(a, 3 * r + cc)]);
     const size_t q0 = 64 * (size_t)sell_ptr[a >> 6] + (a & 63);
     const int len = row_ptr[a + 1] - row_ptr[a];
     for (int s = 0; s < len; s++) {
@@ -111,7 +126,7 @@ __global__ void k_tb_load(int N, const int *node_blk, const TBand *bands, double
         if (cn < B.n0 || cn >= n1) continue;
         const int jc = 3 * (cn - B.n0);
         for (int r = 0; r < 3; r++)
-            for (int cc = 0; cc < 3; cc++) tb_at(AB, B, ia + r, jc + cc) = offd[sell_vidx(q, 3 * r + cc)];
+            for (int cc = 0; cc < 3; cc++) put(ia + r, jc + cc, offd[sell_vidx(q, 3 * r + cc)]);
     }
 }
 
@@ -373,14 +388,15 @@ __device__ __forceinline__ void lu64(d4 (&D)[2], Lu64 &S, double *LI, double *UI
     if (threadIdx.x == 0) *guard = S.hit;   // every pivot was before the last barriers
 }
 
-// Panel 0's diagonal block, one workgroup per band (every later panel's is
-// factored by k_tb_step of the panel before, which updates it last).
+// Panel 0's diagonal block, one workgroup per band, or with `shared` that of the
+// shared rows' first panel (every other panel's is factored by k_tb_step of the
+// panel before, which updates it last).
 __global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const double *AB, double *LI, double *UI,
-                                                   int *guard, const int *mask) {
+                                                   int *guard, bool shared, const int *mask) {
     __shared__ Lu64 S;
     const TBand B = band_rec(bands, blockIdx.x);
-    if (mask && !mask[B.inst]) return;
-    const int kb = min(TB, B.m);
+    if ((mask && !mask[B.inst]) || (shared && (B.part < 0 || B.rev))) return;
+    const int k = shared ? B.na : 0, c0 = k * TB, kb = min(TB, B.m - c0);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wi = wv & 3, wj = wv >> 2, lo = lane & 15, hi = lane >> 4;
     d4 D[2];
@@ -390,10 +406,22 @@ __global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const dou
 #pragma unroll
         for (int r = 0; r < 4; r++) {   // past a short block: the identity
             const int j = 32 * wj + 16 * t + hi + 4 * r;
-            const double v = tb_get(AB, B, min(i, kb - 1), min(j, kb - 1));
+            const double v = tb_get(AB, B, c0 + min(i, kb - 1), c0 + min(j, kb - 1));
             D[t][r] = (i < kb && j < kb) ? v : (i == j ? 1.0 : 0.0);
         }
-    lu64(D, S, LI + 4096 * B.toff, UI + 4096 * B.toff, guard + B.toff, lane, wi, wj);
+    lu64(D, S, LI + 4096 * (B.toff + k), UI + 4096 * (B.toff + k), guard + B.toff + k, lane, wi, wj);
+}
+
+// The band from the end's updates of the shared rows onto the other band's, which
+// hold the matrix: one workgroup per column.
+__global__ void __launch_bounds__(256) k_tb_merge(const TBand *bands, double *AB, const int *mask) {
+    const TBand B = band_rec(bands, blockIdx.y);
+    if (B.part < 0 || B.rev || (mask && !mask[B.inst])) return;
+    const int j = TB * B.na + blockIdx.x;
+    if (j >= B.m) return;
+    const TBand Q = bands[B.part];
+    for (int i = max(TB * B.na, j - B.w) + (int)threadIdx.x; i < min(B.m, j + B.w + 1); i += 256)
+        tb_at(AB, B, i, j) += tb_get(AB, Q, B.mtot - 1 - i, B.mtot - 1 - j);
 }
 
 // Panel k: the trailing window A[r0:r1, r0:r1] -= (A[r0:r1, panel] U_k^-1) (L_k^-1 A[panel, r0:r1])
@@ -408,14 +436,17 @@ __global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const dou
 // block, not the matrix cores, are what a panel waits for.  The workgroup of the
 // window's first tile, the next panel's diagonal block, goes on to factor it.
 __global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, double *AB, double *LI, double *UI, int *guard,
-                                                int k, int gt, const int *mask) {
+                                                   int step, int amax, int gt, const int *mask) {
     constexpr int LD = TB + 2;   // operand reads of 16 rows x 2 columns hit distinct banks
     __shared__ union {
         struct { double Xs[TB * LD], Us[TB * LD], Ls[4][16][64]; } p;
         Lu64 S;
     } sm;
     const TBand B = band_rec(bands, blockIdx.y);
-    if (k + 1 >= B.nt || (mask && !mask[B.inst])) return;   // the last panel has no window
+    // the bands of blocks factored from both ends reach their shared rows at one step, amax
+    const int k = B.part < 0 ? step : step - (amax - B.na);
+    if (k < 0 || k + 1 >= B.nt || (mask && !mask[B.inst])) return;   // the last panel has no window
+    if (B.rev && k >= B.na) return;
     const int c0 = k * TB;
     const int r0 = c0 + TB, r1 = min(B.m, r0 + B.w);
     const int I = blockIdx.x % gt, J = blockIdx.x / gt;
@@ -500,7 +531,7 @@ __global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, double *A
             C[t][r] = C[t][r] - acc[t][r];
             if (i < cl && j < cl) tb_at(AB, B, i, j) = C[t][r];
         }
-    if (!next) return;
+    if (!next || k + 1 == B.na) return;   // the shared rows' first panel waits for k_tb_merge
     const int kb1 = min(TB, B.m - r0);
 #pragma unroll
     for (int t = 0; t < 2; t++)
@@ -527,7 +558,7 @@ __global__ void __launch_bounds__(64) k_tb_inv(const TBand *bands, const double 
     __shared__ double X[TB][TB + 1];
     const TBand B = band_rec(bands, blockIdx.y);
     const int k = blockIdx.x;
-    if (k >= B.nt || (mask && !mask[B.inst])) return;
+    if (k >= (B.rev ? B.na : B.nt) || (mask && !mask[B.inst])) return;
     const int c0 = k * TB, kb = min(TB, B.m - c0), t = threadIdx.x;
     double *Lk = LI + 4096 * (B.toff + k), *Uk = UI + 4096 * (B.toff + k);
     const int lo = t & 15, hi = t >> 4;
@@ -589,7 +620,7 @@ __global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB
     __shared__ double Ms[TB][TB + 1];   // Ms[q][col]: the inverse
     const TBand B = band_rec(bands, blockIdx.z);
     const int k = blockIdx.x;
-    if (k >= B.nt || (mask && !mask[B.inst])) return;
+    if (k >= (B.rev ? B.na : B.nt) || (mask && !mask[B.inst])) return;
     const bool low = (int)blockIdx.y < gf;
     const int g = (low ? (int)blockIdx.y : (int)blockIdx.y - gf) + 1;
     const int c0 = k * TB, kb = min(TB, B.m - c0);
@@ -669,22 +700,26 @@ __device__ __forceinline__ double await_value(const double *p, bool want) {
     return __longlong_as_double((long long)u);
 }
 
-// The right-hand side into band order (nodes of no block skipped), the two
-// output vectors to NOT_YET, the tickets to zero.
-__global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, const int *node_blk, const TBand *bands,
-                                                   const double *x, double *xb, double *yb, double *zb, int *tick) {
+// The right-hand side into band order (nodes of no block skipped; the band from
+// the end has zeros on the shared rows), the two output vectors to NOT_YET, the
+// tickets to zero.
+__global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, int nbot, const int *node_blk,
+                                                   const TBand *bands, const double *x, double *xb, double *yb,
+                                                   double *zb, int *tick) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int b = a; b < 2 * nband; b += gridDim.x * blockDim.x) tick[b] = 0;
+    for (int b = a; b < 3 * nband; b += gridDim.x * blockDim.x) tick[b] = 0;
     if (a >= N) return;
     const int bk = node_blk[a];
     if (bk < 0) return;
-    const TBand B = bands[bk];
-    const size_t o = B.xoff + 3 * (size_t)(a - B.n0);
+    const TBand B = bands[nbot + bk];
+    const TBand Q = bands[max(B.part, 0)];
     const double ny = __longlong_as_double((long long)NOT_YET);
     for (int v = 0; v < 3; v++) {
-        xb[o + v] = x[vidx3(a, v)];
-        yb[o + v] = ny;
-        zb[o + v] = ny;
+        const int i = 3 * (a - B.n0) + v;
+        const double xv = x[vidx3(a, v)];
+        auto put = [&](size_t o, double r) { xb[o] = r; yb[o] = ny; zb[o] = ny; };
+        if (i < B.m) put(B.xoff + i, xv);
+        if (B.part >= 0 && i >= TB * B.na) put(Q.xoff + B.mtot - 1 - i, i < B.m ? 0.0 : xv);
     }
 }
 
@@ -707,21 +742,27 @@ struct SweepLds {
     int ready;       // values handed over since the last barrier
     int rows[2][4];  // the next row and those claimed after it
 };
+// Rows: FWD all, upwards from 0; else nrows of them downwards from `first`.  A
+// band from the end has no factors for the shared rows: FWD its columns before
+// them, so that y is what it subtracts there, which `other` (FWD, the band from
+// the start: the other's y, read backwards) adds; downwards the shared rows'
+// values are x, not z, and stand in out already.
 template <bool FWD>
-__device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const double *in, double *out, int *tick,
-                                         SweepLds &S) {
+__device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const double *in, double *out,
+                                         const double *other, int first, int nrows, int *tick, SweepLds &S) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool server = wv == SW_W;
     // t-th row in sweep order; its number of tiles; the j-th of them in the order their values finish
-    auto row_of = [&](int t) { return FWD ? t : B.nt - 1 - t; };
+    auto row_of = [&](int t) { return FWD ? t : first - t; };
+    auto ktop = [&](int i) { return B.rev ? min(i, B.na) : i; };   // FWD: end of the row's columns
     auto ntiles = [&](int i) {
         if (FWD) {
             const int d = TB * i - TB - B.w;   // column tile k reaches row tile i when 64 k > d
-            return i - (d < 0 ? 0 : d / TB + 1);
+            return max(0, ktop(i) - (d < 0 ? 0 : d / TB + 1));
         }
         return min(B.nt - 1, (TB * i + TB + B.w - 1) / TB) - i;
     };
-    auto kcol = [&](int i, int n, int j) { return FWD ? i - n + j : i + n - j; };
+    auto kcol = [&](int i, int n, int j) { return FWD ? ktop(i) - n + j : i + n - j; };
     if (threadIdx.x == 64 * SW_W) {
         S.rows[0][0] = atomicAdd(tick, 1);
         S.ready = 0;
@@ -749,9 +790,10 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
             else if (q1 == INT_MAX) q1 = t;
             else q2 = t;
         };
-        while (cur < B.nt) {
+        while (cur < nrows) {
             const int i = row_of(cur), n = ntiles(i), r = TB * i + lane;
-            const double xi = FWD ? in[B.xoff + min(r, B.m - 1)] : await_value(in + B.xoff + min(r, B.m - 1), true);
+            double xi = FWD ? in[B.xoff + min(r, B.m - 1)] : await_value(in + B.xoff + min(r, B.m - 1), true);
+            if (FWD && other && i >= B.na) xi += await_value(other + B.mtot - 1 - min(r, B.m - 1), true);
             if (n == 0) claim();
             for (int j = 0; j < n; j++) {
                 const int d = TB * kcol(i, n, j) + lane;
@@ -784,7 +826,7 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
     } else {
         const int c8 = 8 * wv;
         double m[SW_PF][8];
-        long long tag[SW_PF];   // row (in sweep order) and tile whose entries m[s] holds
+        long long tag[SW_PF] = {-1, -1, -1, -1};   // row (in sweep order) and tile whose entries m[s] holds
         auto id = [&](int t, int j) { return ((long long)t << 32) | j; };
         auto fetch = [&](double (&d)[8], int t, int j) {
             const int i = row_of(t), n = ntiles(i), k = kcol(i, n, j);
@@ -795,7 +837,7 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
             for (int u = 0; u < 8; u++) d[u] = p[(size_t)min(c8 + u, kb - 1) * (2 * B.wp)];
         };
         int q[2] = {INT_MAX, INT_MAX};   // the rows after cur, as far as they are known
-        int j = 0, n = cur < B.nt ? ntiles(row_of(cur)) : 0;
+        int j = 0, n = cur < nrows ? ntiles(row_of(cur)) : 0;
         // the entries of the `ahead`-th tile from (cur, j) into d, and its tag.  Always
         // eight loads, so that the number in flight is known where one is waited
         // for: past the known rows an earlier tile again (row 1 has one
@@ -804,22 +846,22 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
             int t = cur, jj = j + ahead, nn = n;
 #pragma unroll
             for (int a = 0; a < 2; a++)
-                if (jj >= nn && t < B.nt) {
+                if (jj >= nn && t < nrows) {
                     jj -= nn;
                     t = q[a];
-                    nn = t < B.nt ? ntiles(row_of(t)) : 0;
+                    nn = t < nrows ? ntiles(row_of(t)) : 0;
                 }
-            const bool got = t < B.nt && jj < nn;
+            const bool got = t < nrows && jj < nn;
             if (!got) { t = 1; jj = 0; }
             fetch(d, t, jj);
             return got ? id(t, jj) : -1LL;
         };
-        if (B.nt > 1) {
+        if (nrows > 1) {
 #pragma unroll
             for (int s = 0; s < SW_PF; s++) tag[s] = prefetch(m[s], s);
         }
         double acc = 0.0;
-        while (cur < B.nt) {
+        while (cur < nrows) {
 #pragma unroll
             for (int s = 0; s < SW_PF; s++) {
                 while (j == n) {   // the row is done
@@ -831,7 +873,7 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
                     parity ^= 1;
                     j = 0;
                     acc = 0.0;
-                    n = cur < B.nt ? ntiles(row_of(cur)) : -1;
+                    n = cur < nrows ? ntiles(row_of(cur)) : -1;
                     __syncthreads();
                 }
                 if (n < 0) break;   // no rows left
@@ -863,28 +905,42 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
     __syncthreads();   // the LDS is free for the next sweep
 }
 
+// Where blocks are factored from both ends, SHARED: the forward sweep of every
+// band and the backward sweep of the shared rows; then, those applied
+// (k_tb_apply), REST: the backward sweep of all others.  ALL: no such block.
+// Workgroups of bands from the end come first in the grid: the other bands'
+// wait for theirs, which wait for nothing outside the band.
+enum { SW_ALL, SW_SHARED, SW_REST };
 __global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, const double *AB, const double *xb, double *yb,
-                                                    double *zb, int *tick, const int *done, const int *mask,
+                                                    double *zb, int *tick, int phase, const int *done, const int *mask,
                                                     const KScal *sc) {
     __shared__ SweepLds S;
     const int stop = *done;   // the band record and the flag fetched together
     const TBand B = band_rec(bands, blockIdx.y, stop);
     // ensembles: the band's model, converged or outside the mask, is skipped
     if (stop || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
-    tb_sweep<true>(B, AB, xb, yb, tick + 2 * blockIdx.y, S);
-    tb_sweep<false>(B, AB, yb, zb, tick + 2 * blockIdx.y + 1, S);
+    tick += 3 * blockIdx.y;
+    if (phase != SW_REST) {
+        const bool top = B.part >= 0 && !B.rev;
+        tb_sweep<true>(B, AB, xb, yb, top ? yb + bands[B.part].xoff : nullptr, 0, B.nt, tick, S);
+        if (top) tb_sweep<false>(B, AB, yb, zb, nullptr, B.nt - 1, B.nt - B.na, tick + 1, S);
+    }
+    if (phase != SW_SHARED) tb_sweep<false>(B, AB, yb, zb, nullptr, B.na - 1, B.na, tick + 2, S);
 }
 
 // The backward sweep's diagonal inverses, and back into node order: x_k = UI_k z_k,
 // one workgroup of four waves per tile (16 columns each, partial sums added in
-// wave order).  A model that has converged, or is outside the mask, keeps x.
-__global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, const double *UI, const double *zb, double *x,
-                                                  const int *done, const int *mask, const KScal *sc) {
+// wave order).  `shared`: of the shared rows, which the band from the end
+// receives too; else of the others.  A model that has converged, or is outside
+// the mask, keeps x.
+__global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, const double *UI, double *zb, double *x,
+                                                  bool shared, const int *done, const int *mask, const KScal *sc) {
     __shared__ double part[4][TB];
     const int stop = *done;
     const TBand B = band_rec(bands, blockIdx.y, stop);
-    const int k = blockIdx.x;
-    if (stop || k >= B.nt || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
+    if (shared && (B.part < 0 || B.rev)) return;
+    const int k = blockIdx.x + (shared ? B.na : 0);
+    if (stop || k >= (shared ? B.nt : B.na) || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c0 = TB * k, kb = min(TB, B.m - c0);
     const double *M = UI + 4096 * (B.toff + k);
@@ -899,8 +955,10 @@ __global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, const doub
     part[wv][lane] = s;
     __syncthreads();
     if (wv != 0 || lane >= kb) return;
-    const int d = c0 + lane;
-    x[vidx3(B.n0 + d / 3, d % 3)] = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+    const int d = B.rev ? B.mtot - 1 - (c0 + lane) : c0 + lane;
+    s = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+    x[vidx3(B.n0 + d / 3, d % 3)] = s;
+    if (shared) zb[bands[B.part].xoff + B.mtot - 1 - d] = s;
 }
 
 void tband_free(Ctx *c) {
@@ -910,7 +968,19 @@ void tband_free(Ctx *c) {
     c->tb_bands = nullptr; c->tb_AB = nullptr; c->tb_LI = nullptr; c->tb_UI = nullptr; c->tb_int = nullptr;
     c->tb_xb = nullptr; c->tb_yb = nullptr; c->tb_zb = nullptr;
     c->tb_nband = 0; c->tb_maxnt = 0; c->tb_gt = 0; c->tb_gf = 0; c->tb_size = 0;
-    c->tb_h_nt.clear(); c->tb_h_inst.clear();
+    c->tb_h_nt.clear(); c->tb_h_inst.clear(); c->tb_h_na.clear();
+    c->tb_nbot = 0; c->tb_maxs = 0;
+}
+
+// Panels from each end of a block of m DOFs and half bandwidth w, 0: one band.
+// From both ends the chain of dependent panels is the longer end's and the
+// shared rows' (at least w of them, so that the ends do not couple), plus a merge
+// and a diagonal block on their own, about one panel's time; from one end it is
+// all of the block's.  Short ends are not worth the sweeps' extra launches.
+static int twist_panels(int m, int w) {
+    const int nt = (m + TB - 1) / TB, a = m > w ? (m - w) / (2 * TB) : 0;
+    const int shared = m - 2 * TB * a;
+    return a >= 3 && a + (shared + TB - 1) / TB + 2 < nt ? a : 0;
 }
 
 // Bands of the node blocks (nodes [s0[b], s1[b]) of model inst[b]) with
@@ -919,38 +989,61 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
                             const std::vector<int> &inst, const std::vector<int> &w) {
     tband_free(c);
     const int nblk = (int)w.size();
-    std::vector<TBand> h(nblk);
-    size_t off = 0, toff = 0, xoff = 0;
-    int maxnt = 0, maxw = 0;
-    for (int b = 0; b < nblk; b++) {
-        TBand &B = h[b];
-        B.n0 = s0[b];
-        B.m = 3 * (s1[b] - s0[b]);
-        B.w = w[b];
-        B.wp = w[b] + TB;
-        B.nt = (B.m + TB - 1) / TB;
-        B.pad = 0;
-        B.inst = inst[b];
-        B.pad2 = 0;
-        B.off = off;
-        B.toff = toff;
-        B.xoff = xoff;
-        off += (size_t)B.m * (2 * B.wp + 1);
-        toff += B.nt;
-        xoff += B.m;
-        maxnt = std::max(maxnt, B.nt);
-        maxw = std::max(maxw, B.w);
-    }
     size_t freeb = 0, totalb = 0;
     (void)hipMemGetInfo(&freeb, &totalb);
-    const size_t nint = toff + 2 * (size_t)nblk;   // a guard flag per tile, two tickets per band
-    const size_t need = sizeof(double) * (off + 2 * 4096 * toff + 3 * xoff) + sizeof(int) * nint;
-    if (need + ((size_t)2 << 30) > freeb)
+    std::vector<TBand> h;
+    size_t off = 0, toff = 0, xoff = 0, nint = 0, need = 0;
+    int maxnt = 0, maxw = 0;
+    // blocks from both ends take s rows more each; where that does not fit, one band each
+    for (const bool twist : {true, false}) {
+        std::vector<int> top(nblk);
+        int nbot = 0;
+        for (int b = 0; b < nblk; b++) {
+            top[b] = twist ? twist_panels(3 * (s1[b] - s0[b]), w[b]) : 0;
+            nbot += top[b] > 0;
+        }
+        h.assign(nbot + nblk, TBand{});
+        off = toff = xoff = 0;
+        maxnt = maxw = c->tb_maxs = 0;
+        for (int b = 0, bot = 0; b < nblk; b++) {
+            const int mtot = 3 * (s1[b] - s0[b]);
+            for (int rev = 0; rev <= (top[b] > 0); rev++) {
+                TBand &B = h[rev ? bot : nbot + b];
+                B.n0 = s0[b];
+                B.m = top[b] ? mtot - TB * top[b] : mtot;   // all but the other end's rows
+                B.w = w[b];
+                B.wp = w[b] + TB;
+                B.nt = (B.m + TB - 1) / TB;
+                B.na = top[b] ? top[b] : B.nt;
+                B.part = top[b] ? (rev ? nbot + b : bot) : -1;
+                B.rev = rev;
+                B.mtot = mtot;
+                B.pad = 0;
+                B.inst = inst[b];
+                B.off = off;
+                B.toff = toff;
+                B.xoff = xoff;
+                off += (size_t)B.m * (2 * B.wp + 1);
+                toff += B.nt;
+                xoff += B.m;
+                maxnt = std::max(maxnt, B.nt);
+                maxw = std::max(maxw, B.w);
+                if (top[b]) c->tb_maxs = std::max(c->tb_maxs, B.m - TB * B.na);
+            }
+            bot += top[b] > 0;
+        }
+        c->tb_nbot = nbot;
+        nint = toff + 3 * h.size();   // a guard flag per tile, three tickets per band
+        need = sizeof(double) * (off + 2 * 4096 * toff + 3 * xoff) + sizeof(int) * nint;
+        if (need + ((size_t)2 << 30) <= freeb) break;
+        if (twist && nbot > 0) continue;
         return "tiled band LU: " + std::to_string(need >> 20) + " MiB of band storage do not fit in the free " +
                std::to_string(freeb >> 20) + " MiB; raise nblock" +
                (c->ninst ? ", or step the models in groups that fit" : "");
-    if (hipMalloc((void **)&c->tb_bands, sizeof(TBand) * nblk) != hipSuccess ||
-        hipMemcpy(c->tb_bands, h.data(), sizeof(TBand) * nblk, hipMemcpyHostToDevice) != hipSuccess ||
+    }
+    const int nband = (int)h.size();
+    if (hipMalloc((void **)&c->tb_bands, sizeof(TBand) * nband) != hipSuccess ||
+        hipMemcpy(c->tb_bands, h.data(), sizeof(TBand) * nband, hipMemcpyHostToDevice) != hipSuccess ||
         hipMalloc((void **)&c->tb_AB, sizeof(double) * off) != hipSuccess ||
         hipMalloc((void **)&c->tb_LI, sizeof(double) * 4096 * toff) != hipSuccess ||
         hipMalloc((void **)&c->tb_UI, sizeof(double) * 4096 * toff) != hipSuccess ||
@@ -961,15 +1054,20 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
         tband_free(c);
         return "hipMalloc failed for the tiled band LU";
     }
-    c->tb_nband = nblk;
+    c->tb_nband = nband;
     c->tb_maxnt = maxnt;
-    c->tb_h_nt.resize(nblk);
-    c->tb_h_inst.resize(nblk);
-    for (int b = 0; b < nblk; b++) { c->tb_h_nt[b] = h[b].nt; c->tb_h_inst[b] = h[b].inst; }
+    c->tb_h_nt.resize(nband);
+    c->tb_h_inst.resize(nband);
+    c->tb_h_na.resize(nband);
+    for (int b = 0; b < nband; b++) {
+        c->tb_h_nt[b] = h[b].nt;
+        c->tb_h_inst[b] = h[b].inst;
+        c->tb_h_na[b] = h[b].part < 0 ? -1 : h[b].na;
+    }
     c->tb_gt = (maxw + TB - 1) / TB;
     c->tb_gf = (maxw + 2 * TB - 2) / TB;   // tiles below (above) a panel that its L (U) reaches
     c->tb_size = off;
-    c->tb_guard = c->tb_int + 2 * nblk;
+    c->tb_guard = c->tb_int + 3 * nband;
     return "";
 }
 
@@ -993,13 +1091,37 @@ void launch_tband_setup(Ctx *c) {
     if (nt == 0) return;
     launch_zero(c, c->tb_AB, c->tb_size);
     hipLaunchKernelGGL(k_tb_load, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->node_blk,
-                       c->tb_bands, c->tb_AB, c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, mask);
+                       c->tb_bands, c->tb_nbot, c->tb_AB, c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, mask);
     const int gt = std::max(1, c->tb_gt);
-    hipLaunchKernelGGL(k_tb_diag, dim3(c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
-                       c->tb_UI, c->tb_guard, mask);
-    for (int k = 0; k + 1 < nt; k++)
+    // the step at which the active models' shared rows begin, and the steps in all
+    int amax = 0, steps = 0;
+    auto each_active = [&](auto f) {
+        for (int b = 0; b < c->tb_nband; b++)
+            if (!mask || c->h_inst_mask[c->tb_h_inst[b]]) f(b);
+    };
+    each_active([&](int b) { amax = std::max(amax, c->tb_h_na[b]); });
+    each_active([&](int b) {
+        steps = std::max(steps, c->tb_h_nt[b] - 1 + (c->tb_h_na[b] < 0 ? 0 : amax - c->tb_h_na[b]));
+    });
+    auto diag = [&](bool shared) {
+        hipLaunchKernelGGL(k_tb_diag, dim3(c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
+                           c->tb_UI, c->tb_guard, shared, mask);
+    };
+    diag(false);
+    for (int k = 0; k < steps; k++) {
+        if (amax > 0 && k == amax) {
+            hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands,
+                               c->tb_AB, mask);
+            diag(true);
+        }
         hipLaunchKernelGGL(k_tb_step, dim3(gt * gt, c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_LI, c->tb_UI, c->tb_guard, k, gt, mask);
+                           c->tb_LI, c->tb_UI, c->tb_guard, k, amax, gt, mask);
+    }
+    if (amax > 0 && steps == amax) {   // shared rows of one panel
+        hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_AB,
+                           mask);
+        diag(true);
+    }
     hipLaunchKernelGGL(k_tb_inv, dim3(nt, c->tb_nband), dim3(64), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
                        c->tb_UI, c->tb_guard, mask);
     const int gf = std::max(1, c->tb_gf);
@@ -1014,7 +1136,7 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     const int nt = tb_active_nt(c);
     if (nt == 0) return;
     hipLaunchKernelGGL(k_tb_gather, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->tb_nband,
-                       c->node_blk, c->tb_bands, x, c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int);
+                       c->tb_nbot, c->node_blk, c->tb_bands, x, c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int);
     // one model: its done flag, or the first band record's pad (always 0),
     // read beside the band record; ensembles: each band's model's flag
     const int *done = (sc && !mask) ? &sc->done : &c->tb_bands[0].pad;
@@ -1023,10 +1145,22 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     // row always waiting; any number is correct, and with many bands one
     // workgroup each already fills the chip
     const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 512 / c->tb_nband));
-    hipLaunchKernelGGL(k_tb_sweep, dim3(g, c->tb_nband), dim3(SW_NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_xb,
-                       c->tb_yb, c->tb_zb, c->tb_int, done, mask, msc);
-    hipLaunchKernelGGL(k_tb_apply, dim3(nt, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_UI, c->tb_zb, x,
-                       done, mask, msc);
+    auto sweep = [&](int phase) {
+        hipLaunchKernelGGL(k_tb_sweep, dim3(g, c->tb_nband), dim3(SW_NT), 0, c->stream, c->tb_bands, c->tb_AB,
+                           c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int, phase, done, mask, msc);
+    };
+    auto apply = [&](bool shared, int tiles) {
+        hipLaunchKernelGGL(k_tb_apply, dim3(tiles, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_UI,
+                           c->tb_zb, x, shared, done, mask, msc);
+    };
+    if (c->tb_nbot > 0) {
+        sweep(SW_SHARED);
+        apply(true, (c->tb_maxs + TB - 1) / TB);
+        sweep(SW_REST);
+    } else {
+        sweep(SW_ALL);
+    }
+    apply(false, nt);
 }
 
 }  // namespace sw2

@@ -10,9 +10,9 @@ couples to, <= 21), bounded here by 1e-13 of the largest entry.
 import numpy as np
 import pytest
 
-from gpu_helpers import say
+from gpu_helpers import bits_equal, say
 from adhv8_kraken_amd import mesh
-from adhv8_kraken_amd.sw2 import SW2Model, default_opts
+from adhv8_kraken_amd.sw2 import SW2Ensemble, SW2Model, default_opts
 
 pytestmark = pytest.mark.gpu
 
@@ -38,9 +38,11 @@ def _system(g, seed):
 
 
 # (cells along, cells across, node blocks): DOFs 12 (part of one tile), 192 = 3 tiles in a
-# band of 17, 195, 693, reaches of 33 and 34 tiles, blocks of 64 and 128 DOFs and their remainders
+# band of 17, 195, 693, reaches of 33 and 34 tiles, blocks of 64 and 128 DOFs and their remainders;
+# 390, 396 and 456 DOFs: the last block in one band, three panels from each end with one shared panel and with two
 @pytest.mark.parametrize("ncx,ncy,nblock", [(1, 1, 1), (15, 3, 1), (12, 4, 1), (20, 10, 1), (4, 700, 1), (3, 720, 1),
-                                            (20, 10, 2), (42, 5, 5), (31, 20, 9)])
+                                            (20, 10, 2), (42, 5, 5), (31, 20, 9),
+                                            (64, 1, 1), (65, 1, 1), (75, 1, 1)])
 def test_apply_is_the_block_inverse(ncx, ncy, nblock):
     import scipy.sparse as sp
     import scipy.sparse.linalg as sl
@@ -93,3 +95,21 @@ def test_backward_sweep_divides_by_the_pivot_itself(node):
     ref = sl.splu(S.tocsc()).solve(v[rest])
     assert np.abs(y[rest] - ref).max() < 1e-13 * np.abs(ref).max()
     g.close()
+
+
+def test_models_of_one_band_and_of_two_factor_together():
+    """One to 60 tiles, factored from one end and from both, in one ensemble:
+    the bands meet their shared rows at one launch, and each model takes the
+    steps it takes alone, bit for bit."""
+    ps = [mesh.bumpy_channel(*c, seed=k) for k, c in enumerate([(3, 1), (64, 1), (65, 1), (75, 1), (200, 4), (30, 40)])]
+    opts = default_opts(preconditioner=1, nblock=1, lu_tiled=1, max_nonlin_it=4, tol_nonlin=1e-9)
+    e = SW2Ensemble(ps, opts)
+    rs = e.timestep()
+    for k, p in enumerate(ps):
+        g = SW2Model(p, opts)
+        r = g.timestep()
+        say(f"  {3 * p.nnodes} DOFs: {r['iterations']} iterations")
+        assert r["iterations"] == rs[k]["iterations"] and bits_equal(r["hist_max"], rs[k]["hist_max"])
+        assert all(bits_equal(a, b) for a, b in zip(g.get_state()[:2], e.get_state(k)))
+        g.close()
+    e.close()
