@@ -259,6 +259,8 @@ struct Ctx {
     int *ilu_rnode, *ilu_lptr, *ilu_uptr, *ilu_lcol, *ilu_ucol, *ilu_lsrc, *ilu_usrc, *ilu_tptr;
     int4 *ilu_upd;
     double *ilu_Lw, *ilu_Uw, *ilu_Dw, *ilu_Dinv, *ilu_w;   // FP64 factor work, colour-ordered vector
+    double *ilu_xw;                        // the backward sweep's x in colour order
+    int *ilu_tick;                         // tickets of the two sweeps
     void *ilu_L, *ilu_U, *ilu_D;           // the apply's factors (FP64 or FP32) and U_ii^-1
     // restarted GMRES (opts.krylov = 1), allocated on first use
     double *gm_V;          // basis, GMRES restart + 1 vectors of 3 Np

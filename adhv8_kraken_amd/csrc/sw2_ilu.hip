@@ -23,8 +23,10 @@
 //
 // Apply (in place on a node-ordered vector): forward sweeps z_i = v_i -
 // sum L_ik z_k over the colours in order, backward sweeps
-// x_i = U_ii^-1 (z_i - sum U_ij x_j) in reverse order, one launch per colour
-// and sweep; the colour-ordered work vector w holds z, then x.
+// x_i = U_ii^-1 (z_i - sum U_ij x_j) in reverse order.  A sweep is one launch in
+// which rows wait for the values they need (k_ilu_flow), or for large systems a
+// launch per colour; the colour-ordered work vector w holds z (with a launch
+// per colour then x).
 //
 // Storage: like the SpMV's SELL-64 blocks, slices of 64 consecutive rows (in
 // colour order) with a per-slice slot count; value e of slot b of the row in
@@ -35,6 +37,7 @@
 #include <numeric>
 
 #include "sw2_ctx.h"
+#include "sw2_flow.h"
 
 namespace sw2 {
 
@@ -176,6 +179,100 @@ __global__ void __launch_bounds__(256) k_ilu_bwd(IluView V, int r0, int r1, cons
     }
 }
 
+// A whole sweep in one launch: a workgroup takes the next 256 rows in the
+// sweep's order (a ticket), and a row polls its neighbours' values, which are
+// words handed over (sw2_flow.h), as far as they come before it.  Rows are taken
+// in order, so the first unfinished ones belong to a running workgroup and wait
+// only for finished ones.  FWD: z into w from the vector; else x into xw and the
+// vector, from w.  Each sweep empties what the other waits on next: FWD its row
+// of xw, the backward sweep its row of w once it has read it; each sets the
+// other's ticket back.  Same operations as k_ilu_fwd and k_ilu_bwd.
+template <typename FT, bool FWD>
+__global__ void __launch_bounds__(256) k_ilu_flow(IluView V, const FT *F, const FT *Dinv, double *vec, double *w,
+                                                  double *xw, int *tick, const KScal *sc) {
+    if (sc && sc->done) return;
+    __shared__ int unit;
+    if (threadIdx.x == 0) {
+        const int t = atomicAdd(tick + (FWD ? 0 : 1), 1);
+        if (t == 0) tick[FWD ? 1 : 0] = 0;
+        unit = FWD ? t : gridDim.x - 1 - t;
+    }
+    __syncthreads();
+    const int r = 256 * unit + threadIdx.x;
+    if (r >= V.Rp) return;
+    const int node = V.rnode[r];
+    if (node < 0) return;   // padding: no row waits for it
+    const int s = r >> 6, lane = r & 63;
+    const int *ptr = FWD ? V.lptr : V.uptr, *col = FWD ? V.lcol : V.ucol;
+    const double *near = FWD ? w : xw;
+    const int b1 = ptr[s + 1];
+    double z[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        if constexpr (FWD) {
+            z[j] = vec[vidx3(node, j)];
+            put_raw(xw + ilu_w(r, j), Slot<double>::EMPTY);
+        } else {
+            z[j] = __builtin_bit_cast(double, peek(w + ilu_w(r, j)));
+            put_raw(w + ilu_w(r, j), Slot<double>::EMPTY);
+        }
+    }
+    constexpr int C = 6;   // slots whose blocks are loaded before their values are waited for
+    for (int b = ptr[s]; b < b1; b += C) {
+        int k[C];
+        FT f[C][9];
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const int bi = min(b + i, b1 - 1);
+            k[i] = b + i < b1 ? col[64 * (size_t)bi + lane] : -1;
+#pragma unroll
+            for (int e = 0; e < 9; e++) f[i][e] = F[ilu_v(bi, e, lane)];
+        }
+        double x[C][3];
+        for (;;) {
+            bool all = true;
+#pragma unroll
+            for (int i = 0; i < C; i++)
+                if (k[i] >= 0)
+#pragma unroll
+                    for (int j = 0; j < 3; j++) {
+                        const auto u = peek(near + ilu_w(k[i], j));
+                        all = all && u != Slot<double>::EMPTY;
+                        x[i][j] = __builtin_bit_cast(double, u);
+                    }
+            if (!__any(!all)) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+#pragma unroll
+        for (int i = 0; i < C; i++)
+            if (k[i] >= 0) {
+                double y[3];
+                blk_mul(f[i], 1, x[i], y);
+                z[0] -= y[0]; z[1] -= y[1]; z[2] -= y[2];
+            }
+    }
+    if constexpr (FWD) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) put(w + ilu_w(r, j), z[j]);
+    } else {
+        double x[3];
+        blk_mul(Dinv + ilu_v(s, 0, lane), 64, z, x);
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            put(xw + ilu_w(r, j), x[j]);
+            vec[vidx3(node, j)] = x[j];
+        }
+    }
+}
+
+__global__ void k_ilu_empty(size_t n, double *a, double *b, int *tick) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 2) tick[i] = 0;
+    if (i >= n) return;
+    put_raw(a + i, Slot<double>::EMPTY);
+    put_raw(b + i, Slot<double>::EMPTY);
+}
+
 static IluView iview(Ctx *c) { return IluView{c->ilu_Rp, c->ilu_rnode, c->ilu_lptr, c->ilu_uptr, c->ilu_lcol, c->ilu_ucol}; }
 
 void ilu_free(Ctx *c) {
@@ -311,6 +408,8 @@ std::string ilu_structure(Ctx *c) {
               alloc((void **)&c->ilu_Dw, sizeof(double) * 9 * (size_t)Rp) &&
               alloc((void **)&c->ilu_Dinv, sizeof(double) * 9 * (size_t)Rp) &&
               alloc((void **)&c->ilu_w, sizeof(double) * 3 * (size_t)Rp) &&
+              alloc((void **)&c->ilu_xw, sizeof(double) * 3 * (size_t)Rp) &&
+              alloc((void **)&c->ilu_tick, sizeof(int) * 2) &&
               alloc((void **)&c->ilu_L, fsz * 9 * std::max<size_t>(nl, 1)) &&
               alloc((void **)&c->ilu_U, fsz * 9 * std::max<size_t>(nu, 1)) &&
               alloc((void **)&c->ilu_D, fsz * 9 * (size_t)Rp);
@@ -325,6 +424,9 @@ std::string ilu_structure(Ctx *c) {
     c->ilu_nl = nl;
     c->ilu_nu = nu;
     c->ilu_f32 = c->opts.precision >= 1;
+    const size_t n3 = 3 * (size_t)Rp;
+    hipLaunchKernelGGL(k_ilu_empty, dim3((unsigned)((n3 + 255) / 256 + 1)), dim3(256), 0, c->stream, n3, c->ilu_w,
+                       c->ilu_xw, c->ilu_tick);
     c->ilu_ready = 1;
     return "";
 }
@@ -357,10 +459,26 @@ void launch_ilu_setup(Ctx *c) {
     }
 }
 
+// Rows up to which a sweep runs in one launch: there a colour's launch (4.6 us
+// at 20,000 rows) is longer than a hand-over, above it the neighbours' values,
+// read past the L2, cost more than they save.  A time step's solves, ms, a launch
+// per colour / per sweep: 1,891 rows 1.68 / 1.25, 20,301 1.79 / 1.23, 80,400
+// 2.29 / 1.75, 125,751 2.32 / 2.07, 180,901 2.52 / 2.48 (FP64 3.11 / 2.86),
+// 246,051 2.70 / 2.82, 501,501 4.15 / 4.52.
+constexpr int FLOW_ROWS = 200000;
+
 template <typename FT>
 static void ilu_sweeps(Ctx *c, double *x, const KScal *sc) {
     IluView V = iview(c);
     const FT *L = (const FT *)c->ilu_L, *U = (const FT *)c->ilu_U, *D = (const FT *)c->ilu_D;
+    if (V.Rp <= FLOW_ROWS) {
+        const dim3 g(nblocks_for(V.Rp, 256));
+        hipLaunchKernelGGL((k_ilu_flow<FT, true>), g, dim3(256), 0, c->stream, V, L, D, x, c->ilu_w, c->ilu_xw,
+                           c->ilu_tick, sc);
+        hipLaunchKernelGGL((k_ilu_flow<FT, false>), g, dim3(256), 0, c->stream, V, U, D, x, c->ilu_w, c->ilu_xw,
+                           c->ilu_tick, sc);
+        return;
+    }
     for (int k = 0; k < c->ilu_ncolor; k++) {
         const int r0 = c->h_ilu_cstart[k], r1 = c->h_ilu_cstart[k + 1];
         hipLaunchKernelGGL(k_ilu_fwd<FT>, dim3(nblocks_for(r1 - r0, 256)), dim3(256), 0, c->stream, V, r0, r1, L, x,

@@ -27,40 +27,12 @@
 // block polls all blocks' partials, and the neighbours' values are read past
 // the L2).
 
+#include "sw2_flow.h"
 #include "sw2_krylov.h"
 
 namespace sw2 {
 
 namespace {
-
-// An empty slot: a NaN no arithmetic produces.
-template <typename T>
-struct Slot;
-template <>
-struct Slot<double> {
-    using U = unsigned long long;
-    static constexpr U EMPTY = 0xfff8dead0badf00dull, QNAN = 0x7ff8000000000000ull;
-};
-template <>
-struct Slot<float> {
-    using U = unsigned;
-    static constexpr U EMPTY = 0xffdeadadu, QNAN = 0x7fc00000u;
-};
-
-template <typename T>
-__device__ __forceinline__ typename Slot<T>::U peek(const T *p) {
-    return __hip_atomic_load((const typename Slot<T>::U *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void put_raw(T *p, typename Slot<T>::U u) {
-    __hip_atomic_store((typename Slot<T>::U *)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void put(T *p, T v) {
-    typename Slot<T>::U u = __builtin_bit_cast(typename Slot<T>::U, v);
-    if (u == Slot<T>::EMPTY) u = Slot<T>::QNAN;
-    put_raw(p, u);
-}
 
 // x of the lane 32 (16) further, cyclically: halves of the wave (rows of 16) exchanged
 __device__ __forceinline__ double swap32(double x) {
