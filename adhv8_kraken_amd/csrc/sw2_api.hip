@@ -493,7 +493,8 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     UP(col, c.h_col.data(), c.nnz);
     UP(sell_ptr, sell_ptr.data(), c.nslice + 1);
     UP(sell_col, sell_col.data(), c.nsell);
-    UP(offd_pos, c.h_offd_pos.data(), c.h_offd_pos.size());
+    if ((rc = dalloc(h, &c.offd_pos, c.h_offd_pos.size()))) { adh_sw2_hip_destroy(h); return rc; }
+    launch_offd_pos(&c);
     UP(slot_ptr, slot_ptr.data(), c.ndslots + 1);
     UP(slot_src, slot_src.data(), slot_src.size());
     {   // element block -> its position in the slot-ordered contributor list
@@ -525,7 +526,8 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
         std::vector<double> w(may ? run_slot_words(c.run_max_blocks) : 1);
         for (double &x : w) memcpy(&x, &empty, sizeof x);
         UP(run_slots, w.data(), w.size());
-        UP(run_xch, (const double *)nullptr, may ? run_vector_words(c.Np) : 1);
+        // emptied by the first solve
+        if ((rc = dalloc(h, &c.run_xch, may ? run_vector_words(c.Np) : 1))) { adh_sw2_hip_destroy(h); return rc; }
     }
     UP(run_quit, (const int *)nullptr, 2 * nmod);
     c.red.maxblocks = nblocks_for(N, 256) + 8;

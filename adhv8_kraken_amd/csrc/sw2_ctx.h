@@ -193,7 +193,7 @@ struct Ctx {
     Norms *norms, *h_norms;  // [max(1, ninst)]
     int *h_flag;           // pinned scratch
     Stage stage;
-    int *offd_pos;         // device copy of h_offd_pos
+    int *offd_pos;         // the same as h_offd_pos, on the device
     ElemData ed;
     // Ensemble of independent models sharing one mesh ("batch"): model i owns
     // the node range [inst_node0[i], inst_node0[i] + inst_N[i]) starting on a
@@ -350,6 +350,7 @@ void launch_inc(Ctx *c, double factor_on_sol);   // state += sol
 void launch_scale_sol(Ctx *c, double f);          // sol *= f
 void launch_inc_flip(Ctx *c);                     // state += sol, then sol = -sol
 void launch_setup(Ctx *c, bool guess = true);   // guess: sol holds an initial guess, scaled with the system
+void launch_offd_pos(Ctx *c);
 void launch_scal_init(Ctx *c, int max_it);
 void launch_krylov_prologue(Ctx *c);
 void launch_krylov_iters(Ctx *c, int k);

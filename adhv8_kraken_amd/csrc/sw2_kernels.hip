@@ -20,7 +20,7 @@ namespace sw2 {
 
 int nblocks_for(int n, int bs) { return n <= 0 ? 1 : (n + bs - 1) / bs; }
 
-static void launch_resid2d_split(Ctx *c, const ElemData &D);
+static void launch_resid_split(Ctx *c, const ElemData &D, bool edges);
 
 // The refined forms (precision >= 1) store the element Jacobian blocks in
 // FP32 (the matrix they assemble is stored in FP32 anyway); the FP64 form in
@@ -32,11 +32,13 @@ static float *em32_of(Ctx *c) { return c->opts.precision >= 1 ? (float *)c->EM :
 // WET lists hold triangles with positive depths, run without clipping code.
 // Software pipeline: the triangle id two iterations ahead and its node ids
 // one iteration ahead are loaded while the current triangle is computed.
+// block / nblocks: of the workgroups that share the list
 template <bool WET, int BS>
-__global__ void __launch_bounds__(BS) k_resid2d_list(ElemData D, const int *list, const int *count, double *ER) {
+__device__ __forceinline__ void resid_list(const ElemData &D, const int *list, const int *count, double *ER, int block,
+                                           int nblocks) {
     const int n = *count;
-    const int stride = gridDim.x * blockDim.x;
-    int li = blockIdx.x * blockDim.x + threadIdx.x;
+    const int stride = nblocks * BS;
+    int li = block * BS + threadIdx.x;
     int ie_a = li < n ? list[li] : 0;
     int ie_b = li + stride < n ? list[li + stride] : 0;
     int nd_a[3] = {0, 0, 0};
@@ -61,8 +63,12 @@ __global__ void __launch_bounds__(BS) k_resid2d_list(ElemData D, const int *list
     }
 }
 
-__global__ void __launch_bounds__(128) k_resid1d(ElemData D, int B, double *ER1) {
-    int ie = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool WET, int BS>
+__global__ void __launch_bounds__(BS) k_resid2d_list(ElemData D, const int *list, const int *count, double *ER) {
+    resid_list<WET, BS>(D, list, count, ER, blockIdx.x, gridDim.x);
+}
+
+__device__ __forceinline__ void resid_edge(const ElemData &D, int ie, int B, double *ER1) {
     if (ie >= B) return;
     d3 r[3];
     boundary_resid(D, ie, 0.0, 0, PERTURB_NONE, 0, true, r);
@@ -73,6 +79,19 @@ __global__ void __launch_bounds__(128) k_resid1d(ElemData D, int B, double *ER1)
         o[3 * i + 1] = r[i].y_eq;
         o[3 * i + 2] = r[i].c_eq;
     }
+}
+
+// The general list and the boundary edges in one launch: each is mostly launch
+// time (an empty list 3.4 us, 128 edges 4.2).  With WET the wet list too, where
+// its workgroups fit beside: this kernel holds one wave a SIMD, the wet list's
+// own two.
+template <bool WET, int BS>
+__global__ void __launch_bounds__(BS) k_resid_all(ElemData D, const int *wet, const int *gen, const int *count,
+                                                  double *ER, int nwet, int ngen, int B, double *ER1) {
+    const int b = blockIdx.x;
+    if (WET && b < nwet) resid_list<true, BS>(D, wet, count, ER, b, nwet);
+    else if (b < nwet + ngen) resid_list<false, BS>(D, gen, count + 1, ER, b - nwet, ngen);
+    else resid_edge(D, (b - nwet - ngen) * BS + threadIdx.x, B, ER1);
 }
 
 // residual[3n..] = -(sum of element contributions) in ascending element
@@ -216,9 +235,8 @@ void launch_resid(Ctx *c, bool norms) {
     if (!c->pre_valid) launch_old_terms(c);
     ElemData D = c->ed;
     D.first_elem = c->first_elem;
-    launch_resid2d_split(c, D);
-    double *er1 = c->ER + 9 * (size_t)c->E;
-    if (c->B) hipLaunchKernelGGL(k_resid1d, dim3(nblocks_for(c->B, 128)), dim3(128), 0, c->stream, D, c->B, er1);
+    launch_resid_split(c, D, true);
+    const double *er1 = c->ER + 9 * (size_t)c->E;
     const int nb = nblocks_for(c->N, 256);
     if (!norms) {
         hipLaunchKernelGGL(k_resid_gather<false>, dim3(nb), dim3(256), 0, c->stream, c->N, c->n2e_ptr, c->n2e,
@@ -533,16 +551,15 @@ __device__ __forceinline__ void lds_column(const ElemData &DL, const SRC &S, int
 // all nine, one node's three, or one (unit w: group w / (9 / COLS), part w
 // mod that).  With more than one column the terms of the unperturbed triangles
 // (Base) are formed once after the staging.
+// block / nblocks: of the workgroups that share the list; srec, slog: LDS
 template <bool WET, int BS, int COLS>
-__global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list, const int *count, int b0, int b1,
-                                                  int b2, const int *blkpos, double *EM, float *EM32) {
-    if (WET) stamp(D.ts);
+__device__ __forceinline__ void jac_lds_list(const ElemData &D, const int *list, const int *count, int b0, int b1,
+                                             int b2, const int *blkpos, double *EM, float *EM32, int block,
+                                             int nblocks, double (&srec)[BS / 64][32][LREC], crlog::tables &slog) {
     constexpr int WPB = BS / 64, PARTS = 9 / COLS;
-    __shared__ double srec[WPB][32][LREC];
-    __shared__ crlog::tables slog;
     const int n = *count;
     const int nunits = PARTS * ((n + 31) >> 5);
-    if ((int)blockIdx.x * WPB >= nunits) return;   // the whole block has no unit (uniform exit)
+    if (block * WPB >= nunits) return;   // the whole block has no unit (uniform exit)
     // the friction law's log table copied to LDS: its lookup is the one
     // data-dependent load of the element code
     {
@@ -557,14 +574,14 @@ __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list
     const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool minus = lane >= 32;
     double *rec = &srec[wib][lane & 31][0];
-    const int wstride = gridDim.x * WPB;
+    const int wstride = nblocks * WPB;
     // software pipeline: the triangle id two units ahead and its node ids one
     // unit ahead are loaded while the current unit is computed
     auto tri_of = [&](int w) {
         const int g = w / PARTS, l = g * 32 + (lane & 31);
         return list[l < n ? l : g * 32];
     };
-    int w = blockIdx.x * WPB + wib;
+    int w = block * WPB + wib;
     int ie_a = w < nunits ? tri_of(w) : 0;
     int ie_b = w + wstride < nunits ? tri_of(w + wstride) : 0;
     int nd_a[3] = {0, 0, 0};
@@ -619,9 +636,17 @@ __global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list
     }
 }
 
-__global__ void __launch_bounds__(128) k_jac1d(ElemData D, int B, int b0, int b1, const int *blkpos1, double *EM,
-                                               float *EM32) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool WET, int BS, int COLS>
+__global__ void __launch_bounds__(BS, 2) k_jac2d_lds(ElemData D, const int *list, const int *count, int b0, int b1,
+                                                  int b2, const int *blkpos, double *EM, float *EM32) {
+    __shared__ double srec[BS / 64][32][LREC];
+    __shared__ crlog::tables slog;
+    if (WET) stamp(D.ts);
+    jac_lds_list<WET, BS, COLS>(D, list, count, b0, b1, b2, blkpos, EM, EM32, blockIdx.x, gridDim.x, srec, slog);
+}
+
+__device__ __forceinline__ void jac_edge(const ElemData &D, int t, int B, int b0, int b1, const int *blkpos1, double *EM,
+                                         float *EM32) {
     if (t >= 6 * B) return;
     int ie = t / 6, q = t % 6, j = q / 3, var = q % 3;
     double col[9];
@@ -639,6 +664,30 @@ __global__ void __launch_bounds__(128) k_jac1d(ElemData D, int B, int b0, int b1
             else EM[o + 3 * r + var] = col[3 * i + r];
         }
     }
+}
+
+__global__ void __launch_bounds__(128) k_jac1d(ElemData D, int B, int b0, int b1, const int *blkpos1, double *EM,
+                                               float *EM32) {
+    jac_edge(D, blockIdx.x * blockDim.x + threadIdx.x, B, b0, b1, blkpos1, EM, EM32);
+}
+
+// Both lists (LDS layout) and the boundary edges in one launch: an empty general
+// list costs 4.0 us on its own and 128 edges 5.8, of 25 that the wet list takes
+// at 1,600 triangles.
+template <int BS, int COLS>
+__global__ void __launch_bounds__(BS, 2) k_jac_all(ElemData D, const int *wet, const int *gen, const int *count,
+                                                   int b0, int b1, int b2, const int *blkpos, double *EM, float *EM32,
+                                                   int nwet, int ngen, int B, const int *blkpos1) {
+    __shared__ double srec[BS / 64][32][LREC];
+    __shared__ crlog::tables slog;
+    stamp(D.ts);
+    const int b = blockIdx.x;
+    if (b < nwet)
+        jac_lds_list<true, BS, COLS>(D, wet, count, b0, b1, b2, blkpos, EM, EM32, b, nwet, srec, slog);
+    else if (b < nwet + ngen)
+        jac_lds_list<false, BS, COLS>(D, gen, count + 1, b0, b1, b2, blkpos, EM, EM32, b - nwet, ngen, srec, slog);
+    else
+        jac_edge(D, (b - nwet - ngen) * BS + threadIdx.x, B, b0, b1, blkpos1, EM, EM32);
 }
 
 // Splits the triangles into those whose three depths stay positive under the
@@ -829,18 +878,69 @@ void launch_list_phase(Ctx *c, int phase, int bs, int grid, int layout) {
     launch_list(c, D, phase, bs, grid, layout);
 }
 
-static void launch_jac2d_split(Ctx *c, const ElemData &D) {
-    if (!c->E) return;
-    if (!c->split_valid) launch_split(c);
-    launch_list(c, D, 0, c->tune.bs[0], c->tune.grid[0], c->tune.layout[0]);
-    launch_list(c, D, 1, c->tune.bs[1], c->tune.grid[1], c->tune.layout[1]);
+// Workgroup size of the launches over both lists, where neither list's own launch
+// shape asks for another
+constexpr int JAC_ALL_BS = 256, RES_ALL_BS = 128;
+// Triangles up to which the wet list runs beside the others.  Residuals: above,
+// more than one wave a SIMD is at work and the wet list is faster in its own
+// launch (44 us at 250,000 triangles).  Jacobians: both lists' code at once
+// overruns the instruction caches, 148 against 59 + 74 us at 50,176 triangles of
+// which half are partly dry; at 31,486 wet ones it saves 10 of 65.  (Edges and an
+// empty general list alone in that kernel: 18 us, in their own 13.)
+constexpr int RES_ALL_TRIS = 65536, JAC_ALL_TRIS = 32768;
+
+// The element Jacobians of both lists and, with `edges`, the boundary's.
+static void launch_jac_split(Ctx *c, const ElemData &D, bool edges) {
+    const int B = edges ? c->B : 0;
+    const int *blkpos1 = c->blkpos + 9 * (size_t)c->E;
+    if (c->E && !c->split_valid) launch_split(c);
+    const bool all = c->E && c->E <= JAC_ALL_TRIS && c->tune.bs[0] == JAC_ALL_BS && c->tune.bs[1] == JAC_ALL_BS &&
+                     c->tune.layout[0] >= 2 && c->tune.layout[1] == c->tune.layout[0];
+    if (!all) {
+        if (c->E) {
+            launch_list(c, D, 0, c->tune.bs[0], c->tune.grid[0], c->tune.layout[0]);
+            launch_list(c, D, 1, c->tune.bs[1], c->tune.grid[1], c->tune.layout[1]);
+        }
+        if (B)
+            hipLaunchKernelGGL(k_jac1d, dim3(nblocks_for(6 * B, 128)), dim3(128), 0, c->stream, D, B, c->loc_bc[0],
+                               c->loc_bc[1], blkpos1, c->EM, em32_of(c));
+        return;
+    }
+    const int groups = (c->E + 31) / 32;
+    const int cols = c->tune.layout[0] == 2 ? 1 : jac_columns(groups);
+    const int need = nblocks_for(9 / cols * groups, JAC_ALL_BS / 64);
+    const int nwet = std::min(c->tune.grid[0], need), ngen = std::min(c->tune.grid[1], need);
+    const dim3 g(nwet + ngen + (B ? nblocks_for(6 * B, JAC_ALL_BS) : 0));
+    auto launch = [&](auto n) {
+        hipLaunchKernelGGL((k_jac_all<JAC_ALL_BS, decltype(n)::value>), g, dim3(JAC_ALL_BS), 0, c->stream, D,
+                           c->elist_wet, c->elist_gen, c->ecount, c->loc_bc[0], c->loc_bc[1], c->loc_bc[2], c->blkpos,
+                           c->EM, em32_of(c), nwet, ngen, B, blkpos1);
+    };
+    static_assert((JAC_ALL_TRIS + 31) / 32 < 2 * JAC_WAVES, "never nine columns a wave");
+    if (cols == 1) launch(std::integral_constant<int, 1>());
+    else launch(std::integral_constant<int, 3>());
 }
 
-static void launch_resid2d_split(Ctx *c, const ElemData &D) {
-    if (!c->E) return;
-    if (!c->split_valid) launch_split(c);
-    launch_list(c, D, 2, c->tune.bs[2], c->tune.grid[2], c->tune.layout[2]);
-    launch_list(c, D, 3, c->tune.bs[3], c->tune.grid[3], c->tune.layout[3]);
+// The element residuals of both lists and, with `edges`, the boundary's.
+static void launch_resid_split(Ctx *c, const ElemData &D, bool edges) {
+    const int B = edges ? c->B : 0;
+    double *er1 = c->ER + 9 * (size_t)c->E;
+    if (c->E && !c->split_valid) launch_split(c);
+    const int need = c->E ? nblocks_for(c->E, RES_ALL_BS) : 0;
+    const bool beside = c->E <= RES_ALL_TRIS && c->tune.bs[2] == RES_ALL_BS && c->tune.bs[3] == RES_ALL_BS;
+    if (c->E && !beside) launch_list(c, D, 2, c->tune.bs[2], c->tune.grid[2], c->tune.layout[2]);
+    if (c->E && c->tune.bs[3] != RES_ALL_BS)
+        launch_list(c, D, 3, c->tune.bs[3], c->tune.grid[3], c->tune.layout[3]);
+    const int nwet = beside ? std::min(c->tune.grid[2], need) : 0;
+    const int ngen = c->tune.bs[3] == RES_ALL_BS ? std::min(c->tune.grid[3], need) : 0;
+    const dim3 g(nwet + ngen + (B ? nblocks_for(B, RES_ALL_BS) : 0));
+    if (g.x == 0) return;
+    if (beside)
+        hipLaunchKernelGGL((k_resid_all<true, RES_ALL_BS>), g, dim3(RES_ALL_BS), 0, c->stream, D, c->elist_wet,
+                           c->elist_gen, c->ecount, c->ER, nwet, ngen, B, er1);
+    else
+        hipLaunchKernelGGL((k_resid_all<false, RES_ALL_BS>), g, dim3(RES_ALL_BS), 0, c->stream, D, c->elist_wet,
+                           c->elist_gen, c->ecount, c->ER, nwet, ngen, B, er1);
 }
 
 void launch_jacobian(Ctx *c) {
@@ -849,10 +949,7 @@ void launch_jacobian(Ctx *c) {
     D.first_elem = nullptr;
     D.ts = c->h_ts + TS_LOAD;
     c->em32 = em32_of(c) != nullptr;
-    launch_jac2d_split(c, D);
-    if (c->B)
-        hipLaunchKernelGGL(k_jac1d, dim3(nblocks_for(6 * c->B, 128)), dim3(128), 0, c->stream, D, c->B, c->loc_bc[0],
-                           c->loc_bc[1], c->blkpos + 9 * (size_t)c->E, c->EM, em32_of(c));
+    launch_jac_split(c, D, true);
 }
 
 // Ordered block assembly.  The element kernels store each 3x3 block at its
@@ -977,14 +1074,14 @@ void launch_jac2d_only(Ctx *c) {
     if (!c->pre_valid) launch_old_terms(c);
     ElemData D = c->ed;
     D.first_elem = nullptr;
-    launch_jac2d_split(c, D);
+    launch_jac_split(c, D, false);
 }
 
 void launch_resid2d_only(Ctx *c) {
     if (!c->pre_valid) launch_old_terms(c);
     ElemData D = c->ed;
     D.first_elem = c->first_elem;
-    launch_resid2d_split(c, D);
+    launch_resid_split(c, D, false);
 }
 
 void launch_assemble_only(Ctx *c) { launch_assemble(c); }

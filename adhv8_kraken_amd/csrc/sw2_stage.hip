@@ -53,9 +53,22 @@ __global__ void __launch_bounds__(256) k_stage_in(StageMap m, size_t first, size
     }
 }
 
+// SELL slot of each off-diagonal block, by row
+__global__ void k_offd_pos(int N, const int *row_ptr, const int *sell_ptr, int *pos) {
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    const int p0 = row_ptr[n], p1 = row_ptr[n + 1];
+    for (int p = p0; p < p1; p++) pos[p] = 64 * (sell_ptr[n >> 6] + p - p0) + (n & 63);
+}
+
 constexpr size_t word(const StageMap &m) { return m.kind == StageMap::INTS ? sizeof(int) : sizeof(double); }
 
 }  // namespace
+
+void launch_offd_pos(Ctx *c) {
+    hipLaunchKernelGGL(k_offd_pos, dim3(nblocks_for(c->N, 256)), dim3(256), 0, c->stream, c->N, c->row_ptr,
+                       c->sell_ptr, c->offd_pos);
+}
 
 hipError_t Stage::wait(int h) {
     if (!pending[h]) return hipSuccess;

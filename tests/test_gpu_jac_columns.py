@@ -1,6 +1,7 @@
 """The element Jacobian's column split at the edges of its rule: one column a
 wave up to 7,264 triangles, three up to 131,040, nine above; a last group of
-fewer than 32 triangles, and one triangle group in all.  Every split computes
+fewer than 32 triangles, and one triangle group in all; both sides of 32,768,
+up to which both lists and the edges share a launch.  Every split computes
 the same columns from the same inputs, so the assembled system equals the
 lane-per-column kernel's bit for bit.
 """
@@ -15,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("cells", [(4, 4), (17, 1), (56, 64), (227, 16), (56, 65), (252, 260), (256, 256)])
+@pytest.mark.parametrize("cells", [(4, 4), (17, 1), (56, 64), (227, 16), (56, 65), (128, 128), (128, 129),
+                                   (252, 260), (256, 256)])
 def test_column_split_equals_lane_kernel(cells, precision):
     p = mesh.floodplain(*cells)
     out = []

@@ -1,6 +1,7 @@
 """The wet / general triangle lists and the fused residual norms at the edges of
 their block counts: one triangle block and its remainder, 1,024 count blocks (a
-block's first round of counts to add up) and more.  On a partly dry floodplain,
+block's first round of counts to add up) and more, and 65,536 triangles, up to
+which both lists share a launch.  On a partly dry floodplain,
 where both lists are filled, residual and opening norms equal the oracle's (the
 residual bit for bit, the l2 norm to the rounding of another summation order:
 N eps of its square).
@@ -15,7 +16,7 @@ from adhv8_kraken_amd.sw2 import default_opts
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("cells", [(1, 1), (16, 8), (13, 10), (512, 256), (640, 250)])
+@pytest.mark.parametrize("cells", [(1, 1), (16, 8), (13, 10), (256, 128), (256, 129), (512, 256), (640, 250)])
 def test_lists_and_norms_equal_oracle(cells):
     p = mesh.floodplain(*cells)
     o, g = pair(p, None, default_opts(max_nonlin_it=1, tol_nonlin=1e30))
