@@ -35,3 +35,19 @@ def test_column_split_equals_lane_kernel(cells, precision):
     for a, b in zip(*out):
         assert np.isfinite(a).all() and np.abs(a).max() > 0.0
         assert bits_equal(a, b)
+
+
+def test_autotuned_jacobian_is_no_slower_than_the_default():
+    """The autotuner's times are those of its launches: the shape it keeps runs
+    as fast as it says (twice that at most, a single timing of a launch of 0.2
+    ms) and no slower than the default's (within a quarter)."""
+    g = SW2Model(mesh.bumpy_channel(400, 200), default_opts(precision=1))
+    g.shift(); g.init(); g.resid()
+    before = g.time_kernel(1, 20)
+    chosen = g.autotune(3)
+    after = g.time_kernel(1, 20)
+    say(f"  default {before:.4f} ms, tuned {after:.4f} ms, {chosen['jac_wet']}")
+    assert 0.5 * after < chosen["jac_wet"]["ms"] < 2.0 * after
+    assert after < 1.25 * before
+    assert 0.0 < chosen["res_wet"]["ms"] < 0.8 * chosen["jac_wet"]["ms"]
+    g.close()
