@@ -289,6 +289,12 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     c.N = m->nnodes; c.E = m->nelems2d; c.B = m->nelems1d; c.M = m->nmat;
     c.Np = (c.N + 63) & ~63;
     c.kgraph_prec = -1;
+    // Launch shapes of the wet lists before any tuning.  us at 1M / 250,000 /
+    // 160,000 / 50,000 triangles: Jacobian, 256 threads and 4,096 workgroups 752 /
+    // 221 / 165 / 62, 128 and 8,192 734 / 216 / 164 / 64; residual, 128 threads and
+    // 4,096 workgroups 141 / 41 / 35 / 17, 2,048 of them 159 / 41 / 35 / 17 (a third
+    // round of workgroups nearly empty).
+    if (m->nelems2d > 131040) { c.tune.bs[0] = 128; c.tune.grid[0] = 8192; }
     c.run_cap[0] = c.run_cap[1] = c.run_prec = -1;
     c.run_max_blocks = nblocks_for(c.N, 256);
     c.run_limit = 200000;   // 2 ms: a hand-over takes 2 to 5 us when every block is resident
