@@ -138,10 +138,10 @@ def jacobian_roofline(g, p):
     every triangle's 18 perturbed residuals evaluated in full, as the
     reference does (the pressure block for the 6 depth perturbations only,
     fe_sw2_body_resid.c:761-862), counted with rocprofv3 FP64 instruction
-    counters on the column-uniform kernel that does exactly that (layout 2,
-    committed summary) -- over the live HIP-event time of the kernel in use.
-    The default kernel executes less (the drag coefficient shared by a
-    triangle's u and v columns); its own count is reported beside it."""
+    counters on a column-uniform kernel that did exactly that (committed
+    summary) -- over the live HIP-event time of the kernel in use.  The
+    default kernel executes less (terms that a perturbation leaves as they are
+    are formed once per triangle); its own count is reported beside it."""
     kernel, kname = JAC_KERNELS[g.get_tuning().layout[0]]
     ms = g.time_kernel(1, reps=5)
     flops = executed = traffic = None
