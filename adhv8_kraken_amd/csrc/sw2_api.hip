@@ -297,7 +297,10 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     if (m->nelems2d > 131040) { c.tune.bs[0] = 128; c.tune.grid[0] = 8192; }
     c.run_cap[0] = c.run_cap[1] = c.run_prec = -1;
     c.run_max_blocks = nblocks_for(c.N, 256);
-    c.run_limit = 200000;   // 2 ms: a hand-over takes 2 to 5 us when every block is resident
+    // 0.3 ms: a hand-over takes 3 to 13 us when every block is resident, and what a
+    // time-out costs is small (two threads' 500 x 250 models, which do not fit
+    // together, six steps each: 24.8 ms, with 2 ms 27, a kernel per step 23.4)
+    c.run_limit = 30000;
     if (opts) {
         int rc0 = check_opts(opts);
         if (rc0) { delete h; return rc0; }
@@ -985,9 +988,10 @@ static void chunk_plan(const Ctx &c, int &first, int &more) {
 // The solve as one kernel where the models fit on the GPU (sw2_run.hip).
 // *done: every model finished; otherwise a hand-over timed out or the system
 // does not take this form, and the caller solves from the prologue.  After a
-// time-out the next solves are left to the other form: what held the CUs
-// (another stream's or program's long kernels) may still do.
-constexpr int RUN_PAUSE = 64;
+// time-out the next solves are left to the other form, twice as many after
+// each in a row: what held the CUs (another stream's or program's kernels) may
+// still do.
+constexpr int RUN_PAUSE = 64, RUN_PAUSE_DOUBLINGS = 6;
 static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     *done = false;
     if (c.run_pause > 0) { c.run_pause--; return 0; }
@@ -996,7 +1000,12 @@ static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     HIPCHK(hipStreamSynchronize(c.stream));
     *done = true;
     for (int i = 0; i < n; i++) *done = *done && c.h_ksc[i].done;
-    if (!*done) { c.run_pause = RUN_PAUSE; c.run_dirty = 1; }
+    if (*done) {
+        c.run_giveups = 0;
+    } else {
+        c.run_pause = RUN_PAUSE << std::min(c.run_giveups++, RUN_PAUSE_DOUBLINGS);
+        c.run_dirty = 1;
+    }
     return 0;
 }
 
@@ -1766,7 +1775,7 @@ extern "C" int adh_sw2_hip_get_tuning(adh_sw2_hip *h, adh_sw2_tuning *out) {
 extern "C" int adh_sw2_hip_set_solve_wait(adh_sw2_hip *h, long long ticks) {
     if (!h) return fail(ADH_SW2_EINVAL, "null argument");
     h->c.run_limit = ticks;
-    h->c.run_pause = 0;
+    h->c.run_pause = h->c.run_giveups = 0;
     return 0;
 }
 

@@ -229,6 +229,7 @@ struct Ctx {
     int run_cap[2];        // blocks the GPU holds at once in form run_prec, at one and two a CU (-1: not asked yet)
     int run_max_blocks;    // 256-node blocks of the largest model
     int run_pause;         // solves left to the kernel-per-step form after a hand-over timed out
+    int run_giveups;       // such solves in a row
     long long run_limit;   // bound of a hand-over's wait, 100 MHz ticks
     // profile-LU (OP BLK) preconditioner, built on demand for opts.nblock
     int band_nblock;       // block count of the current band structure (0 = none)

@@ -308,7 +308,7 @@ int adh_sw2_hip_set_tuning(adh_sw2_hip *h, const adh_sw2_tuning *t);
 
 /* Block-Jacobi BiCGSTAB solves of models of up to 131,072 nodes run as one
  * kernel whose workgroups wait for each other.  A wait longer than `ticks` of
- * a 100 MHz clock (default 200000, 2 ms) ends it, and the solve is repeated
+ * a 100 MHz clock (default 30000, 0.3 ms) ends it, and the solve is repeated
  * as a kernel per step, with the same result; below 0 every solve is.  No
  * counterpart in the reference. */
 int adh_sw2_hip_set_solve_wait(adh_sw2_hip *h, long long ticks);

@@ -12,7 +12,7 @@ from adhv8_kraken_amd import mesh
 from adhv8_kraken_amd.sw2 import SW2Ensemble, SW2Model, default_opts
 
 pytestmark = pytest.mark.gpu
-PER_STEP, NO_WAIT, DEFAULT = -1, 0, 200000
+PER_STEP, NO_WAIT, DEFAULT = -1, 0, 30000
 
 
 def _flipped(p, every):
@@ -82,3 +82,34 @@ def test_one_kernel_solve_of_more_models_than_fit_at_once(precision):
         assert [q["lin_its"] for q in r] == [q["lin_its"] for q in runs[0][0]]
         for a, b in zip(s, runs[0][1]):
             assert all(bits_equal(x, y) for x, y in zip(a, b))
+
+
+def test_models_of_three_threads_that_do_not_fit_together():
+    """Three handles stepped by three threads at once, 315 blocks each of the 512
+    that the GPU holds: whichever solves find the CUs taken give up and are
+    repeated, and every model ends where it ends alone, bit for bit."""
+    import threading
+    ps = [mesh.bumpy_channel(401, 199, seed=k) for k in range(3)]
+    opts = default_opts(max_nonlin_it=3, tol_nonlin=1e-9)
+
+    def steps(p):
+        g = SW2Model(p, opts)
+        for _ in range(3):
+            g.timestep()
+        s = g.get_state()
+        g.close()
+        return s
+
+    alone = [steps(p) for p in ps]
+    together = [None] * 3
+
+    def run(k):
+        together[k] = steps(ps[k])
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(alone, together):
+        assert b is not None and all(bits_equal(x, y) for x, y in zip(a, b))
