@@ -259,7 +259,9 @@ struct Ctx {
     std::vector<void *> ilu_allocs;
     int *ilu_rnode, *ilu_lptr, *ilu_uptr, *ilu_lcol, *ilu_ucol, *ilu_lsrc, *ilu_usrc, *ilu_tptr;
     int4 *ilu_upd;
-    double *ilu_Lw, *ilu_Uw, *ilu_Dw, *ilu_Dinv, *ilu_w;   // FP64 factor work, colour-ordered vector
+    double *ilu_Uw, *ilu_Dinv, *ilu_w;     // FP64 upper blocks and inverses, colour-ordered vector
+    double *ilu_spill;                     // rows under factorisation that the LDS does not hold
+    int ilu_maxblk;                        // blocks of a row at most (with the padding of its slice)
     double *ilu_xw;                        // the backward sweep's x in colour order
     int *ilu_tick;                         // tickets of the two sweeps
     void *ilu_L, *ilu_U, *ilu_D;           // the apply's factors (FP64 or FP32) and U_ii^-1
@@ -274,34 +276,52 @@ __device__ __forceinline__ void stamp(long long *ts) {
     if (ts && blockIdx.x == 0 && threadIdx.x == 0) *ts = wall_clock64();
 }
 
-// 3x3 block inverse by Gauss-Jordan with partial pivoting (block-Jacobi set-up)
+// 3x3 block inverse by Gauss-Jordan with partial pivoting (block-Jacobi and
+// ILU set-up).  The row exchange is a select per entry: indexed by the pivot row
+// the array lies in scratch memory, which made an ILU(0) colour without any
+// update 27 us long.
 __device__ __forceinline__ void inv3(const double (&d)[9], double (&inv)[9]) {
     double a[3][6];
+#pragma unroll
     for (int r = 0; r < 3; r++)
+#pragma unroll
         for (int c = 0; c < 3; c++) {
             a[r][c] = d[3 * r + c];
             a[r][3 + c] = (r == c) ? 1.0 : 0.0;
         }
+#pragma unroll
     for (int k = 0; k < 3; k++) {
         int p = k;
-        for (int r = k + 1; r < 3; r++) if (fabs(a[r][k]) > fabs(a[p][k])) p = r;
-        if (p != k)
-            for (int c = 0; c < 6; c++) { double t = a[k][c]; a[k][c] = a[p][c]; a[p][c] = t; }
+        double big = a[k][k];
+#pragma unroll
+        for (int r = k + 1; r < 3; r++)
+            if (fabs(a[r][k]) > fabs(big)) { p = r; big = a[r][k]; }
+#pragma unroll
+        for (int r = k + 1; r < 3; r++)
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                const double u = a[k][c], v = a[r][c];
+                a[k][c] = p == r ? v : u;
+                a[r][c] = p == r ? u : v;
+            }
         double piv = a[k][k];
         if (fabs(piv) < SMALL) piv = (piv < 0) ? -SMALL : SMALL;
-        double ip = 1.0 / piv;
+        const double ip = 1.0 / piv;
+#pragma unroll
         for (int c = 0; c < 6; c++) a[k][c] *= ip;
+#pragma unroll
         for (int r = 0; r < 3; r++) {
             if (r == k) continue;
-            double f = a[r][k];
+            const double f = a[r][k];
+#pragma unroll
             for (int c = 0; c < 6; c++) a[r][c] -= f * a[k][c];
         }
     }
+#pragma unroll
     for (int r = 0; r < 3; r++)
+#pragma unroll
         for (int c = 0; c < 3; c++) inv[3 * r + c] = a[r][3 + c];
 }
-
-
 
 // value index of entry e (0..8) of SELL slot q
 __host__ __device__ __forceinline__ size_t sell_vidx(size_t q, int e) {

@@ -17,8 +17,7 @@
 //     L_ik = A_ik U_kk^-1,   A_ij -= L_ik U_kj  for j in row i with pos(j) > pos(k)
 // (j = i included), then U_ii = A_ii and U_ij = A_ij for the upper j.  Rows
 // of one colour depend only on rows of smaller colours, so each colour is
-// one launch with a thread per row; the (k, j) update lists are built once
-// on the host.  The factors are formed in FP64 from the scaled system and
+// one launch; the (k, j) update lists are built once on the host.  The factors are formed in FP64 from the scaled system and
 // stored in FP64 (precision 0) or FP32 (precision 1).
 //
 // Apply (in place on a node-ordered vector): forward sweeps z_i = v_i -
@@ -59,74 +58,137 @@ struct IluView {
 __device__ __forceinline__ size_t ilu_v(size_t slot_base, int e, int lane) { return 9 * 64 * slot_base + 64 * e + lane; }
 __device__ __forceinline__ size_t ilu_w(int r, int k) { return 3 * (size_t)(r & ~63) + 64 * k + (r & 63); }
 
-// Copies the scaled system into the factor work arrays (FP64).
-template <typename MT>
-__global__ void __launch_bounds__(256) k_ilu_load(IluView V, const int *lsrc, const int *usrc, const MT *diag,
-                                                  const MT *offd, double *Lw, double *Uw, double *Dw) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= V.Rp) return;
+// One colour of the factorisation, a workgroup per 64-row slice.  A row's blocks
+// (its lower slots, upper slots and diagonal) are taken from the scaled system
+// into LDS, a block per wave, where one wave's updates change them, and leave in
+// the apply's precision; the
+// upper blocks and U_ii^-1, which later colours read, also in FP64 (Uw, Dinv; the
+// apply's own arrays when those are FP64).  upd[tptr[r] .. tptr[r+1]) lists, in
+// the order of the row's lower slots, (lower slot b, U slot of row k holding
+// U_kj, target): target >= 0 an L slot of row r, -1 - t a U slot t of row r, and
+// INT_MIN the diagonal; an update's block is fetched while the one before is
+// applied.  80,400 nodes, four colours: 64 us a set-up (9 us for the first
+// colour, which has no updates, 15 to 21 for the others); with the row in
+// memory, a copy in before and copies out after it 158, with one wave for all
+// 134 (its code is run once and waits to be fetched).
+// IN_LDS = false: rows of more blocks than the LDS holds stay in `spill`.
+constexpr int FAC_W = 8;   // waves
+template <typename MT, typename FT, bool IN_LDS>
+__global__ void __launch_bounds__(64 * FAC_W) k_ilu_factor(IluView V, int s0, const int *lsrc, const int *usrc,
+                                                   const MT *diag, const MT *offd, const int *tptr, const int4 *upd,
+                                                   double *Uw, double *Dinv, FT *L, FT *U, FT *Df, double *spill,
+                                                   int maxblk) {
+    extern __shared__ double lds[];
+    double *row = IN_LDS ? lds : spill + 576 * (size_t)maxblk * blockIdx.x;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int s = s0 + blockIdx.x, r = 64 * s + lane;
     const int node = V.rnode[r];
-    const int s = r >> 6, lane = r & 63;
-    for (int e = 0; e < 9; e++) Dw[ilu_v(s, e, lane)] = node >= 0 ? (double)diag[didx9(node, e)] : (e % 4 == 0 ? 1.0 : 0.0);
-    for (int b = V.lptr[s]; b < V.lptr[s + 1]; b++) {
-        const int q = lsrc[64 * (size_t)b + lane];
-        for (int e = 0; e < 9; e++) Lw[ilu_v(b, e, lane)] = q >= 0 ? (double)offd[sell_vidx((size_t)q, e)] : 0.0;
+    const int l0 = V.lptr[s], nl = V.lptr[s + 1] - l0, u0 = V.uptr[s], nu = V.uptr[s + 1] - u0;
+    auto at = [&](int b, int e) -> double & { return row[64 * (9 * b + e) + lane]; };
+    const int dg = nl + nu;
+    for (int b = wv; b <= dg; b += FAC_W) {
+        double x[9];
+        if (b == dg) {
+#pragma unroll
+            for (int e = 0; e < 9; e++) x[e] = node >= 0 ? (double)diag[didx9(node, e)] : (e % 4 == 0 ? 1.0 : 0.0);
+        } else {
+            const int q = b < nl ? lsrc[64 * (size_t)(l0 + b) + lane] : usrc[64 * (size_t)(u0 + b - nl) + lane];
+#pragma unroll
+            for (int e = 0; e < 9; e++) x[e] = q >= 0 ? (double)offd[sell_vidx((size_t)q, e)] : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < 9; e++) at(b, e) = x[e];
     }
-    for (int b = V.uptr[s]; b < V.uptr[s + 1]; b++) {
-        const int q = usrc[64 * (size_t)b + lane];
-        for (int e = 0; e < 9; e++) Uw[ilu_v(b, e, lane)] = q >= 0 ? (double)offd[sell_vidx((size_t)q, e)] : 0.0;
-    }
-}
-
-// One colour of the factorisation.  upd[tptr[r] .. tptr[r+1]) lists, in the
-// order of the row's lower slots, (lower slot b, U slot of row k holding
-// U_kj, target): target >= 0 an L slot of row r, -1 - t a U slot t of row r,
-// and INT_MIN the diagonal.  Dinv holds U_kk^-1 of the rows already factored.
-__global__ void __launch_bounds__(256) k_ilu_factor(IluView V, int r0, int r1, const int *tptr, const int4 *upd,
-                                                    double *Lw, double *Uw, double *Dw, double *Dinv) {
-    const int r = r0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= r1) return;
-    const int s = r >> 6, lane = r & 63;
-    int t = tptr[r];
-    const int t1 = tptr[r + 1];
-    if (V.rnode[r] >= 0) {
-        for (int b = V.lptr[s]; b < V.lptr[s + 1]; b++) {
-            const int k = V.lcol[64 * (size_t)b + lane];
-            if (k < 0) continue;
-            // L_ik = A_ik U_kk^-1
-            double a[9], l[9];
-            for (int e = 0; e < 9; e++) a[e] = Lw[ilu_v(b, e, lane)];
-            const size_t dk = ilu_v(k >> 6, 0, k & 63);
+    __syncthreads();
+    if (wv == 0 && node >= 0 && nl > 0) {
+        const int4 none = make_int4(-1, 0, 0, 0);
+        const int t0 = tptr[r], t1 = tptr[r + 1];
+        auto entry = [&](int i) { return i < t1 ? upd[i] : none; };
+        auto block = [&](const int4 &u, double (&x)[9]) {
+            if (u.x >= 0)
+#pragma unroll
+                for (int e = 0; e < 9; e++) x[e] = Uw[ilu_v((size_t)u.y >> 6, 0, u.y & 63) + 64 * e];
+        };
+        // L_ik = A_ik U_kk^-1 of the lower slots up to `want`; the next slot's column
+        // and inverse are on their way
+        auto column = [&](int b) { return b < nl ? V.lcol[64 * (size_t)(l0 + b) + lane] : -1; };
+        auto inverse = [&](int k, double (&x)[9]) {
+            if (k >= 0)
+#pragma unroll
+                for (int e = 0; e < 9; e++) x[e] = Dinv[ilu_v(k >> 6, 0, k & 63) + 64 * e];
+        };
+        int b = -1, k = column(0), kn = column(1);
+        double dk[9] = {}, l[9] = {};
+        inverse(k, dk);
+        auto to_slot = [&](int want) {
+            while (b < want) {
+                b++;
+                if (k >= 0) {
+                    double x[9];
+#pragma unroll
+                    for (int e = 0; e < 9; e++) x[e] = at(b, e);
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+#pragma unroll
+                        for (int j = 0; j < 3; j++)
+                            l[3 * i + j] = x[3 * i] * dk[j] + x[3 * i + 1] * dk[3 + j] + x[3 * i + 2] * dk[6 + j];
+#pragma unroll
+                    for (int e = 0; e < 9; e++) at(b, e) = l[e];
+                }
+                k = kn;
+                inverse(k, dk);
+                kn = column(b + 2);
+            }
+        };
+        // A_ij -= L_ik U_kj
+        auto apply = [&](const int4 &u, const double (&x)[9]) {
+            to_slot(u.x - l0);
+            const int to = u.z == INT_MIN ? dg : (u.z >= 0 ? u.z - l0 : nl + (-1 - u.z) - u0);
+#pragma unroll
             for (int i = 0; i < 3; i++)
+#pragma unroll
                 for (int j = 0; j < 3; j++)
-                    l[3 * i + j] = a[3 * i] * Dinv[dk + 64 * j] + a[3 * i + 1] * Dinv[dk + 64 * (3 + j)] +
-                                   a[3 * i + 2] * Dinv[dk + 64 * (6 + j)];
-            for (int e = 0; e < 9; e++) Lw[ilu_v(b, e, lane)] = l[e];
-            // A_ij -= L_ik U_kj
-            for (; t < t1 && upd[t].x == b; t++) {
-                const int4 u = upd[t];
-                const size_t src = ilu_v((size_t)u.y >> 6, 0, u.y & 63);
-                double *dst;
-                if (u.z == INT_MIN) dst = Dw + ilu_v(s, 0, lane);
-                else if (u.z >= 0) dst = Lw + ilu_v(u.z, 0, lane);
-                else dst = Uw + ilu_v(-1 - u.z, 0, lane);
-                for (int i = 0; i < 3; i++)
-                    for (int j = 0; j < 3; j++)
-                        dst[64 * (3 * i + j)] -= l[3 * i] * Uw[src + 64 * j] + l[3 * i + 1] * Uw[src + 64 * (3 + j)] +
-                                                 l[3 * i + 2] * Uw[src + 64 * (6 + j)];
+                    at(to, 3 * i + j) -= l[3 * i] * x[j] + l[3 * i + 1] * x[3 + j] + l[3 * i + 2] * x[6 + j];
+        };
+        // two entries a turn, each block in registers of its own: one is fetched while the other is applied
+        int4 ua = entry(t0), ub = entry(t0 + 1);
+        double xa[9] = {}, xb[9] = {};
+        block(ua, xa);
+        for (int t = t0; t < t1; t += 2) {
+            block(ub, xb);
+            const int4 uc = entry(t + 2), ud = entry(t + 3);
+            apply(ua, xa);
+            block(uc, xa);
+            if (ub.x >= 0) apply(ub, xb);
+            ua = uc;
+            ub = ud;
+        }
+        to_slot(nl - 1);
+    }
+    __syncthreads();
+    for (int b = wv; b <= dg; b += FAC_W) {
+        double x[9];
+#pragma unroll
+        for (int e = 0; e < 9; e++) x[e] = at(b, e);
+        if (b == dg) {
+            double inv[9];
+            inv3(x, inv);
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                Dinv[ilu_v(s, e, lane)] = inv[e];
+                if constexpr (sizeof(FT) < sizeof(double)) Df[ilu_v(s, e, lane)] = (FT)inv[e];
+            }
+        } else if (b < nl) {
+#pragma unroll
+            for (int e = 0; e < 9; e++) L[ilu_v(l0 + b, e, lane)] = (FT)x[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                Uw[ilu_v(u0 + b - nl, e, lane)] = x[e];
+                if constexpr (sizeof(FT) < sizeof(double)) U[ilu_v(u0 + b - nl, e, lane)] = (FT)x[e];
             }
         }
     }
-    double d[9], inv[9];
-    for (int e = 0; e < 9; e++) d[e] = Dw[ilu_v(s, e, lane)];
-    inv3(d, inv);
-    for (int e = 0; e < 9; e++) Dinv[ilu_v(s, e, lane)] = inv[e];
-}
-
-template <typename FT>
-__global__ void k_ilu_store(size_t n, const double *a, FT *b) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = (FT)a[i];
 }
 
 // forward sweep of one colour: w_r = v_node - sum_b L_b w_col
@@ -282,6 +344,9 @@ void ilu_free(Ctx *c) {
     c->ilu_ncolor = 0;
 }
 
+// blocks of a 64-row slice's rows that fit in the 64 KB of LDS a launch has
+constexpr int ILU_LDS_BLOCKS = (64 << 10) / (576 * 8);
+
 // Greedy colouring, colour-ordered rows, the lower/upper slot structure and
 // the update lists, built once per pattern.  Returns an error text or "".
 std::string ilu_structure(Ctx *c) {
@@ -394,6 +459,11 @@ std::string ilu_structure(Ctx *c) {
         return true;
     };
     const size_t fsz = c->opts.precision >= 1 ? sizeof(float) : sizeof(double);
+    // blocks of a row at most, and whether they leave the 64 KB of LDS a launch has
+    int maxblk = 1;
+    for (int sl = 0; sl < nsl; sl++) maxblk = std::max(maxblk, lptr[sl + 1] - lptr[sl] + uptr[sl + 1] - uptr[sl] + 1);
+    const bool spill = maxblk > ILU_LDS_BLOCKS;
+    c->ilu_maxblk = maxblk;
     bool ok = up_dev((void **)&c->ilu_rnode, rnode.data(), sizeof(int) * Rp) &&
               up_dev((void **)&c->ilu_lptr, lptr.data(), sizeof(int) * lptr.size()) &&
               up_dev((void **)&c->ilu_uptr, uptr.data(), sizeof(int) * uptr.size()) &&
@@ -403,16 +473,20 @@ std::string ilu_structure(Ctx *c) {
               up_dev((void **)&c->ilu_usrc, usrc.data(), sizeof(int) * usrc.size()) &&
               up_dev((void **)&c->ilu_tptr, tptr.data(), sizeof(int) * tptr.size()) &&
               up_dev((void **)&c->ilu_upd, upd.data(), sizeof(int4) * upd.size()) &&
-              alloc((void **)&c->ilu_Lw, sizeof(double) * 9 * std::max<size_t>(nl, 1)) &&
-              alloc((void **)&c->ilu_Uw, sizeof(double) * 9 * std::max<size_t>(nu, 1)) &&
-              alloc((void **)&c->ilu_Dw, sizeof(double) * 9 * (size_t)Rp) &&
-              alloc((void **)&c->ilu_Dinv, sizeof(double) * 9 * (size_t)Rp) &&
+              alloc((void **)&c->ilu_spill, spill ? sizeof(double) * 9 * (size_t)Rp * maxblk : sizeof(double)) &&
               alloc((void **)&c->ilu_w, sizeof(double) * 3 * (size_t)Rp) &&
               alloc((void **)&c->ilu_xw, sizeof(double) * 3 * (size_t)Rp) &&
               alloc((void **)&c->ilu_tick, sizeof(int) * 2) &&
               alloc((void **)&c->ilu_L, fsz * 9 * std::max<size_t>(nl, 1)) &&
               alloc((void **)&c->ilu_U, fsz * 9 * std::max<size_t>(nu, 1)) &&
               alloc((void **)&c->ilu_D, fsz * 9 * (size_t)Rp);
+    if (ok && fsz < sizeof(double))   // the FP64 upper blocks and inverses that the factorisation reads
+        ok = alloc((void **)&c->ilu_Uw, sizeof(double) * 9 * std::max<size_t>(nu, 1)) &&
+             alloc((void **)&c->ilu_Dinv, sizeof(double) * 9 * (size_t)Rp);
+    else if (ok) {
+        c->ilu_Uw = (double *)c->ilu_U;
+        c->ilu_Dinv = (double *)c->ilu_D;
+    }
     if (!ok) {
         ilu_free(c);
         return "hipMalloc failed for the ILU(0) factors";
@@ -431,32 +505,26 @@ std::string ilu_structure(Ctx *c) {
     return "";
 }
 
-// Loads the scaled system, factors colour by colour, stores the factors in
-// the apply's precision.
-void launch_ilu_setup(Ctx *c) {
+// Factors the scaled system colour by colour into the apply's precision.
+template <typename MT, typename FT>
+static void ilu_factor(Ctx *c, const MT *diag, const MT *offd) {
     IluView V = iview(c);
-    const int nb = nblocks_for(c->ilu_Rp, 256);
-    if (c->ilu_f32)
-        hipLaunchKernelGGL(k_ilu_load<float>, dim3(nb), dim3(256), 0, c->stream, V, c->ilu_lsrc, c->ilu_usrc,
-                           c->diag32, c->offd32, c->ilu_Lw, c->ilu_Uw, c->ilu_Dw);
-    else
-        hipLaunchKernelGGL(k_ilu_load<double>, dim3(nb), dim3(256), 0, c->stream, V, c->ilu_lsrc, c->ilu_usrc,
-                           c->diag, c->offd, c->ilu_Lw, c->ilu_Uw, c->ilu_Dw);
+    const bool in_lds = c->ilu_maxblk <= ILU_LDS_BLOCKS;
     for (int k = 0; k < c->ilu_ncolor; k++) {
-        const int r0 = c->h_ilu_cstart[k], r1 = c->h_ilu_cstart[k + 1];
-        hipLaunchKernelGGL(k_ilu_factor, dim3(nblocks_for(r1 - r0, 256)), dim3(256), 0, c->stream, V, r0, r1,
-                           c->ilu_tptr, c->ilu_upd, c->ilu_Lw, c->ilu_Uw, c->ilu_Dw, c->ilu_Dinv);
+        const int s0 = c->h_ilu_cstart[k] / 64, s1 = c->h_ilu_cstart[k + 1] / 64;
+        auto launch = [&](auto kern, size_t lds) {
+            hipLaunchKernelGGL(kern, dim3(s1 - s0), dim3(64 * FAC_W), lds, c->stream, V, s0, c->ilu_lsrc, c->ilu_usrc, diag,
+                               offd, c->ilu_tptr, c->ilu_upd, c->ilu_Uw, c->ilu_Dinv, (FT *)c->ilu_L, (FT *)c->ilu_U,
+                               (FT *)c->ilu_D, c->ilu_spill, c->ilu_maxblk);
+        };
+        if (in_lds) launch(k_ilu_factor<MT, FT, true>, sizeof(double) * 576 * (size_t)c->ilu_maxblk);
+        else launch(k_ilu_factor<MT, FT, false>, 0);
     }
-    const size_t nl9 = 9 * c->ilu_nl, nu9 = 9 * c->ilu_nu, nd9 = 9 * (size_t)c->ilu_Rp;
-    if (c->ilu_f32) {
-        hipLaunchKernelGGL(k_ilu_store<float>, dim3(nblocks_for((int)nl9, 256)), dim3(256), 0, c->stream, nl9, c->ilu_Lw, (float *)c->ilu_L);
-        hipLaunchKernelGGL(k_ilu_store<float>, dim3(nblocks_for((int)nu9, 256)), dim3(256), 0, c->stream, nu9, c->ilu_Uw, (float *)c->ilu_U);
-        hipLaunchKernelGGL(k_ilu_store<float>, dim3(nblocks_for((int)nd9, 256)), dim3(256), 0, c->stream, nd9, c->ilu_Dinv, (float *)c->ilu_D);
-    } else {
-        hipLaunchKernelGGL(k_ilu_store<double>, dim3(nblocks_for((int)nl9, 256)), dim3(256), 0, c->stream, nl9, c->ilu_Lw, (double *)c->ilu_L);
-        hipLaunchKernelGGL(k_ilu_store<double>, dim3(nblocks_for((int)nu9, 256)), dim3(256), 0, c->stream, nu9, c->ilu_Uw, (double *)c->ilu_U);
-        hipLaunchKernelGGL(k_ilu_store<double>, dim3(nblocks_for((int)nd9, 256)), dim3(256), 0, c->stream, nd9, c->ilu_Dinv, (double *)c->ilu_D);
-    }
+}
+
+void launch_ilu_setup(Ctx *c) {
+    if (c->ilu_f32) ilu_factor<float, float>(c, c->diag32, c->offd32);
+    else ilu_factor<double, double>(c, c->diag, c->offd);
 }
 
 // Rows up to which a sweep runs in one launch: there a colour's launch (4.6 us

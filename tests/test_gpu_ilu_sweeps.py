@@ -34,6 +34,34 @@ def test_apply_matches_the_cpu_factors_at_unit_edges(cells):
     g.close()
 
 
+def _wheel():
+    """A 20 x 20 channel with one node of twelve neighbours: the edges around it
+    turned towards it.  Its slice's rows hold more blocks than the LDS."""
+    p = mesh.bumpy_channel(20, 20)
+    e = [list(t) for t in p.e2d.reshape(-1, 3)]
+    hub = p.nnodes // 2
+    for t in [t for t in e if hub in t]:
+        k = t.index(hub)
+        a, b = t[(k + 1) % 3], t[(k + 2) % 3]
+        u = next(x for x in e if x is not t and a in x and b in x)
+        c = next(n for n in u if n not in (a, b))
+        t[:] = [hub, a, c]
+        u[:] = [hub, c, b]
+    p.e2d = np.array(e, dtype=p.e2d.dtype).reshape(p.e2d.shape)
+    return p
+
+
+def test_factors_of_rows_beyond_the_lds():
+    g = _stepped(_wheel(), 3, 0)
+    D, O, rp, col = _scaled_system(g)
+    assert np.diff(rp).max() == 12
+    M = BlockILU0(D, O, colour_order(g.ilu_colors()[0])[1])
+    v = np.random.default_rng(1).uniform(-1, 1, 3 * g.N)
+    ref = M.apply(v)
+    assert np.abs(g.precond_apply(v) - ref).max() <= 1e-12 * np.abs(ref).max()
+    g.close()
+
+
 @pytest.mark.parametrize("cells", [(440, 440), (455, 450)])
 def test_apply_is_exact_without_fill_on_both_sides_of_the_rule(cells):
     g = SW2Model(mesh.bumpy_channel(*cells), default_opts(preconditioner=3))
