@@ -693,8 +693,8 @@ __global__ void __launch_bounds__(BS, 2) k_jac_all(ElemData D, const int *wet, c
 // Splits the triangles into those whose three depths stay positive under the
 // -eps perturbation of the FD Jacobian (h - eps(h) > 0, the exact operation
 // the perturbed residual performs) and the rest, as two ordered lists: block
-// counts, a one-block scan, then the ordered scatter (no same-address
-// atomics, which serialise across the whole grid).
+// counts, then the ordered scatter (no same-address atomics, which serialise
+// across the whole grid).
 __device__ __forceinline__ bool tri_stays_wet(int ie, const int *e2d, const double *head) {
     bool w = true;
     for (int i = 0; i < 3; i++) {
