@@ -546,7 +546,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     if ((rc = alloc_solver(h))) { adh_sw2_hip_destroy(h); return rc; }
     if (hipHostMalloc((void **)&c.h_ksc, sizeof(KScal) * nmod) != hipSuccess ||
         hipHostMalloc((void **)&c.h_norms, sizeof(Norms) * nmod) != hipSuccess ||
-        hipHostMalloc((void **)&c.h_flag, 64) != hipSuccess ||
+        hipHostMalloc((void **)&c.h_gave_up, sizeof(int)) != hipSuccess ||
         hipHostMalloc((void **)&c.h_ts, sizeof(long long) * TS_N) != hipSuccess || c.stage.create() != hipSuccess) {
         adh_sw2_hip_destroy(h);
         return fail(ADH_SW2_ENOMEM, "hipHostMalloc failed");
@@ -601,7 +601,7 @@ extern "C" void adh_sw2_hip_destroy(adh_sw2_hip *h) {
     for (void *p : h->allocs) (void)hipFree(p);
     if (c.h_ksc) (void)hipHostFree(c.h_ksc);
     if (c.h_norms) (void)hipHostFree(c.h_norms);
-    if (c.h_flag) (void)hipHostFree(c.h_flag);
+    if (c.h_gave_up) (void)hipHostFree(c.h_gave_up);
     if (c.h_ts) (void)hipHostFree(c.h_ts);
     c.stage.destroy();
     for (int i = 0; i < 2; i++) if (c.ev[i]) (void)hipEventDestroy(c.ev[i]);
@@ -990,7 +990,11 @@ static void chunk_plan(const Ctx &c, int &first, int &more) {
 // does not take this form, and the caller solves from the prologue.  After a
 // time-out the next solves are left to the other form, twice as many after
 // each in a row: what held the CUs (another stream's or program's kernels) may
-// still do.
+// still do.  A time-out at the last hand-over can leave every model finished
+// (the solution is stored before it), but the blocks that gave up have not
+// emptied their parts of the hand-over vectors, whose words the next solve would
+// take for its own: whether any wait timed out is therefore told by the kernel
+// apart from the models' results.
 constexpr int RUN_PAUSE = 64, RUN_PAUSE_DOUBLINGS = 6;
 static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     *done = false;
@@ -1000,12 +1004,9 @@ static int krylov_one_kernel(Ctx &c, bool zero_guess, bool *done) {
     HIPCHK(hipStreamSynchronize(c.stream));
     *done = true;
     for (int i = 0; i < n; i++) *done = *done && c.h_ksc[i].done;
-    if (*done) {
-        c.run_giveups = 0;
-    } else {
-        c.run_pause = RUN_PAUSE << std::min(c.run_giveups++, RUN_PAUSE_DOUBLINGS);
-        c.run_dirty = 1;
-    }
+    c.run_dirty = *c.h_gave_up || !*done;
+    if (*done) c.run_giveups = 0;
+    else c.run_pause = RUN_PAUSE << std::min(c.run_giveups++, RUN_PAUSE_DOUBLINGS);
     return 0;
 }
 

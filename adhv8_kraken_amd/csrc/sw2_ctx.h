@@ -191,7 +191,7 @@ struct Ctx {
     KScal *h_ksc;          // pinned, [max(1, ninst)]
     Red red;
     Norms *norms, *h_norms;  // [max(1, ninst)]
-    int *h_flag;           // pinned scratch
+    int *h_gave_up;        // pinned: a wait of the one-kernel solve (sw2_run.hip) ended without result
     Stage stage;
     int *offd_pos;         // the same as h_offd_pos, on the device
     ElemData ed;

@@ -93,7 +93,9 @@ __device__ __forceinline__ double uniform(double x) {
 // A wait gives up (all blocks do, then) after `limit` ticks of the 100 MHz
 // clock: another program's kernels may hold the CUs that this model's
 // remaining blocks wait for.  The caller then repeats the solve with the
-// kernel-per-step form.
+// kernel-per-step form.  At the last hand-over some blocks may give up and others
+// pass: the solve is then whole, but those that gave up leave their parts of the
+// vectors filled, so the host is told of every give-up and empties all vectors.
 constexpr int RING = 3, PARTS = 3, VRING = 4;
 using HO = Slot<double>;
 // Place of a partial: eight blocks' words to a 256-byte piece.  All blocks poll
@@ -107,6 +109,7 @@ struct HandOver {
     int nblk, k0, k1, blk;     // blocks in all, the model's range, this one
     int turn;
     int *quit;                 // the model's give-up flag
+    int *gave_up;              // the same for the host, of all models: the vectors are to be emptied
     long long limit;
     double (*shp)[4], (*shr)[4];
     int *shq;
@@ -116,8 +119,10 @@ struct HandOver {
     }
     // the wait that began at t0 is over without result
     __device__ __forceinline__ bool give_up(long long t0, int spin) {
-        if (wall_clock64() - t0 > limit) put_raw((float *)quit, 1u);
-        else if ((spin & 15) != 15 || !peek((float *)quit)) return false;
+        if (wall_clock64() - t0 > limit) {
+            put_raw((float *)quit, 1u);
+            *gave_up = 1;
+        } else if ((spin & 15) != 15 || !peek((float *)quit)) return false;
         *shq = 1;
         return true;
     }
@@ -266,7 +271,7 @@ template <typename P, int K, int OCC>
 __global__ void __launch_bounds__(256, OCC)
     k_bcg_run(int N, size_t n3, KVecs<P> V, typename P::V *xch, const int *sell_col, const double *rhs,
               const double *scale, double *sol, KScal *sc, KScal *host, const int *blk_inst, const int *inst_blk0, double *slots,
-              int parity, int *quit, long long limit) {
+              int parity, int *quit, int *gave_up, long long limit) {
     using T = typename P::V;
     using MT = typename P::M;
     // AGAIN: the neighbours' r in LDS instead of their Ap, which is read a second
@@ -292,6 +297,7 @@ __global__ void __launch_bounds__(256, OCC)
     H.blk = lb;
     H.turn = 0;
     H.quit = quit + 2 * m + parity;
+    H.gave_up = gave_up;
     H.limit = limit;
     H.shp = shp;
     H.shr = shr;
@@ -554,11 +560,12 @@ bool run_k(Ctx *c, bool zero_guess) {
                            VRING * n3, xch);
     }
     for (int i = 0; i < (c->ninst ? c->ninst : 1); i++) c->h_ksc[i].done = 0;   // the kernel sets what it finishes
+    *c->h_gave_up = 0;
     c->run_parity ^= 1;
     hipLaunchKernelGGL((k_bcg_run<P, K, OCC>), dim3(nb), dim3(256), 0, c->stream, c->N, n3, vecs<P>(c), xch,
                        c->sell_col, c->R, c->scale, zero_guess ? c->sol : nullptr, c->ksc, c->h_ksc,
                        c->ninst ? c->blk_inst : nullptr, c->ninst ? c->inst_blk0 : nullptr, c->run_slots,
-                       c->run_parity, c->run_quit, c->run_limit);
+                       c->run_parity, c->run_quit, c->h_gave_up, c->run_limit);
     return true;
 }
 
