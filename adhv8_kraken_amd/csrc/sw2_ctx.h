@@ -247,7 +247,7 @@ struct Ctx {
     size_t tb_size;
     TBand *tb_bands;
     double *tb_AB, *tb_LI, *tb_UI, *tb_xb, *tb_yb, *tb_zb;
-    int *tb_int, *tb_guard;   // sweep tickets [3 bands], then a guard flag per tile (tb_guard)
+    int *tb_int, *tb_guard;   // sweep tickets [3 bands], the claims of bands, then a guard flag per tile (tb_guard)
     int tb_nbot;           // bands running upwards, before all others; block b's other band is tb_nbot + b
     int tb_maxs;           // shared rows of the block with most of them
     std::vector<int> tb_h_na;   // host copy: panels before the shared rows, -1: a block in one band

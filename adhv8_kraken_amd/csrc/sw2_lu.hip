@@ -702,12 +702,12 @@ __device__ __forceinline__ double await_value(const double *p, bool want) {
 
 // The right-hand side into band order (nodes of no block skipped; the band from
 // the end has zeros on the shared rows), the two output vectors to NOT_YET, the
-// tickets to zero.
+// tickets (three a band, and the claims of bands) to zero.
 __global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, int nbot, const int *node_blk,
                                                    const TBand *bands, const double *x, double *xb, double *yb,
                                                    double *zb, int *tick) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int b = a; b < 3 * nband; b += gridDim.x * blockDim.x) tick[b] = 0;
+    for (int b = a; b < 3 * nband + 1; b += gridDim.x * blockDim.x) tick[b] = 0;
     if (a >= N) return;
     const int bk = node_blk[a];
     if (bk < 0) return;
@@ -739,6 +739,7 @@ constexpr int SW_RING = 32;              // values handed over between two barri
 struct SweepLds {
     double x[SW_RING][TB];
     double part[2][SW_W][TB];
+    int unit;        // SW_SHARED: the workgroup's place in the order of claims
     int ready;       // values handed over since the last barrier
     int rows[2][4];  // the next row and those claimed after it
 };
@@ -908,18 +909,27 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
 // Where blocks are factored from both ends, SHARED: the forward sweep of every
 // band and the backward sweep of the shared rows; then, those applied
 // (k_tb_apply), REST: the backward sweep of all others.  ALL: no such block.
-// Workgroups of bands from the end come first in the grid: the other bands'
-// wait for theirs, which wait for nothing outside the band.
+// In SHARED the bands from the start wait for those from the end, which wait for
+// nothing outside the band and come first in the list of bands.  A workgroup
+// takes its band by ticket (`claim`), so whatever order the workgroups start in,
+// every band from the end has its workgroups running before one waits for it.
+// (200 x 100 cells: both sweeps 1.83 ms, 1.84 with a band per grid index.)
 enum { SW_ALL, SW_SHARED, SW_REST };
 __global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, const double *AB, const double *xb, double *yb,
-                                                    double *zb, int *tick, int phase, const int *done, const int *mask,
-                                                    const KScal *sc) {
+                                                    double *zb, int *tick, int *claim, int phase, const int *done,
+                                                    const int *mask, const KScal *sc) {
     __shared__ SweepLds S;
+    int band = blockIdx.y;
+    if (phase == SW_SHARED) {
+        if (threadIdx.x == 0) S.unit = atomicAdd(claim, 1);
+        __syncthreads();
+        band = __builtin_amdgcn_readfirstlane(S.unit) / (int)gridDim.x;
+    }
     const int stop = *done;   // the band record and the flag fetched together
-    const TBand B = band_rec(bands, blockIdx.y, stop);
+    const TBand B = band_rec(bands, band, stop);
     // ensembles: the band's model, converged or outside the mask, is skipped
     if (stop || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
-    tick += 3 * blockIdx.y;
+    tick += 3 * band;
     if (phase != SW_REST) {
         const bool top = B.part >= 0 && !B.rev;
         tb_sweep<true>(B, AB, xb, yb, top ? yb + bands[B.part].xoff : nullptr, 0, B.nt, tick, S);
@@ -1033,7 +1043,7 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
             bot += top[b] > 0;
         }
         c->tb_nbot = nbot;
-        nint = toff + 3 * h.size();   // a guard flag per tile, three tickets per band
+        nint = toff + 3 * h.size() + 1;   // a guard flag per tile, three tickets per band, the claims
         need = sizeof(double) * (off + 2 * 4096 * toff + 3 * xoff) + sizeof(int) * nint;
         if (need + ((size_t)2 << 30) <= freeb) break;
         if (twist && nbot > 0) continue;
@@ -1067,7 +1077,7 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     c->tb_gt = (maxw + TB - 1) / TB;
     c->tb_gf = (maxw + 2 * TB - 2) / TB;   // tiles below (above) a panel that its L (U) reaches
     c->tb_size = off;
-    c->tb_guard = c->tb_int + 3 * nband;
+    c->tb_guard = c->tb_int + 3 * nband + 1;
     return "";
 }
 
@@ -1147,7 +1157,7 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 512 / c->tb_nband));
     auto sweep = [&](int phase) {
         hipLaunchKernelGGL(k_tb_sweep, dim3(g, c->tb_nband), dim3(SW_NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int, phase, done, mask, msc);
+                           c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int, c->tb_int + 3 * c->tb_nband, phase, done, mask, msc);
     };
     auto apply = [&](bool shared, int tiles) {
         hipLaunchKernelGGL(k_tb_apply, dim3(tiles, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_UI,
