@@ -118,6 +118,7 @@ hipError_t Stage::out(hipStream_t st, const StageMap &m, void *user, size_t coun
 }
 
 hipError_t Stage::finish_out(hipStream_t st) {
+    if (nseg[cur] == 0) return hipStreamSynchronize(st);   // nothing goes to the caller: the call's work is waited for
     hipError_t e = turn_over(st);   // drains the half before
     const hipError_t d = drain(cur ^ 1);
     nseg[0] = nseg[1] = 0;
