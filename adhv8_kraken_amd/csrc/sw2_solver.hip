@@ -153,8 +153,8 @@ __global__ void k_to_f32(size_t n, const double *a, float *b) {
                                c->diag32, c->offd32, c->dinv32, c->h_ts + TS_SETUP);                                \
         else                                                                                                        \
             hipLaunchKernelGGL((k_scale_apply<F32, BJ, K, false>), dim3(nb), dim3(256), 0, c->stream, c->N,         \
-                               c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, c->scale, c->R, c->sol,      \
-                               c->dinv, c->diag32, c->offd32, c->dinv32, c->h_ts + TS_SETUP);                       \
+                               c->diag, c->offd, c->row_ptr, c->sell_ptr, c->sell_col, c->scale, c->R, x0, c->dinv, \
+                               c->diag32, c->offd32, c->dinv32, c->h_ts + TS_SETUP);                                \
     } while (0)
 #define SW2_SCALE_SWITCH(F32, BJ)                           \
     switch (c->kuni) {                                      \
@@ -664,19 +664,23 @@ __global__ void __launch_bounds__(256) k_pl_omega(int N, KVecs<P> V, double *par
 // deck 3e-14) and returns u as the reference does; a nearly singular one (the
 // partly dry floodplain, 224 x 112 nodes) was seen at 8e-7, and without the
 // step its Newton history left the oracle's by 2.4e-7 of its first entry,
-// with it by 1.2e-8.
+// with it by 1.2e-8.  mask (ensembles): a model that the step leaves out, and the
+// gaps between models, keep their sol, as with the one-kernel solve: it is the
+// model's last correction, whose norm its next step reports first.
 constexpr double REFINE_ABOVE = 1e-12;
 
 template <typename T, bool ZERO>
 __global__ void k_bcg_epi(int N3, const T *u, const double *scale, double *sol, const double *r, const KScal *sc,
-                          const int *node_inst) {
+                          const int *node_inst, const int *mask) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N3) return;
-    double x = (double)u[i];
-    if (r) {
-        const int m = node_inst ? node_inst[64 * (i / 192) + (i & 63)] : 0;
-        if (m >= 0 && sc[m].done && sc[m].it == 0 && sc[m].rnorm > REFINE_ABOVE * sc[m].bnorm) x += r[i];
+    int m = 0;
+    if (mask) {
+        m = node_inst[64 * (i / 192) + (i & 63)];
+        if (m < 0 || !mask[m]) return;
     }
+    double x = (double)u[i];
+    if (r && sc[m].done && sc[m].it == 0 && sc[m].rnorm > REFINE_ABOVE * sc[m].bnorm) x += r[i];
     x += ZERO ? 0.0 : sol[i];
     x *= scale[i];
     sol[i] = x;
@@ -844,9 +848,9 @@ void launch_krylov_epilogue(Ctx *c, bool zero_guess) {
     const bool lu = c->opts.preconditioner == 1 && c->opts.krylov == 0 && c->band_tiled && c->opts.nblock == 1 &&
                     c->opts.precision != 2;
     const double *r = lu ? c->kr : nullptr;
-    const int *ni = c->ninst ? c->node_inst : nullptr;
+    const int *ni = c->node_inst, *mask = c->ninst ? c->inst_mask : nullptr;
 #define SW2_EPI(T, Z, U) \
-    hipLaunchKernelGGL((k_bcg_epi<T, Z>), g, dim3(256), 0, c->stream, n3, U, c->scale, c->sol, r, c->ksc, ni)
+    hipLaunchKernelGGL((k_bcg_epi<T, Z>), g, dim3(256), 0, c->stream, n3, U, c->scale, c->sol, r, c->ksc, ni, mask)
     if (c->opts.precision == 2) {
         if (zero_guess) SW2_EPI(float, true, c->fu);
         else SW2_EPI(float, false, c->fu);
