@@ -414,8 +414,8 @@ __global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const dou
 
 // The band from the end's updates of the shared rows onto the other band's, which
 // hold the matrix: one workgroup per column.
-__global__ void __launch_bounds__(256) k_tb_merge(const TBand *bands, double *AB, const int *mask) {
-    const TBand B = band_rec(bands, blockIdx.y);
+__global__ void __launch_bounds__(256) k_tb_merge(const TBand *bands, int b0, double *AB, const int *mask) {
+    const TBand B = band_rec(bands, b0 + blockIdx.y);
     if (B.part < 0 || B.rev || (mask && !mask[B.inst])) return;
     const int j = TB * B.na + blockIdx.x;
     if (j >= B.m) return;
@@ -435,14 +435,14 @@ __global__ void __launch_bounds__(256) k_tb_merge(const TBand *bands, double *AB
 // and at the usual band widths (a few tiles) the launch and the next diagonal
 // block, not the matrix cores, are what a panel waits for.  The workgroup of the
 // window's first tile, the next panel's diagonal block, goes on to factor it.
-__global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, double *AB, double *LI, double *UI, int *guard,
-                                                   int step, int amax, int gt, const int *mask) {
+__global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, int b0, double *AB, double *LI, double *UI,
+                                                   int *guard, int step, int amax, int gt, const int *mask) {
     constexpr int LD = TB + 2;   // operand reads of 16 rows x 2 columns hit distinct banks
     __shared__ union {
         struct { double Xs[TB * LD], Us[TB * LD], Ls[4][16][64]; } p;
         Lu64 S;
     } sm;
-    const TBand B = band_rec(bands, blockIdx.y);
+    const TBand B = band_rec(bands, b0 + blockIdx.y);
     // the bands of blocks factored from both ends reach their shared rows at one step, amax
     const int k = B.part < 0 ? step : step - (amax - B.na);
     if (k < 0 || k + 1 >= B.nt || (mask && !mask[B.inst])) return;   // the last panel has no window
@@ -552,11 +552,11 @@ __global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, double *A
 // with the guarded one: U^-1 L^-1 with L's multipliers guarded and U's own
 // diagonal, formed column by column from the block's LU (rare).  One workgroup
 // of a wave per tile, column t in lane t.
-__global__ void __launch_bounds__(64) k_tb_inv(const TBand *bands, const double *AB, double *LI, double *UI,
+__global__ void __launch_bounds__(64) k_tb_inv(const TBand *bands, int b0, const double *AB, double *LI, double *UI,
                                                const int *guard, const int *mask) {
     __shared__ double D[TB][TB + 1];
     __shared__ double X[TB][TB + 1];
-    const TBand B = band_rec(bands, blockIdx.y);
+    const TBand B = band_rec(bands, b0 + blockIdx.y);
     const int k = blockIdx.x;
     if (k >= (B.rev ? B.na : B.nt) || (mask && !mask[B.inst])) return;
     const int c0 = k * TB, kb = min(TB, B.m - c0), t = threadIdx.x;
@@ -614,11 +614,11 @@ __global__ void __launch_bounds__(64) k_tb_inv(const TBand *bands, const double 
 // the band's TB extra diagonals (entries within w + 63 of the diagonal), which
 // is what they are stored for.  One workgroup of 256 threads per tile, a 4 x 4
 // register block each from LDS.
-__global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, double *AB, const double *G, const double *UI,
-                                                  int gf, const int *mask) {
+__global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, int b0, double *AB, const double *G,
+                                                  const double *UI, int gf, const int *mask) {
     __shared__ double As[TB][TB];       // As[q][row]: the tile, column q
     __shared__ double Ms[TB][TB + 1];   // Ms[q][col]: the inverse
-    const TBand B = band_rec(bands, blockIdx.z);
+    const TBand B = band_rec(bands, b0 + blockIdx.z);
     const int k = blockIdx.x;
     if (k >= (B.rev ? B.na : B.nt) || (mask && !mask[B.inst])) return;
     const bool low = (int)blockIdx.y < gf;
@@ -915,11 +915,11 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
 // every band from the end has its workgroups running before one waits for it.
 // (200 x 100 cells: both sweeps 1.83 ms, 1.84 with a band per grid index.)
 enum { SW_ALL, SW_SHARED, SW_REST };
-__global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, const double *AB, const double *xb, double *yb,
+__global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, int b0, const double *AB, const double *xb, double *yb,
                                                     double *zb, int *tick, int *claim, int phase, const int *done,
                                                     const int *mask, const KScal *sc) {
     __shared__ SweepLds S;
-    int band = blockIdx.y;
+    int band = b0 + blockIdx.y;
     if (phase == SW_SHARED) {
         if (threadIdx.x == 0) S.unit = atomicAdd(claim, 1);
         __syncthreads();
@@ -943,11 +943,11 @@ __global__ void __launch_bounds__(SW_NT) k_tb_sweep(const TBand *bands, const do
 // wave order).  `shared`: of the shared rows, which the band from the end
 // receives too; else of the others.  A model that has converged, or is outside
 // the mask, keeps x.
-__global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, const double *UI, double *zb, double *x,
+__global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, int b0, const double *UI, double *zb, double *x,
                                                   bool shared, const int *done, const int *mask, const KScal *sc) {
     __shared__ double part[4][TB];
     const int stop = *done;
-    const TBand B = band_rec(bands, blockIdx.y, stop);
+    const TBand B = band_rec(bands, b0 + blockIdx.y, stop);
     if (shared && (B.part < 0 || B.rev)) return;
     const int k = blockIdx.x + (shared ? B.na : 0);
     if (stop || k >= (shared ? B.nt : B.na) || (mask && (!mask[B.inst] || (sc && sc[B.inst].done)))) return;
@@ -1081,6 +1081,14 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     return "";
 }
 
+// Launches with a grid row (or layer) per band: HIP takes 65,536 of them, a
+// partition may have more bands.  f(first band, bands)
+constexpr int BANDS_A_LAUNCH = 32768;
+template <typename F>
+static void each_launch(const Ctx *c, F f) {
+    for (int b0 = 0; b0 < c->tb_nband; b0 += BANDS_A_LAUNCH) f(b0, std::min(BANDS_A_LAUNCH, c->tb_nband - b0));
+}
+
 // the models the masked launches of an ensemble work on (null: every band)
 static const int *tb_mask(const Ctx *c) { return c->ninst ? c->inst_mask : nullptr; }
 
@@ -1118,25 +1126,28 @@ void launch_tband_setup(Ctx *c) {
                            c->tb_UI, c->tb_guard, shared, mask);
     };
     diag(false);
-    for (int k = 0; k < steps; k++) {
-        if (amax > 0 && k == amax) {
-            hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands,
-                               c->tb_AB, mask);
-            diag(true);
-        }
-        hipLaunchKernelGGL(k_tb_step, dim3(gt * gt, c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_LI, c->tb_UI, c->tb_guard, k, amax, gt, mask);
-    }
-    if (amax > 0 && steps == amax) {   // shared rows of one panel
-        hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_AB,
-                           mask);
+    auto merge = [&]() {
+        each_launch(c, [&](int b0, int nb) {
+            hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, nb), dim3(256), 0, c->stream, c->tb_bands, b0, c->tb_AB,
+                               mask);
+        });
         diag(true);
+    };
+    for (int k = 0; k < steps; k++) {
+        if (amax > 0 && k == amax) merge();
+        each_launch(c, [&](int b0, int nb) {
+            hipLaunchKernelGGL(k_tb_step, dim3(gt * gt, nb), dim3(NT), 0, c->stream, c->tb_bands, b0, c->tb_AB,
+                               c->tb_LI, c->tb_UI, c->tb_guard, k, amax, gt, mask);
+        });
     }
-    hipLaunchKernelGGL(k_tb_inv, dim3(nt, c->tb_nband), dim3(64), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
-                       c->tb_UI, c->tb_guard, mask);
+    if (amax > 0 && steps == amax) merge();   // shared rows of one panel
     const int gf = std::max(1, c->tb_gf);
-    hipLaunchKernelGGL(k_tb_scale, dim3(nt, 2 * gf, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands,
-                       c->tb_AB, c->tb_LI, c->tb_UI, gf, mask);
+    each_launch(c, [&](int b0, int nb) {
+        hipLaunchKernelGGL(k_tb_inv, dim3(nt, nb), dim3(64), 0, c->stream, c->tb_bands, b0, c->tb_AB, c->tb_LI,
+                           c->tb_UI, c->tb_guard, mask);
+        hipLaunchKernelGGL(k_tb_scale, dim3(nt, 2 * gf, nb), dim3(256), 0, c->stream, c->tb_bands, b0, c->tb_AB,
+                           c->tb_LI, c->tb_UI, gf, mask);
+    });
 }
 
 // sc: the Krylov scalars (one per model) whose done flags end the sweeps, or
@@ -1155,13 +1166,17 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     // row always waiting; any number is correct, and with many bands one
     // workgroup each already fills the chip
     const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 512 / c->tb_nband));
-    auto sweep = [&](int phase) {
-        hipLaunchKernelGGL(k_tb_sweep, dim3(g, c->tb_nband), dim3(SW_NT), 0, c->stream, c->tb_bands, c->tb_AB,
-                           c->tb_xb, c->tb_yb, c->tb_zb, c->tb_int, c->tb_int + 3 * c->tb_nband, phase, done, mask, msc);
+    auto sweep = [&](int phase) {   // SW_SHARED's claims count on from launch to launch
+        each_launch(c, [&](int b0, int nb) {
+            hipLaunchKernelGGL(k_tb_sweep, dim3(g, nb), dim3(SW_NT), 0, c->stream, c->tb_bands, b0, c->tb_AB, c->tb_xb,
+                               c->tb_yb, c->tb_zb, c->tb_int, c->tb_int + 3 * c->tb_nband, phase, done, mask, msc);
+        });
     };
     auto apply = [&](bool shared, int tiles) {
-        hipLaunchKernelGGL(k_tb_apply, dim3(tiles, c->tb_nband), dim3(256), 0, c->stream, c->tb_bands, c->tb_UI,
-                           c->tb_zb, x, shared, done, mask, msc);
+        each_launch(c, [&](int b0, int nb) {
+            hipLaunchKernelGGL(k_tb_apply, dim3(tiles, nb), dim3(256), 0, c->stream, c->tb_bands, b0, c->tb_UI,
+                               c->tb_zb, x, shared, done, mask, msc);
+        });
     };
     if (c->tb_nbot > 0) {
         sweep(SW_SHARED);

@@ -1,11 +1,13 @@
 """The tiled band LU's sweeps with more bands than the GPU holds workgroups: 900
 models factored from both ends, 1,800 bands, where the bands from the start
 wait for those from the end.  Every model takes the step it takes alone, bit for
-bit.
+bit.  And with more bands than a grid has rows.
 """
+import numpy as np
 import pytest
 
 from gpu_helpers import bits_equal, say
+from test_gpu_lu_tiles import _system
 from adhv8_kraken_amd import mesh
 from adhv8_kraken_amd.sw2 import SW2Ensemble, SW2Model, default_opts
 
@@ -29,3 +31,31 @@ def test_more_two_ended_bands_than_workgroups_fit():
             assert all(bits_equal(a, b) for a, b in zip(s, e.get_state(i)))
         g.close()
     e.close()
+
+
+@pytest.mark.parametrize("blocks", [32769, 66000])
+def test_more_bands_than_a_grid_has_rows(blocks):
+    """Blocks of a few nodes, one more than a launch takes (the last block holds the
+    1,392 nodes that are left over, factored from both ends) and more than HIP's
+    grids have rows.  The system is diagonally dominant (condition below 10), so
+    M^-1 v is the exact block inverse's to 1e-13 of its largest entry, as in
+    test_gpu_lu_tiles.py."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as sl
+    p = mesh.bumpy_channel(659, 299)   # 198,000 nodes
+    N = p.nnodes
+    g = SW2Model(p, default_opts(preconditioner=1, nblock=blocks, lu_tiled=1))
+    diag, offd, A = _system(g, 3)
+    v = np.random.default_rng(5).uniform(-1.0, 1.0, 3 * N)
+    g.set_system(diag, offd, v)
+    s = g.linear_sys_setup()
+    S = (sp.diags(s) @ A @ sp.diags(s)).tocoo()
+    block = lambda i: np.minimum(i // 3 // (N // blocks), blocks - 1)   # noqa: E731
+    keep = block(S.row) == block(S.col)
+    inside = sp.csc_matrix((S.data[keep], (S.row[keep], S.col[keep])), shape=S.shape)
+    ref = sl.splu(inside, permc_spec="NATURAL").solve(v)
+    for rep in range(2):
+        err = np.abs(g.precond_apply(v) - ref).max() / np.abs(ref).max()
+        say(f"  {blocks} blocks, apply {rep}: {err:.1e}")
+        assert err < 1e-13
+    g.close()
