@@ -8,13 +8,15 @@
 // factors are those of the skyline LU; only the rounding order of the
 // updates differs).
 //
-// Here: the partition, and the LU of blocks of at most a tile (64 DOFs), one
-// workgroup per block (right-looking band update, a barrier per pivot) and one
-// wavefront per solve (forward unit-lower, backward upper, the block's
-// right-hand side in LDS).  Larger blocks go to the tiled band LU (sw2_lu.hip).
+// Here: the partition, and the LU with one workgroup per block (right-looking
+// band update, a barrier per pivot) and one wavefront per solve (forward
+// unit-lower, backward upper, the block's right-hand side in LDS), for blocks of
+// at most a tile (64 DOFs) and for many short and narrow ones.  Others go to the
+// tiled band LU (sw2_lu.hip).
 // This is the robust preconditioner for steps with large Courant numbers, where
 // 3x3 block Jacobi stalls.
 #include <algorithm>
+#include <cmath>
 #include <string>
 
 #include "sw2_ctx.h"
@@ -128,6 +130,39 @@ void band_free(Ctx *c) {
     c->band_max_n = 0;
 }
 
+// The expected time (us) of a set-up and 20 applications, about what a solve
+// takes, of blocks of n DOFs and half bandwidth w, with one workgroup per block
+// and with the tiled LU.  Each is the longest block's chain of dependent steps
+// and what all blocks take together: a pivot or row at a time and the band's
+// updates and bytes there; panels, tiles of 64 DOFs and their products here.
+// The constants are fitted to 79 partitions of ten meshes (1,891 to 501,501 nodes,
+// blocks of 66 to 4,000 DOFs, w from 5 to 1,500); the LU it picks was at most 1.08
+// times as slow there as the other.  Set-up + ten iterations measured, ms, workgroup /
+// tiled: 21 blocks of 258 DOFs, w 98, 8.8 / 1.2; 280 of 66, w 5, 1.7 / 1.4; 3,663 of 66,
+// w 5, 3.7 / 7.1; 1,259 of 192, w 5, 6.7 / 4.0; 22,795 of 66, w 5, 13 / 41; 5,831 of 258,
+// w 5, 17 / 27; 2,383 of 384, w 188, 129 / 25.
+struct LuCost {
+    double chain_set = 0, chain_app = 0, dofs = 0, updates = 0, band = 0, tiles = 0, products = 0, panels = 0;
+    void add(double n, double w) {
+        chain_set = std::max(chain_set, n * (0.8 + 8e-4 * w * w));
+        chain_app = std::max(chain_app, n * (0.87 + 7e-3 * w));
+        dofs += n;
+        updates += n * w * w;
+        band += n * w;
+        const double nt = std::ceil(n / 64), reach = std::min(nt, std::ceil(w / 64));
+        panels = std::max(panels, nt);
+        tiles += nt;
+        products += reach * nt - reach * (reach + 1) / 2;
+    }
+    double workgroup() const {
+        return chain_set + 7e-4 * dofs + 3.3e-6 * updates + 20 * (chain_app + 2.3e-4 * dofs + 7e-6 * band);
+    }
+    double tiled() const {
+        return 60 + 22 * panels + 0.12 * tiles + 0.2 * products +
+               20 * (25 + 3 * panels + 0.025 * tiles + 0.012 * products);
+    }
+};
+
 // Builds the block partition and band offsets for `nblock` blocks
 // (node_order.c:64-104 serial partition: N/nblock consecutive nodes per
 // block, the last block taking the rest).  An ensemble partitions each model's
@@ -165,6 +200,7 @@ std::string band_structure(Ctx *c, int nblock) {
     std::vector<int> w(nbk), node_blk(N, -1);
     std::vector<size_t> off(nbk + 1, 0);
     int max_n = 0;
+    LuCost cost;
     for (int b = 0; b < nbk; b++) {
         int maxd = 0;
         for (int a = s0[b]; a < s1[b]; a++) {
@@ -177,21 +213,22 @@ std::string band_structure(Ctx *c, int nblock) {
         w[b] = 3 * maxd + 2;
         const int nb = 3 * (s1[b] - s0[b]);
         max_n = std::max(max_n, nb);
+        cost.add(nb, w[b]);
         off[b + 1] = off[b] + (size_t)nb * (2 * w[b] + 1);
     }
-    // The tiled band LU takes every partition whose largest block exceeds a
-    // tile: the one-workgroup LU pays a global-memory round trip and a barrier
-    // per pivot (set-up + one application, 40 x 20 cells: one block of 2,583
-    // DOFs 12.9 + 2.7 ms against 1.0 + 0.21, ten of 258 1.2 + 0.32 against
-    // 0.19 + 0.07, 41 of 63 0.09 + 0.09 against 0.08 + 0.05).  Below, the one-
-    // workgroup LU is the faster one and needs no 64 x 64 inverses per block
-    // (300 x 100 cells, 7,600 blocks of 12 DOFs: 0.16 + 0.19 ms against 0.83 +
-    // 0.35, and 20 MB against 1.1 GB).  Ensembles always take the tiled LU, and so
+    // The tiled band LU takes a partition whose largest block exceeds a tile, where
+    // it is the faster one: the one-workgroup LU pays a global-memory round trip and
+    // a barrier per pivot (set-up + one application, 40 x 20 cells: one block of
+    // 2,583 DOFs 12.9 + 2.7 ms against 1.0 + 0.21, ten of 258 1.2 + 0.32 against
+    // 0.19 + 0.07, 41 of 63 0.09 + 0.09 against 0.08 + 0.05), the tiled one the
+    // 64 x 64 inverses of every tile, also of a short or narrow block's (300 x 100
+    // cells, 7,600 blocks of 12 DOFs: 0.83 + 0.35 ms and 1.1 GB against 0.16 + 0.19
+    // and 20 MB).  Ensembles always take the tiled LU, and so
     // does opts.lu_tiled; a partition whose tiles do not fit in device memory
     // falls back to the one-workgroup LU where that can hold its blocks.
     const bool small_ok = !c->ninst && !c->opts.lu_tiled && max_n <= BAND_MAX_DOF &&
                           off[nbk] * sizeof(double) <= BAND_MAX_BYTES;
-    if (!small_ok || max_n > 64) {
+    if (!small_ok || (max_n > 64 && cost.tiled() <= cost.workgroup())) {
         if (hipMalloc((void **)&c->node_blk, sizeof(int) * N) != hipSuccess ||
             hipMemcpy(c->node_blk, node_blk.data(), sizeof(int) * N, hipMemcpyHostToDevice) != hipSuccess) {
             band_free(c);

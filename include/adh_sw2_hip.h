@@ -107,10 +107,10 @@ typedef struct {
     int krylov;          /* 0 (default): BiCGSTAB (solv_bcgstab.c); 1: restarted GMRES(30), left-preconditioned,
                             stopping on the Arnoldi 2-norm of the preconditioned residual (no counterpart in the
                             reference; single models, precision 0 or 1) */
-    int lu_tiled;        /* preconditioner 1: 0 (default) factors node blocks of up to 21 nodes with one
-                            workgroup each and larger ones (up to OP BLK 1, the whole matrix) with the tiled
-                            band LU; 1 uses the tiled band LU for every block (an ensemble handle
-                            always does) */
+    int lu_tiled;        /* preconditioner 1: 0 (default) factors node blocks with one workgroup each where
+                            none has more than 21 nodes, or where there are many short and narrow ones
+                            (thousands), and else (up to OP BLK 1, the whole matrix) with the tiled band LU;
+                            1 uses the tiled band LU for every block (an ensemble handle always does) */
 } adh_sw2_opts;
 
 typedef struct {
