@@ -515,7 +515,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     UP(elist_wet, (const int *)nullptr, E);
     UP(elist_gen, (const int *)nullptr, E);
     UP(ecount, (const int *)nullptr, 2);
-    UP(esplit, (const int *)nullptr, 2 * (size_t)nblocks_for(E, 256) + 2);
+    UP(esplit, (const int *)nullptr, split_words(E));
     c.pre_valid = 0;
     UP(ER, (const double *)nullptr, 9 * (size_t)E + 6 * (size_t)B);
     UP(EM, (const double *)nullptr, 81 * (size_t)E + 36 * (size_t)B);

@@ -156,7 +156,7 @@ struct Ctx {
     size_t ndslots;               // N diagonal slots + one slot per SELL position
     // work
     int *elist_wet, *elist_gen, *ecount;  // FD-Jacobian triangle lists [E], [E], counts [2]
-    int *esplit;                          // per-block counts / offsets of the split [E/256 + 1]
+    int *esplit;                          // the split's per-block counts, and their sums by runs [split_words(E)]
     int split_valid;                      // the lists match the current depths
     // launch shape of the four list kernels (Jacobian wet/general, residual
     // wet/general): block size and grid-stride grid size
@@ -409,5 +409,6 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc);
 void launch_probe(const double *x, int n, const crlog::tables *t, double *lg, double *sq, double *dv);
 
 int nblocks_for(int n, int bs);
+size_t split_words(int E);
 
 }  // namespace sw2

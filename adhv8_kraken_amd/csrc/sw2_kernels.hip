@@ -734,28 +734,57 @@ __global__ void __launch_bounds__(256) k_split_count(int E, const int *e2d, cons
     }
 }
 
+// Above SPLIT_DIRECT count blocks: sums of SPLIT_RUN consecutive counts of each
+// list, a workgroup each.
+constexpr int SPLIT_RUN = 1024, SPLIT_DIRECT = 6144;
+__global__ void __launch_bounds__(256) k_split_sums(int nb, const int *bcount, int *sums) {
+    __shared__ int part[4];
+    const int *c = bcount + (size_t)blockIdx.y * nb;
+    const int b0 = blockIdx.x * SPLIT_RUN;
+    int s = 0;
+#pragma unroll
+    for (int u = 0; u < SPLIT_RUN / 256; u++) {
+        const int b = b0 + u * 256 + threadIdx.x;
+        s += b < nb ? c[b] : 0;
+    }
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.y * gridDim.x + blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+}
+
 // A block's place in the two lists is the sum of the counts before it, which
 // it adds up itself: 1M triangles, 3,906 counts, take less time that way than
-// a scan kernel's launch (3.5 us), and fewer take next to none.  The last block
-// leaves the totals in counts.
+// a scan kernel's launch (3.5 us), and fewer take next to none.  What all blocks
+// add grows with the square of the triangles, so above SPLIT_DIRECT they add the
+// sums of whole runs before them and the counts of their own run alone.
+// Counts, sums and lists, us, by runs / directly: 1M triangles 16.6 / 15.6, 1.5M
+// 25.0 / 23.6, 2M 28.1 / 30.9, 4M 49 / 71, 13.5M 146 / 496.
+// The last block leaves the totals in counts.
 __global__ void __launch_bounds__(256) k_split_write(int E, const int *e2d, const double *head, const int *elem_inst,
-                                                     const int *mask, const int *bcount, int *counts, int *wet,
-                                                     int *gen) {
+                                                     const int *mask, const int *bcount, const int *sums, int *counts,
+                                                     int *wet, int *gen) {
     __shared__ int wc[2][4], before[2][4];
     {
         int s0 = 0, s1 = 0;
-        constexpr int U = 4;
-        for (int b = threadIdx.x; b < (int)blockIdx.x; b += U * 256) {
-            int x[U][2];
+        // entries first .. last - 1 of the two arrays of n
+        auto add = [&](const int *a, int n, int first, int last) {
+            constexpr int U = 4;
+            for (int b = first + threadIdx.x; b < last; b += U * 256) {
+                int x[U][2];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool in = b + u * 256 < (int)blockIdx.x;
-                x[u][0] = in ? bcount[b + u * 256] : 0;
-                x[u][1] = in ? bcount[gridDim.x + b + u * 256] : 0;
+                for (int u = 0; u < U; u++) {
+                    const bool in = b + u * 256 < last;
+                    x[u][0] = in ? a[b + u * 256] : 0;
+                    x[u][1] = in ? a[n + b + u * 256] : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) { s0 += x[u][0]; s1 += x[u][1]; }
             }
-#pragma unroll
-            for (int u = 0; u < U; u++) { s0 += x[u][0]; s1 += x[u][1]; }
-        }
+        };
+        const int run = sums ? (int)blockIdx.x / SPLIT_RUN : 0;
+        if (sums) add(sums, (gridDim.x + SPLIT_RUN - 1) / SPLIT_RUN, 0, run);
+        add(bcount, gridDim.x, run * SPLIT_RUN, blockIdx.x);
         for (int o = 32; o > 0; o >>= 1) { s0 += __shfl_xor(s0, o, 64); s1 += __shfl_xor(s1, o, 64); }
         if ((threadIdx.x & 63) == 0) { before[0][threadIdx.x >> 6] = s0; before[1][threadIdx.x >> 6] = s1; }
     }
@@ -781,6 +810,13 @@ __global__ void __launch_bounds__(256) k_split_write(int E, const int *e2d, cons
     if (g) gen[bef_g + __popcll(bg & below)] = ie;
 }
 
+static int split_runs(int nb) { return (nb + SPLIT_RUN - 1) / SPLIT_RUN; }
+// ints of the count blocks' arrays of a mesh of E triangles
+size_t split_words(int E) {
+    const int nb = nblocks_for(E, 256);
+    return 2 * (size_t)nb + 2 * (size_t)split_runs(nb);
+}
+
 // ordered wet / general triangle lists for the current depths (and, for
 // ensembles, the models being iterated)
 static void launch_split(Ctx *c) {
@@ -789,8 +825,13 @@ static void launch_split(Ctx *c) {
     const int *mask = c->ninst ? c->inst_mask : nullptr;
     hipLaunchKernelGGL(k_split_count, dim3(nb), dim3(256), 0, c->stream, c->E, c->e2d, c->head, c->elem_inst, mask,
                        c->esplit, c->h_ts + TS_RESID);
+    int *sums = nullptr;
+    if (nb > SPLIT_DIRECT) {
+        sums = c->esplit + 2 * (size_t)nb;
+        hipLaunchKernelGGL(k_split_sums, dim3(split_runs(nb), 2), dim3(256), 0, c->stream, nb, c->esplit, sums);
+    }
     hipLaunchKernelGGL(k_split_write, dim3(nb), dim3(256), 0, c->stream, c->E, c->e2d, c->head, c->elem_inst, mask,
-                       c->esplit, c->ecount, c->elist_wet, c->elist_gen);
+                       c->esplit, sums, c->ecount, c->elist_wet, c->elist_gen);
     c->split_valid = 1;
 }
 
