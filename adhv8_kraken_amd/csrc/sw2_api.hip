@@ -538,7 +538,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
         // emptied by the first solve
         if ((rc = dalloc(h, &c.run_xch, may ? run_vector_words(c.Np) : 1))) { adh_sw2_hip_destroy(h); return rc; }
     }
-    UP(run_quit, (const int *)nullptr, 2 * nmod);
+    UP(run_quit, (const int *)nullptr, 2 * nmod + 2);
     c.red.maxblocks = nblocks_for(N, 256) + 8;
     UP(red.part, (const double *)nullptr, 4 * (size_t)c.red.maxblocks);
     UP(red.count, (const unsigned *)nullptr, 8);
@@ -1325,10 +1325,22 @@ extern "C" int adh_sw2_hip_timestep(adh_sw2_hip *h, adh_sw2_report *rep, int *ve
 // model's arithmetic is the single-model arithmetic: same block partitions,
 // same reduction order, same element code.
 
+// the contents of inst_mask
+static std::vector<int> mask_and_blocks(const Ctx &c, const std::vector<int> &m) {
+    std::vector<int> both(m);
+    int before = 0;
+    for (int i = 0; i < c.ninst; i++) {
+        both.push_back(before);
+        before += m[i] ? nblocks_for(c.h_inst_N[i], 256) : 0;
+    }
+    return both;
+}
+
 static int set_mask(Ctx &c, const std::vector<int> &m) {
     if (m == c.h_inst_mask) return 0;   // the device and the element lists have it already
     c.split_valid = 0;  // the element lists hold the masked models only
-    HIPCHK(hipMemcpyAsync(c.inst_mask, m.data(), sizeof(int) * c.ninst, hipMemcpyHostToDevice, c.stream));
+    const std::vector<int> both = mask_and_blocks(c, m);
+    HIPCHK(hipMemcpyAsync(c.inst_mask, both.data(), sizeof(int) * both.size(), hipMemcpyHostToDevice, c.stream));
     c.h_inst_mask = m;
     // the host vector may change before the copy runs
     HIPCHK(hipStreamSynchronize(c.stream));
@@ -1603,10 +1615,12 @@ extern "C" int adh_sw2_hip_batch_create(const adh_sw2_mesh *meshes, int n, const
     inst_blk0[n] = (c.N + 255) / 256;
     c.run_max_blocks = 0;
     for (int i = 0; i < n; i++) c.run_max_blocks = std::max(c.run_max_blocks, inst_blk0[i + 1] - inst_blk0[i]);
+    std::vector<int> both(mask);   // see mask_and_blocks
+    both.insert(both.end(), inst_blk0.begin(), inst_blk0.begin() + n);
     auto up = [&](auto **dst, const auto *src, size_t cnt) -> int { return dupload(h, dst, src, cnt); };
     if ((rc = up(&c.blk_inst, blk_inst.data(), blk_inst.size())) || (rc = up(&c.inst_blk0, inst_blk0.data(), n + 1)) ||
         (rc = up(&c.inst_nodes, inst_nodes.data(), n)) || (rc = up(&c.node_inst, node_inst.data(), node_inst.size())) ||
-        (rc = up(&c.inst_mask, mask.data(), n)) || (rc = up(&c.elem_inst, elem_inst.data(), elem_inst.size())) ||
+        (rc = up(&c.inst_mask, both.data(), both.size())) || (rc = up(&c.elem_inst, elem_inst.data(), elem_inst.size())) ||
         (rc = up(&c.edge_inst, edge_inst.data(), edge_inst.size())) || (rc = up(&c.dt_inst, dts.data(), n)) ||
         (rc = up(&c.loc_bc_inst, loc_bc.data(), loc_bc.size()))) {
         adh_sw2_hip_destroy(h);

@@ -205,7 +205,8 @@ struct Ctx {
     int *inst_blk0;        // [ninst+1] first 256-node block of each model
     int *inst_nodes;       // [ninst] nodes of each model (the l2 norm's count)
     int *node_inst;        // [Np] model of each node (gap nodes: the model before them)
-    int *inst_mask;        // [ninst] 1 = the masked node kernels update this model
+    int *inst_mask;        // [ninst] 1 = the masked node kernels update this model; then [ninst] the
+                           // 256-node blocks of such models before this one
     std::vector<int> h_inst_mask;   // its host copy
     int *elem_inst, *edge_inst;
     double *dt_inst;
@@ -224,7 +225,7 @@ struct Ctx {
     double *run_slots;     // two sets of hand-over slots, used by turns (run_parity)
     double *run_xch;       // the hand-over vectors
     int run_dirty;         // run_xch is to be emptied first
-    int *run_quit;         // [2 max(1, ninst)] give-up flags
+    int *run_quit;         // [2 max(1, ninst)] give-up flags, then by parity [2] the blocks that are through
     int run_parity, run_prec;
     int run_cap[2];        // blocks the GPU holds at once in form run_prec, at one and two a CU (-1: not asked yet)
     int run_max_blocks;    // 256-node blocks of the largest model

@@ -27,6 +27,8 @@
 // block polls all blocks' partials, and the neighbours' values are read past
 // the L2).
 
+#include <algorithm>
+
 #include "sw2_flow.h"
 #include "sw2_krylov.h"
 
@@ -92,7 +94,12 @@ __device__ __forceinline__ double uniform(double x) {
 //
 // A wait gives up (all blocks do, then) after `limit` ticks of the 100 MHz
 // clock: another program's kernels may hold the CUs that this model's
-// remaining blocks wait for.  The caller then repeats the solve with the
+// remaining blocks wait for.  In an ensemble with more blocks than the GPU
+// holds it may also be the launch's own earlier models: the clock stands while
+// blocks before the model's first are at work, which end, or give up, in their
+// time.  (With that time counted, 256 channels of 13.4M triangles in all gave up
+// their first solve in FP64 after 17 ms and left the next ones to the other form,
+// 277 M triangle-Newton/s instead of 309.)  The caller repeats the solve with the
 // kernel-per-step form.  At the last hand-over some blocks may give up and others
 // pass: the solve is then whole, but those that gave up leave their parts of the
 // vectors filled, so the host is told of every give-up and empties all vectors.
@@ -104,26 +111,47 @@ __host__ __device__ __forceinline__ size_t slot_at(int t, int k, int b, int nblk
     return (((size_t)t * PARTS + k) * ((nblk + 7) / 8) + (b >> 3)) * 32 + (b & 7);
 }
 
+// An ensemble's block's, in LDS: in registers it would be held through the solve.
+// Times are the low halves of the clock's.
+struct Wait {
+    int quit;                  // the model gives up (one model's too)
+    int ahead;                 // blocks of the launch before the model's first, 0 once they are through
+    unsigned from;             // time at which they were last found at work
+    int *ended;                // the launch's blocks that are through
+};
+
+template <bool ENS>
 struct HandOver {
     double *set;               // this launch's partials [turn][partial][256-node block]
     int nblk, k0, k1, blk;     // blocks in all, the model's range, this one
     int turn;
     int *quit;                 // the model's give-up flag
     int *gave_up;              // the same for the host, of all models: the vectors are to be emptied
-    long long limit;
+    unsigned limit;
     double (*shp)[4], (*shr)[4];
-    int *shq;
+    Wait *shw;
 
     __device__ __forceinline__ double *slot(int t, int k, int b) const {
         return set + slot_at(t, k, b, nblk);
     }
     // the wait that began at t0 is over without result
-    __device__ __forceinline__ bool give_up(long long t0, int spin) {
-        if (wall_clock64() - t0 > limit) {
+    __device__ __forceinline__ bool give_up(unsigned t0, int spin) {
+        const bool look = (spin & 15) == 15;
+        bool late = (unsigned)wall_clock64() - t0 > limit;
+        if (!look && !late) return false;
+        if constexpr (ENS) {
+            if (shw->ahead > 0) {
+                if ((int)peek((float *)shw->ended) < shw->ahead) shw->from = (unsigned)wall_clock64();
+                else shw->ahead = 0;
+            }
+            // signed: another wave may have found them at work after this one's look at the clock
+            late = late && (int)((unsigned)wall_clock64() - shw->from) > (int)limit;
+        }
+        if (late) {
             put_raw((float *)quit, 1u);
             *gave_up = 1;
-        } else if ((spin & 15) != 15 || !peek((float *)quit)) return false;
-        *shq = 1;
+        } else if (!look || !peek((float *)quit)) return false;
+        shw->quit = 1;
         return true;
     }
 
@@ -157,7 +185,7 @@ struct HandOver {
         double acc[K];
 #pragma unroll
         for (int k = 0; k < K; k++) acc[k] = 0.0;
-        const long long t0 = wall_clock64();
+        const unsigned t0 = (unsigned)wall_clock64();
         bool ok = true;
         constexpr int W = 2;
         for (int b0 = k0 + threadIdx.x; b0 < k1 && ok; b0 += W * 256) {
@@ -204,7 +232,7 @@ struct HandOver {
             if (lane == 0) shr[k][wid] = x;
         }
         __syncthreads();
-        const bool quit_now = *shq != 0;
+        const bool quit_now = shw->quit != 0;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             double x = shr[k][0];
@@ -266,12 +294,23 @@ struct Rows {
     }
 };
 
-// OCC blocks on a CU: 512 registers a lane with one, 256 with two
-template <typename P, int K, int OCC>
+// counts an ensemble's block at its end, whichever way it leaves
+template <bool ENS>
+struct Leaver {
+    const Wait &w;
+    __device__ __forceinline__ ~Leaver() {
+        if (ENS && threadIdx.x == 0) atomicAdd(w.ended, 1);
+    }
+};
+
+// OCC blocks on a CU: 512 registers a lane with one, 256 with two.  ENS: an
+// ensemble's models (one model without what only they need: with it a solve of
+// 125,751 nodes in FP64 was 2 % longer, all of it registers)
+template <typename P, int K, int OCC, bool ENS>
 __global__ void __launch_bounds__(256, OCC)
     k_bcg_run(int N, size_t n3, KVecs<P> V, typename P::V *xch, const int *sell_col, const double *rhs,
-              const double *scale, double *sol, KScal *sc, KScal *host, const int *blk_inst, const int *inst_blk0, double *slots,
-              int parity, int *quit, int *gave_up, long long limit) {
+              const double *scale, double *sol, KScal *sc, KScal *host, const int *blk_inst, const int *inst_blk0,
+              const int *blocks_before, double *slots, int parity, int *quit, int *gave_up, int *ended, unsigned limit) {
     using T = typename P::V;
     using MT = typename P::M;
     // AGAIN: the neighbours' r in LDS instead of their Ap, which is read a second
@@ -279,13 +318,13 @@ __global__ void __launch_bounds__(256, OCC)
     constexpr bool AGAIN = OCC == 2 && sizeof(MT) == 8 && K > 4;
     __shared__ T nbP[K][3][256], nbX[K][3][256], q[3][256];
     __shared__ double shp[PARTS][4], shr[PARTS][4];
-    __shared__ int shq;
+    __shared__ Wait shw;
     const int lb = blockIdx.x, nblk = gridDim.x, tid = threadIdx.x;
     int m = 0, nend = N;
-    HandOver H;
+    HandOver<ENS> H;
     H.k0 = 0;
     H.k1 = nblk;
-    if (blk_inst) {
+    if constexpr (ENS) {
         m = blk_inst[2 * lb];
         nend = blk_inst[2 * lb + 1];
         H.k0 = inst_blk0[m];
@@ -301,21 +340,28 @@ __global__ void __launch_bounds__(256, OCC)
     H.limit = limit;
     H.shp = shp;
     H.shr = shr;
-    H.shq = &shq;
+    H.shw = &shw;
     if (tid < RING * PARTS) put_raw(slots + (1 - parity) * nset + slot_at(0, tid, lb, nblk), HO::EMPTY);
     const bool first = lb == H.k0;
     if (tid == 0) {
-        shq = 0;
+        shw.quit = 0;
         if (first) put_raw((float *)(quit + 2 * m + 1 - parity), 0u);
+        if constexpr (ENS) {
+            shw.ahead = blocks_before[m];
+            shw.from = (unsigned)wall_clock64() - limit - 1;
+            shw.ended = ended + parity;
+            if (lb == 0) put_raw((float *)(ended + 1 - parity), 0u);
+        }
     }
     sc += m;
     host += m;
     const int max_it = sc->max_it;
     const double atol = sc->atol, rtol = sc->rtol;
-    if (blk_inst && max_it <= 0) {   // a model the ensemble's step leaves out
+    if (ENS && max_it <= 0) {   // a model the ensemble's step leaves out
         if (first && tid == 0) sc->done = host->done = 1;
         return;
     }
+    const Leaver<ENS> through{shw};
     // threads past the model's end repeat its last row and keep the result to themselves
     const bool live = lb * 256 + tid < nend;
     const int n = live ? lb * 256 + tid : nend - 1;
@@ -357,9 +403,9 @@ __global__ void __launch_bounds__(256, OCC)
 #pragma unroll
         for (int j = 0; j < 3; j++) v[0] = fmax(v[0], fabs((double)u[j]));
         if (!live) v[0] = 0.0;
-        __syncthreads();   // shq
-        H.publish<1, 1, 0>(v);
-        if (!H.collect<1, 1>(out, X, cc, g)) return;
+        __syncthreads();   // shw
+        H.template publish<1, 1, 0>(v);
+        if (!H.template collect<1, 1>(out, X, cc, g)) return;
         turn_vector();
         bnorm = out[0];
     }
@@ -377,8 +423,8 @@ __global__ void __launch_bounds__(256, OCC)
         }
         give(r);
         if (!live) v[0] = v[1] = 0.0;
-        H.publish<2, 1, 3>(v);
-        if (!H.collect<2, 1>(out, X, cc, rn)) return;
+        H.template publish<2, 1, 3>(v);
+        if (!H.template collect<2, 1>(out, X, cc, rn)) return;
         turn_vector();
         rnorm = out[0];
         rho = out[1];
@@ -405,8 +451,8 @@ __global__ void __launch_bounds__(256, OCC)
 #pragma unroll
             for (int j = 0; j < 3; j++) v[0] += (double)q[j][tid] * (double)ap[j];
             if (!live) v[0] = v[1] = 0.0;
-            H.publish<2, 2, 3>(v);
-            if (!H.collect<2, 2>(out, X, cc, g)) return;
+            H.template publish<2, 2, 3>(v);
+            if (!H.template collect<2, 2>(out, X, cc, g)) return;
             turn_vector();
             if (it > 0) {
                 rnorm = out[1];
@@ -442,8 +488,8 @@ __global__ void __launch_bounds__(256, OCC)
                 v[2] += (double)as[j] * (double)q[j][tid];
             }
             if (!live) v[0] = v[1] = v[2] = 0.0;
-            H.publish<3, 0, 3>(v);
-            if (!H.collect<3, 0>(out, X, cc, g)) return;
+            H.template publish<3, 0, 3>(v);
+            if (!H.template collect<3, 0>(out, X, cc, g)) return;
             turn_vector();
             omega = uniform(out[0] / out[1]);
             rhop = rho;
@@ -508,8 +554,8 @@ __global__ void __launch_bounds__(256, OCC)
         }
     // every block has come this far: the model's first block reports, and all empty their vectors
     double v[1] = {0.0}, out[1];
-    H.publish<1, 0, 0>(v);
-    if (!H.collect<1, 0>(out, (const T *)nullptr, cc, g)) return;
+    H.template publish<1, 0, 0>(v);
+    if (!H.template collect<1, 0>(out, (const T *)nullptr, cc, g)) return;
     if (live)
         for (int t = 0; t < VRING; t++)
 #pragma unroll
@@ -533,22 +579,22 @@ __global__ void k_run_empty(size_t n, T *x) {
 }
 
 // Blocks that the GPU holds at once, 0 where the system is not for this form.
-template <typename P, int K, int OCC>
+template <typename P, int K, int OCC, bool ENS>
 int run_capacity() {
     int per_cu = 0, dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bcg_run<P, K, OCC>, 256, 0) != hipSuccess) {
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bcg_run<P, K, OCC, ENS>, 256, 0) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
     }
     return per_cu * cus;
 }
 
-template <typename P, int K, int OCC>
+template <typename P, int K, int OCC, bool ENS>
 bool run_k(Ctx *c, bool zero_guess) {
     int &cap = c->run_cap[OCC - 1];
-    if (cap < 0) cap = run_capacity<P, K, OCC>();
+    if (cap < 0) cap = run_capacity<P, K, OCC, ENS>();
     if (c->run_max_blocks > cap) return false;
     using T = typename P::V;
     const int nb = nblocks_for(c->N, 256);
@@ -562,10 +608,12 @@ bool run_k(Ctx *c, bool zero_guess) {
     for (int i = 0; i < (c->ninst ? c->ninst : 1); i++) c->h_ksc[i].done = 0;   // the kernel sets what it finishes
     *c->h_gave_up = 0;
     c->run_parity ^= 1;
-    hipLaunchKernelGGL((k_bcg_run<P, K, OCC>), dim3(nb), dim3(256), 0, c->stream, c->N, n3, vecs<P>(c), xch,
+    hipLaunchKernelGGL((k_bcg_run<P, K, OCC, ENS>), dim3(nb), dim3(256), 0, c->stream, c->N, n3, vecs<P>(c), xch,
                        c->sell_col, c->R, c->scale, zero_guess ? c->sol : nullptr, c->ksc, c->h_ksc,
-                       c->ninst ? c->blk_inst : nullptr, c->ninst ? c->inst_blk0 : nullptr, c->run_slots,
-                       c->run_parity, c->run_quit, c->h_gave_up, c->run_limit);
+                       c->ninst ? c->blk_inst : nullptr, c->ninst ? c->inst_blk0 : nullptr,
+                       c->ninst ? c->inst_mask + c->ninst : nullptr, c->run_slots, c->run_parity, c->run_quit,
+                       c->h_gave_up, c->run_quit + 2 * (c->ninst ? c->ninst : 1),
+                       (unsigned)std::min(c->run_limit, 1000000000LL));
     return true;
 }
 
@@ -579,28 +627,33 @@ bool run_k(Ctx *c, bool zero_guess) {
 // eight neighbours: the LDS takes one block.  More blocks than the GPU holds
 // (512, 131,072 nodes), more or fewer neighbours, or slices of unequal width:
 // the kernel-per-step form.
-template <typename P, int K>
+template <typename P, int K, bool ENS>
 bool run_occ(Ctx *c, bool zero_guess) {
     constexpr bool WIDE = sizeof(typename P::M) == 8;
-    if constexpr (K > 6) return run_k<P, K, 1>(c, zero_guess);
+    if constexpr (K > 6) return run_k<P, K, 1, ENS>(c, zero_guess);
     else {
         if constexpr (WIDE && K > 4)
-            if (run_k<P, K, 1>(c, zero_guess)) return true;
-        return run_k<P, K, 2>(c, zero_guess);
+            if (run_k<P, K, 1, ENS>(c, zero_guess)) return true;
+        return run_k<P, K, 2, ENS>(c, zero_guess);
+    }
+}
+
+template <typename P, bool ENS>
+bool run_e(Ctx *c, bool zero_guess) {
+    switch (c->kuni) {
+        case 3: return run_occ<P, 3, ENS>(c, zero_guess);
+        case 4: return run_occ<P, 4, ENS>(c, zero_guess);
+        case 5: return run_occ<P, 5, ENS>(c, zero_guess);
+        case 6: return run_occ<P, 6, ENS>(c, zero_guess);
+        case 7: return run_occ<P, 7, ENS>(c, zero_guess);
+        case 8: return run_occ<P, 8, ENS>(c, zero_guess);
+        default: return false;
     }
 }
 
 template <typename P>
 bool run_p(Ctx *c, bool zero_guess) {
-    switch (c->kuni) {
-        case 3: return run_occ<P, 3>(c, zero_guess);
-        case 4: return run_occ<P, 4>(c, zero_guess);
-        case 5: return run_occ<P, 5>(c, zero_guess);
-        case 6: return run_occ<P, 6>(c, zero_guess);
-        case 7: return run_occ<P, 7>(c, zero_guess);
-        case 8: return run_occ<P, 8>(c, zero_guess);
-        default: return false;
-    }
+    return c->ninst ? run_e<P, true>(c, zero_guess) : run_e<P, false>(c, zero_guess);
 }
 
 }  // namespace

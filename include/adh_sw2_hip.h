@@ -308,7 +308,8 @@ int adh_sw2_hip_set_tuning(adh_sw2_hip *h, const adh_sw2_tuning *t);
 
 /* Block-Jacobi BiCGSTAB solves of models of up to 131,072 nodes run as one
  * kernel whose workgroups wait for each other.  A wait longer than `ticks` of
- * a 100 MHz clock (default 30000, 0.3 ms) ends it, and the solve is repeated
+ * a 100 MHz clock (default 30000, 0.3 ms; at most 10 s; in an ensemble not
+ * counting the time that models before hold the GPU) ends it, and the solve is repeated
  * as a kernel per step, with the same result; below 0 every solve is.  No
  * counterpart in the reference. */
 int adh_sw2_hip_set_solve_wait(adh_sw2_hip *h, long long ticks);
