@@ -10,7 +10,7 @@ import pytest
 
 from gpu_helpers import bits_equal, say
 from adhv8_kraken_amd import mesh
-from adhv8_kraken_amd.sw2 import SW2Ensemble, default_opts
+from adhv8_kraken_amd.sw2 import YES, SW2Ensemble, default_opts
 
 pytestmark = pytest.mark.gpu
 
@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("precision", [0, 1, 2])
 def test_waiting_for_the_models_before_does_not_end_a_solve(precision):
     ps = [mesh.bumpy_channel(507, 201, seed=k) for k in range(4)]   # 401 blocks each, 512 at once
-    opts = default_opts(precision=precision, max_nonlin_it=1, max_lin_it=150, lin_rtol=0.0, lin_atol=0.0)
+    # one Newton iteration a step, accepted; 30 and more iterations in its solve
+    opts = default_opts(precision=precision, max_nonlin_it=1, tol_nonlin=1e30, max_lin_it=150, lin_rtol=1e-13, lin_atol=0.0)
     e = SW2Ensemble(ps, opts)
 
     def step(wait):
@@ -27,8 +28,10 @@ def test_waiting_for_the_models_before_does_not_end_a_solve(precision):
         e.set_solve_wait(wait)
         e.get_state(0)
         t0 = time.perf_counter()
-        e.timestep()
-        return time.perf_counter() - t0
+        rs = e.timestep()
+        t = time.perf_counter() - t0
+        assert all(r["verdict"] == YES and r["lin_its"] >= 30 for r in rs)
+        return t
 
     step(-1)
     want = [e.get_state(i) for i in range(len(ps))]
@@ -36,6 +39,7 @@ def test_waiting_for_the_models_before_does_not_end_a_solve(precision):
     default = min(step(30000) for _ in range(3))
     say(f"  precision {precision}: {1e3 * long:.2f} ms with a bound of 10 s, {1e3 * default:.2f} with 0.3 ms")
     assert default < 1.3 * long
+    assert not any(bits_equal(w[0], p.head0) for w, p in zip(want, ps))
     for i, w in enumerate(want):
         assert all(bits_equal(a, b) for a, b in zip(w, e.get_state(i)))
     e.close()
