@@ -28,6 +28,10 @@
 // the L2).
 
 #include <algorithm>
+#include <functional>
+#include <queue>
+#include <utility>
+#include <vector>
 
 #include "sw2_flow.h"
 #include "sw2_krylov.h"
@@ -591,11 +595,49 @@ int run_capacity() {
     return per_cu * cus;
 }
 
+// Whether an ensemble's solve is expected to be shorter so than as a kernel per
+// step.  A model has the GPU's places for its blocks until it is through, and the
+// next ones start in order as places come free: models of just over half the GPU
+// run one at a time, with nearly half of the GPU idle, while the kernels of the
+// other form are filled by all models together.  us an iteration (of ten, the
+// set-up of a solve included), measured with models of 60 to 512 blocks, six
+// neighbours: a model of B blocks in FP64 10.2 + 0.011 B with one block a CU, 16.2 +
+// 0.025 B with two, FP32 entries 9.3 + 0.0185 B, all FP32 9 + 0.0172 B; a kernel per
+// step 18 and 0.07, 0.0453, 0.039 for every block.  A step of ten iterations, ms, per
+// step / so: 24 models of 260 blocks FP64 11.4 / 12.4, 12 of 350 7.5 / 7.7, 12 of 450 9.5 /
+// 9.1, 30 of 150 (one block a CU) 8.4 / 8.8; refined 24 of 260 9.2 / 9.3, 16 of 320 7.5 / 7.1.
+template <typename P, int OCC>
+bool run_pays(const Ctx *c, int cap) {
+    if (!c->ninst) return true;
+    constexpr bool WIDE = sizeof(typename P::M) == 8, F32 = sizeof(typename P::V) == 4;
+    constexpr double A = WIDE ? (OCC == 1 ? 10.2 : 16.2) : (F32 ? 9.0 : 9.3);
+    constexpr double B = WIDE ? (OCC == 1 ? 0.011 : 0.025) : (F32 ? 0.0172 : 0.0185);
+    constexpr double STEP = WIDE ? 0.07 : (F32 ? 0.039 : 0.0453);
+    using Busy = std::pair<double, int>;   // until when, how many places
+    std::priority_queue<Busy, std::vector<Busy>, std::greater<Busy>> busy;
+    double now = 0.0, end = 0.0, per_step = 18.0;
+    int places = cap;
+    for (int i = 0; i < c->ninst; i++) {
+        if (!c->h_inst_mask[i]) continue;
+        const int nb = nblocks_for(c->h_inst_N[i], 256);
+        while (places < nb) {
+            now = std::max(now, busy.top().first);
+            places += busy.top().second;
+            busy.pop();
+        }
+        places -= nb;
+        busy.emplace(now + A + B * nb, nb);
+        end = std::max(end, now + A + B * nb);
+        per_step += STEP * nb;
+    }
+    return end <= per_step;
+}
+
 template <typename P, int K, int OCC, bool ENS>
 bool run_k(Ctx *c, bool zero_guess) {
     int &cap = c->run_cap[OCC - 1];
     if (cap < 0) cap = run_capacity<P, K, OCC, ENS>();
-    if (c->run_max_blocks > cap) return false;
+    if (c->run_max_blocks > cap || !run_pays<P, OCC>(c, cap)) return false;
     using T = typename P::V;
     const int nb = nblocks_for(c->N, 256);
     const size_t n3 = 3 * (size_t)c->Np;
@@ -626,7 +668,8 @@ bool run_k(Ctx *c, bool zero_guess) {
 // 69 / 117, 16,008 81 / 138, 65,341 115 / 146; FP32 entries: equal.  Seven and
 // eight neighbours: the LDS takes one block.  More blocks than the GPU holds
 // (512, 131,072 nodes), more or fewer neighbours, or slices of unequal width:
-// the kernel-per-step form.
+// the kernel-per-step form.  An ensemble takes the first of these that pays
+// (run_pays).
 template <typename P, int K, bool ENS>
 bool run_occ(Ctx *c, bool zero_guess) {
     constexpr bool WIDE = sizeof(typename P::M) == 8;
