@@ -276,6 +276,17 @@ static int alloc_solver(adh_sw2_hip *h) {
 
 // ninst > 0: the mesh is the union of an ensemble of ninst models (see
 // adh_sw2_hip_batch_create); the per-model scalars are sized for them.
+// Launch shapes of the lists before any tuning.  Wet lists, us at 1M / 250,000 /
+// 160,000 / 50,000 triangles: Jacobian, 256 threads and 4,096 workgroups 752 /
+// 221 / 165 / 62, 128 and 8,192 734 / 216 / 164 / 64; residual, 128 threads and
+// 4,096 workgroups 141 / 41 / 35 / 17, 2,048 of them 159 / 41 / 35 / 17 (a third
+// round of workgroups nearly empty).
+static Ctx::Tuning default_tuning(int E) {
+    Ctx::Tuning t;
+    if (E > 131040) { t.bs[0] = 128; t.grid[0] = 8192; }
+    return t;
+}
+
 static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_hip **out, int ninst) {
     if (!out) return fail(ADH_SW2_EINVAL, "out is NULL");
     *out = nullptr;
@@ -289,12 +300,7 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     c.N = m->nnodes; c.E = m->nelems2d; c.B = m->nelems1d; c.M = m->nmat;
     c.Np = (c.N + 63) & ~63;
     c.kgraph_prec = -1;
-    // Launch shapes of the wet lists before any tuning.  us at 1M / 250,000 /
-    // 160,000 / 50,000 triangles: Jacobian, 256 threads and 4,096 workgroups 752 /
-    // 221 / 165 / 62, 128 and 8,192 734 / 216 / 164 / 64; residual, 128 threads and
-    // 4,096 workgroups 141 / 41 / 35 / 17, 2,048 of them 159 / 41 / 35 / 17 (a third
-    // round of workgroups nearly empty).
-    if (m->nelems2d > 131040) { c.tune.bs[0] = 128; c.tune.grid[0] = 8192; }
+    c.tune = default_tuning(m->nelems2d);
     c.run_cap[0] = c.run_cap[1] = c.run_prec = -1;
     c.run_max_blocks = nblocks_for(c.N, 256);
     // 0.3 ms: a hand-over takes 3 to 13 us when every block is resident, and what a
@@ -1828,6 +1834,19 @@ extern "C" int adh_sw2_hip_autotune(adh_sw2_hip *h, int reps, adh_sw2_tuning *ou
     static const int GRID[8] = {256, 512, 1024, 2048, 4096, 8192, 16384, 32768};
     adh_sw2_tuning best;
     adh_sw2_hip_get_tuning(h, &best);
+    // ms a launch, one warm-up and reps timed ones
+    auto time_ms = [&](auto launch, double *ms) -> int {
+        launch();
+        (void)hipEventRecord(c.ev[0], c.stream);
+        for (int r = 0; r < reps; r++) launch();
+        (void)hipEventRecord(c.ev[1], c.stream);
+        HIPCHK(hipEventSynchronize(c.ev[1]));
+        HIPCHK(hipGetLastError());
+        float total = 0.f;
+        HIPCHK(hipEventElapsedTime(&total, c.ev[0], c.ev[1]));
+        *ms = (double)total / reps;
+        return 0;
+    };
     for (int phase = 0; phase < 4; phase++) {
         const int items = (phase < 2 ? 18 : 1) * cnt[phase & 1];
         if (items == 0) continue;
@@ -1839,15 +1858,8 @@ extern "C" int adh_sw2_hip_autotune(adh_sw2_hip *h, int reps, adh_sw2_tuning *ou
                 for (int gi = 0; gi < 8; gi++) {
                     const int g = std::min(GRID[gi], full);
                     if (gi > 0 && std::min(GRID[gi - 1], full) == g) continue;   // same shape as the previous one
-                    launch_list_phase(&c, phase, b, g, layout);
-                    (void)hipEventRecord(c.ev[0], c.stream);
-                    for (int r = 0; r < reps; r++) launch_list_phase(&c, phase, b, g, layout);
-                    (void)hipEventRecord(c.ev[1], c.stream);
-                    HIPCHK(hipEventSynchronize(c.ev[1]));
-                    HIPCHK(hipGetLastError());
-                    float total = 0.f;
-                    HIPCHK(hipEventElapsedTime(&total, c.ev[0], c.ev[1]));
-                    const double ms = (double)total / reps;
+                    double ms = 0.0;
+                    if ((rc = time_ms([&]() { launch_list_phase(&c, phase, b, g, layout); }, &ms))) return rc;
                     if (ms < tbest) {
                         tbest = ms;
                         best.block[phase] = b;
@@ -1859,10 +1871,35 @@ extern "C" int adh_sw2_hip_autotune(adh_sw2_hip *h, int reps, adh_sw2_tuning *ou
             }
         }
     }
-    for (int k = 0; k < 4; k++) {
-        c.tune.bs[k] = best.block[k];
-        c.tune.grid[k] = best.grid[k];
-        c.tune.layout[k] = best.layout[k];
+    // The default shapes let the two lists and the edges share launches, which the
+    // lists' own best ones may not: whichever makes the whole of a Jacobian, or a
+    // residual, the shorter one stays.
+    const Ctx::Tuning dflt = default_tuning(c.E);
+    for (const int p : {0, 2}) {
+        auto take = [&](const int *bs, const int *grid, const int *layout) {
+            for (int k = p; k < p + 2; k++) { c.tune.bs[k] = bs[k]; c.tune.grid[k] = grid[k]; c.tune.layout[k] = layout[k]; }
+        };
+        double own = 0.0, whole = 0.0;
+        auto elements = [&]() { launch_elements(&c, p == 0); };
+        take(best.block, best.grid, best.layout);
+        if ((rc = time_ms(elements, &own))) return rc;
+        take(dflt.bs, dflt.grid, dflt.layout);
+        if ((rc = time_ms(elements, &whole))) return rc;
+        if (own < whole) {
+            take(best.block, best.grid, best.layout);
+        } else {
+            for (int k = p; k < p + 2; k++) {
+                best.block[k] = dflt.bs[k]; best.grid[k] = dflt.grid[k]; best.layout[k] = dflt.layout[k];
+                best.ms[k] = 0.0;
+                if (cnt[k & 1] > 0 && !lists_joined(&c, p) &&
+                    (rc = time_ms([&]() { launch_list_phase(&c, k, dflt.bs[k], dflt.grid[k], dflt.layout[k]); }, &best.ms[k])))
+                    return rc;
+            }
+        }
+        if (lists_joined(&c, p)) {
+            best.ms[p] = std::min(own, whole);
+            best.ms[p + 1] = 0.0;
+        }
     }
     if (out) *out = best;
     return sync_check(c);

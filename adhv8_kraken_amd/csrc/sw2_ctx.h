@@ -390,6 +390,8 @@ void launch_resid2d_only(Ctx *c);
 void launch_assemble_only(Ctx *c);
 void ensure_lists(Ctx *c);
 void launch_list_phase(Ctx *c, int phase, int bs, int grid, int layout);
+void launch_elements(Ctx *c, bool jacobian);
+bool lists_joined(const Ctx *c, int phase);
 std::string ilu_structure(Ctx *c);
 void ilu_free(Ctx *c);
 void launch_ilu_setup(Ctx *c);

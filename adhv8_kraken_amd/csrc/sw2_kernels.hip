@@ -926,8 +926,10 @@ constexpr int JAC_ALL_BS = 256, RES_ALL_BS = 128;
 // more than one wave a SIMD is at work and the wet list is faster in its own
 // launch (44 us at 250,000 triangles).  Jacobians: both lists' code at once
 // overruns the instruction caches, 148 against 59 + 74 us at 50,176 triangles of
-// which half are partly dry; at 31,486 wet ones it saves 10 of 65.  (Edges and an
-// empty general list alone in that kernel: 18 us, in their own 13.)
+// which half are partly dry; below the line it is the shorter one, whole loads of
+// 1,600 / 13,794 / 32,768 triangles 37 / 54 / 77 against 43 / 62 / 83 us all wet and 42 / 74 / 111
+// against 55 / 107 / 121 with 40 % of them partly dry.  (Edges and an empty general list
+// alone in that kernel at 250,000 triangles: 18 us, in their own 13.)
 constexpr int RES_ALL_TRIS = 65536, JAC_ALL_TRIS = 32768;
 
 // The element Jacobians of both lists and, with `edges`, the boundary's.
@@ -935,9 +937,7 @@ static void launch_jac_split(Ctx *c, const ElemData &D, bool edges) {
     const int B = edges ? c->B : 0;
     const int *blkpos1 = c->blkpos + 9 * (size_t)c->E;
     if (c->E && !c->split_valid) launch_split(c);
-    const bool all = c->E && c->E <= JAC_ALL_TRIS && c->tune.bs[0] == JAC_ALL_BS && c->tune.bs[1] == JAC_ALL_BS &&
-                     c->tune.layout[0] >= 2 && c->tune.layout[1] == c->tune.layout[0];
-    if (!all) {
+    if (!(c->E && lists_joined(c, 0))) {
         if (c->E) {
             launch_list(c, D, 0, c->tune.bs[0], c->tune.grid[0], c->tune.layout[0]);
             launch_list(c, D, 1, c->tune.bs[1], c->tune.grid[1], c->tune.layout[1]);
@@ -968,7 +968,7 @@ static void launch_resid_split(Ctx *c, const ElemData &D, bool edges) {
     double *er1 = c->ER + 9 * (size_t)c->E;
     if (c->E && !c->split_valid) launch_split(c);
     const int need = c->E ? nblocks_for(c->E, RES_ALL_BS) : 0;
-    const bool beside = c->E <= RES_ALL_TRIS && c->tune.bs[2] == RES_ALL_BS && c->tune.bs[3] == RES_ALL_BS;
+    const bool beside = lists_joined(c, 2);
     if (c->E && !beside) launch_list(c, D, 2, c->tune.bs[2], c->tune.grid[2], c->tune.layout[2]);
     if (c->E && c->tune.bs[3] != RES_ALL_BS)
         launch_list(c, D, 3, c->tune.bs[3], c->tune.grid[3], c->tune.layout[3]);
@@ -991,6 +991,25 @@ void launch_jacobian(Ctx *c) {
     D.ts = c->h_ts + TS_LOAD;
     c->em32 = em32_of(c) != nullptr;
     launch_jac_split(c, D, true);
+}
+
+// the launches of a Jacobian's (else a residual's) element kernels, edges included,
+// as they run with the tuning in force; for the autotuner
+void launch_elements(Ctx *c, bool jacobian) {
+    if (!c->pre_valid) launch_old_terms(c);
+    ElemData D = c->ed;
+    D.first_elem = jacobian ? nullptr : c->first_elem;
+    if (jacobian) launch_jac_split(c, D, true);
+    else launch_resid_split(c, D, true);
+}
+
+// Whether phase 0's or 2's list runs in one launch with the next phase's.
+bool lists_joined(const Ctx *c, int phase) {
+    const Ctx::Tuning &t = c->tune;
+    if (phase == 0)
+        return c->E <= JAC_ALL_TRIS && t.bs[0] == JAC_ALL_BS && t.bs[1] == JAC_ALL_BS && t.layout[0] >= 2 &&
+               t.layout[1] == t.layout[0];
+    return c->E <= RES_ALL_TRIS && t.bs[2] == RES_ALL_BS && t.bs[3] == RES_ALL_BS;
 }
 
 // Ordered block assembly.  The element kernels store each 3x3 block at its

@@ -315,7 +315,10 @@ int adh_sw2_hip_set_tuning(adh_sw2_hip *h, const adh_sw2_tuning *t);
 int adh_sw2_hip_set_solve_wait(adh_sw2_hip *h, long long ticks);
 /* Times every candidate shape of each list kernel on the handle's current
  * state and triangle lists (HIP events on the library's stream, one warm-up
- * and `reps` timed launches per shape), keeps the fastest and returns it.
+ * and `reps` timed launches per shape), keeps the fastest and returns it --
+ * or the default shapes of a pair of lists where these make the whole of its
+ * launches, boundary edges included, the shorter one.  Where a pair shares one
+ * launch, ms of its first list is that launch's and ms of its second 0.
  * For an ensemble the lists cover every model.  Leaves the state unchanged. */
 int adh_sw2_hip_autotune(adh_sw2_hip *h, int reps, adh_sw2_tuning *out);
 
