@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "sw2_ctx.h"
+#include "sw2_flow.h"
 
 using namespace sw2;
 
@@ -535,11 +536,10 @@ static int create_impl(const adh_sw2_mesh *m, const adh_sw2_opts *opts, adh_sw2_
     UP(ksc, (const KScal *)nullptr, nmod);
     UP(norms, (const Norms *)nullptr, nmod);
     {
-        const unsigned long long empty = 0xfff8dead0badf00dull;   // Slot<double>::EMPTY of sw2_run.hip
         // the one-kernel solve's hand-over storage; a single model beyond RUN_BLOCKS never takes it
         const bool may = ninst > 0 || c.run_max_blocks <= RUN_BLOCKS;
         std::vector<double> w(may ? run_slot_words(c.run_max_blocks) : 1);
-        for (double &x : w) memcpy(&x, &empty, sizeof x);
+        std::fill(w.begin(), w.end(), __builtin_bit_cast(double, Slot<double>::EMPTY));
         UP(run_slots, w.data(), w.size());
         // emptied by the first solve
         if ((rc = dalloc(h, &c.run_xch, may ? run_vector_words(c.Np) : 1))) { adh_sw2_hip_destroy(h); return rc; }

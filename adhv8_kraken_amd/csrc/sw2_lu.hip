@@ -56,6 +56,7 @@
 #include <vector>
 
 #include "sw2_ctx.h"
+#include "sw2_flow.h"
 
 namespace sw2 {
 
@@ -674,34 +675,21 @@ __global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, int b0, do
 // One kernel runs both sweeps as a dataflow over 64-row tiles: a workgroup takes
 // the next tile row in order (a ticket), adds up its tiles' products as the
 // rows they need are finished, and publishes its 64 values.  A value is its own
-// ready flag: the output vectors hold NOT_YET until it is stored, values travel
-// by agent-scope atomic stores and loads (past the XCDs' private L2s), and a
-// reader polls the value itself, so a hand-over is one store and one load and
-// needs no fence.  Tickets make it free of deadlock whatever is resident: rows
+// ready flag (sw2_flow.h): the output vectors hold EMPTY until it is stored.  Tickets make it free of deadlock whatever is resident: rows
 // are claimed in order, so the lowest unfinished row belongs to a running
 // workgroup and waits only for finished ones.
-constexpr unsigned long long NOT_YET = 0xfff8dead0badf00dull;   // a NaN no arithmetic produces
-
-__device__ __forceinline__ void publish(double *p, double v) {
-    unsigned long long u = (unsigned long long)__double_as_longlong(v);
-    if (u == NOT_YET) u = 0x7ff8000000000000ull;
-    __hip_atomic_store((unsigned long long *)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long peek(const double *p) {
-    return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // the value at p in every lane with `want`, waiting until all of the wave's are there
 __device__ __forceinline__ double await_value(const double *p, bool want) {
-    unsigned long long u = want ? peek(p) : 0ull;
-    while (__any(u == NOT_YET)) {
+    Slot<double>::U u = want ? peek(p) : 0ull;
+    while (__any(u == Slot<double>::EMPTY)) {
         __builtin_amdgcn_s_sleep(1);
-        if (u == NOT_YET) u = peek(p);
+        if (u == Slot<double>::EMPTY) u = peek(p);
     }
     return __longlong_as_double((long long)u);
 }
 
 // The right-hand side into band order (nodes of no block skipped; the band from
-// the end has zeros on the shared rows), the two output vectors to NOT_YET, the
+// the end has zeros on the shared rows), the two output vectors to EMPTY, the
 // tickets (three a band, and the claims of bands) to zero.
 __global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, int nbot, const int *node_blk,
                                                    const TBand *bands, const double *x, double *xb, double *yb,
@@ -713,11 +701,11 @@ __global__ void __launch_bounds__(256) k_tb_gather(int N, int nband, int nbot, c
     if (bk < 0) return;
     const TBand B = bands[nbot + bk];
     const TBand Q = bands[max(B.part, 0)];
-    const double ny = __longlong_as_double((long long)NOT_YET);
+    const double empty = __builtin_bit_cast(double, Slot<double>::EMPTY);
     for (int v = 0; v < 3; v++) {
         const int i = 3 * (a - B.n0) + v;
         const double xv = x[vidx3(a, v)];
-        auto put = [&](size_t o, double r) { xb[o] = r; yb[o] = ny; zb[o] = ny; };
+        auto put = [&](size_t o, double r) { xb[o] = r; yb[o] = empty; zb[o] = empty; };
         if (i < B.m) put(B.xoff + i, xv);
         if (B.part >= 0 && i >= TB * B.na) put(Q.xoff + B.mtot - 1 - i, i < B.m ? 0.0 : xv);
     }
@@ -815,7 +803,7 @@ __device__ __forceinline__ void tb_sweep(const TBand &B, const double *AB, const
             double s = S.part[parity][0][lane];
 #pragma unroll
             for (int w = 1; w < SW_W; w++) s += S.part[parity][w][lane];
-            if (r < B.m) publish(out + B.xoff + r, xi - s);
+            if (r < B.m) put(out + B.xoff + r, xi - s);
             cur = q0;
             q0 = q1;
             q1 = q2;
