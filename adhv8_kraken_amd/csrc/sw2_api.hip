@@ -951,7 +951,7 @@ static void drop_graphs(Ctx &c) {
 // k BiCGSTAB iterations: a captured graph of the 3k kernels and their
 // finishers, replayed (captured on first use for this k)
 static int run_iters(Ctx &c, int k) {
-    if (k > KGRAPH_MAX || !c.opts.graphs || c.band_tiled) {   // the tiled LU's sweeps: a launch per tile, eager
+    if (k > KGRAPH_MAX || !c.opts.graphs || c.band_tiled) {   // the tiled LU: the flags are read after every iteration
         launch_krylov_iters(&c, k);
         HIPCHK(hipGetLastError());
         return 0;
@@ -1044,8 +1044,9 @@ static int krylov(Ctx &c, int *lin_it, int *verdict, bool zero_guess) {
     int first, more;
     chunk_plan(c, first, more);
     int left = lin_it_cap(c);
-    // with the tiled band LU an iteration is two sweeps of a launch per tile:
-    // the flag is read after the prologue and after every iteration instead
+    // with the tiled band LU an iteration is two applications of up to tens of ms,
+    // and a direct solve ends at the prologue: the flag is read after the
+    // prologue and after every iteration instead
     if (c.opts.preconditioner == 1 && c.band_tiled) {
         first = more = 1;
         HIPCHK(hipMemcpyAsync(c.h_ksc, c.ksc, sizeof(KScal), hipMemcpyDeviceToHost, c.stream));

@@ -664,7 +664,7 @@ __global__ void __launch_bounds__(256) k_pl_omega(int N, KVecs<P> V, double *par
 // deck 3e-14) and returns u as the reference does; a nearly singular one (the
 // partly dry floodplain, 224 x 112 nodes) was seen at 8e-7, and without the
 // step its Newton history left the oracle's by 2.4e-7 of its first entry,
-// with it by 1.2e-8.  mask (ensembles): a model that the step leaves out, and the
+// with it by 7.9e-9 (an LU by substitution, without the inverses: 4.0e-9).  mask (ensembles): a model that the step leaves out, and the
 // gaps between models, keep their sol, as with the one-kernel solve: it is the
 // model's last correction, whose norm its next step reports first.
 constexpr double REFINE_ABOVE = 1e-12;

@@ -508,8 +508,10 @@ def profile_lu_bytes(p, nblock: int = 1) -> int:
     block of n nodes has m = 3 n DOFs and pattern half bandwidth w = 3 d + 2
     (d: the largest node-number distance of two nodes of one element inside
     the block); it stores the band, m (2 (w + 64) + 1) doubles, the inverses
-    of its 64 x 64 diagonal factor tiles (2 x 4096 doubles per 64 DOFs), two
-    band-ordered vectors and one panel copy (8,256 doubles)."""
+    of its 64 x 64 diagonal factor tiles (2 x 4096 doubles per 64 DOFs), and its
+    share of the vectors and flags (counted as 2 m + 8,256 doubles).  A block
+    factored from both ends holds the rows that both reach, at least w of them,
+    twice; where that does not fit the library factors it from one end."""
     N = int(p.nnodes)
     nb = min(max(1, int(nblock)), N)
     inc = max(1, N // nb)

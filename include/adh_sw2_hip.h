@@ -144,7 +144,9 @@ int adh_sw2_hip_geometry(adh_sw2_hip *h, double *djac, double *grad, double *dja
 int adh_sw2_hip_pattern_nnz(adh_sw2_hip *h);
 int adh_sw2_hip_pattern(adh_sw2_hip *h, int *row_ptr, int *col);
 
-/* SSW_2D state (head, vel, old_*, older_*); vel arrays interleaved (x,y). */
+/* SSW_2D state (head, vel, old_*, older_*); vel arrays interleaved (x,y).
+ * set_state has copied the arrays when it returns; the device takes them over
+ * before anything that is called later. */
 int adh_sw2_hip_set_state(adh_sw2_hip *h, const double *head, const double *vel, const double *old_head,
                           const double *old_vel, const double *older_head, const double *older_vel);
 int adh_sw2_hip_get_state(adh_sw2_hip *h, double *head, double *vel, double *old_head, double *old_vel,
