@@ -244,9 +244,10 @@ struct Ctx {
     // workgroup band LU's size, or opts.lu_tiled): band_tiled selects it
     int band_tiled, band_lu_tiled_opt;
     int tb_nband, tb_maxnt, tb_gt, tb_gf;
-    std::vector<int> tb_h_nt, tb_h_inst;   // host copies: each band's panels and model
+    std::vector<int> tb_h_nt, tb_h_inst, tb_h_gt;   // host copies: each band's panels, model and window tiles a side
     size_t tb_size;
     TBand *tb_bands;
+    double *tb_P;          // a step's L and U panels, where they are formed on their own
     double *tb_AB, *tb_LI, *tb_UI, *tb_xb, *tb_yb, *tb_zb;
     int *tb_int, *tb_guard;   // sweep tickets [3 bands], the claims of bands, then a guard flag per tile (tb_guard)
     int tb_nbot;           // bands running upwards, before all others; block b's other band is tb_nbot + b

@@ -26,7 +26,10 @@
 //              with the guarded pivots) on the matrix cores; the workgroup of the
 //              first tile, the next panel's diagonal block, goes on to factor
 //              it and to invert both factors (lu64).
-// k_tb_diag factors the diagonal blocks that no panel comes before.  Then
+// k_tb_diag factors the diagonal blocks that no panel comes before.  Where a
+// step's tiles are more than the GPU takes at once, every tile's own L and U
+// panel would be most of the work: k_tb_panel forms them once a panel, k_tb_update
+// the products, k_tb_diag the next diagonal block, with the same operations.  Then
 // k_tb_inv forms G_k = U~^-1 L^-1 of every diagonal block and k_tb_scale
 // multiplies every off-diagonal tile by its column's, so that the substitutions
 // are matrix-vector work in which only a tile's input is serial: k_tb_sweep runs
@@ -93,6 +96,12 @@ __device__ __forceinline__ TBand band_rec(const TBand *bands, int b, int flag = 
     asm volatile("" ::"s"(B.m), "s"(B.w), "s"(B.wp), "s"(B.nt), "s"(B.inst), "s"(B.off), "s"(B.toff), "s"(B.xoff),
                  "s"(B.na), "s"(B.part), "s"(B.rev), "s"(B.mtot), "s"(flag));
     return B;
+}
+
+// The panel that a band eliminates at a step: bands of blocks factored from both
+// ends reach their shared rows at one step, amax.
+__device__ __forceinline__ int panel_at(const TBand &B, int step, int amax) {
+    return B.part < 0 ? step : step - (amax - B.na);
 }
 
 __device__ __forceinline__ double guarded(double piv) { return fabs(piv) > SMALL ? piv : SMALL; }
@@ -389,15 +398,24 @@ __device__ __forceinline__ void lu64(d4 (&D)[2], Lu64 &S, double *LI, double *UI
     if (threadIdx.x == 0) *guard = S.hit;   // every pivot was before the last barriers
 }
 
-// Panel 0's diagonal block, one workgroup per band, or with `shared` that of the
-// shared rows' first panel (every other panel's is factored by k_tb_step of the
-// panel before, which updates it last).
+// A diagonal block, one workgroup per band: panel 0's, that of the shared rows'
+// first panel, or (DIAG_NEXT) that of the panel after the one that `step` has
+// eliminated, where k_tb_step does not do it.
+enum { DIAG_FIRST = -1, DIAG_SHARED = -2 };
 __global__ void __launch_bounds__(NT, 2) k_tb_diag(const TBand *bands, const double *AB, double *LI, double *UI,
-                                                   int *guard, bool shared, const int *mask) {
+                                                   int *guard, int step, int amax, const int *mask) {
     __shared__ Lu64 S;
     const TBand B = band_rec(bands, blockIdx.x);
-    if ((mask && !mask[B.inst]) || (shared && (B.part < 0 || B.rev))) return;
-    const int k = shared ? B.na : 0, c0 = k * TB, kb = min(TB, B.m - c0);
+    if (mask && !mask[B.inst]) return;
+    int k = 0;
+    if (step == DIAG_SHARED) {
+        if (B.part < 0 || B.rev) return;
+        k = B.na;
+    } else if (step >= 0) {
+        k = panel_at(B, step, amax) + 1;
+        if (k < 1 || k >= B.nt || k == B.na || (B.rev && k > B.na)) return;
+    }
+    const int c0 = k * TB, kb = min(TB, B.m - c0);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wi = wv & 3, wj = wv >> 2, lo = lane & 15, hi = lane >> 4;
     d4 D[2];
@@ -444,8 +462,7 @@ __global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, int b0, d
         Lu64 S;
     } sm;
     const TBand B = band_rec(bands, b0 + blockIdx.y);
-    // the bands of blocks factored from both ends reach their shared rows at one step, amax
-    const int k = B.part < 0 ? step : step - (amax - B.na);
+    const int k = panel_at(B, step, amax);
     if (k < 0 || k + 1 >= B.nt || (mask && !mask[B.inst])) return;   // the last panel has no window
     if (B.rev && k >= B.na) return;
     const int c0 = k * TB;
@@ -543,6 +560,136 @@ __global__ void __launch_bounds__(NT, 2) k_tb_step(const TBand *bands, int b0, d
         }
     __syncthreads();   // the products' LDS reads are done
     lu64(C, sm.S, LI + 4096 * (B.toff + k + 1), UI + 4096 * (B.toff + k + 1), guard + B.toff + k + 1, lane, wi, wj);
+}
+
+// The same in parts: four ninths of the products of k_tb_step with wide windows, and four
+// workgroups a CU, so that one's loads run beside another's products.  Bound by the
+// window's way through memory (columns of 64 rows, on no line's start): 1000 x 500
+// cells in 16 blocks, 18,432 tiles a panel, 386 us an update, 3.1 TB/s and 25
+// TFLOP/s (factorisation 360 ms; 623 by k_tb_step, 401 with a substitution launch
+// and an update by vector FMAs).  k_tb_panel: a workgroup per 64 rows of the L panel (blockIdx.x
+// < gt) or 64 columns of the U panel, as k_tb_step forms them, into P: 2 gt tiles
+// a band, in the order in which the matrix cores take them, [block][q][lane]:
+// L[16 block + lane % 16][4 q + lane / 16], U[4 q + lane / 16][16 block + lane % 16].
+__global__ void __launch_bounds__(NT, 2) k_tb_panel(const TBand *bands, int b0, const double *AB, const double *LI,
+                                                    const double *UI, double *P, int step, int amax, int gt,
+                                                    const int *mask) {
+    constexpr int LD = TB + 2;
+    __shared__ double Xs[TB * LD];
+    const TBand B = band_rec(bands, b0 + blockIdx.y);
+    const int k = panel_at(B, step, amax);
+    if (k < 0 || k + 1 >= B.nt || (mask && !mask[B.inst])) return;
+    if (B.rev && k >= B.na) return;
+    const bool low = (int)blockIdx.x < gt;
+    const int c0 = k * TB, r0 = c0 + TB, r1 = min(B.m, r0 + B.w);
+    const int t0 = r0 + TB * (low ? (int)blockIdx.x : (int)blockIdx.x - gt);
+    if (t0 >= r1) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wi = wv & 3, wj = wv >> 2, lo = lane & 15, hi = lane >> 4;
+    double *out = P + 4096 * (2 * (size_t)gt * (b0 + blockIdx.y) + blockIdx.x) + 1024 * wi;
+    // the wave's block columns (rows) of the product: wj and 3 - wj, with wj + 1 and 4 - wj blocks
+    const double *inv = (low ? UI : LI) + 4096 * (B.toff + k);
+    double iv[20], av[16];
+#pragma unroll
+    for (int z = 0; z < 20; z++) {
+        const int blk = z < 4 * (wj + 1) ? wj : 3 - wj, q = z < 4 * (wj + 1) ? z : z - 4 * (wj + 1);
+        iv[z] = inv[64 * (4 * q + hi) + 16 * blk + lo];
+    }
+    if (low) {
+        const int i = t0 + 16 * wi + lo;
+#pragma unroll
+        for (int q = 0; q < 16; q++) av[q] = tb_get(AB, B, min(i, r1 - 1), c0 + 4 * q + hi);
+#pragma unroll
+        for (int q = 0; q < 16; q++) av[q] = i < r1 ? av[q] : 0.0;
+    } else {
+        double xv[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
+            xv[u] = tb_get(AB, B, c0 + row, min(t0 + col, r1 - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int e = threadIdx.x + NT * u, row = e & (TB - 1), col = e >> 6;
+            Xs[LD * col + row] = t0 + col < r1 ? xv[u] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 16; q++) av[q] = Xs[LD * (16 * wi + lo) + 4 * q + hi];
+    }
+    auto products = [&](auto WJ) {
+        constexpr int J0 = decltype(WJ)::value;
+        d4 p0 = {0.0, 0.0, 0.0, 0.0}, p1 = p0;
+#pragma unroll
+        for (int q = 0; q < 16 - 4 * J0; q++) {
+            if (q < 4 * (J0 + 1)) p0 = low ? mfma4(iv[q], av[q], p0) : mfma4(av[q], iv[q], p0);
+            const double v = iv[4 * (J0 + 1) + q];
+            p1 = low ? mfma4(v, av[q], p1) : mfma4(av[q], v, p1);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if (low) {
+                out[64 * (4 * J0 + r) + lane] = p0[r];
+                out[64 * (4 * (3 - J0) + r) + lane] = p1[r];
+            } else {   // U[16 block + lo][column hi + 4 r]
+                const int to = 64 * (lo >> 2) + 16 * (lo & 3) + hi + 4 * r;
+                out[64 * 4 * J0 + to] = p0[r];
+                out[64 * 4 * (3 - J0) + to] = p1[r];
+            }
+        }
+    };
+    if (wj == 0) products(std::integral_constant<int, 0>());
+    else products(std::integral_constant<int, 1>());
+}
+
+// Panel k's window from P: a workgroup of four waves per 64 x 64 tile, 32 x 32 a wave.
+__global__ void __launch_bounds__(256, 4) k_tb_update(const TBand *bands, int b0, double *AB, const double *P, int step,
+                                                      int amax, int gt, const int *mask) {
+    const TBand B = band_rec(bands, b0 + blockIdx.y);
+    const int k = panel_at(B, step, amax);
+    if (k < 0 || k + 1 >= B.nt || (mask && !mask[B.inst])) return;
+    if (B.rev && k >= B.na) return;
+    const int r0 = k * TB + TB, r1 = min(B.m, r0 + B.w);
+    const int I = blockIdx.x % gt, J = blockIdx.x / gt;
+    const int i0 = r0 + TB * I, j0 = r0 + TB * J;
+    if (i0 >= r1 || j0 >= r1) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wi = 2 * (wv & 1), wj = 2 * (wv >> 1), lo = lane & 15, hi = lane >> 4;
+    const double *Pb = P + 4096 * (2 * (size_t)gt * (b0 + blockIdx.y));
+    const double *Lp = Pb + 4096 * I + 1024 * wi + lane, *Up = Pb + 4096 * (gt + J) + 1024 * wj + lane;
+    const int i = i0 + 16 * wi + lo, j = j0 + 16 * wj + hi;
+    d4 C[2][2], acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                C[a][t][r] = tb_get(AB, B, min(i + 16 * a, r1 - 1), min(j + 16 * t + 4 * r, r1 - 1));
+                acc[a][t][r] = 0.0;
+            }
+#pragma unroll 4
+    for (int q = 0; q < 16; q++) {
+        double l[2], u[2];
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            l[a] = Lp[1024 * a + 64 * q];
+            u[a] = Up[1024 * a + 64 * q];
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) acc[a][t] = mfma4(u[t], l[a], acc[a][t]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int ii = i + 16 * a, jj = j + 16 * t + 4 * r;
+                if (ii < r1 && jj < r1) tb_at(AB, B, ii, jj) = C[a][t][r] - acc[a][t][r];
+            }
 }
 
 // Every panel's diagonal block inverse for the sweeps, in the place of its
@@ -675,9 +822,10 @@ __global__ void __launch_bounds__(256) k_tb_scale(const TBand *bands, int b0, do
 // One kernel runs both sweeps as a dataflow over 64-row tiles: a workgroup takes
 // the next tile row in order (a ticket), adds up its tiles' products as the
 // rows they need are finished, and publishes its 64 values.  A value is its own
-// ready flag (sw2_flow.h): the output vectors hold EMPTY until it is stored.  Tickets make it free of deadlock whatever is resident: rows
-// are claimed in order, so the lowest unfinished row belongs to a running
-// workgroup and waits only for finished ones.
+// ready flag (sw2_flow.h): the output vectors hold EMPTY until it is stored.
+// Tickets make it free of deadlock whatever is resident: rows are claimed in
+// order, so the lowest unfinished row belongs to a running workgroup and waits
+// only for finished ones.
 // the value at p in every lane with `want`, waiting until all of the wave's are there
 __device__ __forceinline__ double await_value(const double *p, bool want) {
     Slot<double>::U u = want ? peek(p) : 0ull;
@@ -961,12 +1109,13 @@ __global__ void __launch_bounds__(256) k_tb_apply(const TBand *bands, int b0, co
 
 void tband_free(Ctx *c) {
     for (void *p : {(void *)c->tb_bands, (void *)c->tb_AB, (void *)c->tb_LI, (void *)c->tb_UI, (void *)c->tb_xb,
-                    (void *)c->tb_yb, (void *)c->tb_zb, (void *)c->tb_int})
+                    (void *)c->tb_yb, (void *)c->tb_zb, (void *)c->tb_int, (void *)c->tb_P})
         if (p) (void)hipFree(p);
     c->tb_bands = nullptr; c->tb_AB = nullptr; c->tb_LI = nullptr; c->tb_UI = nullptr; c->tb_int = nullptr;
+    c->tb_P = nullptr;
     c->tb_xb = nullptr; c->tb_yb = nullptr; c->tb_zb = nullptr;
     c->tb_nband = 0; c->tb_maxnt = 0; c->tb_gt = 0; c->tb_gf = 0; c->tb_size = 0;
-    c->tb_h_nt.clear(); c->tb_h_inst.clear(); c->tb_h_na.clear();
+    c->tb_h_nt.clear(); c->tb_h_inst.clear(); c->tb_h_na.clear(); c->tb_h_gt.clear();
     c->tb_nbot = 0; c->tb_maxs = 0;
 }
 
@@ -981,6 +1130,15 @@ static int twist_panels(int m, int w) {
     return a >= 3 && a + (shared + TB - 1) / TB + 2 < nt ? a : 0;
 }
 
+// Window tiles of a step over all bands above which the panels are formed on their
+// own: two for each CU, which holds one workgroup of k_tb_step.  Below, the parts'
+// two launches more and the panels' way through memory cost more than the products
+// formed again.  Factorisation in one launch a panel and in parts, ms, at about the
+// given tiles a step: 200 13.8 and 17.1 (800 x 100 cells, nblock 4), 400 35.0 and 35.5
+// (400 x 200, 2), 450 76.8 and 102 (400 x 300, 1), 600 31.1 and 27.9 (400 x 200, 3),
+// 1,150 355 and 319 (500 x 500, 1), 5,600 19.9 and 13.0 (400 x 200, 28).
+constexpr size_t PARTS_TILES = 512;
+
 // Bands of the node blocks (nodes [s0[b], s1[b]) of model inst[b]) with
 // pattern half bandwidths w[] (DOFs).  Returns an error text or "".
 std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vector<int> &s1,
@@ -990,7 +1148,7 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     size_t freeb = 0, totalb = 0;
     (void)hipMemGetInfo(&freeb, &totalb);
     std::vector<TBand> h;
-    size_t off = 0, toff = 0, xoff = 0, nint = 0, need = 0;
+    size_t off = 0, toff = 0, xoff = 0, nint = 0, need = 0, npart = 0;
     int maxnt = 0, maxw = 0;
     // blocks from both ends take s rows more each; where that does not fit, one band each
     for (const bool twist : {true, false}) {
@@ -1032,8 +1190,14 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
         }
         c->tb_nbot = nbot;
         nint = toff + 3 * h.size() + 1;   // a guard flag per tile, three tickets per band, the claims
+        size_t tiles = 0;   // of a step; with one tile a band nothing is formed twice
+        for (const TBand &B : h) tiles += (size_t)((B.w + TB - 1) / TB) * ((B.w + TB - 1) / TB);
+        npart = maxw > TB && tiles > PARTS_TILES ? 2 * 4096 * (size_t)((maxw + TB - 1) / TB) * h.size() : 0;
         need = sizeof(double) * (off + 2 * 4096 * toff + 3 * xoff) + sizeof(int) * nint;
-        if (need + ((size_t)2 << 30) <= freeb) break;
+        if (need + ((size_t)2 << 30) <= freeb) {
+            if (need + sizeof(double) * npart + ((size_t)2 << 30) > freeb) npart = 0;   // one launch a panel then
+            break;
+        }
         if (twist && nbot > 0) continue;
         return "tiled band LU: " + std::to_string(need >> 20) + " MiB of band storage do not fit in the free " +
                std::to_string(freeb >> 20) + " MiB; raise nblock" +
@@ -1048,7 +1212,8 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
         hipMalloc((void **)&c->tb_xb, sizeof(double) * xoff) != hipSuccess ||
         hipMalloc((void **)&c->tb_yb, sizeof(double) * xoff) != hipSuccess ||
         hipMalloc((void **)&c->tb_zb, sizeof(double) * xoff) != hipSuccess ||
-        hipMalloc((void **)&c->tb_int, sizeof(int) * nint) != hipSuccess) {
+        hipMalloc((void **)&c->tb_int, sizeof(int) * nint) != hipSuccess ||
+        (npart && hipMalloc((void **)&c->tb_P, sizeof(double) * npart) != hipSuccess)) {
         tband_free(c);
         return "hipMalloc failed for the tiled band LU";
     }
@@ -1057,10 +1222,12 @@ std::string tband_structure(Ctx *c, const std::vector<int> &s0, const std::vecto
     c->tb_h_nt.resize(nband);
     c->tb_h_inst.resize(nband);
     c->tb_h_na.resize(nband);
+    c->tb_h_gt.resize(nband);
     for (int b = 0; b < nband; b++) {
         c->tb_h_nt[b] = h[b].nt;
         c->tb_h_inst[b] = h[b].inst;
         c->tb_h_na[b] = h[b].part < 0 ? -1 : h[b].na;
+        c->tb_h_gt[b] = (h[b].w + TB - 1) / TB;
     }
     c->tb_gt = (maxw + TB - 1) / TB;
     c->tb_gf = (maxw + 2 * TB - 2) / TB;   // tiles below (above) a panel that its L (U) reaches
@@ -1109,20 +1276,33 @@ void launch_tband_setup(Ctx *c) {
     each_active([&](int b) {
         steps = std::max(steps, c->tb_h_nt[b] - 1 + (c->tb_h_na[b] < 0 ? 0 : amax - c->tb_h_na[b]));
     });
-    auto diag = [&](bool shared) {
+    auto diag = [&](int step) {
         hipLaunchKernelGGL(k_tb_diag, dim3(c->tb_nband), dim3(NT), 0, c->stream, c->tb_bands, c->tb_AB, c->tb_LI,
-                           c->tb_UI, c->tb_guard, shared, mask);
+                           c->tb_UI, c->tb_guard, step, amax, mask);
     };
-    diag(false);
+    diag(DIAG_FIRST);
     auto merge = [&]() {
         each_launch(c, [&](int b0, int nb) {
             hipLaunchKernelGGL(k_tb_merge, dim3(c->tb_maxs, nb), dim3(256), 0, c->stream, c->tb_bands, b0, c->tb_AB,
                                mask);
         });
-        diag(true);
+        diag(DIAG_SHARED);
     };
+    size_t tiles = 0;
+    each_active([&](int b) { tiles += (size_t)c->tb_h_gt[b] * c->tb_h_gt[b]; });
+    const bool parts = c->tb_P && tiles > PARTS_TILES;
     for (int k = 0; k < steps; k++) {
         if (amax > 0 && k == amax) merge();
+        if (parts) {
+            each_launch(c, [&](int b0, int nb) {
+                hipLaunchKernelGGL(k_tb_panel, dim3(2 * gt, nb), dim3(NT), 0, c->stream, c->tb_bands, b0, c->tb_AB,
+                                   c->tb_LI, c->tb_UI, c->tb_P, k, amax, gt, mask);
+                hipLaunchKernelGGL(k_tb_update, dim3(gt * gt, nb), dim3(256), 0, c->stream, c->tb_bands, b0,
+                                   c->tb_AB, c->tb_P, k, amax, gt, mask);
+            });
+            diag(k);
+            continue;
+        }
         each_launch(c, [&](int b0, int nb) {
             hipLaunchKernelGGL(k_tb_step, dim3(gt * gt, nb), dim3(NT), 0, c->stream, c->tb_bands, b0, c->tb_AB,
                                c->tb_LI, c->tb_UI, c->tb_guard, k, amax, gt, mask);
