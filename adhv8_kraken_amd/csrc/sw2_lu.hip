@@ -1331,9 +1331,12 @@ void launch_tband_solve(Ctx *c, double *x, const KScal *sc) {
     const int *done = (sc && !mask) ? &sc->done : &c->tb_bands[0].pad;
     const KScal *msc = mask ? sc : nullptr;
     // a workgroup per tile of a row's reach and one more keep the chain's next
-    // row always waiting; any number is correct, and with many bands one
-    // workgroup each already fills the chip
-    const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 512 / c->tb_nband));
+    // row always waiting; any number is correct.  With many bands one for each CU is
+    // the line: two on some CUs slow the rows that the bands' chains wait for.  Four
+    // iterations' solve at 256 and 512 of them, ms: 1000 x 500 cells nblock 16 136
+    // and 185, 50 84.7 and 110; 400 x 200 nblock 16 9.6 and 12.2; 1500 x 40 nblock
+    // 32 2.8 and 4.3 (only 1000 x 500 nblock 8 the other way, 163 and 141).
+    const int g = std::max(1, std::min(std::min(c->tb_gf + 2, nt), 256 / c->tb_nband));
     auto sweep = [&](int phase) {   // SW_SHARED's claims count on from launch to launch
         each_launch(c, [&](int b0, int nb) {
             hipLaunchKernelGGL(k_tb_sweep, dim3(g, nb), dim3(SW_NT), 0, c->stream, c->tb_bands, b0, c->tb_AB, c->tb_xb,
