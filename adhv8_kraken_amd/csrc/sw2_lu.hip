@@ -1144,13 +1144,14 @@ static int twist_panels(int m, int w) {
 }
 
 // Window tiles of a step over all bands above which the panels are formed on their
-// own: two for each CU, which holds one workgroup of k_tb_step.  Below, the parts'
-// two launches more and the panels' way through memory cost more than the products
-// formed again.  Factorisation in one launch a panel and in parts, ms, at about the
-// given tiles a step: 200 13.8 and 17.1 (800 x 100 cells, nblock 4), 400 35.0 and 35.5
-// (400 x 200, 2), 450 76.8 and 102 (400 x 300, 1), 600 31.1 and 27.9 (400 x 200, 3),
-// 1,150 355 and 319 (500 x 500, 1), 5,600 19.9 and 13.0 (400 x 200, 28).
-constexpr size_t PARTS_TILES = 512;
+// own: three for each CU, which holds one workgroup of k_tb_step.  Below, the parts'
+// two launches more and the panels' way through memory cost as much as the products
+// formed again, or more.  Factorisation in one launch a panel and in parts, ms, at about
+// the given tiles a step: 200 13.8 and 17.1 (800 x 100 cells, nblock 4), 400 35.0 and
+// 35.5 (400 x 200, 2), 450 76.8 and 102 (400 x 300, 1), 600 31.1 and 27.9 (400 x 200,
+// 3), 900 72.4 and 73.6 (400 x 300, 2), 1,150 355 and 319 (500 x 500, 1), 5,600 19.9
+// and 13.0 (400 x 200, 28); a floodplain's three steps at 650 31.8 and 34.3 s.
+constexpr size_t PARTS_TILES = 768;
 
 // Bands of the node blocks (nodes [s0[b], s1[b]) of model inst[b]) with
 // pattern half bandwidths w[] (DOFs).  Returns an error text or "".

@@ -16,9 +16,9 @@ from adhv8_kraken_amd.sw2 import SW2Ensemble, SW2Model, default_opts
 pytestmark = pytest.mark.gpu
 
 
-# half bandwidths of 5 tiles with the last one part full and of 3 full ones; blocks from both
-# ends (880 DOFs, last block 1,683) and from one (635; 255, narrower than its last panel's window)
-@pytest.mark.parametrize("ncx,ncy,nblock", [(60, 100, 21), (60, 100, 29), (80, 61, 60)])
+# windows of 5 tiles a side with the last one part full and of up to 3; blocks from both ends
+# (879 DOFs) and from one (576; 165, all of it the first panel's window; the last one 381)
+@pytest.mark.parametrize("ncx,ncy,nblock", [(60, 100, 21), (60, 100, 32), (80, 61, 90)])
 def test_apply_is_the_block_inverse(ncx, ncy, nblock):
     """The system is diagonally dominant (condition below 10), so M^-1 v is the exact
     block inverse's to 1e-13 of its largest entry, as in test_gpu_lu_tiles.py."""
@@ -45,7 +45,7 @@ def test_apply_is_the_block_inverse(ncx, ncy, nblock):
 
 def test_an_ensemble_takes_the_steps_of_its_models_alone():
     """Bands of no window, of one tile a side and of two to seven, from one end and
-    from both, over 512 tiles in all until models have converged and fewer after."""
+    from both, over 768 tiles in all until models have converged and fewer after."""
     cells = [(3, 1), (64, 1), (75, 1), (200, 4), (30, 40), (12, 130)]
     kinds = [mesh.bumpy_channel(*c, seed=k) for k, c in enumerate(cells)]
     ps = [kinds[k % 6] for k in range(48)]
